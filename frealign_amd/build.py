@@ -21,6 +21,7 @@ SOURCES = [
     "fr_fft.hip",
     "fr_prep.hip",
     "fr_extract.hip",
+    "fr_cc3m.hip",
     "fr_insert.hip",
     "fr_final.hip",
     "fr_stats.hip",

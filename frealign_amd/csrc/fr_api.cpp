@@ -197,6 +197,52 @@ int fr_ctx::cc3m_tables(const fr::Cc3mArgs& a, fr::Cc3mTables* t) {
   return 0;
 }
 
+int fr_ctx::cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t) {
+  const int M = fr::cc3m_band_grid(a.nsam, a.maxr2), rb = fr::cc3m_band_rb(a.maxr2);
+  const std::pair<int, int> dk(M, rb), pk(a.maxr1 * a.maxr1, a.maxr2 * a.maxr2);
+  auto di = band_dft_tabs.find(dk);
+  if (di == band_dft_tabs.end()) {
+    std::vector<float> h;
+    fr::cc3m_band_dft(M, rb, h);
+    float* d = nullptr;
+    if (int r = upload_table(h, &d)) return r;
+    di = band_dft_tabs.emplace(dk, d).first;
+  }
+  t->dft = di->second;
+  auto pi = band_pair_tabs.find(pk);
+  if (pi == band_pair_tabs.end()) {
+    std::vector<int> h;
+    fr::cc3m_band_pairs(pk.first, pk.second, rb, h);
+    int* d = nullptr;
+    if (int r = upload_table(h, &d)) return r;
+    pi = band_pair_tabs.emplace(pk, d).first;
+  }
+  t->pairs = pi->second;
+  const auto rk = std::make_tuple(a.nsam, a.ri2, a.ri3);
+  auto ri = ring_tabs.find(rk);
+  if (ri == ring_tabs.end()) {
+    std::vector<float> h;
+    RingTab rt;
+    rt.cnt = fr::cc3m_fused_ring_q(a.nsam, a.ri2, a.ri3, h);
+    if (int r = upload_table(h, &rt.d)) return r;
+    ri = ring_tabs.emplace(rk, rt).first;
+  }
+  t->ring = ri->second.d;
+  t->ring_cnt = ri->second.cnt;
+  const auto wk = std::make_tuple(a.nsam, M, a.ri2, a.ri3, a.rih, a.halfw);
+  auto wi = band_wmap_tabs.find(wk);
+  if (wi == band_wmap_tabs.end()) {
+    std::vector<float> full, w;
+    fr::cc3m_fused_wmap(a.nsam, a.ri2, a.ri3, a.rih, a.halfw, full);
+    fr::cc3m_band_wmap(a.nsam, M, full, w);
+    float* d = nullptr;
+    if (int r = upload_table(w, &d)) return r;
+    wi = band_wmap_tabs.emplace(wk, d).first;
+  }
+  t->wmap = wi->second;
+  return 0;
+}
+
 fr_ctx::Tune fr_ctx::tune_for(int nsam) const {
   auto it = tune.find(nsam);
   return it == tune.end() ? Tune{} : it->second;
@@ -269,6 +315,9 @@ int fr_destroy(fr_ctx* c) {
   if (c->hpin) (void)hipHostFree(c->hpin);
   if (c->d_kidx) (void)hipFree(c->d_kidx);
   for (auto& e : c->dft_tabs) (void)hipFree(e.second);
+  for (auto& e : c->band_dft_tabs) (void)hipFree(e.second);
+  for (auto& e : c->band_pair_tabs) (void)hipFree(e.second);
+  for (auto& e : c->band_wmap_tabs) (void)hipFree(e.second);
   for (auto& e : c->pts_tabs) (void)hipFree(e.second);
   for (auto& e : c->ring_tabs) (void)hipFree(e.second.d);
   for (auto& e : c->wmap_tabs) (void)hipFree(e.second);
@@ -400,7 +449,7 @@ namespace fr {
 int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                const float* d_ctff, const int* d_pidx, const float* d_dm, const float* d_shift,
                const float* d_amag, int maxr1, int maxr2, float rbfact, const float* d_fsct,
-               const float* ring, float* d_score, int cc3) {
+               const float* ring, float* d_score, int cc3, bool unit_amag) {
   CTX_CHECK(c);
   SIZE_CHECK(nsam);
   FR_CHECK(n >= 0 && d_a3df && d_spec && d_ctff && d_pidx && d_dm && d_shift && d_amag &&
@@ -412,14 +461,24 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
   a.cc3 = cc3;
   const fr_ctx::Tune tn = c->tune_for(nsam);
   if (fr::cc3m_fused_ok(nsam, maxr2) && tn.cc3m_fused) {
+    // the items with AMAG = 1 on the band's own grid, the others (unless there
+    // are none) on the NSAM grid
     Cc3mTables tabs;
-    if (int r = c->cc3m_tables(a, &tabs)) return r;
+    Cc3mBandTables band;
+    if (int r = c->cc3m_band_tables(a, &band)) return r;
+    if (!unit_amag)
+      if (int r = c->cc3m_tables(a, &tabs)) return r;
     int pslot = c->prof_begin(kProfCc3m);
     for (int o = 0; o < n; o += 65535) {
       a.n = n - o < 65535 ? n - o : 65535;
+      if (int r = launch_cc3m_band(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o,
+                                   d_dm + 9 * (size_t)o, d_shift + 2 * (size_t)o, d_amag + o,
+                                   d_fsct, band, d_score + o, tn.cc3m_blocks))
+        return r;
+      if (unit_amag) continue;
       if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o,
                                     d_dm + 9 * (size_t)o, d_shift + 2 * (size_t)o, d_amag + o,
-                                    d_fsct, tabs, d_score + o, tn.cc3m_blocks))
+                                    d_fsct, tabs, d_score + o, -1, nullptr, nullptr, true))
         return r;
     }
     c->prof_end(pslot);
@@ -1278,8 +1337,8 @@ int fr_rescore_batch(fr_ctx* c, int nsam, int np, int k, const float* d_a3df, co
   if (int r = launch_cand_items(*c, np, k, d_top_o, d_top_row, nbank, d_dm_bank, nsamr, pidx, dm,
                                 sh, am))
     return r;
-  if (int r = fr_cc3m_batch(c, nsam, (int)n, d_a3df, d_outc, d_ctff, pidx, dm, sh, am, maxr1,
-                            maxr2, rbfact, d_fsct, ring, d_score))
+  if (int r = cc3m_batch(c, nsam, (int)n, d_a3df, d_outc, d_ctff, pidx, dm, sh, am, maxr1, maxr2,
+                         rbfact, d_fsct, ring, d_score, 0, true))
     return r;
   return launch_best_cand(*c, np, k, d_top_o, d_score, d_best);
 }
@@ -1354,10 +1413,12 @@ int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d
     memcpy(h + o_sh, hsh, sizeof(float) * 2 * m);
     memcpy(h + o_am, ham, sizeof(float) * m);
     FR_HIP(hipMemcpyAsync(dbuf, h, o_sc, hipMemcpyHostToDevice, c->stream));
-    if (int r = fr_cc3m_batch(c, nsam, m, d_a3df, d_spec, d_ctff, (const int*)dbuf,
-                              (const float*)(dbuf + o_dm), (const float*)(dbuf + o_sh),
-                              (const float*)(dbuf + o_am), maxr1, maxr2, rbfact, d_fsct, ring,
-                              dsc))
+    bool unit = true;
+    for (int i = 0; i < m; i++) unit &= ham[i] == 1.0f;
+    if (int r = cc3m_batch(c, nsam, m, d_a3df, d_spec, d_ctff, (const int*)dbuf,
+                           (const float*)(dbuf + o_dm), (const float*)(dbuf + o_sh),
+                           (const float*)(dbuf + o_am), maxr1, maxr2, rbfact, d_fsct, ring, dsc,
+                           0, unit))
       return r;
     FR_HIP(hipMemcpyAsync(h + o_sc, dsc, sizeof(float) * m, hipMemcpyDeviceToHost, c->stream));
     FR_HIP(hipStreamSynchronize(c->stream));

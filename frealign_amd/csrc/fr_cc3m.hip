@@ -1,0 +1,556 @@
+// fr_cc3m.hip -- CC3M (cc3m.f:8-169) on the band's own grid.
+//
+// CC3M extracts a section on the annulus MAXR1 <= r < MAXR2, goes to real
+// space on the NSAM x NSAM grid, applies MASKCOS2 and comes back, and reads
+// only the annulus again.  With R = MAXR2 - 1 the largest frequency on either
+// side, the masked band is
+//   out[k] = sum_j W[k - j] X[j],   |k|, |j| <= R,
+// W the transform of the mask's weights: only its frequencies up to 2 R
+// matter.  So the same numbers come from any M x M grid with M >= 4 R + 1
+// that carries the mask with W cut at M/2 - 1 (what aliases falls outside the
+// band), whatever NSAM is: 64, 96 or 128 points for MAXR2 <= 16, 24, 32.
+// The mean that MASKCOS2 takes over its ring is linear in the band (the table
+// Q, formed on the NSAM grid).  This needs the weights of one AMAG; the kernel
+// takes the items with AMAG = 1 and leaves the others to the NSAM-grid form.
+//
+// One workgroup per item, persistent over a contiguous run of items (the
+// candidates of one particle reuse its CTF and spectrum, held in registers).
+// Every pass is a product with T[m][2i] = cos(2 pi i m/M), T[m][2i+1] =
+// -sin(2 pi i m/M) on the FP32 matrix cores, folded over the table's
+// symmetry: rows m and M - m of T differ by the sign of the sines, so only
+// m <= M/2 is held and each product gives both.
+//   column c2c  Y[m][c]   = sum_J T[m][.] B[c][.]   B: the +-J pairs
+//   row c2r     x[r][m]   = sum_I T[r][.] w_I Y[m][.]
+//   mask        y = (x - mean) w, the same w at r and M - r
+//   row r2c     Z[m][k]   = sum_r T[r][k] y[r][m]  (+ M mean at k = 0)
+//   column r2c  out[j][k] = sum_m T[m][j] Z[m][k]
+// then the shell sums of cc3m.f:117-150, each thread its own (I, +-J) pairs,
+// reduced by shell in a fixed order.
+//
+// What bounds it: at MAXR2 = 32 an item takes 1,808 16x16x4 FP32 MFMA (6 us
+// of one CU's matrix cores) against 4,896 on a 256 grid.  LDS is 71 KB (149 KB
+// on the 256 grid), so two workgroups share a CU and one's gathers and sums
+// run under the other's products.  8,192 items of a 256 box: 544 us against
+// 1,387 us on the 256 grid.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <vector>
+
+#include "fr_common.h"
+#include "fr_extract.h"
+#include "fr_kernels.h"
+
+namespace fr {
+
+namespace {
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float fx4;
+
+__device__ inline fx4 mfma4(float a, float b, fx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// sum over the 16 lanes of a row, in every lane, on the vector ALU
+template <int kCtrl>
+__device__ inline float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf,
+                                                        false));
+}
+__device__ inline float row16_sum(float v) {
+  v = dpp_add<0xB1>(v);   // quad_perm 1,0,3,2
+  v = dpp_add<0x4E>(v);   // quad_perm 2,3,0,1
+  v = dpp_add<0x141>(v);  // row_half_mirror
+  return dpp_add<0x140>(v);  // row_mirror
+}
+
+template <int RB, int M>
+struct BandShape {
+  static constexpr int kThreads = RB == 32 ? 512 : 256;
+  static constexpr int kWaves = kThreads / 64;
+  static constexpr int kK = 2 * RB;      // reals per row: RB frequencies
+  static constexpr int kP = kK + 4;      // LDS row pitch (floats): conflict-free operand reads
+  static constexpr int kPairs = RB * RB / kThreads;  // (I, |J|) pairs per thread
+  static constexpr int kT = (M / 2 + 1) * kP, kY = M * kP, kB = kK * kP;
+  // T, Y/Z (then the pairs' sums), B/out, the shells' terms
+  static constexpr int kLds = kT + kY + kB;
+  static_assert(3 * RB * RB <= kY, "the pairs' sums use the Y buffer");
+  static_assert(M / 16 <= kWaves, "one row block per wave");
+};
+
+template <int RB, int M>
+__global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
+    k_cc3m_band(int nsam, int nitem, float rbfact,
+                const float2* __restrict__ a3df, const float* __restrict__ dm,
+                const int* __restrict__ pidx, const float2* __restrict__ ctff,
+                const float2* __restrict__ spec, const float* __restrict__ shift,
+                const float* __restrict__ amag_arr, const float* __restrict__ fsct,
+                const float* __restrict__ tab, const int* __restrict__ pairs,
+                const float* __restrict__ ring_tab, int ring_cnt,
+                const float* __restrict__ wmap, float* __restrict__ score, int flip) {
+  using S = BandShape<RB, M>;
+  constexpr int kThr = S::kThreads, kK = S::kK, kP = S::kP, kPr = S::kPairs, H = M / 2;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* Ts = lds;          // [M/2 + 1][kP]
+  float* Ys = Ts + S::kT;   // [M][kP]
+  float* Bs = Ys + S::kY;   // [kK][kP]
+  __shared__ float red_s[S::kWaves];
+  __shared__ float2 phx[RB], phy[RB];  // e^{i SHX I}, e^{i SHY J}
+  __shared__ double term[RB][2];       // per shell: R_k WGT and WGT^2 sum |SAMP|^2
+
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int la = lane & 15, lg = lane >> 4;
+  const int jc = nsam / 2 + 1;
+  const size_t ic = (size_t)nsam * jc;
+  auto ld2 = [](const float* p) { return *reinterpret_cast<const float2*>(p); };
+
+  const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
+
+  // ---- what does not depend on the item
+  for (int e = tid; e < (H + 1) * (kK / 4); e += kThr) {
+    const int r = e / (kK / 4), q = e % (kK / 4);
+    *reinterpret_cast<float4*>(Ts + r * kP + 4 * q) =
+        *reinterpret_cast<const float4*>(tab + (size_t)r * kK + 4 * q);
+  }
+  // this thread's pairs (I, +-J): the ring table's entries, the place of the
+  // pair's sums in shell order (below 0: off the band)
+  float4 qv[kPr];
+  int pos[kPr];
+#pragma unroll
+  for (int u = 0; u < kPr; u++) {
+    const int e = tid + u * kThr, i = e / RB, jj = e % RB;
+    const float2 a = ld2(ring_tab + (2 * i) * kCc3mRingPitch + 2 * jj);
+    const float2 b = ld2(ring_tab + (2 * i + 1) * kCc3mRingPitch + 2 * jj);
+    qv[u] = make_float4(a.x, a.y, b.x, b.y);
+    pos[u] = pairs[kCc3mPairHdr + e];
+  }
+  // this 16-lane row's shell: its pairs, point count, weight and sign rule
+  const int sh = 1 + (tid >> 4);
+  const int sb0 = pairs[sh], sb1 = pairs[sh + 1];
+  const int top = min(nsam / 2, kCc3mShells);
+  const bool used = sh < top && sb1 > sb0;
+  const float wgt = expf(-rbfact * (float)(sh * sh));
+  const bool absr = used && !flip && fsct[sh] < 0.95f;
+  // shells with points (SUM1 of cc3m.f:139-167)
+  double nshell = 0.0;
+  for (int s = 1; s < top && s <= RB; s++)
+    if (pairs[s + 1] > pairs[s]) nshell += 1.0;
+  // mask weights of this wave's row block
+  const int m0 = wave * 16, m = m0 + la;
+  const bool rows = m0 < M;
+  float2 cpos[kPr], cneg[kPr];
+  int pprev = -1;
+
+  for (int it = it0; it < it1; it++) {
+    if (amag_arr[it] != 1.0f) continue;  // the NSAM-grid form's item
+    const int p = pidx[it];
+    if (p != pprev) {
+      pprev = p;
+      const float2* cp = ctff + (size_t)p * 2 * ic;
+#pragma unroll
+      for (int u = 0; u < kPr; u++) {
+        cpos[u] = cneg[u] = make_float2(0.f, 0.f);
+        if (pos[u] >= 0) {
+          const int e = tid + u * kThr, i = e / RB, jj = e % RB;
+          const size_t ip = (size_t)i + (size_t)jc * jj;
+          const size_t in = (size_t)i + (size_t)jc * wrapn(-jj, nsam);
+          float2 cr = cp[ip], cl = cp[ip + ic];
+          cpos[u] = make_float2(cr.x + cl.x, cr.y - cl.y);
+          cr = cp[in], cl = cp[in + ic];
+          cneg[u] = make_float2(cr.x + cl.x, cr.y - cl.y);
+        }
+      }
+    }
+    if (tid < 2 * RB) {
+      float sn, cs;
+      sincosf(shift[2 * it + (tid < RB ? 0 : 1)] * (float)(tid % RB), &sn, &cs);
+      (tid < RB ? phx : phy)[tid % RB] = make_float2(cs, sn);
+    }
+    // ---- B[c][k], c = (I, re|im), k = (J, cos|sin), from the CTF-multiplied
+    // section (cc3m.f:74-112); the ring sum on the way
+    float rsum = 0.f;
+    {
+      const float* d = dm + 9 * (size_t)it;
+      const float scal = 1.0f / (float)nsam / (float)nsam;
+#pragma unroll
+      for (int u = 0; u < kPr; u++) {
+        // one pair's gathers in flight at a time: two pairs' do not fit the registers
+        if (u) __builtin_amdgcn_sched_barrier(0);
+        const int e = tid + u * kThr, i = e / RB, jj = e % RB;
+        cf ap = {0.f, 0.f}, an = ap;
+        if (pos[u] >= 0) {
+          ap = ainterpo_dev(nsam, a3df, d, i, jj);
+          an = ainterpo_dev(nsam, a3df, d, i, -jj);
+        }
+        if (flip) {  // cc3.f:86-89
+          if (cpos[u].x < 0.0f) ap = cf{-ap.re, -ap.im};
+          if (cneg[u].x < 0.0f) an = cf{-an.re, -an.im};
+        } else {
+          ap = cmul(ap, cf{cpos[u].x, cpos[u].y});
+          an = cmul(an, cf{cneg[u].x, cneg[u].y});
+        }
+        const cf xp = cscale(ap, scal), xn = jj ? cscale(an, scal) : cf{0.f, 0.f};
+        const cf P = cadd(xp, xn);
+        const cf Q = jj ? csub(xp, xn) : cf{0.f, 0.f};
+        // Y_re = P_re T_re + Q_im T_im, Y_im = P_im T_re - Q_re T_im
+        *reinterpret_cast<float2*>(Bs + (2 * i) * kP + 2 * jj) = make_float2(P.re, Q.im);
+        *reinterpret_cast<float2*>(Bs + (2 * i + 1) * kP + 2 * jj) = make_float2(P.im, -Q.re);
+        rsum += qv[u].x * P.re + qv[u].y * Q.im + qv[u].z * P.im - qv[u].w * Q.re;
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
+    if (lane == 0) red_s[wave] = rsum;
+    __syncthreads();
+
+    // ---- column c2c, times the c2r weight: for m < M/2, E against the cosine
+    // rows of B and O against its sine rows give Y[m] = E + O, Y[M-m] = E - O
+    {
+      constexpr int kTiles = (H / 16) * (kK / 16);
+#pragma unroll
+      for (int t0 = 0; t0 < kTiles; t0 += S::kWaves) {
+        const int t = t0 + wave;
+        if (kTiles % S::kWaves && t >= kTiles) break;
+        const int y0 = (t / (kK / 16)) * 16, c0 = (t % (kK / 16)) * 16;
+        fx4 e = {0.f, 0.f, 0.f, 0.f}, o = e;
+#pragma unroll
+        for (int ks = 0; ks < RB / 4; ks++) {
+          const float2 tv = ld2(Ts + (y0 + la) * kP + 8 * ks + 2 * lg);
+          const float2 bv = ld2(Bs + (c0 + la) * kP + 8 * ks + 2 * lg);
+          e = mfma4(tv.x, bv.x, e);
+          o = mfma4(tv.y, bv.y, o);
+        }
+        const float wc = (c0 + la) < 2 ? 1.0f : 2.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int y = y0 + 4 * lg + i;
+          Ys[y * kP + c0 + la] = (e[i] + o[i]) * wc;
+          if (y) Ys[(M - y) * kP + c0 + la] = (e[i] - o[i]) * wc;
+        }
+      }
+      // row M/2: Y[c] = sum_J (-1)^J B[c][cos J], eight threads per column
+      const int c = tid >> 3, q = tid & 7;
+      float y = 0.f;
+#pragma unroll
+      for (int j = 0; j < RB; j += 8) y += Bs[c * kP + 2 * (j + q)];
+      if (q & 1) y = -y;
+      y += __shfl_xor(y, 1, 64);
+      y += __shfl_xor(y, 2, 64);
+      y += __shfl_xor(y, 4, 64);
+      if (q == 0) Ys[H * kP + c] = y * (c < 2 ? 1.0f : 2.0f);
+    }
+    __syncthreads();
+
+    // ---- rows of this wave's block: E and O of a tile of T rows r < M/2 give
+    // x[r] = E + O and x[M-r] = E - O; y = (x - mean) w (the same w at r and
+    // M - r); Z's cosine part takes y[r] + y[M-r], its sine part y[r] - y[M-r]
+    fx4 w[M / 32];
+    float wh = 0.f;
+    if (rows) {
+#pragma unroll
+      for (int t = 0; t < M / 32; t++)
+        w[t] = *reinterpret_cast<const fx4*>(wmap + (size_t)m * M + 16 * t + 4 * lg);
+      wh = wmap[(size_t)m * M + H];
+    }
+    float tot = 0.f;
+#pragma unroll
+    for (int k = 0; k < S::kWaves; k++) tot += red_s[k];
+    const float mean = ring_cnt ? tot / (float)ring_cnt : tot;
+    if (rows) {
+      float2 yv[RB / 4];
+#pragma unroll
+      for (int ks = 0; ks < RB / 4; ks++) yv[ks] = ld2(Ys + m * kP + 8 * ks + 2 * lg);
+      fx4 zc[RB / 16], zs[RB / 16];
+#pragma unroll
+      for (int kt = 0; kt < RB / 16; kt++) zc[kt] = zs[kt] = fx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < M / 32; t++) {
+        __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
+        fx4 e = {0.f, 0.f, 0.f, 0.f}, o = e, sp, sm;
+#pragma unroll
+        for (int ks = 0; ks < RB / 4; ks++) {
+          const float2 tv = ld2(Ts + (16 * t + la) * kP + 8 * ks + 2 * lg);
+          e = mfma4(tv.x, yv[ks].x, e);
+          o = mfma4(tv.y, yv[ks].y, o);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float ya = (e[i] + o[i] - mean) * w[t][i];
+          float yb = (e[i] - o[i] - mean) * w[t][i];
+          if (t == 0 && i == 0 && lg == 0) yb = 0.f;  // r = 0: its own partner
+          sp[i] = ya + yb;
+          sm[i] = ya - yb;
+        }
+        // k-step i takes r = 16t + 4 lg + i: the C layout of E, O is the B layout
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int kt = 0; kt < RB / 16; kt++) {
+            const float2 tv = ld2(Ts + (16 * t + 4 * lg + i) * kP + 2 * (16 * kt + la));
+            zc[kt] = mfma4(tv.x, sp[i], zc[kt]);
+            zs[kt] = mfma4(tv.y, sm[i], zs[kt]);
+          }
+      }
+      // row M/2: x = sum_I (-1)^I wYre[m][I], I = 4 ks + lg
+      float xs = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < RB / 4; ks++) xs += yv[ks].x;
+      xs = (lg & 1) ? -xs : xs;
+      xs += __shfl_xor(xs, 16, 64);
+      xs += __shfl_xor(xs, 32, 64);
+      const float yh = (xs - mean) * wh;
+#pragma unroll
+      for (int kt = 0; kt < RB / 16; kt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) zc[kt][i] += (i & 1) ? -yh : yh;
+      if (lg == 0) zc[0][0] += mean * (float)M;  // k = 0, the mean's own term
+      // this wave alone read rows m0 .. m0 + 15 of Ys
+#pragma unroll
+      for (int kt = 0; kt < RB / 16; kt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          *reinterpret_cast<float2*>(Ys + m * kP + 2 * (16 * kt + 4 * lg + i)) =
+              make_float2(zc[kt][i], zs[kt][i]);
+    }
+    __syncthreads();
+
+    // the pairs' spectrum, in flight under the column r2c
+    float2 spos[kPr], sneg[kPr];
+#pragma unroll
+    for (int u = 0; u < kPr; u++) {
+      const int e = tid + u * kThr, i = e / RB, jj = e % RB;
+      spos[u] = sneg[u] = make_float2(0.f, 0.f);
+      if (pos[u] >= 0) {
+        const float2* sp = spec + (size_t)p * ic + i;
+        spos[u] = sp[(size_t)jc * jj];
+        sneg[u] = sp[(size_t)jc * wrapn(-jj, nsam)];
+      }
+    }
+    // ---- column r2c, folded over m: cosine rows take Z[m] + Z[M-m], sine
+    // rows Z[m] - Z[M-m] (m = 0 and M/2 are their own partners)
+    {
+      constexpr int kTiles = (RB / 16) * (kK / 16);
+      if (wave < kTiles) {
+        const int j0 = (wave / (kK / 16)) * 16, c0 = (wave % (kK / 16)) * 16;
+        fx4 ac = {0.f, 0.f, 0.f, 0.f}, as = ac;
+        // rows m = 4 s + lg upward and their partners M - m downward, each from
+        // one base and a constant offset per step
+        constexpr int kSteps = M / 8;
+        const float* zp = Ys + lg * kP + c0 + la;
+        const float* zq = Ys + (M - 4 * (kSteps - 1) - lg) * kP + c0 + la;
+        const float* tp = Ts + lg * kP + 2 * (j0 + la);
+#pragma unroll
+        for (int s = 0; s < kSteps; s++) {
+          const float za = zp[4 * s * kP];
+          // m = 0 has no partner (its row M does not exist)
+          const float zb = s ? zq[4 * (kSteps - 1 - s) * kP]
+                             : Ys[(lg ? M - lg : 0) * kP + c0 + la];
+          const float2 tv = ld2(tp + 4 * s * kP);
+          const bool alone = s == 0 && lg == 0;
+          ac = mfma4(tv.x, alone ? za : za + zb, ac);
+          as = mfma4(tv.y, alone ? 0.f : za - zb, as);
+        }
+        // m = M/2: T = (-1)^j, no sine
+        const float zh = Ys[H * kP + c0 + la];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float c = ac[i] + ((i & 1) ? -zh : zh);
+          Bs[(j0 + 4 * lg + i) * kP + c0 + la] = c;
+          Bs[(RB + j0 + 4 * lg + i) * kP + c0 + la] = as[i];
+        }
+      }
+    }
+    __syncthreads();
+
+    // ---- cc3m.f:117-150: shifted particle x conj(masked projection) of this
+    // thread's pairs, to the pair's place in shell order
+#pragma unroll
+    for (int u = 0; u < kPr; u++) {
+      if (pos[u] < 0) continue;
+      const int e = tid + u * kThr, i = e / RB, jj = e % RB;
+      const float2 c = ld2(Bs + jj * kP + 2 * i), s = ld2(Bs + (RB + jj) * kP + 2 * i);
+      const float2 ex = phx[i], ey = phy[jj];
+      const float2 apv = make_float2(c.x - s.y, c.y + s.x);
+      // REAL(SAMP CONJG(AINPO)) with SAMP = SPEC e^{i (SHX I + SHY J)}
+      auto corr = [&](float2 v, float2 a, float cs, float sn) {
+        const float re = v.x * a.x + v.y * a.y, im = v.y * a.x - v.x * a.y;
+        return re * cs - im * sn;
+      };
+      float q = corr(spos[u], apv, ex.x * ey.x - ex.y * ey.y, ex.x * ey.y + ex.y * ey.x);
+      float s2 = spos[u].x * spos[u].x + spos[u].y * spos[u].y;
+      float a2 = apv.x * apv.x + apv.y * apv.y;
+      if (jj) {
+        const float2 anv = make_float2(c.x + s.y, c.y - s.x);
+        q += corr(sneg[u], anv, ex.x * ey.x + ex.y * ey.y, ex.y * ey.x - ex.x * ey.y);
+        s2 += sneg[u].x * sneg[u].x + sneg[u].y * sneg[u].y;
+        a2 += anv.x * anv.x + anv.y * anv.y;
+      }
+      Ys[pos[u]] = q;
+      Ys[RB * RB + pos[u]] = s2;
+      Ys[2 * RB * RB + pos[u]] = a2;
+    }
+    __syncthreads();
+    // one 16-lane row per shell, a fixed order; cc3m.f:139-167
+    {
+      float q = 0.f, s2 = 0.f, a2 = 0.f;
+      for (int e = sb0 + la; e < sb1; e += 16) {
+        q += Ys[e];
+        s2 += Ys[RB * RB + e];
+        a2 += Ys[2 * RB * RB + e];
+      }
+      q = row16_sum(q);
+      s2 = row16_sum(s2);
+      a2 = row16_sum(a2);
+      if (la == 0) {
+        float r = q / sqrtf(a2);
+        if (absr) r = fabsf(r);
+        term[sh - 1][0] = used ? (double)(r * wgt) : 0.0;
+        term[sh - 1][1] = used ? (double)(wgt * wgt * s2) : 0.0;
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {
+      double s3 = lane < RB ? term[lane][0] : 0.0, s2 = lane < RB ? term[lane][1] : 0.0;
+      for (int off = RB / 2; off > 0; off >>= 1) {
+        s3 += __shfl_xor(s3, off, 64);
+        s2 += __shfl_xor(s2, off, 64);
+      }
+      if (lane == 0) {
+        if (nshell * s2 != 0.0) s3 = s3 / sqrt(nshell * s2);
+        score[it] = (float)s3;
+      }
+    }
+  }
+}
+
+}  // namespace
+
+int cc3m_band_grid(int nsam, int maxr2) {
+  if (maxr2 > 32 || maxr2 < 1) return 0;
+  const int need = maxr2 <= 16 ? 64 : maxr2 <= 24 ? 96 : 128;
+  // the particle's own grid where it is one of the sizes and no larger
+  return (nsam == 64 || nsam == 96 || nsam == 128) && nsam < need ? nsam : need;
+}
+
+int cc3m_band_rb(int maxr2) { return maxr2 <= 16 ? 16 : 32; }
+
+// T[m][2i] = cos(2 pi i m/M), T[m][2i+1] = -sin(2 pi i m/M), m = 0 .. M/2
+void cc3m_band_dft(int M, int rb, std::vector<float>& tab) {
+  tab.assign((size_t)(M / 2 + 1) * 2 * rb, 0.f);
+  for (int m = 0; m <= M / 2; m++)
+    for (int i = 0; i < rb; i++) {
+      const double ph = 2.0 * M_PI * (double)((i * m) % M) / (double)M;
+      tab[(size_t)m * 2 * rb + 2 * i] = (float)std::cos(ph);
+      tab[(size_t)m * 2 * rb + 2 * i + 1] = (float)-std::sin(ph);
+    }
+}
+
+// Offsets of the shells INT(SQRT(FLOAT(I*I+J*J))+0.5) in the list of the pairs
+// (I, |J|) of the band sorted by shell, then each pair's place in it
+void cc3m_band_pairs(int maxr12, int maxr22, int rb, std::vector<int>& out) {
+  std::vector<std::vector<int>> by(kCc3mShells + 1);
+  for (int i = 0; i < rb; i++)
+    for (int j = 0; j < rb; j++) {
+      const int r2 = i * i + j * j;
+      if (r2 >= maxr12 && r2 < maxr22) by[(int)(sqrtf((float)r2) + 0.5f)].push_back(i * rb + j);
+    }
+  out.assign((size_t)kCc3mPairHdr + rb * rb, -1);
+  int n = 0;
+  for (int s = 0; s < kCc3mPairHdr; s++) {
+    out[s] = n;
+    if (s <= kCc3mShells)
+      for (int e : by[s]) out[kCc3mPairHdr + e] = n++;
+  }
+}
+
+// The mask on the M grid, [m][n]: the NSAM-grid weights of cc3m_fused_wmap
+// with their transform cut at M/2 - 1 (M = NSAM: the weights themselves).
+// They are even in both axes, so cosines do.
+void cc3m_band_wmap(int nsam, int M, const std::vector<float>& full, std::vector<float>& w) {
+  if (M == nsam) {
+    w = full;
+    return;
+  }
+  const int h = nsam / 2, Q = M / 2;  // frequencies 0 .. Q - 1
+  std::vector<double> cosn(nsam), cosm(M);
+  for (int k = 0; k < nsam; k++) cosn[k] = std::cos(2.0 * M_PI * k / nsam);
+  for (int k = 0; k < M; k++) cosm[k] = std::cos(2.0 * M_PI * k / M);
+  auto mult = [&](int n) { return n == 0 || n == h ? 1.0 : 2.0; };
+  // a[q][m] = sum_n w[m][n] cos(2 pi q n/N), m = 0 .. N/2
+  std::vector<double> a((size_t)Q * (h + 1), 0.0), f((size_t)Q * Q, 0.0);
+  for (int q = 0; q < Q; q++)
+    for (int m = 0; m <= h; m++) {
+      double s = 0.0;
+      for (int n = 0; n <= h; n++)
+        s += mult(n) * (double)full[(size_t)m * nsam + n] * cosn[(long long)q * n % nsam];
+      a[(size_t)q * (h + 1) + m] = s;
+    }
+  for (int q = 0; q < Q; q++)
+    for (int p = 0; p < Q; p++) {
+      double s = 0.0;
+      for (int m = 0; m <= h; m++)
+        s += mult(m) * a[(size_t)q * (h + 1) + m] * cosn[(long long)p * m % nsam];
+      f[(size_t)p * Q + q] = s / ((double)nsam * nsam) * (p ? 2.0 : 1.0) * (q ? 2.0 : 1.0);
+    }
+  // b[p][n] = sum_q f[p][q] cos(2 pi q n/M), then the rows
+  std::vector<double> b((size_t)Q * M, 0.0);
+  for (int p = 0; p < Q; p++)
+    for (int n = 0; n < M; n++) {
+      double s = 0.0;
+      for (int q = 0; q < Q; q++) s += f[(size_t)p * Q + q] * cosm[q * n % M];
+      b[(size_t)p * M + n] = s;
+    }
+  w.assign((size_t)M * M, 0.f);
+  for (int m = 0; m < M; m++)
+    for (int n = 0; n < M; n++) {
+      double s = 0.0;
+      for (int p = 0; p < Q; p++) s += b[(size_t)p * M + n] * cosm[p * m % M];
+      w[(size_t)m * M + n] = (float)s;
+    }
+}
+
+namespace {
+template <int RB, int M>
+int launch_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
+                const float* ctff, const int* pidx, const float* dm, const float* shift,
+                const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
+                int blocks) {
+  using S = BandShape<RB, M>;
+  auto fn = k_cc3m_band<RB, M>;
+  const size_t lds = sizeof(float) * S::kLds;
+  FR_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)lds));
+  int grid = 0;
+  if (int r = cc3m_grid(c, (const void*)fn, S::kThreads, lds, a.n, blocks, &grid)) return r;
+  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(S::kThreads), lds, c.stream, a.nsam, a.n, a.rbfact,
+                     reinterpret_cast<const float2*>(a3df), dm, pidx,
+                     reinterpret_cast<const float2*>(ctff), reinterpret_cast<const float2*>(spec),
+                     shift, amag, fsct, t.dft, t.pairs, t.ring, t.ring_cnt, t.wmap, score, a.cc3);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+}  // namespace
+
+int launch_cc3m_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
+                     const float* ctff, const int* pidx, const float* dm, const float* shift,
+                     const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
+                     int blocks) {
+  if (a.n <= 0) return 0;
+  FR_CHECK(t.dft && t.pairs && t.ring && t.wmap, "band CC3M tables missing");
+  const int M = cc3m_band_grid(a.nsam, a.maxr2), rb = cc3m_band_rb(a.maxr2);
+  if (rb == 16 && M == 64)
+    return launch_band<16, 64>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
+                               blocks);
+  if (rb == 32 && M == 64)
+    return launch_band<32, 64>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
+                               blocks);
+  if (rb == 32 && M == 96)
+    return launch_band<32, 96>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
+                               blocks);
+  if (rb == 32 && M == 128)
+    return launch_band<32, 128>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
+                                blocks);
+  return fail("band CC3M: no grid for MAXR2 %d", a.maxr2);
+}
+
+}  // namespace fr

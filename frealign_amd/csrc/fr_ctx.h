@@ -38,6 +38,11 @@ struct fr_ctx : public fr::Ctx {
   // per (NSAM, RI2, RI3, RIH, HALFW)
   std::map<std::tuple<int, float, float, float, float>, float*> wmap_tabs;
   int cc3m_tables(const fr::Cc3mArgs& a, fr::Cc3mTables* t);
+  std::map<std::pair<int, int>, float*> band_dft_tabs;         // per (M, frequencies held)
+  std::map<std::pair<int, int>, int*> band_pair_tabs;          // per (MAXR1^2, MAXR2^2)
+  // per (NSAM, M, RI2, RI3, RIH, HALFW)
+  std::map<std::tuple<int, int, float, float, float, float>, float*> band_wmap_tabs;
+  int cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t);
   // launch choices per box size (set by fr_autotune_cc3m)
   struct Tune {
     int cc3m_fused = 1;   // band-pruned fused CC3M where it applies
@@ -52,11 +57,12 @@ struct fr_ctx : public fr::Ctx {
 };
 
 namespace fr {
-// fr_cc3m_batch (cc3 = 0) and fr_cc3_batch (cc3 = 1)
+// fr_cc3m_batch (cc3 = 0) and fr_cc3_batch (cc3 = 1).  unit_amag: the caller
+// knows that every AMAG is 1
 int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                const float* d_ctff, const int* d_pidx, const float* d_dm, const float* d_shift,
                const float* d_amag, int maxr1, int maxr2, float rbfact, const float* d_fsct,
-               const float* ring, float* d_score, int cc3);
+               const float* ring, float* d_score, int cc3, bool unit_amag = false);
 // fr_refine_batch with the symmetry matrix SM applied to every DM (null: identity)
 int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                  const float* d_ctff, const int* pidx, const float* amag, float* par,

@@ -4,6 +4,9 @@
 
 namespace fr {
 
+// two neighbouring points of the half-volume, 8-byte aligned
+typedef float PointPair __attribute__((ext_vector_type(4), aligned(8)));
+
 // AINTERPO3DS (ainterpo3ds.f:22-98, IPAD=1) evaluated at X3 = DM*(I,J): the
 // plane coordinates are formed in the reference's FP32 operation order
 // (X3 = DM(1)*I + DM(4)*J, no FMA), and the eight corners use the same
@@ -52,10 +55,20 @@ __device__ inline cf ainterpo_dev(int nsam, const float2* __restrict__ a3df, con
   const float az0 = 1.0f - fabsf(z - (float)ns), az1 = 1.0f - fabsf(z - (float)nt);
   const size_t my0 = (size_t)jc * wrapn(ms, nsam), my1 = (size_t)jc * wrapn(mt, nsam);
   const size_t nz0 = (size_t)jc * nsam * wrapn(ns, nsam), nz1 = (size_t)jc * nsam * wrapn(nt, nsam);
-  float2 c000 = a3df[ls + my0 + nz0], c100 = a3df[lt + my0 + nz0];
-  float2 c010 = a3df[ls + my1 + nz0], c110 = a3df[lt + my1 + nz0];
-  float2 c001 = a3df[ls + my0 + nz1], c101 = a3df[lt + my0 + nz1];
-  float2 c011 = a3df[ls + my1 + nz1], c111 = a3df[lt + my1 + nz1];
+  // LS and LT are neighbours (or the same point at JC-1): one 16-byte load
+  // takes both from the pair that starts at min(LS, JC-2)
+  const int lb = min(ls, jc - 2);
+  const bool sl = ls != lb, tl = lt != lb;
+  auto pair = [&](size_t row, float2& s0, float2& t0) {
+    const PointPair v = *reinterpret_cast<const PointPair*>(a3df + row + lb);
+    s0 = sl ? make_float2(v[2], v[3]) : make_float2(v[0], v[1]);
+    t0 = tl ? make_float2(v[2], v[3]) : make_float2(v[0], v[1]);
+  };
+  float2 c000, c100, c010, c110, c001, c101, c011, c111;
+  pair(my0 + nz0, c000, c100);
+  pair(my1 + nz0, c010, c110);
+  pair(my0 + nz1, c001, c101);
+  pair(my1 + nz1, c011, c111);
   float w000 = ax0 * ay0 * az0, w100 = ax1 * ay0 * az0, w010 = ax0 * ay1 * az0, w110 = ax1 * ay1 * az0;
   float w001 = ax0 * ay0 * az1, w101 = ax1 * ay0 * az1, w011 = ax0 * ay1 * az1, w111 = ax1 * ay1 * az1;
   float re = c000.x * w000 + c100.x * w100 + c010.x * w010 + c110.x * w110 + c001.x * w001 +

@@ -258,7 +258,7 @@ __global__ void __launch_bounds__(kFT)
                  const int* __restrict__ pts, const float* __restrict__ ring_tab, int ring_cnt,
                  const float* __restrict__ wmap, float ri2,
                  float ri3, float rih, float halfw, float* score, Cc3mWindow win,
-                 int* __restrict__ wcode, int flip) {
+                 int* __restrict__ wcode, int flip, int skip_unit) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int hrow = nsam / 2 + 1;
   float* Ts = lds;                      // [nsam/2 + 1][kFP]: the folded table TF
@@ -288,7 +288,16 @@ __global__ void __launch_bounds__(kFT)
     return (up && (k & 1)) ? -v : v;
   };
 
-  // ---- stage TF once; the workgroup then takes items blockIdx.x, +gridDim.x, ...
+  // a contiguous run of items per workgroup: consecutive items of one
+  // particle (a particle's candidates) reuse its band spectrum in LDS
+  const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
+  if (skip_unit) {
+    bool any = false;
+    for (int it = it0 + tid; it < it1; it += kFT) any |= amag_arr[it] != 1.0f;
+    if (!__syncthreads_or(any)) return;
+  }
+  // ---- stage TF once; the workgroup then takes its items
   for (int e = tid; e < hrow * (kFK / 4); e += kFT) {
     int n = e / (kFK / 4), q = e % (kFK / 4);
     *reinterpret_cast<float4*>(Ts + n * kFP + 4 * q) =
@@ -302,12 +311,9 @@ __global__ void __launch_bounds__(kFT)
   float qv[64 * 64 / kFT];
 #pragma unroll
   for (int r = 0; r < 64 * 64 / kFT; r++) qv[r] = ring_tab ? ring_tab[tid + r * kFT] : 0.f;
-  // a contiguous run of items per workgroup: consecutive items of one
-  // particle (a particle's candidates) reuse its band spectrum in LDS
-  const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
-  const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
   int pprev = -1;
   for (int it = it0; it < it1; it++) {
+  if (skip_unit && amag_arr[it] == 1.0f) continue;
   const int p = pidx[it];
   const bool newp = p != pprev;
   pprev = p;
@@ -1046,10 +1052,25 @@ void cc3m_fused_wmap(int nsam, float ri2, float ri3, float rih, float halfw,
   }
 }
 
+int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks, int* grid) {
+  *grid = (blocks > 0 && blocks < n) ? blocks : n;
+  if (blocks >= 0) return 0;
+  if (c.cus <= 0) {
+    hipDeviceProp_t prop;
+    FR_HIP(hipGetDeviceProperties(&prop, c.device));
+    c.cus = prop.multiProcessorCount;
+  }
+  int per_cu = 0;
+  FR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds));
+  const long long full = (long long)c.cus * (per_cu > 0 ? per_cu : 1);
+  if (full < n) *grid = (int)full;
+  return 0;
+}
+
 int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
                       const float* ctff, const int* pidx, const float* dm, const float* shift,
                       const float* amag, const float* fsct, const Cc3mTables& t, float* score,
-                      int blocks, const Cc3mWindow* win, int* wcode) {
+                      int blocks, const Cc3mWindow* win, int* wcode, bool skip_unit) {
   if (a.n <= 0) return 0;
   FR_CHECK(cc3m_fused_ok(a.nsam, a.maxr2), "fused CC3M needs NSAM %% 32 == 0, NSAM <= 256, MAXR2 <= 32");
   FR_CHECK(t.dft && t.pts, "fused CC3M tables missing");
@@ -1064,21 +1085,10 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
   }
   const void* fn = win ? (const void*)k_cc3m_fused<true> : (const void*)k_cc3m_fused<false>;
   FR_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  // persistent grid: `blocks` workgroups (0: one per item; below 0: one full
-  // wave of workgroups), each looping over items, so that the tables are
-  // staged once per workgroup rather than once per item
-  int grid = (blocks > 0 && blocks < a.n) ? blocks : a.n;
-  if (blocks < 0) {
-    if (c.cus <= 0) {
-      hipDeviceProp_t prop;
-      FR_HIP(hipGetDeviceProperties(&prop, c.device));
-      c.cus = prop.multiProcessorCount;
-    }
-    int per_cu = 0;
-    FR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kFT, lds));
-    const long long full = (long long)c.cus * (per_cu > 0 ? per_cu : 1);
-    if (full < a.n) grid = (int)full;
-  }
+  // persistent: each workgroup loops over items, so that the tables are staged
+  // once per workgroup rather than once per item
+  int grid = 0;
+  if (int r = cc3m_grid(c, fn, kFT, lds, a.n, blocks, &grid)) return r;
   if (win)
     hipLaunchKernelGGL(k_cc3m_fused<true>, dim3((unsigned)grid), dim3(kFT), lds, c.stream, a.nsam,
                        a.n, a.maxr1 * a.maxr1, a.maxr2 * a.maxr2, a.rbfact,
@@ -1086,7 +1096,7 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
                        t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w, wcode,
-                       a.cc3);
+                       a.cc3, (int)skip_unit);
   else
     hipLaunchKernelGGL(k_cc3m_fused<false>, dim3((unsigned)grid), dim3(kFT), lds, c.stream,
                        a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2 * a.maxr2, a.rbfact,
@@ -1094,7 +1104,7 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
                        t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w,
-                       (int*)nullptr, a.cc3);
+                       (int*)nullptr, a.cc3, (int)skip_unit);
   FR_HIP(hipGetLastError());
   return 0;
 }

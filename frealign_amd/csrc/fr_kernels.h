@@ -159,9 +159,38 @@ struct Cc3mWindow {
   int nsx, nsy;
   float dsx, dsy;
 };
+// skip_unit: leave the items with AMAG = 1 alone
 int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
                       const float* ctff, const int* pidx, const float* dm, const float* shift,
                       const float* amag, const float* fsct, const Cc3mTables& t, float* score,
-                      int blocks = 0, const Cc3mWindow* win = nullptr, int* wcode = nullptr);
+                      int blocks = 0, const Cc3mWindow* win = nullptr, int* wcode = nullptr,
+                      bool skip_unit = false);
+// The launch's workgroups: `blocks` (0: one per item; below 0: what the device
+// holds at once), at most one per item.
+int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks, int* grid);
+
+// CC3M on the band's own M x M grid (fr_cc3m.hip), for the items with AMAG = 1;
+// the others are left alone.  cc3m_band_grid: M, or 0 where there is none.
+int cc3m_band_grid(int nsam, int maxr2);
+int cc3m_band_rb(int maxr2);  // frequencies per axis the kernel holds: 16 or 32
+// Constant tables (device pointers, owned by the context): the DFT table of the
+// M grid, the band's (I, |J|) pairs in shell order, Q and the ring's pixel
+// count as in Cc3mTables, the mask on the M grid.
+constexpr int kCc3mPairHdr = 36;    // shell offsets in front of the pairs' places
+constexpr int kCc3mRingPitch = 64;  // row length of Q
+struct Cc3mBandTables {
+  const float* dft = nullptr;
+  const int* pairs = nullptr;
+  const float* ring = nullptr;
+  int ring_cnt = 0;
+  const float* wmap = nullptr;
+};
+void cc3m_band_dft(int M, int rb, std::vector<float>& tab);
+void cc3m_band_pairs(int maxr12, int maxr22, int rb, std::vector<int>& out);
+void cc3m_band_wmap(int nsam, int M, const std::vector<float>& full, std::vector<float>& w);
+int launch_cc3m_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
+                     const float* ctff, const int* pidx, const float* dm, const float* shift,
+                     const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
+                     int blocks);
 
 }  // namespace fr

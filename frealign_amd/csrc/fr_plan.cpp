@@ -39,6 +39,7 @@ struct fr_plan {
   PrepGlobals g{};
   Cc3mArgs ca{};
   Cc3mTables tabs;  // fused CC3M tables (owned by the context)
+  Cc3mBandTables band;
   int nsym = 0;
   int jsym[8] = {};
   float symop[72] = {};
@@ -85,9 +86,13 @@ int enqueue(fr_plan* p) {
                         c->stream));
   Cc3mArgs a = p->ca;
   a.n = nb;
-  if (p->fused) {
+  if (p->fused) {  // as cc3m_batch: a batch's AMAG is not known at capture
+    if (int r = launch_cc3m_band(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm,
+                                 p->d_shift, p->d_amag, p->fsct, p->band, p->d_score, p->blocks))
+      return r;
     if (int r = launch_cc3m_fused(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm,
-                                  p->d_shift, p->d_amag, p->fsct, p->tabs, p->d_score, p->blocks))
+                                  p->d_shift, p->d_amag, p->fsct, p->tabs, p->d_score, -1,
+                                  nullptr, nullptr, true))
       return r;
   } else {
     if (int r = launch_cc3m(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm, p->d_shift,
@@ -228,7 +233,9 @@ int fr_plan_create(fr_ctx* c, int nsam, int nb, const float* d_a3df, const float
   if (!p->fused && (r = dalloc(&p->d_work, img * nb))) return fail(r);
   if ((r = dalloc(&p->d_ins, insert_scratch_bytes(nsam, nb, nb * ncopy)))) return fail(r);
   if ((r = dalloc(&p->d_part, 2 * prep_partials_count(nsam, nb)))) return fail(r);
-  if (p->fused && (r = c->cc3m_tables(p->ca, &p->tabs))) return fail(r);
+  if (p->fused && ((r = c->cc3m_tables(p->ca, &p->tabs)) ||
+                   (r = c->cc3m_band_tables(p->ca, &p->band))))
+    return fail(r);
   std::vector<int> pid(nb);
   for (int b = 0; b < nb; b++) pid[b] = b;
   if (hipMemcpy(p->d_pidx, pid.data(), sizeof(int) * nb, hipMemcpyHostToDevice) != hipSuccess)
