@@ -27,11 +27,11 @@
 // then the shell sums of cc3m.f:117-150, each thread its own (I, +-J) pairs,
 // reduced by shell in a fixed order.
 //
-// What bounds it: at MAXR2 = 32 an item takes 1,808 16x16x4 FP32 MFMA (6 us
+// What bounds it: at MAXR2 = 32 an item takes 1,536 16x16x4 FP32 MFMA (5 us
 // of one CU's matrix cores) against 4,896 on a 256 grid.  LDS is 71 KB (149 KB
 // on the 256 grid), so two workgroups share a CU and one's gathers and sums
-// run under the other's products.  8,192 items of a 256 box: 544 us against
-// 1,387 us on the 256 grid.
+// run under the other's products.  8,192 items of a 256 box: 380 us against
+// 1,370 us on the 256 grid.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -98,8 +98,7 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
   __shared__ float2 phx[RB], phy[RB];  // e^{i SHX I}, e^{i SHY J}
   __shared__ double term[RB][2];       // per shell: R_k WGT and WGT^2 sum |SAMP|^2
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int la = lane & 15, lg = lane >> 4;
+  const int tid0 = threadIdx.x;
   const int jc = nsam / 2 + 1;
   const size_t ic = (size_t)nsam * jc;
   auto ld2 = [](const float* p) { return *reinterpret_cast<const float2*>(p); };
@@ -108,25 +107,18 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
   const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
 
   // ---- what does not depend on the item
-  for (int e = tid; e < (H + 1) * (kK / 4); e += kThr) {
+  for (int e = tid0; e < (H + 1) * (kK / 4); e += kThr) {
     const int r = e / (kK / 4), q = e % (kK / 4);
     *reinterpret_cast<float4*>(Ts + r * kP + 4 * q) =
         *reinterpret_cast<const float4*>(tab + (size_t)r * kK + 4 * q);
   }
-  // this thread's pairs (I, +-J): the ring table's entries, the place of the
-  // pair's sums in shell order (below 0: off the band)
-  float4 qv[kPr];
+  // this thread's pairs (I, +-J): the place of the pair's sums in shell order
+  // (below 0: off the band)
   int pos[kPr];
 #pragma unroll
-  for (int u = 0; u < kPr; u++) {
-    const int e = tid + u * kThr, i = e / RB, jj = e % RB;
-    const float2 a = ld2(ring_tab + (2 * i) * kCc3mRingPitch + 2 * jj);
-    const float2 b = ld2(ring_tab + (2 * i + 1) * kCc3mRingPitch + 2 * jj);
-    qv[u] = make_float4(a.x, a.y, b.x, b.y);
-    pos[u] = pairs[kCc3mPairHdr + e];
-  }
+  for (int u = 0; u < kPr; u++) pos[u] = pairs[kCc3mPairHdr + tid0 + u * kThr];
   // this 16-lane row's shell: its pairs, point count, weight and sign rule
-  const int sh = 1 + (tid >> 4);
+  const int sh = 1 + (tid0 >> 4);
   const int sb0 = pairs[sh], sb1 = pairs[sh + 1];
   const int top = min(nsam / 2, kCc3mShells);
   const bool used = sh < top && sb1 > sb0;
@@ -136,14 +128,21 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
   double nshell = 0.0;
   for (int s = 1; s < top && s <= RB; s++)
     if (pairs[s + 1] > pairs[s]) nshell += 1.0;
-  // mask weights of this wave's row block
-  const int m0 = wave * 16, m = m0 + la;
-  const bool rows = m0 < M;
   float2 cpos[kPr], cneg[kPr];
   int pprev = -1;
 
   for (int it = it0; it < it1; it++) {
     if (amag_arr[it] != 1.0f) continue;  // the NSAM-grid form's item
+    // Opaque copies, made anew for each item: addresses formed from them and
+    // values loaded through them are not kept across items, which would cost
+    // more registers (as spills, read back through L2) than forming them again.
+    int tid = tid0;
+    const float *wtab = wmap, *qtab = ring_tab;
+    asm volatile("" : "+v"(tid), "+s"(wtab), "+s"(qtab));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int la = lane & 15, lg = lane >> 4;
+    const int m0 = wave * 16, m = m0 + la;
+    const bool rows = m0 < M;
     const int p = pidx[it];
     if (p != pprev) {
       pprev = p;
@@ -172,6 +171,7 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     float rsum = 0.f;
     {
       const float* d = dm + 9 * (size_t)it;
+      const bool inner = ainterpo_inner(jc, d, RB);
       const float scal = 1.0f / (float)nsam / (float)nsam;
 #pragma unroll
       for (int u = 0; u < kPr; u++) {
@@ -180,8 +180,13 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
         const int e = tid + u * kThr, i = e / RB, jj = e % RB;
         cf ap = {0.f, 0.f}, an = ap;
         if (pos[u] >= 0) {
-          ap = ainterpo_dev(nsam, a3df, d, i, jj);
-          an = ainterpo_dev(nsam, a3df, d, i, -jj);
+          if (inner) {
+            ap = ainterpo_inner_dev(nsam, jc, a3df, d, i, jj);
+            an = ainterpo_inner_dev(nsam, jc, a3df, d, i, -jj);
+          } else {
+            ap = ainterpo_dev(nsam, a3df, d, i, jj);
+            an = ainterpo_dev(nsam, a3df, d, i, -jj);
+          }
         }
         if (flip) {  // cc3.f:86-89
           if (cpos[u].x < 0.0f) ap = cf{-ap.re, -ap.im};
@@ -196,7 +201,9 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
         // Y_re = P_re T_re + Q_im T_im, Y_im = P_im T_re - Q_re T_im
         *reinterpret_cast<float2*>(Bs + (2 * i) * kP + 2 * jj) = make_float2(P.re, Q.im);
         *reinterpret_cast<float2*>(Bs + (2 * i + 1) * kP + 2 * jj) = make_float2(P.im, -Q.re);
-        rsum += qv[u].x * P.re + qv[u].y * Q.im + qv[u].z * P.im - qv[u].w * Q.re;
+        const float2 qa = ld2(qtab + (2 * i) * kCc3mRingPitch + 2 * jj);
+        const float2 qb = ld2(qtab + (2 * i + 1) * kCc3mRingPitch + 2 * jj);
+        rsum += qa.x * P.re + qa.y * Q.im + qb.x * P.im - qb.y * Q.re;
       }
     }
     for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
@@ -249,8 +256,8 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     if (rows) {
 #pragma unroll
       for (int t = 0; t < M / 32; t++)
-        w[t] = *reinterpret_cast<const fx4*>(wmap + (size_t)m * M + 16 * t + 4 * lg);
-      wh = wmap[(size_t)m * M + H];
+        w[t] = *reinterpret_cast<const fx4*>(wtab + (size_t)m * M + 16 * t + 4 * lg);
+      wh = wtab[(size_t)m * M + H];
     }
     float tot = 0.f;
 #pragma unroll
