@@ -78,7 +78,9 @@ struct BandShape {
   static_assert(M / 16 <= kWaves, "one row block per wave");
 };
 
-template <int RB, int M>
+// kWin: instead of the score, each item's cross-spectrum sums and differences
+// over +-J for every pair, and its shells' |AINPO|^2 and norm, for k_cc3m_window
+template <int RB, int M, bool kWin>
 __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     k_cc3m_band(int nsam, int nitem, float rbfact,
                 const float2* __restrict__ a3df, const float* __restrict__ dm,
@@ -87,7 +89,8 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
                 const float* __restrict__ amag_arr, const float* __restrict__ fsct,
                 const float* __restrict__ tab, const int* __restrict__ pairs,
                 const float* __restrict__ ring_tab, int ring_cnt,
-                const float* __restrict__ wmap, float* __restrict__ score, int flip) {
+                const float* __restrict__ wmap, float* __restrict__ score, int flip,
+                Cc3mWinBuf wb) {
   using S = BandShape<RB, M>;
   constexpr int kThr = S::kThreads, kK = S::kK, kP = S::kP, kPr = S::kPairs, H = M / 2;
   extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -378,6 +381,29 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
       const float2 c = ld2(Bs + jj * kP + 2 * i), s = ld2(Bs + (RB + jj) * kP + 2 * i);
       const float2 ex = phx[i], ey = phy[jj];
       const float2 apv = make_float2(c.x - s.y, c.y + s.x);
+      if constexpr (kWin) {
+        // C = SPEC CONJG(AINPO) e^{i (SHX I + SHY J)} at the window's centre
+        auto cross = [&](float2 v, float2 a, float cs, float sn) {
+          const float re = v.x * a.x + v.y * a.y, im = v.y * a.x - v.x * a.y;
+          return make_float2(re * cs - im * sn, re * sn + im * cs);
+        };
+        const float2 cp =
+            cross(spos[u], apv, ex.x * ey.x - ex.y * ey.y, ex.x * ey.y + ex.y * ey.x);
+        float2 cn = make_float2(0.f, 0.f);
+        float s2 = spos[u].x * spos[u].x + spos[u].y * spos[u].y;
+        float a2 = apv.x * apv.x + apv.y * apv.y;
+        if (jj) {
+          const float2 anv = make_float2(c.x + s.y, c.y - s.x);
+          cn = cross(sneg[u], anv, ex.x * ey.x + ex.y * ey.y, ex.y * ey.x - ex.x * ey.y);
+          s2 += sneg[u].x * sneg[u].x + sneg[u].y * sneg[u].y;
+          a2 += anv.x * anv.x + anv.y * anv.y;
+        }
+        wb.cross[(size_t)it * wb.npair + pos[u]] =
+            make_float4(cp.x + cn.x, cp.y + cn.y, cp.x - cn.x, cp.y - cn.y);
+        Ys[RB * RB + pos[u]] = s2;
+        Ys[2 * RB * RB + pos[u]] = a2;
+        continue;
+      }
       // REAL(SAMP CONJG(AINPO)) with SAMP = SPEC e^{i (SHX I + SHY J)}
       auto corr = [&](float2 v, float2 a, float cs, float sn) {
         const float re = v.x * a.x + v.y * a.y, im = v.y * a.x - v.x * a.y;
@@ -401,14 +427,18 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     {
       float q = 0.f, s2 = 0.f, a2 = 0.f;
       for (int e = sb0 + la; e < sb1; e += 16) {
-        q += Ys[e];
+        if (!kWin) q += Ys[e];
         s2 += Ys[RB * RB + e];
         a2 += Ys[2 * RB * RB + e];
       }
       q = row16_sum(q);
       s2 = row16_sum(s2);
       a2 = row16_sum(a2);
-      if (la == 0) {
+      if (kWin && la == 0) {
+        wb.a2[(size_t)it * kCc3mWinShells + sh - 1] = a2;
+        term[sh - 1][1] = used ? (double)(wgt * wgt * s2) : 0.0;
+      }
+      if (!kWin && la == 0) {
         float r = q / sqrtf(a2);
         if (absr) r = fabsf(r);
         term[sh - 1][0] = used ? (double)(r * wgt) : 0.0;
@@ -417,15 +447,150 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     }
     __syncthreads();
     if (wave == 0) {
-      double s3 = lane < RB ? term[lane][0] : 0.0, s2 = lane < RB ? term[lane][1] : 0.0;
+      double s3 = !kWin && lane < RB ? term[lane][0] : 0.0, s2 = lane < RB ? term[lane][1] : 0.0;
       for (int off = RB / 2; off > 0; off >>= 1) {
         s3 += __shfl_xor(s3, off, 64);
         s2 += __shfl_xor(s2, off, 64);
       }
       if (lane == 0) {
-        if (nshell * s2 != 0.0) s3 = s3 / sqrt(nshell * s2);
-        score[it] = (float)s3;
+        if (kWin) {
+          wb.norm[it] = nshell * s2 != 0.0 ? sqrt(nshell * s2) : 1.0;
+        } else {
+          if (nshell * s2 != 0.0) s3 = s3 / sqrt(nshell * s2);
+          score[it] = (float)s3;
+        }
       }
+    }
+  }
+}
+
+// ---- CC3M at every shift of a window (cc3m.f:117-167): with C the item's
+// cross spectrum at the window's centre, S and D its sums and differences over
+// +-J, and a, b the shift's offsets, the shell sums are
+//   Re sum C e^{i (a I + b J)} = T1 - T2 - T3 - T4,
+//   T1 = sum Re S cos aI cos bJ,   T2 = sum Im D cos aI sin bJ,
+//   T3 = sum Im S sin aI cos bJ,   T4 = sum Re D sin aI sin bJ,
+// and -a or -b only change signs: four products over a quarter of the window.
+// Per shell each is a matrix product of 16 items by the shell's pairs with the
+// pairs by the quarter's shifts, on the FP32 matrix cores.  One wave takes 16
+// items; the phase factors are formed from two small tables, and a shell's
+// terms join FP64 sums per shift, as in the score.
+// On the vector units, one item a workgroup and one shift a lane, the sums were
+// most of the window's time: 52,728 items of a 128 box x 81 shifts took 10.6 ms,
+// and take 2.6 ms.
+constexpr int kWinWaves = 4, kWinItems = 16 * kWinWaves;
+constexpr int kWinHalf = kCc3mWinMax / 2 + 1;  // offsets 0 .. 5 per axis
+
+template <int NT>
+__global__ void __launch_bounds__(64 * kWinWaves)
+    k_cc3m_window(int nitem, int rb, int top, float rbfact, const int* __restrict__ pairs,
+                  const float* __restrict__ fsct, const float* __restrict__ amag_arr, int flip,
+                  Cc3mWindow win, Cc3mWinBuf wb, float* __restrict__ score,
+                  int* __restrict__ code) {
+  __shared__ float2 tx[32][kWinHalf], ty[32][kWinHalf];  // (cos, sin) of a dsx I, b dsy J
+  __shared__ unsigned short ij[32 * 32];                 // the pairs in shell order
+  const int tid = threadIdx.x, lane = tid & 63, la = lane & 15, lg = lane >> 4;
+  for (int e = tid; e < 32 * kWinHalf; e += 64 * kWinWaves) {
+    const int i = e / kWinHalf, a = e % kWinHalf;
+    float sn, cs;
+    sincosf((float)a * win.dsx * (float)i, &sn, &cs);
+    tx[i][a] = make_float2(cs, sn);
+    sincosf((float)a * win.dsy * (float)i, &sn, &cs);
+    ty[i][a] = make_float2(cs, sn);
+  }
+  for (int e = tid; e < rb * rb; e += 64 * kWinWaves) {
+    const int p = pairs[kCc3mPairHdr + e];
+    if (p >= 0) ij[p] = (unsigned short)((e / rb) | ((e % rb) << 8));
+  }
+  __syncthreads();
+  const int base = (blockIdx.x * kWinWaves + (tid >> 6)) * 16;
+  if (base >= nitem) return;
+  const int hx = win.nsx / 2, hy = win.nsy / 2, nq = (hx + 1) * (hy + 1);
+  int qa[NT], qb[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int n = min(16 * t + la, nq - 1);
+    qa[t] = n / (hy + 1);
+    qb[t] = n % (hy + 1);
+  }
+  const float4* row = wb.cross + (size_t)min(base + la, nitem - 1) * wb.npair;
+  double acc[NT][4][4];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) acc[t][i][k] = 0.0;
+  for (int sh = 1; sh < top && sh <= rb; sh++) {
+    const int b0 = pairs[sh], b1 = pairs[sh + 1];
+    if (b0 == b1) continue;
+    fx4 T[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) T[t][k] = fx4{0.f, 0.f, 0.f, 0.f};
+    for (int e0 = b0; e0 < b1; e0 += 4) {
+      const int e = e0 + lg;
+      float4 v = row[min(e, b1 - 1)];
+      if (e >= b1) v = make_float4(0.f, 0.f, 0.f, 0.f);
+      const int pk = ij[min(e, b1 - 1)], i = pk & 0xff, j = pk >> 8;
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const float2 x = tx[i][qa[t]], y = ty[j][qb[t]];
+        T[t][0] = mfma4(v.x, x.x * y.x, T[t][0]);
+        T[t][1] = mfma4(v.w, x.x * y.y, T[t][1]);
+        T[t][2] = mfma4(v.y, x.y * y.x, T[t][2]);
+        T[t][3] = mfma4(v.z, x.y * y.y, T[t][3]);
+      }
+    }
+    const float wgt = expf(-rbfact * (float)(sh * sh));
+    const bool absr = !flip && fsct[sh] < 0.95f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int it = min(base + 4 * lg + i, nitem - 1);
+      const float ra = sqrtf(wb.a2[(size_t)it * kCc3mWinShells + sh - 1]);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const float u = T[t][0][i], w = T[t][1][i], x = T[t][2][i], y = T[t][3][i];
+        float r[4] = {(u - w) - (x + y), (u + w) - (x - y), (u - w) + (x + y), (u + w) + (x - y)};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          r[k] = r[k] / ra;
+          if (absr) r[k] = fabsf(r[k]);
+          acc[t][i][k] += (double)(r[k] * wgt);
+        }
+      }
+    }
+  }
+  // the first maximum of each item in window order (IX outer, IY inner)
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int it = base + 4 * lg + i;
+    const double norm = wb.norm[min(it, nitem - 1)];
+    float bv = -3.0e38f;
+    int bs = 0x7fffffff;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float v = (float)(acc[t][i][k] / norm);
+        const int s = (hx + (k & 2 ? -qa[t] : qa[t])) * win.nsy + hy + (k & 1 ? -qb[t] : qb[t]);
+        if (v > bv || (v == bv && s < bs)) {
+          bv = v;
+          bs = s;
+        }
+      }
+    for (int off = 8; off > 0; off >>= 1) {
+      const float ov = __shfl_xor(bv, off, 64);
+      const int os = __shfl_xor(bs, off, 64);
+      if (ov > bv || (ov == bv && os < bs)) {
+        bv = ov;
+        bs = os;
+      }
+    }
+    if (la == 0 && it < nitem && amag_arr[it] == 1.0f) {
+      score[it] = bv;
+      code[it] = bs < win.nsx * win.nsy ? bs : 0;
     }
   }
 }
@@ -516,23 +681,72 @@ void cc3m_band_wmap(int nsam, int M, const std::vector<float>& full, std::vector
     }
 }
 
+int cc3m_band_npair(int maxr12, int maxr22, int rb) {
+  int n = 0;
+  for (int i = 0; i < rb; i++)
+    for (int j = 0; j < rb; j++) n += i * i + j * j >= maxr12 && i * i + j * j < maxr22;
+  return n;
+}
+
+size_t cc3m_window_bytes(int npair) {
+  return sizeof(float4) * (size_t)npair + sizeof(float) * kCc3mWinShells + sizeof(double);
+}
+
+Cc3mWinBuf cc3m_window_buf(void* base, int npair, size_t n) {
+  Cc3mWinBuf b;
+  b.npair = npair;
+  b.cross = static_cast<float4*>(base);
+  b.norm = reinterpret_cast<double*>(b.cross + (size_t)npair * n);
+  b.a2 = reinterpret_cast<float*>(b.norm + n);
+  return b;
+}
+
 namespace {
-template <int RB, int M>
-int launch_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
-                const float* ctff, const int* pidx, const float* dm, const float* shift,
-                const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
-                int blocks) {
+struct BandCall {
+  const float *a3df, *spec, *ctff;
+  const int* pidx;
+  const float *dm, *shift, *amag, *fsct;
+};
+
+template <int RB, int M, bool kWin>
+int launch_band(Ctx& c, const Cc3mArgs& a, const BandCall& p, const Cc3mBandTables& t,
+                float* score, int blocks, const Cc3mWinBuf& wb) {
   using S = BandShape<RB, M>;
-  auto fn = k_cc3m_band<RB, M>;
+  auto fn = k_cc3m_band<RB, M, kWin>;
   const size_t lds = sizeof(float) * S::kLds;
   FR_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)lds));
   int grid = 0;
   if (int r = cc3m_grid(c, (const void*)fn, S::kThreads, lds, a.n, blocks, &grid)) return r;
-  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(S::kThreads), lds, c.stream, a.nsam, a.n, a.rbfact,
-                     reinterpret_cast<const float2*>(a3df), dm, pidx,
-                     reinterpret_cast<const float2*>(ctff), reinterpret_cast<const float2*>(spec),
-                     shift, amag, fsct, t.dft, t.pairs, t.ring, t.ring_cnt, t.wmap, score, a.cc3);
+  hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(S::kThreads), lds, c.stream, a.nsam, a.n,
+                     a.rbfact, reinterpret_cast<const float2*>(p.a3df), p.dm, p.pidx,
+                     reinterpret_cast<const float2*>(p.ctff),
+                     reinterpret_cast<const float2*>(p.spec), p.shift, p.amag, p.fsct, t.dft,
+                     t.pairs, t.ring, t.ring_cnt, t.wmap, score, a.cc3, wb);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
+template <bool kWin>
+int launch_any(Ctx& c, const Cc3mArgs& a, const BandCall& p, const Cc3mBandTables& t,
+               float* score, int blocks, const Cc3mWinBuf& wb) {
+  FR_CHECK(t.dft && t.pairs && t.ring && t.wmap, "band CC3M tables missing");
+  const int M = cc3m_band_grid(a.nsam, a.maxr2), rb = cc3m_band_rb(a.maxr2);
+  if (rb == 16 && M == 64) return launch_band<16, 64, kWin>(c, a, p, t, score, blocks, wb);
+  if (rb == 32 && M == 64) return launch_band<32, 64, kWin>(c, a, p, t, score, blocks, wb);
+  if (rb == 32 && M == 96) return launch_band<32, 96, kWin>(c, a, p, t, score, blocks, wb);
+  if (rb == 32 && M == 128) return launch_band<32, 128, kWin>(c, a, p, t, score, blocks, wb);
+  return fail("band CC3M: no grid for MAXR2 %d", a.maxr2);
+}
+
+template <int NT>
+int launch_window(Ctx& c, const Cc3mArgs& a, const float* fsct, const float* amag,
+                  const Cc3mBandTables& t, const Cc3mWindow& win, const Cc3mWinBuf& wb,
+                  float* score, int* code) {
+  const int top = a.nsam / 2 < kCc3mShells ? a.nsam / 2 : kCc3mShells;
+  hipLaunchKernelGGL(k_cc3m_window<NT>, dim3((unsigned)((a.n + kWinItems - 1) / kWinItems)),
+                     dim3(64 * kWinWaves), 0, c.stream, a.n, cc3m_band_rb(a.maxr2), top, a.rbfact,
+                     t.pairs, fsct, amag, a.cc3, win, wb, score, code);
   FR_HIP(hipGetLastError());
   return 0;
 }
@@ -543,21 +757,30 @@ int launch_cc3m_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* 
                      const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
                      int blocks) {
   if (a.n <= 0) return 0;
-  FR_CHECK(t.dft && t.pairs && t.ring && t.wmap, "band CC3M tables missing");
-  const int M = cc3m_band_grid(a.nsam, a.maxr2), rb = cc3m_band_rb(a.maxr2);
-  if (rb == 16 && M == 64)
-    return launch_band<16, 64>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
-                               blocks);
-  if (rb == 32 && M == 64)
-    return launch_band<32, 64>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
-                               blocks);
-  if (rb == 32 && M == 96)
-    return launch_band<32, 96>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
-                               blocks);
-  if (rb == 32 && M == 128)
-    return launch_band<32, 128>(c, a, a3df, spec, ctff, pidx, dm, shift, amag, fsct, t, score,
-                                blocks);
-  return fail("band CC3M: no grid for MAXR2 %d", a.maxr2);
+  return launch_any<false>(c, a, BandCall{a3df, spec, ctff, pidx, dm, shift, amag, fsct}, t, score,
+                           blocks, Cc3mWinBuf{});
+}
+
+int launch_cc3m_band_window(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
+                            const float* ctff, const int* pidx, const float* dm,
+                            const float* shift, const float* amag, const float* fsct,
+                            const Cc3mBandTables& t, const Cc3mWindow& win, void* buf,
+                            float* score, int* code, int blocks) {
+  if (a.n <= 0) return 0;
+  FR_CHECK(buf && code, "window buffers missing");
+  FR_CHECK(win.nsx >= 1 && win.nsy >= 1 && win.nsx <= kCc3mWinMax && win.nsy <= kCc3mWinMax &&
+               win.nsx % 2 == 1 && win.nsy % 2 == 1,
+           "shift window %d x %d: odd sizes up to %d", win.nsx, win.nsy, kCc3mWinMax);
+  const int npair =
+      cc3m_band_npair(a.maxr1 * a.maxr1, a.maxr2 * a.maxr2, cc3m_band_rb(a.maxr2));
+  const Cc3mWinBuf wb = cc3m_window_buf(buf, npair, a.n);
+  if (int r = launch_any<true>(c, a, BandCall{a3df, spec, ctff, pidx, dm, shift, amag, fsct}, t,
+                               score, blocks, wb))
+    return r;
+  const int nq = (win.nsx / 2 + 1) * (win.nsy / 2 + 1);
+  if (nq <= 16) return launch_window<1>(c, a, fsct, amag, t, win, wb, score, code);
+  if (nq <= 32) return launch_window<2>(c, a, fsct, amag, t, win, wb, score, code);
+  return launch_window<3>(c, a, fsct, amag, t, win, wb, score, code);
 }
 
 }  // namespace fr

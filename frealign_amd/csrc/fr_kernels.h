@@ -192,5 +192,22 @@ int launch_cc3m_band(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* 
                      const float* ctff, const int* pidx, const float* dm, const float* shift,
                      const float* amag, const float* fsct, const Cc3mBandTables& t, float* score,
                      int blocks);
+// The same at every shift of a window around the item's: the best score and
+// its index (ix * nsy + iy, the first maximum).  buf: cc3m_window_bytes(the
+// band's pairs) per item, 16-byte aligned.
+constexpr int kCc3mWinShells = 32;
+struct Cc3mWinBuf {
+  float4* cross = nullptr;  // [item][pair] (Re, Im) of C(+J) + C(-J) and C(+J) - C(-J)
+  double* norm = nullptr;   // [item] sqrt(SUM1 SUM2)
+  float* a2 = nullptr;      // [item][shell - 1] sum |AINPO|^2
+  int npair = 0;
+};
+int cc3m_band_npair(int maxr12, int maxr22, int rb);
+size_t cc3m_window_bytes(int npair);
+int launch_cc3m_band_window(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
+                            const float* ctff, const int* pidx, const float* dm,
+                            const float* shift, const float* amag, const float* fsct,
+                            const Cc3mBandTables& t, const Cc3mWindow& win, void* buf,
+                            float* score, int* code, int blocks);
 
 }  // namespace fr

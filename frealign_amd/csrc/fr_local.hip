@@ -120,6 +120,9 @@ __global__ void __launch_bounds__(64)
 }
 
 constexpr int kItemBudget = 1 << 16;  // items per launch
+// bytes of the cross spectra between the two kernels of a launch: they stay in
+// the 256 MB cache next to what else the launch reads
+constexpr size_t kWinBudget = (size_t)160 << 20;
 
 }  // namespace
 
@@ -155,7 +158,13 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
     centre[2 * p + 1] = x[4];
   }
   std::vector<float> am(amag, amag + np);
-  const int chunk_p = std::max(1, std::min(np, kItemBudget / norient));
+  // on the band's own grid where every AMAG is 1, else on the NSAM grid
+  bool unit = true;
+  for (int p = 0; p < np; p++) unit &= fabsf(am[p]) == 1.0f;
+  const size_t win_bytes = cc3m_window_bytes(
+      cc3m_band_npair(maxr1 * maxr1, maxr2 * maxr2, cc3m_band_rb(maxr2)));
+  const size_t budget = unit ? std::min<size_t>(kItemBudget, kWinBudget / win_bytes) : kItemBudget;
+  const int chunk_p = std::max(1, std::min(np, (int)budget / norient));
   const size_t chunk_items = (size_t)chunk_p * norient;
   int err = 0;
   float* d_trig = (float*)c->slot(6, sizeof(float) * (trig.size() + centre.size() + np + 9), &err);
@@ -185,7 +194,15 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
   if (!d_best) return err;
   Cc3mArgs a{nsam, 0, maxr1, maxr2, rbfact, ring[0], ring[1], ring[2], ring[3]};
   Cc3mTables tabs;
-  if (int r = c->cc3m_tables(a, &tabs)) return r;
+  Cc3mBandTables band;
+  void* d_win = nullptr;
+  if (unit) {
+    if (int r = c->cc3m_band_tables(a, &band)) return r;
+    d_win = c->slot(12, win_bytes * chunk_items, &err);
+    if (!d_win) return err;
+  } else if (int r = c->cc3m_tables(a, &tabs)) {
+    return r;
+  }
   const Cc3mWindow win{2 * nsh + 1, 2 * nsh + 1, dsh, dsh};
   const fr_ctx::Tune tn = c->tune_for(nsam);
   std::vector<int> best(3 * (size_t)np);
@@ -199,9 +216,14 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
     float* sc = d_scores ? d_scores + (size_t)p0 * norient : d_sc;
     int* cd = d_codes ? d_codes + (size_t)p0 * norient : d_cd;
     int pslot = c->prof_begin(kProfCc3m);
-    if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai, d_fsct,
-                                  tabs, sc, tn.cc3m_blocks, &win, cd))
+    if (unit) {
+      if (int r = launch_cc3m_band_window(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
+                                          d_fsct, band, win, d_win, sc, cd, tn.cc3m_blocks))
+        return r;
+    } else if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
+                                         d_fsct, tabs, sc, tn.cc3m_blocks, &win, cd)) {
       return r;
+    }
     c->prof_end(pslot);
     hipLaunchKernelGGL(k_local_best, dim3(pc), dim3(64), 0, c->stream, norient, sc, cd,
                        d_best + 3 * (size_t)p0);

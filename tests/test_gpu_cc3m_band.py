@@ -3,7 +3,8 @@
 The two agree up to FP32 rounding for every box size, band and mask: bands at
 the edges of the grids (MAXR2 16 | 17, 24 | 25, 32), boxes smaller than, equal
 to and larger than the grid, one item and more items than workgroups, and
-items whose AMAG is not 1 (taken by another kernel) between the others.
+items whose AMAG is not 1 (taken by another kernel) between the others.  The
+window form is held to the scores at its shifts in the same way.
 
 Bar: both paths run about 2 log2(N^2) + 4 rounded stages (transforms, mask,
 shell sums), each at most 2^-24 of the shells' root mean square, so a score
@@ -76,3 +77,43 @@ def test_band_grid_equals_fft_path(ctx, nsam, maxr1, maxr2, cc3):
         assert np.abs(got - want).max() <= BAR * np.abs(want).max(), (n, halfw)
         again = score(ctx[0], nsam, a, maxr1, maxr2, ring, cc3)
         assert np.array_equal(got, again)
+
+
+@pytest.mark.parametrize("nsam,maxr1,maxr2,nsh", [
+    (64, 1, 16, 0), (64, 2, 31, 2), (96, 0, 24, 3), (96, 2, 25, 4), (128, 2, 32, 5),
+    (160, 2, 14, 1), (256, 1, 32, 4)])
+@pytest.mark.parametrize("amag", [1.0, 1.04])
+def test_window_equals_scores_at_its_shifts(ctx, nsam, maxr1, maxr2, nsh, amag):
+    """Each orientation's best score over the window and its shift, against CC3M at
+    every shift (one, two and three column blocks of the quarter window)."""
+    npart, nang, dang, dsh = 3, 1, 0.02, float(np.float32(2 * np.pi / nsam))
+    ri = 0.42 * nsam
+    ring = np.array([(ri - 3) ** 2, (ri + 3) ** 2, ri - 3, 6.0], np.float32)
+    a3df, spec, ctff = items(nsam, npart, npart, 5 + nsam, False)[:3]
+    fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    rng = np.random.default_rng(nsh)
+    par = np.concatenate([synth.random_orientations(npart, rng), rng.normal(0, 0.1, (npart, 2))], 1)
+    par = par.astype(np.float32)
+    best, sc, code = ctx[0].local_search(
+        nsam, a3df, spec, ctff, par, nang=nang, dang=dang, nsh=nsh, dsh=dsh, maxr1=maxr1,
+        maxr2=maxr2, rbfact=0.002, fsct=fsct, ring=ring, amag=np.full(npart, amag),
+        all_scores=True)
+    k = np.arange(-nang, nang + 1, dtype=np.float32) * np.float32(dang)
+    q = np.arange(-nsh, nsh + 1, dtype=np.float32) * np.float32(dsh)
+    ang = np.stack(np.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3)
+    sh = np.stack(np.meshgrid(q, q, indexing="ij"), -1).reshape(-1, 2)
+    eul = (par[:, None, :3] + ang[None]).reshape(-1, 3)
+    n, ns = len(eul), len(sh)
+    dm = np.repeat(api.rotation(eul, amag=amag), ns, 0)
+    shift = (np.repeat(par[:, 3:], len(ang), 0)[:, None] + sh[None]).reshape(-1, 2)
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a, d)).to(DEV)  # noqa: E731
+    ctx[1].set_cc3m_variant(nsam, False)
+    want = ctx[1].cc3m(nsam, a3df, spec, ctff,
+                       t(np.repeat(np.arange(npart), len(ang) * ns), np.int32), t(dm, np.float32),
+                       t(shift, np.float32), torch.full((n * ns,), amag, device=DEV), maxr1, maxr2,
+                       0.002, fsct, ring).cpu().numpy().reshape(n, ns)
+    sc, code = sc.cpu().numpy().reshape(-1), code.cpu().numpy().reshape(-1)
+    bar = BAR * np.abs(want).max()
+    assert np.abs(sc - want.max(1)).max() <= bar
+    assert (want.max(1) - want[np.arange(n), code] <= 2 * bar).all()
+    assert np.abs(best[:, 5] - want.reshape(npart, -1).max(1)).max() <= bar
