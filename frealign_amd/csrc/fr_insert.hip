@@ -1,5 +1,5 @@
-// fr_insert.hip -- CTF-weighted trilinear Fourier insertion, gathered per
-// voxel tile.
+// fr_insert.hip -- CTF-weighted trilinear Fourier insertion, scattered per voxel
+// tile in LDS.
 //
 // Replaces PINSERT_TRILIN (pinsert_trilin.f:8-244) as driven by PINSERT
 // (pinsert.f:8-195) for a buffer of particles, the A3D3/A3D3_S flush
@@ -9,30 +9,46 @@
 // min(NSAM/2,FLOOR(X3+1))] (and likewise M, N within +-NSAM/2) with the
 // trilinear weight (1-|X3-L|)(1-|Y3-M|)(1-|Z3-N|).
 //
-// Instead of scattering every point with float atomics, each workgroup owns
-// one 8x8x8 tile of the half-volume and each thread one voxel: the tile first
-// lists (in task order) the tasks whose plane passes within reach of it, and
-// each voxel then visits, per listed task, the few plane points (I,J) that can
-// reach it -- those near its projection onto the plane, found through the
-// inverse Gram matrix of the plane's axes -- and re-derives for each the
-// reference's FP32 coordinates and voxel range (same operation order, no FMA
-// contraction), so exactly the scatter's (point, voxel) pairs contribute,
-// with bit-identical terms (the voxel-range test is done as two float
-// comparisons per axis, equivalent to the reference's INT() rules; the J of a
-// candidate row are bounded per axis by a form linear in I).  Tiles near the
-// origin, which every plane crosses, are dispatched first so that they do not
-// trail the launch.  Sums run in a fixed order: the volumes, NKSUM
-// and TTD are deterministic, and no atomics are needed.  The per-point terms
-// (sample x phase ramp x CTF x weight, and CTF^2 x weight) depend only on the
-// particle, so they are formed once per particle.
+// A workgroup owns one 8x8x8 tile of one half-map.  It lists, in task order,
+// the half's tasks whose plane passes within reach of the tile; its four waves
+// take a contiguous quarter of the list each.  A wave takes two tasks at a
+// time, 32 lanes each: the lanes bound the J of 32 rows I against the tile
+// grown by the trilinear reach (a form linear in I), a prefix sum packs the
+// rows, and the points go through 32 at a time, a lane a point: its FP32
+// coordinates and voxel range in the reference's operation order (no FMA
+// contraction), eight corners added to sums in LDS.  A point near a tile's face
+// is visited by the neighbouring tiles too; corners outside the tile are
+// left out.
+//
+// The sums are plain reads and writes: LDS float atomics take about 100 cycles
+// a wave here (measured: 4.4 of 5.1 ms).  No two lanes may then meet in a voxel
+// in one instruction.  Each 32 lanes have sums of their own, and take the
+// plane's points by classes (I mod q, J mod q): q steps of the plane's axes are
+// longer than a cell's diagonal sqrt(3) (q = 2 unless AMAG > 1.15), so the
+// points of a class lie in different cells, and a wave's LDS accesses complete
+// in program order.  The eight sums of a voxel are added in a fixed order at the
+// end: reruns give the same bits, NKSUM and TTD likewise.  No global atomics.
+// Tiles near the origin, which every plane crosses, are dispatched first so
+// that they do not trail the launch.  The per-point terms (sample x phase ramp
+// x CTF x weight, and CTF^2 x weight) depend only on the particle, so they are
+// formed once per particle, J innermost.
+//
+// What bounds it: the vector units (about 300 instructions per 64 lanes' points,
+// near half of them filled) and the latency of a point's eight dependent LDS
+// updates; the sums' 48 KB let three workgroups share a CU.  The gather that this
+// replaces gave each voxel a thread, which tested every point that could reach it,
+// most of them in vain: 64 particles x 14 copies at 256^3 3,790 us, now 1,456;
+// 300 particles in C1 at 150^3 1,150 us, now 310.
 //
 // The _SE variant (PINSERT_TRILIN_SE with NNSTAT = 1,
 // pinsert_trilin_se.f:186-194) also sums, per voxel, the count, |term|^2,
 // |term| and the phase difference to the reference transform of the terms it
-// receives; being per voxel, these ride on the same gather for free.
+// receives, over both halves: its workgroups take the two halves in turn.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
+
+#include <type_traits>
 
 #include "fr_common.h"
 #include "fr_kernels.h"
@@ -42,37 +58,34 @@ namespace fr {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTile = 8;            // voxels per tile edge
-constexpr int kGatherThreads = 512; // one per voxel of a tile
-static_assert(kTile == 8 && kGatherThreads == 512, "the gather maps 8 waves to 4x4x4 sub-cubes");
-constexpr int kChunk = 4096;        // tasks listed per pass
+constexpr int kTile = 8;  // voxels per tile edge
+constexpr int kVox = kTile * kTile * kTile;
+constexpr int kWaves = 4;        // per tile
+constexpr int kSets = 2;         // tasks a wave takes at a time, each with sums of its own
+constexpr int kLanes = 64 / kSets;
+constexpr int kList = kThreads;  // tasks tested per pass
 constexpr int kReduceThreads = 1024;
+static_assert(kThreads == 64 * kWaves && kSets == 2, "32 lanes per set of sums");
 
-// per task, for the candidate search only (never in the sums)
-struct InsertGeo {
-  float nx, ny, nz, nl1;    // plane normal a x b and its L1 norm
-  float h1x, h1y, h1z, r1;  // I = h1 . P for P on the plane; r1 = |h1|_1
-  float h2x, h2y, h2z, r2;  // J = h2 . P; r2 = |h2|_1
-  float rmax2;              // squared reach of the plane's points (+ margin)
-  int valid;
-  int zaxes;                // bit k: |b_k| too small for 1/b_k (axis k bounds no J)
-  float pad_;
-  float ibx, iby, ibz, pad2_;  // 1/b per axis (0 where |b| is tiny)
-  // per axis k, the J of a point I a + J b within 1.02 of coordinate v_k:
-  // J in v_k / b_k - I a_k / b_k -+ 1.02 / |b_k|
-  float sx, sy, sz;         // a_k / b_k
-  float ox, oy, oz;         // 1.02 / |b_k| (3e38 where b_k ~ 0)
-  float pad3_[2];
-};
+// Per task, in the order half 0 then half 1 (task order within a half):
+//   [0] d0 d1 d2 d3   [1] d4 d5 IRREC^2 part
+//   [2] h1 (I = h1 . P for P on the plane), ilo | ihi << 16
+//   [3] h2 (J = h2 . P), bit k: |b_k| too small for 1/b_k (axis k bounds no J)
+//   [4] 1/b per axis, classes per axis   [5] a_k / b_k per axis (0 where b_k ~ 0)
+constexpr int kRec = 6;
 
 __host__ __device__ inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 struct Scratch {
   int* first;        // [nb] first task of each particle (or -1)
-  InsertGeo* geo;    // [ntask]
-  float4* pts;       // [nb][w*w] (samp.re, samp.im, ctfv2, 0)
+  int* ord;          // [ntask] tasks by half
+  int* n0;           // tasks of half 0
+  float4* hit;       // [ntask] plane normal, squared reach (below 0: no plane)
+  float4* rec;       // [ntask][kRec]
+  float4* pts;       // [nb][w*w] (samp.re, samp.im, ctfv2, 0), J innermost
   unsigned long long* pcount;  // [ntiles][2]
   double* pttd;      // [ntiles][2]
+  size_t bytes;
 };
 
 Scratch scratch_layout(void* base, int nsam, int nb, int ntask, int ntiles) {
@@ -80,15 +93,19 @@ Scratch scratch_layout(void* base, int nsam, int nb, int ntask, int ntiles) {
   char* p = static_cast<char*>(base);
   Scratch s;
   size_t o = 0;
-  s.first = reinterpret_cast<int*>(p + o);
-  o += align256(sizeof(int) * (size_t)nb);
-  s.geo = reinterpret_cast<InsertGeo*>(p + o);
-  o += align256(sizeof(InsertGeo) * (size_t)ntask);
-  s.pts = reinterpret_cast<float4*>(p + o);
-  o += align256(sizeof(float4) * (size_t)nb * w * w);
-  s.pcount = reinterpret_cast<unsigned long long*>(p + o);
-  o += align256(sizeof(unsigned long long) * 2 * (size_t)ntiles);
-  s.pttd = reinterpret_cast<double*>(p + o);
+  auto take = [&](auto*& q, size_t n) {
+    q = reinterpret_cast<std::remove_reference_t<decltype(q)>>(p + o);
+    o += align256(sizeof(*q) * n);
+  };
+  take(s.first, (size_t)nb);
+  take(s.ord, (size_t)ntask);
+  take(s.n0, 1);
+  take(s.hit, (size_t)ntask);
+  take(s.rec, (size_t)ntask * kRec);
+  take(s.pts, (size_t)nb * w * w);
+  take(s.pcount, 2 * (size_t)ntiles);
+  take(s.pttd, 2 * (size_t)ntiles);
+  s.bytes = o;
   return s;
 }
 
@@ -96,48 +113,73 @@ void tile_counts(int nsam, int* tx, int* ty, int* tz) {
   const int jc = nsam / 2 + 1;
   *tx = (jc + kTile - 1) / kTile;
   *ty = (nsam + kTile - 1) / kTile;
-  *tz = *ty;
+  *tz = (nsam + kTile - 1) / kTile;
 }
 
-__global__ void __launch_bounds__(kThreads) k_first_clear(int nb, int* first) {
-  const int p = blockIdx.x * kThreads + threadIdx.x;
-  if (p < nb) first[p] = -1;
-}
-
-// the first task of each run of tasks of one particle (tasks come grouped by
-// particle; a particle's copies share its shift, weight and radius)
-__global__ void __launch_bounds__(kThreads)
-    k_first_mark(int ntask, int nb, const InsertTask* __restrict__ tasks, int* first) {
-  const int k = blockIdx.x * kThreads + threadIdx.x;
-  if (k >= ntask) return;
-  const int part = tasks[k].part;
-  if (part < 0 || part >= nb) return;
-  if (k == 0 || tasks[k - 1].part != part) first[part] = k;
+// One workgroup: the tasks of half 0 and then those of half 1, each in task
+// order, and the first task of each run of tasks of one particle (tasks come
+// grouped by particle; a particle's copies share its shift, weight and radius)
+__global__ void __launch_bounds__(1024)
+    k_insert_order(int ntask, int nb, const InsertTask* __restrict__ tasks, int* first, int* ord,
+                   int* n0) {
+  __shared__ int tot[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int p = tid; p < nb; p += 1024) first[p] = -1;
+  int mine = 0;
+  for (int k = tid; k < ntask; k += 1024) mine += tasks[k].half ? 0 : 1;
+  for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
+  if (lane == 0) tot[wave] = mine;
+  __syncthreads();
+  int zeros = 0;
+  for (int q = 0; q < 16; q++) zeros += tot[q];
+  if (tid == 0) *n0 = zeros;
+  int seen0 = 0;  // tasks of half 0 before this pass
+  for (int base = 0; base < ntask; base += 1024) {
+    const int k = base + tid;
+    const bool in = k < ntask;
+    const bool h0 = in && !tasks[k].half;
+    if (in) {
+      const int part = tasks[k].part;
+      if (part >= 0 && part < nb && (k == 0 || tasks[k - 1].part != part)) first[part] = k;
+    }
+    const unsigned long long bal = __ballot(h0);
+    __syncthreads();
+    if (lane == 0) tot[wave] = __popcll(bal);
+    __syncthreads();
+    int before = seen0 + __popcll(bal & ((1ull << lane) - 1ull));
+    for (int q = 0; q < 16; q++) {
+      if (q < wave) before += tot[q];
+      seen0 += tot[q];
+    }
+    if (in) ord[h0 ? before : zeros + k - before] = k;
+  }
 }
 
 // pinsert_trilin.f:60-87: the weighted sample and CTF^2 of every plane point
-// of a particle, exactly as the scatter formed them
+// of a particle, exactly as the reference's scatter forms them; a workgroup
+// takes 16 x 16 points, read with I innermost and written with J innermost
 __global__ void __launch_bounds__(kThreads)
     k_insert_points(int nsam, const int* __restrict__ first,
                     const InsertTask* __restrict__ tasks, const float2* __restrict__ datc,
                     const float2* __restrict__ ctff, float4* pts) {
+  __shared__ float4 turn[16][17];
   const int b = blockIdx.y;
   const int k = first[b];
   if (k < 0) return;
   const InsertTask t = tasks[k];
-  const int jc = nsam / 2 + 1, w = 2 * jc - 1;
+  const int jc = nsam / 2 + 1, w = 2 * jc - 1, nt = (w + 15) / 16;
   const size_t ic = (size_t)nsam * jc;
-  const int e = blockIdx.x * kThreads + threadIdx.x;
-  if (e >= w * w) return;
-  const int i = e % w - (jc - 1);
-  const int j = e / w - (jc - 1);
+  const int bi = (blockIdx.x % nt) * 16, bj = (blockIdx.x / nt) * 16;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  const int i = bi + tx - (jc - 1);
+  const int j = bj + ty - (jc - 1);
   float4 out = make_float4(0.f, 0.f, 0.f, 0.f);
   float g2;
   bool inside;
   {
 #pragma clang fp contract(off)
     g2 = (float)(i * i + j * j);
-    inside = g2 <= (float)t.irrec2;
+    inside = g2 <= (float)t.irrec2 && i < jc && j < jc;
   }
   if (inside) {
     const float2* sp = datc + (size_t)t.part * ic;
@@ -159,75 +201,53 @@ __global__ void __launch_bounds__(kThreads)
     samp = cscale(samp, wgt);
     out = make_float4(samp.re, samp.im, ctfv2, 0.f);
   }
-  pts[(size_t)b * w * w + e] = out;
+  turn[tx][ty] = out;
+  __syncthreads();
+  const int oi = bi + ty, oj = bj + tx;
+  if (oi < w && oj < w) pts[(size_t)b * w * w + (size_t)oi * w + oj] = turn[ty][tx];
 }
 
-// per-task plane geometry for the candidate search (double, then rounded;
-// the margins below cover the rounding)
+// per-task plane geometry for the candidate search (double, then rounded; the
+// margins of the search cover the rounding)
 __global__ void __launch_bounds__(kThreads)
-    k_insert_geo(int ntask, int nsam, const InsertTask* __restrict__ tasks, InsertGeo* geo) {
-  const int k = blockIdx.x * kThreads + threadIdx.x;
-  if (k >= ntask) return;
-  const InsertTask t = tasks[k];
+    k_insert_geo(int ntask, int nb, int nsam, const InsertTask* __restrict__ tasks,
+                 const int* __restrict__ ord, float4* hit, float4* rec) {
+  const int q = blockIdx.x * kThreads + threadIdx.x;
+  if (q >= ntask) return;
+  const InsertTask t = tasks[ord[q]];
   const double ax = t.dm[0], ay = t.dm[1], az = t.dm[2];
   const double bx = t.dm[3], by = t.dm[4], bz = t.dm[5];
-  InsertGeo g;
   const double nx = ay * bz - az * by, ny = az * bx - ax * bz, nz = ax * by - ay * bx;
   const double aa = ax * ax + ay * ay + az * az, bb = bx * bx + by * by + bz * bz;
   const double ab = ax * bx + ay * by + az * bz;
   const double det = aa * bb - ab * ab;
-  g.valid = (t.irrec2 >= 0 && det > 1e-12) ? 1 : 0;
-  const double id = g.valid ? 1.0 / det : 0.0;
-  const double h1x = (bb * ax - ab * bx) * id, h1y = (bb * ay - ab * by) * id,
-               h1z = (bb * az - ab * bz) * id;
-  const double h2x = (aa * bx - ab * ax) * id, h2y = (aa * by - ab * ay) * id,
-               h2z = (aa * bz - ab * az) * id;
-  g.nx = (float)nx;
-  g.ny = (float)ny;
-  g.nz = (float)nz;
-  g.nl1 = (float)(fabs(nx) + fabs(ny) + fabs(nz));
-  g.h1x = (float)h1x;
-  g.h1y = (float)h1y;
-  g.h1z = (float)h1z;
-  g.r1 = (float)(fabs(h1x) + fabs(h1y) + fabs(h1z));
-  g.h2x = (float)h2x;
-  g.h2y = (float)h2y;
-  g.h2z = (float)h2z;
-  g.r2 = (float)(fabs(h2x) + fabs(h2y) + fabs(h2z));
+  const bool valid = t.irrec2 >= 0 && det > 1e-12 && t.part >= 0 && t.part < nb;
+  const double id = valid ? 1.0 / det : 0.0;
   // points reach |P| <= sqrt(IRREC^2 * lambda_max(G)) within the square
   // |I|,|J| <= NSAM/2; a voxel they touch lies within sqrt(3) more
   const double lmax = 0.5 * (aa + bb + sqrt((aa - bb) * (aa - bb) + 4.0 * ab * ab));
   const double jcm = (double)(nsam / 2);
   const double r2pts = t.irrec2 < 2.0 * jcm * jcm ? (double)t.irrec2 : 2.0 * jcm * jcm;
   const double reach = sqrt(r2pts * lmax) + 1.7320508 + 0.01;
-  g.rmax2 = (float)(reach * reach);
-  g.pad_ = 0.f;
+  // classes of points: q steps of the plane's lattice span more than a cell's
+  // diagonal (distances are at least the square root of G's smaller eigenvalue)
+  const double lmin = fmax(aa + bb - lmax, 0.0);
+  const int q2 = valid ? (int)fmin(fmax(ceil(1.7322 / sqrt(lmin)), 2.0), 2.0 * jcm + 1.0) : 2;
+  hit[q] = make_float4((float)nx, (float)ny, (float)nz, valid ? (float)(reach * reach) : -1.f);
   const bool zx = !(fabs(bx) > 1e-6), zy = !(fabs(by) > 1e-6), zz = !(fabs(bz) > 1e-6);
-  g.zaxes = (zx ? 1 : 0) | (zy ? 2 : 0) | (zz ? 4 : 0);
-  g.ibx = zx ? 0.f : (float)(1.0 / bx);
-  g.iby = zy ? 0.f : (float)(1.0 / by);
-  g.ibz = zz ? 0.f : (float)(1.0 / bz);
-  g.pad2_ = 0.f;
-  g.sx = zx ? 0.f : (float)(ax / bx);
-  g.sy = zy ? 0.f : (float)(ay / by);
-  g.sz = zz ? 0.f : (float)(az / bz);
-  // an axis with b_k ~ 0 leaves J free: c_k = s_k = 0 and an unbounded o_k
-  g.ox = zx ? 3.0e38f : (float)(1.02 / fabs(bx));
-  g.oy = zy ? 3.0e38f : (float)(1.02 / fabs(by));
-  g.oz = zz ? 3.0e38f : (float)(1.02 / fabs(bz));
-  g.pad3_[0] = g.pad3_[1] = 0.f;
-  geo[k] = g;
-}
-
-// the logical coordinates stored at index s of a wrapped axis: s itself for
-// s < NSAM/2, s - NSAM for s > NSAM/2, and both +NSAM/2 and -NSAM/2 at s = NSAM/2
-__device__ inline int logical_axis(int s, int nsam, int* v) {
-  const int h = nsam / 2;
-  if (s < h) { v[0] = s; return 1; }
-  if (s > h) { v[0] = s - nsam; return 1; }
-  v[0] = h;
-  v[1] = -h;
-  return 2;
+  float4* r = rec + (size_t)q * kRec;
+  r[0] = make_float4(t.dm[0], t.dm[1], t.dm[2], t.dm[3]);
+  r[1] = make_float4(t.dm[4], t.dm[5], __int_as_float(t.irrec2), __int_as_float(t.part));
+  r[2] = make_float4((float)((bb * ax - ab * bx) * id), (float)((bb * ay - ab * by) * id),
+                     (float)((bb * az - ab * bz) * id),
+                     __int_as_float((int)(unsigned short)t.ilo | (int)t.ihi << 16));
+  r[3] = make_float4((float)((aa * bx - ab * ax) * id), (float)((aa * by - ab * ay) * id),
+                     (float)((aa * bz - ab * az) * id),
+                     __int_as_float((zx ? 1 : 0) | (zy ? 2 : 0) | (zz ? 4 : 0)));
+  r[4] = make_float4(zx ? 0.f : (float)(1.0 / bx), zy ? 0.f : (float)(1.0 / by),
+                     zz ? 0.f : (float)(1.0 / bz), __int_as_float(q2));
+  r[5] = make_float4(zx ? 0.f : (float)(ax / bx), zy ? 0.f : (float)(ay / by),
+                     zz ? 0.f : (float)(az / bz), 0.f);
 }
 
 // logical intervals covered by the storage range [s0, s1] of a wrapped axis
@@ -247,43 +267,23 @@ __device__ inline int logical_ranges(int s0, int s1, int nsam, int* lo, int* hi)
   return n;
 }
 
-// does the plane through the origin with normal g reach the box [lo, hi]
+// does the plane through the origin with normal g.xyz reach the box [lo, hi]
 // grown by one voxel (the trilinear reach), within the plane's disc?
-__device__ inline bool plane_reaches(const InsertGeo& g, float xl, float xh, float yl, float yh,
+__device__ inline bool plane_reaches(const float4& g, float xl, float xh, float yl, float yh,
                                      float zl, float zh) {
   xl -= 1.01f; yl -= 1.01f; zl -= 1.01f;
   xh += 1.01f; yh += 1.01f; zh += 1.01f;
-  const float mn = (g.nx > 0.f ? g.nx * xl : g.nx * xh) + (g.ny > 0.f ? g.ny * yl : g.ny * yh) +
-                   (g.nz > 0.f ? g.nz * zl : g.nz * zh);
-  const float mx = (g.nx > 0.f ? g.nx * xh : g.nx * xl) + (g.ny > 0.f ? g.ny * yh : g.ny * yl) +
-                   (g.nz > 0.f ? g.nz * zh : g.nz * zl);
-  const float slack = 1e-3f * g.nl1 + 1e-3f;
+  const float mn = (g.x > 0.f ? g.x * xl : g.x * xh) + (g.y > 0.f ? g.y * yl : g.y * yh) +
+                   (g.z > 0.f ? g.z * zl : g.z * zh);
+  const float mx = (g.x > 0.f ? g.x * xh : g.x * xl) + (g.y > 0.f ? g.y * yh : g.y * yl) +
+                   (g.z > 0.f ? g.z * zh : g.z * zl);
+  const float slack = 1e-3f * (fabsf(g.x) + fabsf(g.y) + fabsf(g.z)) + 1e-3f;
   if (mn > slack || mx < -slack) return false;
   // nearest point of the box to the origin
   const float cx = xl > 0.f ? xl : (xh < 0.f ? xh : 0.f);
   const float cy = yl > 0.f ? yl : (yh < 0.f ? yh : 0.f);
   const float cz = zl > 0.f ? zl : (zh < 0.f ? zh : 0.f);
-  return cx * cx + cy * cy + cz * cz <= g.rmax2;
-}
-
-// pinsert_trilin.f:88-111 sets, per axis, S = INT(A1) (minus 1 when A1 < 0)
-// with A1 = (X3 + 0.5) - 0.5 and T = INT(A2) (minus 1 when A2 < 0) with
-// A2 = X3 + 1, clamped to the axis's range, and fills the voxels S..T.  For
-// an integer coordinate v inside the range, v >= S exactly when A1 < v + 1
-// (A1 <= v + 1 when v + 1 < 0), and v <= T exactly when A2 >= v (A2 > v when
-// v < 0); the clamps never exclude such a v.  The strict forms are the
-// non-strict ones against the next float toward +infinity, so each bound is
-// one comparison: A1 < range_lo(v) and A2 >= range_hi(v).
-__device__ inline float next_up_neg(float x) {  // x < 0
-  return __int_as_float(__float_as_int(x) - 1);
-}
-__device__ inline float range_lo(int v) {
-  const float f = (float)(v + 1);
-  return v + 1 >= 0 ? f : next_up_neg(f);
-}
-__device__ inline float range_hi(int v) {
-  const float f = (float)v;
-  return v >= 0 ? f : next_up_neg(f);
+  return cx * cx + cy * cy + cz * cz <= g.w;
 }
 
 // pdiff.f:8-24: |phase of b conj(r)|, 0 where the product is 0
@@ -293,227 +293,387 @@ __device__ inline float pdiff_dev(float br, float bi, float2 r) {
   return fabsf(atan2f(ci, cr));
 }
 
+// inclusive prefix sum over each 32 lanes, on the vector ALU
+template <int kCtrl, int kRows>
+__device__ inline int dpp_acc(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, kCtrl, kRows, 0xf, false);
+}
+__device__ inline int half_scan(int v) {
+  v = dpp_acc<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8 within 16 lanes
+  v = dpp_acc<0x112, 0xf>(v);
+  v = dpp_acc<0x114, 0xf>(v);
+  v = dpp_acc<0x118, 0xf>(v);
+  return dpp_acc<0x142, 0xa>(v);  // row_bcast 15 into the odd rows
+}
+
+// LDS written by some lanes of a wave and read by others: the wave's own
+// accesses complete in order, so only the compiler has to be held
+__device__ inline void wave_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+struct Sum {
+  float re, im, c2;  // numerator, CTF^2
+};
+constexpr int kOut = 1 << 20;             // byte offset of a corner outside the tile
+
+// pinsert_trilin.f:88-111 on one axis: the voxels S..T of a point (S = INT(A1),
+// minus 1 for A1 < 0, with A1 = (X + 0.5) - 0.5; T likewise with A2 = X + 1);
+// those outside the tile's [lo, hi], which lies within the reference's clamps,
+// are left out.  T - S is 0, 1 or (at negative integers) 2.
+struct Axis {
+  int s, t;
+  __device__ Axis(float x) {
+#pragma clang fp contract(off)
+    const float a1 = (x + 0.5f) - 0.5f, a2 = x + 1.0f;
+    s = (int)a1;
+    if (a1 < 0.0f) s--;
+    t = (int)a2;
+    if (a2 < 0.0f) t--;
+  }
+  // byte offset of voxel s + k of an axis whose tile holds lo .. lo + n from
+  // offset `at` on, or kOut
+  __device__ int off(int k, int lo, int n, int at, int mul) const {
+    const int v = s + k - lo;
+    return (unsigned)v <= (unsigned)n && (k == 0 || s + k <= t) ? v * mul + at : kOut;
+  }
+};
+
+// the _SE statistics of a voxel
+struct StatSum {
+  float v, a, p;  // |term|^2, |term|, phase difference
+  int n;
+};
+
 template <bool kStats>
-__global__ void __launch_bounds__(kGatherThreads)
-    k_insert_gather(int nsam, int nb, int ntask, int tx, int ty,
-                    const InsertTask* __restrict__ tasks, const InsertGeo* __restrict__ geo,
-                    const float4* __restrict__ pts, float2* num0, float* ctf2_0, float2* num1,
-                    float* ctf2_1, unsigned long long* pcount, double* pttd, InsertStats st) {
-  __shared__ int list[kChunk];
-  __shared__ int wave_tot[kGatherThreads / 64];
-  const int jc = nsam / 2 + 1, w = 2 * jc - 1;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = blockIdx.x;
+struct TileSums {
+  Sum sum[kWaves][kSets * kVox];
+  StatSum st[kStats ? kWaves : 1][kStats ? kSets * kVox : 1];
+  int list[kList];
+  int tot[kWaves];
+  int2 row[kWaves][kSets][kLanes];     // I | first J << 16, start
+  unsigned flag[kWaves][kSets][8];     // a bit where a row starts
+  unsigned long long rc[kWaves];
+  double rt[kWaves];
+};
+
+template <bool kStats>
+__global__ void __launch_bounds__(kThreads)
+    k_insert_scatter(int nsam, int ntask, int tx, int ty, int tz, const int* __restrict__ n0p,
+                     const float4* __restrict__ hit, const float4* __restrict__ rec,
+                     const float4* __restrict__ pts, float2* num0, float* ctf2_0, float2* num1,
+                     float* ctf2_1, unsigned long long* pcount, double* pttd, InsertStats st) {
+  extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  TileSums<kStats>& S = *reinterpret_cast<TileSums<kStats>*>(lds_raw);
+  const int jc = nsam / 2 + 1, h = nsam / 2, w = 2 * jc - 1;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a tile's two halves are neighbouring workgroups (one workgroup with statistics)
+  const int b = kStats ? blockIdx.x : blockIdx.x >> 1;
   // tiles go out slab by slab in order of |logical n|, rows in order of
   // |logical m| (storage rows 0, last, 1, last - 1, ...): the tiles near the
   // origin, which every plane crosses, start first instead of last
   const int tmf = (b / tx) % ty, tnf = b / (tx * ty);
   const int l0 = (b % tx) * kTile;
   const int m0 = ((tmf & 1) ? ty - 1 - (tmf >> 1) : (tmf >> 1)) * kTile;
-  const int n0 = ((tnf & 1) ? ty - 1 - (tnf >> 1) : (tnf >> 1)) * kTile;
-  // the tile's logical boxes (a wrapped axis may split in two)
+  const int n0 = ((tnf & 1) ? tz - 1 - (tnf >> 1) : (tnf >> 1)) * kTile;
   const int l1 = min(l0 + kTile - 1, jc - 1);
+  // the tile's logical boxes (a wrapped axis may split in two)
   int mlo[2], mhi[2], nlo[2], nhi[2];
   const int nmr = logical_ranges(m0, min(m0 + kTile - 1, nsam - 1), nsam, mlo, mhi);
   const int nnr = logical_ranges(n0, min(n0 + kTile - 1, nsam - 1), nsam, nlo, nhi);
-  // this thread's voxel: wave w takes the 4x4x4 sub-cube w of the tile, so
-  // that a plane leaves whole waves idle (their exec mask empty) rather than
-  // most lanes of every wave
-  const int l = l0 + 4 * (wave & 1) + (lane & 3);
-  const int ms_ = m0 + 4 * ((wave >> 1) & 1) + ((lane >> 2) & 3);
-  const int ns_ = n0 + 4 * (wave >> 2) + (lane >> 4);
-  const bool mine = l < jc && ms_ < nsam && ns_ < nsam;
-  int mv[2], nv[2];
-  const int nm = mine ? logical_axis(ms_, nsam, mv) : 0;
-  const int nn = mine ? logical_axis(ns_, nsam, nv) : 0;
-  // the voxel's range tests as thresholds on X3 (see range_lo, range_hi)
-  const float ltl = range_lo(l), utl = range_hi(l);
-  float a0r = 0.f, a0i = 0.f, a0c = 0.f, a1r = 0.f, a1i = 0.f, a1c = 0.f;
-  unsigned c0 = 0u, c1 = 0u;
-  double t0 = 0.0, t1 = 0.0;
-  // _SE statistics of this voxel (both halves), against its reference value
-  float sv = 0.f, sp = 0.f, sa = 0.f;
-  float2 refv = make_float2(0.f, 0.f);
-  if (kStats && mine)
-    refv = reinterpret_cast<const float2*>(
-        st.ref)[(size_t)l + (size_t)jc * ((size_t)ms_ + (size_t)nsam * ns_)];
-  for (int base = 0; base < ntask; base += kChunk) {
-    __syncthreads();  // the previous chunk's list is no longer read
-    const int cnt = min(kChunk, ntask - base);
-    // list the tasks reaching this tile, in task order (ballot compaction)
-    int nlist = 0;
-    for (int k0 = 0; k0 < cnt; k0 += kGatherThreads) {
-      const int k = k0 + tid;
-      bool hit = false;
-      if (k < cnt) {
-        const InsertGeo g = geo[base + k];
-        if (g.valid)
-          for (int a = 0; a < nmr && !hit; a++)
-            for (int c = 0; c < nnr && !hit; c++)
-              hit = plane_reaches(g, (float)l0, (float)l1, (float)mlo[a], (float)mhi[a],
-                                  (float)nlo[c], (float)nhi[c]);
-      }
-      const unsigned long long bal = __ballot(hit);
-      const int before = __popcll(bal & ((1ull << lane) - 1ull));
-      if (lane == 0) wave_tot[wave] = __popcll(bal);
-      __syncthreads();
-      int off = nlist;
-      for (int q = 0; q < wave; q++) off += wave_tot[q];
-      if (hit) list[off + before] = base + k;
-      int tot = 0;
-      for (int q = 0; q < kGatherThreads / 64; q++) tot += wave_tot[q];
-      __syncthreads();
-      nlist += tot;
-    }
-    // gather this voxel's contributions from the listed tasks
-    if (mine) {
-      for (int q = 0; q < nlist; q++) {
-        // the same task for the whole workgroup: scalar loads of its records
-        const int k = __builtin_amdgcn_readfirstlane(list[q]);
-        const InsertGeo g = geo[k];
-        const InsertTask t = tasks[k];
-        if (t.part < 0 || t.part >= nb) continue;
-        const float4* tp = pts + (size_t)t.part * w * w;
-        for (int am = 0; am < nm; am++)
-          for (int an = 0; an < nn; an++) {
-            const int m = mv[am], n = nv[an];
-            const float fl = (float)l, fm = (float)m, fn = (float)n;
-            const float d = g.nx * fl + g.ny * fm + g.nz * fn;
-            if (fabsf(d) > 1.01f * g.nl1 + 1e-3f) continue;
-            const float ci = g.h1x * fl + g.h1y * fm + g.h1z * fn;
-            const float cj = g.h2x * fl + g.h2y * fm + g.h2z * fn;
-            int ilo = (int)ceilf(ci - g.r1 - 0.02f), ihi = (int)floorf(ci + g.r1 + 0.02f);
-            int jlo = (int)ceilf(cj - g.r2 - 0.02f), jhi = (int)floorf(cj + g.r2 + 0.02f);
-            ilo = max(ilo, (int)t.ilo);  // the task's I stripe, within -(JC-1)..JC-1
-            ihi = min(ihi, (int)t.ihi);
-            jlo = max(jlo, -(jc - 1));
-            jhi = min(jhi, jc - 1);
-            // per axis, the J interval of the points within 1.02 of the
-            // voxel, linear in I: [c_k - I s_k - o_k, c_k - I s_k + o_k]
-            // (an axis with b_k ~ 0 bounds no J: tested per I below)
-            const float cx = (g.zaxes & 1) ? 0.f : fl * g.ibx;
-            const float cy = (g.zaxes & 2) ? 0.f : fm * g.iby;
-            const float cz = (g.zaxes & 4) ? 0.f : fn * g.ibz;
-            const float ltm_ = range_lo(m), utm_ = range_hi(m), ltn_ = range_lo(n), utn_ = range_hi(n);
-            for (int i = ilo; i <= ihi; i++) {
-              const float fi = (float)i;
-              const float ex = cx - fi * g.sx, ey = cy - fi * g.sy, ez = cz - fi * g.sz;
-              const float jl = fmaxf(fmaxf((float)jlo, ex - g.ox), fmaxf(ey - g.oy, ez - g.oz));
-              const float jh = fminf(fminf((float)jhi, ex + g.ox), fminf(ey + g.oy, ez + g.oz));
-              if (g.zaxes) {
-                bool none = false;
+  bool live = false;  // a plane reaches the tile: the waves' sums are set up
+  const int rl = lane & (kLanes - 1), slot = lane / kLanes;
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  char* const set = reinterpret_cast<char*>(&S.sum[wave][slot * kVox]);
+
+  for (int half = kStats ? 0 : blockIdx.x & 1; half < (kStats ? 2 : (blockIdx.x & 1) + 1); half++) {
+    const int k0 = half ? *n0p : 0, k1 = half ? ntask : *n0p;
+    unsigned cnt = 0u;
+    unsigned long long cnt64 = 0ull;
+    double ttd = 0.0;
+    for (int box = 0; box < nmr * nnr; box++) {
+      const int ml = mlo[box % nmr], mh = mhi[box % nmr];
+      const int nl = nlo[box / nmr], nh = nhi[box / nmr];
+      // where the box starts in the tile's sums, in bytes
+      constexpr int kB = sizeof(Sum), kM = kTile * kB, kN = kTile * kM;
+      const int ms = ((ml < 0 ? nsam : 0) - m0 + ml) * kM, ns = ((nl < 0 ? nsam : 0) - n0 + nl) * kN;
+      const float cx = 0.5f * (float)(l0 + l1), hx = 0.5f * (float)(l1 - l0) + 1.02f;
+      const float cy = 0.5f * (float)(ml + mh), hy = 0.5f * (float)(mh - ml) + 1.02f;
+      const float cz = 0.5f * (float)(nl + nh), hz = 0.5f * (float)(nh - nl) + 1.02f;
+      for (int base = k0; base < k1; base += kList) {
+        // list the tasks reaching this box, in task order (ballot compaction)
+        const int k = base + tid;
+        bool on = false;
+        if (k < k1) {
+          const float4 g = hit[k];
+          on = g.w >= 0.f && plane_reaches(g, (float)l0, (float)l1, (float)ml, (float)mh,
+                                           (float)nl, (float)nh);
+        }
+        const unsigned long long bal = __ballot(on);
+        __syncthreads();  // the previous list is no longer read
+        if (lane == 0) S.tot[wave] = __popcll(bal);
+        __syncthreads();
+        int nlist = 0, before = 0;
+        for (int q = 0; q < kWaves; q++) {
+          if (q == wave) before = nlist;
+          nlist += S.tot[q];
+        }
+        if (on) S.list[before + __popcll(bal & lt)] = k;
+        __syncthreads();
+        if (nlist && !live) {  // each wave its own
+          live = true;
+          for (int e = lane; e < kSets * kVox; e += 64) {
+            S.sum[wave][e] = Sum{0.f, 0.f, 0.f};
+            if constexpr (kStats) S.st[wave][e] = StatSum{0.f, 0.f, 0.f, 0};
+          }
+          if (rl < 8) S.flag[wave][slot][rl] = 0u;
+          wave_lds();
+        }
+        // this wave's quarter, four tasks at a time
+        const int q0 = nlist * wave / kWaves, q1 = nlist * (wave + 1) / kWaves;
+        for (int qb = q0; qb < q1; qb += kSets) {
+          const int q = qb + slot;
+          const float4* R = rec + (size_t)S.list[min(q, q1 - 1)] * kRec;
+          const float4 r0 = R[0], r1 = R[1], r2 = R[2], r3 = R[3], r4 = R[4], r5 = R[5];
+          const float4* tp = pts + (size_t)__float_as_int(r1.w) * w * w;
+          const int za = __float_as_int(r3.w), ir2 = __float_as_int(r1.z);
+          // classes per axis: the most that either needs
+          int nc = __float_as_int(r4.w);
+          nc = __builtin_amdgcn_readfirstlane(max(nc, __shfl_xor(nc, 32, 64)));
+          const float ci = r2.x * cx + r2.y * cy + r2.z * cz;
+          const float cj = r3.x * cx + r3.y * cy + r3.z * cz;
+          const float ri = fabsf(r2.x) * hx + fabsf(r2.y) * hy + fabsf(r2.z) * hz + 0.02f;
+          const float rj = fabsf(r3.x) * hx + fabsf(r3.y) * hy + fabsf(r3.z) * hz + 0.02f;
+          const float lim = (float)h;
+          const int ilo = max((int)fminf(fmaxf(ceilf(ci - ri), -lim), lim + 1.f),
+                              (int)(short)__float_as_int(r2.w));
+          const int ihi = min((int)fminf(fmaxf(floorf(ci + ri), -lim - 1.f), lim),
+                              __float_as_int(r2.w) >> 16);
+          const float jlo = fmaxf(ceilf(cj - rj), -lim), jhi = fminf(floorf(cj + rj), lim);
+          // per axis, J in (c_k - I a_k) / b_k -+ h_k / |b_k|
+          const float ex = cx * r4.x, ey = cy * r4.y, ez = cz * r4.z;
+          const float ox = za & 1 ? 3.0e38f : hx * fabsf(r4.x);
+          const float oy = za & 2 ? 3.0e38f : hy * fabsf(r4.y);
+          const float oz = za & 4 ? 3.0e38f : hz * fabsf(r4.z);
+          const int nrow = q < q1 ? ihi - ilo + 1 : 0;
+          for (int rb = 0; __any(rb < nrow); rb += kLanes) {
+            const int i = ilo + rb + rl;
+            const float fi = (float)i;
+            int j0 = 0, j1 = -1;
+            if (q < q1 && i <= ihi) {
+              const float jx = ex - fi * r5.x, jy = ey - fi * r5.y, jz = ez - fi * r5.z;
+              const float jl = fmaxf(fmaxf(jlo, jx - ox), fmaxf(jy - oy, jz - oz));
+              const float jh = fminf(fminf(jhi, jx + ox), fminf(jy + oy, jz + oz));
+              bool on = jl <= jh + 0.02f;
+              if (za) {  // an axis with b_k ~ 0: the row is in reach or not
                 const float slack = 1e-3f * (float)jc;
-                if ((g.zaxes & 1) && fabsf(fl - fi * t.dm[0]) > 1.02f + slack * fabsf(t.dm[3]))
-                  none = true;
-                if ((g.zaxes & 2) && fabsf(fm - fi * t.dm[1]) > 1.02f + slack * fabsf(t.dm[4]))
-                  none = true;
-                if ((g.zaxes & 4) && fabsf(fn - fi * t.dm[2]) > 1.02f + slack * fabsf(t.dm[5]))
-                  none = true;
-                if (none) continue;
+                if ((za & 1) && fabsf(cx - fi * r0.x) > hx + slack * fabsf(r0.w)) on = false;
+                if ((za & 2) && fabsf(cy - fi * r0.y) > hy + slack * fabsf(r1.x)) on = false;
+                if ((za & 4) && fabsf(cz - fi * r0.z) > hz + slack * fabsf(r1.y)) on = false;
               }
-              const int j0 = max((int)ceilf(jl - 0.01f), jlo);
-              const int j1 = min((int)floorf(jh + 0.01f), jhi);
-              float xi, yi, zi;
-              {
-#pragma clang fp contract(off)
-                xi = t.dm[0] * fi;
-                yi = t.dm[1] * fi;
-                zi = t.dm[2] * fi;
+              if (on) {
+                j0 = (int)fmaxf(ceilf(jl - 0.01f), jlo);
+                j1 = (int)fminf(floorf(jh + 0.01f), jhi);
               }
-              const int ii = i * i;
-              for (int j = j0; j <= j1; j++) {
-                // pinsert_trilin.f:88-111 in the reference's FP32 order: the
-                // point's X3 and whether this voxel is in its range
-                float x3, y3, z3;
-                bool in;
-                {
+            }
+            const int imod = nc == 2 ? i & 1 : (i + nc * 1024) % nc;
+            const int jmod = nc == 2 ? j0 & 1 : (j0 + nc * 1024) % nc;
+            for (int cls = 0; cls < nc * nc; cls++) {
+              const int ca = nc == 2 ? cls & 1 : cls % nc, cb = nc == 2 ? cls >> 1 : cls / nc;
+              const int f0 = j0 + (cb >= jmod ? cb - jmod : cb - jmod + nc);
+              int c = 0;
+              if (imod == ca && f0 <= j1) c = nc == 2 ? ((j1 - f0) >> 1) + 1 : (j1 - f0) / nc + 1;
+              // a class holds at most 16 of 32 rows: with 16 points of a row at a
+              // time a pass holds at most 256
+              for (int jb = 0; __any(jb < c); jb += 16) {
+                const int cc = min(max(c - jb, 0), 16);
+                const unsigned some = (unsigned)(__ballot(cc > 0) >> (slot * kLanes));
+                const int end = half_scan(cc), start = end - cc;
+                const int total = __shfl(end, slot * kLanes + kLanes - 1, 64);
+                if (cc > 0) {
+                  S.row[wave][slot][__popc(some & ((1u << rl) - 1u))] =
+                      make_int2((i & 0xffff) | (f0 + jb * nc) << 16, start);
+                  atomicOr(&S.flag[wave][slot][start >> 5], 1u << (start & 31));
+                }
+                wave_lds();
+                int before = -1;  // rows started before these 32 points, less one
+                for (int p0 = 0; __any(p0 < total); p0 += kLanes) {
+                  const unsigned mask = S.flag[wave][slot][p0 / kLanes];
+                  const int p = p0 + rl;
+                  const int at = before + (int)__popc(mask & (~0u >> (31 - rl)));
+                  const int2 rw = S.row[wave][slot][max(at, 0)];
+                  before += (int)__popc(mask);
+                  const bool on = p < total;
+                  const int pi = on ? (short)rw.x : 0;
+                  const int pj = on ? (rw.x >> 16) + (p - rw.y) * nc : 0;
+                  const float4 pv = tp[__mul24(pi + h, w) + pj + h];
+                  float x3, y3, z3;
+                  {
 #pragma clang fp contract(off)
-                  const float fj = (float)j;
-                  x3 = xi + t.dm[3] * fj;
-                  y3 = yi + t.dm[4] * fj;
-                  z3 = zi + t.dm[5] * fj;
-                  in = ((x3 + 0.5f) - 0.5f < ltl) & (x3 + 1.0f >= utl) &
-                       ((y3 + 0.5f) - 0.5f < ltm_) & (y3 + 1.0f >= utm_) &
-                       ((z3 + 0.5f) - 0.5f < ltn_) & (z3 + 1.0f >= utn_);
+                    const float fpi = (float)pi, fpj = (float)pj;
+                    x3 = r0.x * fpi + r0.w * fpj;
+                    y3 = r0.y * fpi + r1.x * fpj;
+                    z3 = r0.z * fpi + r1.y * fpj;
+                  }
+                  const Axis X(x3), Y(y3), Z(z3);
+                  const bool inside = on && pi * pi + pj * pj <= ir2;
+                  // corner (kx, ky, kz) of every lane's point: pinsert_trilin.f:113-131,
+                  // the weights' product in its order
+                  auto corner = [&](int off, float bxy, float bz) {
+                    const float box = bxy * bz;
+                    if (off < kOut) {
+                      Sum& t = *reinterpret_cast<Sum*>(set + off);
+                      Sum u = t;
+                      u.re += pv.x * box;
+                      u.im += pv.y * box;
+                      u.c2 += pv.z * box;
+                      t = u;
+                      if constexpr (kStats) {
+                        const int v = off / (int)sizeof(Sum);
+                        const int vm = m0 + (v >> 3 & 7), vn = n0 + (v >> 6);
+                        const float2 ref = reinterpret_cast<const float2*>(
+                            st.ref)[(size_t)(l0 + (v & 7)) +
+                                    (size_t)jc * ((size_t)vm + (size_t)nsam * vn)];
+                        const float br = pv.x * box, bi = pv.y * box, ab = hypotf(br, bi);
+                        StatSum& q2 = S.st[wave][slot * kVox + v];
+                        q2.v += ab * ab;
+                        q2.a += ab;
+                        q2.p += pdiff_dev(br, bi, ref);
+                        q2.n++;
+                      }
+                    }
+                    wave_lds();  // another lane's next corner may be this voxel
+                  };
+                  if (!__any(X.t - X.s > 1 || Y.t - Y.s > 1 || Z.t - Z.s > 1)) {
+                    int ax[2], ay[2], az[2];
+                    float wx[2], wy[2], wz[2];
+#pragma unroll
+                    for (int k = 0; k < 2; k++) {
+                      ax[k] = inside ? X.off(k, l0, l1 - l0, 0, kB) : kOut;
+                      ay[k] = Y.off(k, ml, mh - ml, ms, kM);
+                      az[k] = Z.off(k, nl, nh - nl, ns, kN);
+                      wx[k] = 1.0f - fabsf(x3 - (float)(X.s + k));
+                      wy[k] = 1.0f - fabsf(y3 - (float)(Y.s + k));
+                      wz[k] = 1.0f - fabsf(z3 - (float)(Z.s + k));
+                    }
+                    // NKSUM; TTD's terms over the tile's corners, their weights
+                    // added per axis in 64 bits
+                    auto n2 = [](const int(&o)[2]) { return (o[0] < kOut) + (o[1] < kOut); };
+                    auto w2 = [](const int(&o)[2], const float(&f)[2]) {
+                      return (double)(o[0] < kOut ? f[0] : 0.f) +
+                             (double)(o[1] < kOut ? f[1] : 0.f);
+                    };
+                    const int nv = n2(ax) * n2(ay) * n2(az);
+                    cnt += nv;
+                    if (nv) ttd += (double)pv.z * w2(ax, wx) * w2(ay, wy) * w2(az, wz);
+#pragma unroll
+                    for (int kz = 0; kz < 2; kz++)
+#pragma unroll
+                      for (int ky = 0; ky < 2; ky++)
+#pragma unroll
+                        for (int kx = 0; kx < 2; kx++)
+                          corner(ax[kx] + ay[ky] + az[kz], wx[kx] * wy[ky], wz[kz]);
+                  } else {  // negative integers: three voxels on an axis
+                    for (int kz = 0; kz < 3; kz++)
+                      for (int ky = 0; ky < 3; ky++)
+                        for (int kx = 0; kx < 3; kx++) {
+                          const int off = (inside ? X.off(kx, l0, l1 - l0, 0, kB) : kOut) +
+                                          Y.off(ky, ml, mh - ml, ms, kM) +
+                                          Z.off(kz, nl, nh - nl, ns, kN);
+                          const float bx = 1.0f - fabsf(x3 - (float)(X.s + kx));
+                          const float by = 1.0f - fabsf(y3 - (float)(Y.s + ky));
+                          const float bz = 1.0f - fabsf(z3 - (float)(Z.s + kz));
+                          if (off < kOut) {
+                            cnt++;
+                            ttd += (double)pv.z * (double)bx * (double)by * (double)bz;
+                          }
+                          corner(off, bx * by, bz);
+                        }
+                  }
                 }
-                // I^2 + J^2 <= IRREC^2 (exact in FP32 at these sizes)
-                if (!in || ii + j * j > t.irrec2) continue;
-                const float b3 = 1.0f - fabsf(z3 - fn);
-                const float b2 = (1.0f - fabsf(y3 - fm));
-                const float box = (1.0f - fabsf(x3 - fl)) * b2 * b3;
-                const float4 pv = tp[(size_t)(j + jc - 1) * w + (i + jc - 1)];
-                const float cv = pv.z * box;
-                if (kStats) {
-                  const float br = pv.x * box, bi = pv.y * box;
-                  const float ab = hypotf(br, bi);
-                  sv += ab * ab;
-                  sa += ab;
-                  sp += pdiff_dev(br, bi, refv);
-                }
-                if (t.half) {
-                  a1r += pv.x * box;
-                  a1i += pv.y * box;
-                  a1c += cv;
-                  c1++;
-                  t1 += (double)cv;
-                } else {
-                  a0r += pv.x * box;
-                  a0i += pv.y * box;
-                  a0c += cv;
-                  c0++;
-                  t0 += (double)cv;
-                }
+                wave_lds();
+                if (rl < 8) S.flag[wave][slot][rl] = 0u;
+                wave_lds();
               }
             }
           }
+          cnt64 += cnt;
+          cnt = 0u;
+        }
       }
     }
-  }
-  if (mine) {
-    const size_t v = (size_t)l + (size_t)jc * ((size_t)ms_ + (size_t)nsam * ns_);
-    if (c0) {
-      float2 o = num0[v];
-      num0[v] = make_float2(o.x + a0r, o.y + a0i);
-      ctf2_0[v] += a0c;
+    if (!live) {
+      if (tid == 0) {
+        pcount[2 * (size_t)b + half] = 0;
+        pttd[2 * (size_t)b + half] = 0.0;
+      }
+      continue;
     }
-    if (c1) {
-      float2 o = num1[v];
-      num1[v] = make_float2(o.x + a1r, o.y + a1i);
-      ctf2_1[v] += a1c;
+    // the waves' sums in wave order, into the half-map
+    __syncthreads();
+    float2* num = half ? num1 : num0;
+    float* ctf2 = half ? ctf2_1 : ctf2_0;
+    for (int v = tid; v < kVox; v += kThreads) {
+      const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
+      float re = 0.f, im = 0.f, c2 = 0.f;
+      for (int q = 0; q < kWaves; q++)
+        for (int e = v; e < kSets * kVox; e += kVox) {
+          re += S.sum[q][e].re;
+          im += S.sum[q][e].im;
+          c2 += S.sum[q][e].c2;
+          if (kStats) S.sum[q][e] = Sum{0.f, 0.f, 0.f};
+        }
+      if (l < jc && m < nsam && n < nsam && (re != 0.f || im != 0.f || c2 != 0.f)) {
+        const size_t at = (size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n);
+        const float2 o = num[at];
+        num[at] = make_float2(o.x + re, o.y + im);
+        ctf2[at] += c2;
+      }
     }
-    if (kStats && (c0 | c1)) {
-      st.ksum[v] += (int)(c0 + c1);
-      st.vsum[v] += sv;
-      st.psum[v] += sp;
-      st.asum[v] += sa;
+    // the tile's NKSUM and TTD: a fixed reduction order
+    for (int off = 32; off > 0; off >>= 1) {
+      cnt64 += __shfl_xor(cnt64, off, 64);
+      ttd += __shfl_xor(ttd, off, 64);
+    }
+    if (lane == 0) {
+      S.rc[wave] = cnt64;
+      S.rt[wave] = ttd;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      unsigned long long uc = 0;
+      double ut = 0.0;
+      for (int q = 0; q < kWaves; q++) {
+        uc += S.rc[q];
+        ut += S.rt[q];
+      }
+      pcount[2 * (size_t)b + half] = uc;
+      pttd[2 * (size_t)b + half] = ut;
     }
   }
-  // the tile's NKSUM and TTD: a fixed reduction order
-  __shared__ unsigned long long rc[kGatherThreads / 64][2];
-  __shared__ double rt[kGatherThreads / 64][2];
-  unsigned long long u0 = c0, u1 = c1;
-  for (int off = 32; off > 0; off >>= 1) {
-    u0 += __shfl_xor(u0, off, 64);
-    u1 += __shfl_xor(u1, off, 64);
-    t0 += __shfl_xor(t0, off, 64);
-    t1 += __shfl_xor(t1, off, 64);
-  }
-  if (lane == 0) {
-    rc[wave][0] = u0;
-    rc[wave][1] = u1;
-    rt[wave][0] = t0;
-    rt[wave][1] = t1;
-  }
-  __syncthreads();
-  if (tid < 2) {
-    unsigned long long cc = 0;
-    double tt = 0.0;
-    for (int q = 0; q < kGatherThreads / 64; q++) {
-      cc += rc[q][tid];
-      tt += rt[q][tid];
+  if constexpr (kStats) {
+    if (!live) return;
+    for (int v = tid; v < kVox; v += kThreads) {
+      const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
+      float s2 = 0.f, sa = 0.f, sp = 0.f;
+      int k = 0;
+      for (int q = 0; q < kWaves; q++)
+        for (int e = v; e < kSets * kVox; e += kVox) {
+          s2 += S.st[q][e].v;
+          sa += S.st[q][e].a;
+          sp += S.st[q][e].p;
+          k += S.st[q][e].n;
+        }
+      if (l < jc && m < nsam && n < nsam && k) {
+        const size_t at = (size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n);
+        st.ksum[at] += k;
+        st.vsum[at] += s2;
+        st.psum[at] += sp;
+        st.asum[at] += sa;
+      }
     }
-    pcount[2 * (size_t)b + tid] = cc;
-    pttd[2 * (size_t)b + tid] = tt;
   }
 }
 
@@ -562,13 +722,9 @@ __global__ void __launch_bounds__(kReduceThreads)
 }  // namespace
 
 size_t insert_scratch_bytes(int nsam, int nb, int ntask) {
-  const int jc = nsam / 2 + 1, w = 2 * jc - 1;
   int tx, ty, tz;
   tile_counts(nsam, &tx, &ty, &tz);
-  const size_t ntiles = (size_t)tx * ty * tz;
-  return align256(sizeof(int) * (size_t)nb) + align256(sizeof(InsertGeo) * (size_t)ntask) +
-         align256(sizeof(float4) * (size_t)nb * w * w) +
-         align256(sizeof(unsigned long long) * 2 * ntiles) + align256(sizeof(double) * 2 * ntiles);
+  return scratch_layout(nullptr, nsam, nb, ntask, tx * ty * tz).bytes;
 }
 
 int launch_insert(Ctx& c, int nsam, int nb, int ntask, const InsertTask* d_tasks,
@@ -577,35 +733,36 @@ int launch_insert(Ctx& c, int nsam, int nb, int ntask, const InsertTask* d_tasks
                   void* scratch, const InsertStats* stats) {
   if (ntask <= 0 || nb <= 0) return 0;
   FR_CHECK(scratch != nullptr, "insertion scratch missing");
+  FR_CHECK(nb <= 65535, "too many particles in one insertion (%d)", nb);
   const int jc = nsam / 2 + 1, w = 2 * jc - 1;
   int tx, ty, tz;
   tile_counts(nsam, &tx, &ty, &tz);
   const int ntiles = tx * ty * tz;
   Scratch s = scratch_layout(scratch, nsam, nb, ntask, ntiles);
-  hipLaunchKernelGGL(k_first_clear, dim3((nb + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                     c.stream, nb, s.first);
+  hipLaunchKernelGGL(k_insert_order, dim3(1), dim3(1024), 0, c.stream, ntask, nb, d_tasks, s.first,
+                     s.ord, s.n0);
   FR_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_first_mark, dim3((ntask + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                     c.stream, ntask, nb, d_tasks, s.first);
-  FR_HIP(hipGetLastError());
-  FR_CHECK(nb <= 65535, "too many particles in one insertion (%d)", nb);
-  hipLaunchKernelGGL(k_insert_points, dim3((w * w + kThreads - 1) / kThreads, nb), dim3(kThreads),
-                     0, c.stream, nsam, s.first, d_tasks, reinterpret_cast<const float2*>(d_datc),
+  const int nt = (w + 15) / 16;
+  hipLaunchKernelGGL(k_insert_points, dim3(nt * nt, nb), dim3(kThreads), 0, c.stream, nsam,
+                     s.first, d_tasks, reinterpret_cast<const float2*>(d_datc),
                      reinterpret_cast<const float2*>(d_ctff), s.pts);
   FR_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_insert_geo, dim3((ntask + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                     c.stream, ntask, nsam, d_tasks, s.geo);
+                     c.stream, ntask, nb, nsam, d_tasks, s.ord, s.hit, s.rec);
   FR_HIP(hipGetLastError());
   if (stats) {
     FR_CHECK(stats->ref && stats->ksum && stats->vsum && stats->psum && stats->asum,
              "insertion statistics arrays missing");
-    hipLaunchKernelGGL(k_insert_gather<true>, dim3(ntiles), dim3(kGatherThreads), 0, c.stream,
-                       nsam, nb, ntask, tx, ty, d_tasks, s.geo, s.pts,
-                       reinterpret_cast<float2*>(num0), ctf2_0, reinterpret_cast<float2*>(num1),
-                       ctf2_1, s.pcount, s.pttd, *stats);
+    const size_t lds = sizeof(TileSums<true>);
+    FR_HIP(hipFuncSetAttribute((const void*)k_insert_scatter<true>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_insert_scatter<true>, dim3(ntiles), dim3(kThreads), lds, c.stream, nsam,
+                       ntask, tx, ty, tz, s.n0, s.hit, s.rec, s.pts, reinterpret_cast<float2*>(num0),
+                       ctf2_0, reinterpret_cast<float2*>(num1), ctf2_1, s.pcount, s.pttd, *stats);
   } else {
-    hipLaunchKernelGGL(k_insert_gather<false>, dim3(ntiles), dim3(kGatherThreads), 0, c.stream,
-                       nsam, nb, ntask, tx, ty, d_tasks, s.geo, s.pts,
+    const size_t lds = sizeof(TileSums<false>);
+    hipLaunchKernelGGL(k_insert_scatter<false>, dim3(2 * ntiles), dim3(kThreads), lds, c.stream,
+                       nsam, ntask, tx, ty, tz, s.n0, s.hit, s.rec, s.pts,
                        reinterpret_cast<float2*>(num0), ctf2_0, reinterpret_cast<float2*>(num1),
                        ctf2_1, s.pcount, s.pttd, InsertStats{});
   }
