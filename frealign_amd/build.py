@@ -28,6 +28,7 @@ SOURCES = [
     "fr_search.hip",
     "fr_lists.hip",
     "fr_search_sep.hip",
+    "fr_search_f32.hip",
     "fr_cnn.hip",
     "fr_refine.cpp",
     "fr_sigma.hip",

@@ -40,6 +40,12 @@ int launch_search_sep(Ctx& c, int np, int nbank, int nsamr, int nrow, const int*
                       const void* xa, const void* xb, const float* c2s, const float* sum2,
                       float* score, int* best_row, const int* fb = nullptr,
                       const int* ord = nullptr);
+// the exhaustive FP32 search with separable shifts (fr_search_f32.hip), MAXR2 <=
+// kSepMaxR2: the annulus bank (kc points of kidx, rows of kpad floats) against the
+// particle terms of launch_search_feats
+int launch_search_sep32(Ctx& c, int np, int norient, int maxr2, int kc, int kpad, int nsamr,
+                        const int* kidx, const void* bank, const float* ap, const float* c2,
+                        const float* sum2, float* score, int* best_row);
 int launch_topk(Ctx& c, int nbank, int np, int n, int group, const int* loff, const int* grp,
                 const int* cand, int cap, int topk, const float* score, const int* best_row,
                 int* top_o, int* top_row, float* top_s);

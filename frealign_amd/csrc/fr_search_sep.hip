@@ -31,6 +31,7 @@
 #include "fr_common.h"
 #include "fr_extract.h"
 #include "fr_search.h"
+#include "fr_search_dev.h"
 
 namespace fr {
 
@@ -44,7 +45,6 @@ constexpr int kSepElems = 2048;   // grid points per template (8 x 64 x 4)
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 // grid point of element e = (q * 64 + lane) * 4 + t of the separable layout
 __device__ inline void sep_point(int e, int& I, int& J) {
@@ -66,42 +66,6 @@ __device__ inline unsigned pack_bf16(float lo, float hi) {
 }
 
 __device__ inline bf16x2 as_bf2(unsigned u) { return *reinterpret_cast<bf16x2*>(&u); }
-
-// Wave-wide maximum and sum through DPP row operations (fixed order), the
-// result read from lane 63: a uniform value.
-template <int kCtrl, int kRowMask>
-__device__ inline float dpp_f(float old, float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), kCtrl,
-                                                    kRowMask, 0xF, false));
-}
-
-__device__ inline float wave_max(float v) {
-  const float lo = -3.4e38f;
-  v = fmaxf(v, dpp_f<0xB1, 0xF>(lo, v));   // quad_perm [1,0,3,2]
-  v = fmaxf(v, dpp_f<0x4E, 0xF>(lo, v));   // quad_perm [2,3,0,1]
-  v = fmaxf(v, dpp_f<0x141, 0xF>(lo, v));  // row_half_mirror
-  v = fmaxf(v, dpp_f<0x140, 0xF>(lo, v));  // row_mirror
-  v = fmaxf(v, dpp_f<0x142, 0xA>(lo, v));  // row_bcast15
-  v = fmaxf(v, dpp_f<0x143, 0xC>(lo, v));  // row_bcast31
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
-__device__ inline float wave_sum(float v) {
-  v += dpp_f<0xB1, 0xF>(0.f, v);
-  v += dpp_f<0x4E, 0xF>(0.f, v);
-  v += dpp_f<0x141, 0xF>(0.f, v);
-  v += dpp_f<0x140, 0xF>(0.f, v);
-  v += dpp_f<0x142, 0xA>(0.f, v);
-  v += dpp_f<0x143, 0xC>(0.f, v);
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
-// cos and sin of 2 pi (a mod n) / n: the argument reduced exactly first
-__device__ inline void phase(int a, int n, float& c, float& s) {
-  int r = a % n;
-  if (r < 0) r += n;
-  sincosf(6.283185307179586f * (float)r / (float)n, &s, &c);
-}
 
 // ------------------------------------------------------------------ bank
 __global__ void __launch_bounds__(256)
@@ -271,8 +235,11 @@ __global__ void __launch_bounds__(kSepThreads, 2)
     for (int q = 0; q < 8; q++) tv[q] = src[q * 64];
   };
 
-  // one (particle, template) pair: the 15 x 15 map, then ccp.f's epilogue
-  auto pair = [&](const uint4 (&tv)[8], float& sc, int& row) {
+  // one (particle, template) pair: the 15 x 15 map, then ccp.f's peak; kept in
+  // lane `at` until the chunk's scores are taken
+  float box_l = 0.f, norm_l = 0.f;
+  int row_l = 0;
+  auto pair = [&](const uint4 (&tv)[8], int at) {
     floatx4 acc1[2][2];
 #pragma unroll
     for (int a = 0; a < 2; a++)
@@ -321,39 +288,14 @@ __global__ void __launch_bounds__(kSepThreads, 2)
     floatx4 acc2;
 #pragma unroll
     for (int i = 0; i < 4; i++) acc2[i] = acc2h[0][i] + acc2h[1][i];
-    // lane (g, n) holds map[sx = 4 g + i][sy = n]; ccp.f:229-241: argmax over
-    // the inner 13 x 13, x outer, first maximum: the maximum value across the
-    // wave, then the first (sx, sy) holding it from the lanes' ballots
-    bool ok[4];
-    float m = -3.4e38f;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int sx = 4 * g + i;
-      ok[i] = sx >= 1 && sx <= 13 && n >= 1 && n <= 13;
-      if (ok[i]) m = fmaxf(m, acc2[i]);
+    float box;
+    int row;
+    ccp_peak(acc2, g, n, box, row);
+    if (lane == at) {
+      box_l = box;
+      norm_l = nacc;
+      row_l = row;
     }
-    m = wave_max(m);
-    unsigned long long hit[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) hit[i] = __ballot(ok[i] && acc2[i] == m);
-    int key = 7 * 16 + 7;  // no ordered value (NaN map): the centre
-#pragma unroll
-    for (int sx = 13; sx >= 1; sx--) {
-      const unsigned bits = (unsigned)(hit[sx & 3] >> (16 * (sx >> 2))) & 0xffffu;
-      if (bits) key = sx * 16 + __builtin_ctz(bits);
-    }
-    const int bx = key >> 4, by = key & 15;
-    // ccp.f:242-252: 3 x 3 box sum around the maximum
-    float box = 0.f;
-#pragma unroll
-    for (int dx = -1; dx <= 1; dx++) {
-      const int sxn = bx + dx, ii = sxn & 3;
-      const float v = ii == 0 ? acc2[0] : ii == 1 ? acc2[1] : ii == 2 ? acc2[2] : acc2[3];
-#pragma unroll
-      for (int dy = -1; dy <= 1; dy++) box += __shfl(v, (sxn >> 2) * 16 + by + dy, 64);
-    }
-    sc = (nacc > 0.f && s2 > 0.f) ? box / sqrtf(nacc) / sqrtf(s2) / 9.0f : -3.0e38f;
-    row = bx * 15 + by;
   };
 
   // persistent forms loop over their items; the uniform form is one item
@@ -387,13 +329,6 @@ __global__ void __launch_bounds__(kSepThreads, 2)
       pcur = it.p;
     }
     const int* cl = cand && it.listed ? cand + it.base : nullptr;
-    // the score of an empty column (zero map, no norm): the GEMM form's
-    auto put = [&](int pos, int o, float sc, int row) {
-      if (lane == 0) {
-        score[it.base + pos] = o >= 0 ? sc : -3.0e38f;
-        best_row[it.base + pos] = o >= 0 ? row : 16;
-      }
-    };
     for (int c0 = it.lo; c0 < it.hi; c0 += 64) {
       const int c1 = min(it.hi, c0 + 64);
       // the chunk's bank rows, one per lane, read ahead
@@ -408,22 +343,25 @@ __global__ void __launch_bounds__(kSepThreads, 2)
       load_t(t0, o0);
       // two positions per trip, the next template's loads in flight meanwhile
       for (int pos = c0; pos < c1; pos += 2) {
-        float sc;
-        int row;
         const bool two = pos + 1 < c1;
         if (two) {
           o1 = bank_row(pos + 1);
           load_t(t1, o1);
         }
-        pair(t0, sc, row);
-        put(pos, o0, sc, row);
+        pair(t0, pos - c0);
         if (!two) break;
         if (pos + 2 < c1) {
           o0 = bank_row(pos + 2);
           load_t(t0, o0);
         }
-        pair(t1, sc, row);
-        put(pos + 1, o1, sc, row);
+        pair(t1, pos + 1 - c0);
+      }
+      // a column outside the bank scores as an empty one (zero map, no norm):
+      // the GEMM form's
+      if (c0 + lane < c1) {
+        const size_t e = (size_t)it.base + c0 + lane;
+        score[e] = mine >= 0 ? ccp_score(box_l, norm_l, s2) : -3.0e38f;
+        best_row[e] = mine >= 0 ? row_l : 16;
       }
     }
   }
