@@ -63,6 +63,7 @@ constexpr int kVox = kTile * kTile * kTile;
 constexpr int kWaves = 4;        // per tile
 constexpr int kSets = 2;         // tasks a wave takes at a time, each with sums of its own
 constexpr int kLanes = 64 / kSets;
+constexpr int kSplit = 8;        // shorter task lists are split by classes
 constexpr int kList = kThreads;  // tasks tested per pass
 constexpr int kReduceThreads = 1024;
 static_assert(kThreads == 64 * kWaves && kSets == 2, "32 lanes per set of sums");
@@ -354,6 +355,7 @@ struct TileSums {
   int tot[kWaves];
   int2 row[kWaves][kSets][kLanes];     // I | first J << 16, start
   unsigned flag[kWaves][kSets][8];     // a bit where a row starts
+  unsigned live[kWaves];
   unsigned long long rc[kWaves];
   double rt[kWaves];
 };
@@ -383,7 +385,8 @@ __global__ void __launch_bounds__(kThreads)
   int mlo[2], mhi[2], nlo[2], nhi[2];
   const int nmr = logical_ranges(m0, min(m0 + kTile - 1, nsam - 1), nsam, mlo, mhi);
   const int nnr = logical_ranges(n0, min(n0 + kTile - 1, nsam - 1), nsam, nlo, nhi);
-  bool live = false;  // a plane reaches the tile: the waves' sums are set up
+  unsigned live = 0u;  // this wave's sets that are set up, a bit each
+  bool any = false;    // a plane reaches the tile
   const int rl = lane & (kLanes - 1), slot = lane / kLanes;
   const unsigned long long lt = (1ull << lane) - 1ull;
   char* const set = reinterpret_cast<char*>(&S.sum[wave][slot * kVox]);
@@ -422,17 +425,23 @@ __global__ void __launch_bounds__(kThreads)
         }
         if (on) S.list[before + __popcll(bal & lt)] = k;
         __syncthreads();
-        if (nlist && !live) {  // each wave its own
-          live = true;
-          for (int e = lane; e < kSets * kVox; e += 64) {
-            S.sum[wave][e] = Sum{0.f, 0.f, 0.f};
-            if constexpr (kStats) S.st[wave][e] = StatSum{0.f, 0.f, 0.f, 0};
+        // This wave's quarter of the tasks, two at a time.  A short list is split by
+        // the classes of its points instead, a class (of each four) to a wave: one
+        // wave at work would leave a CU, which holds three tiles, nearly idle.
+        const bool split = nlist < kSplit;
+        const int q0 = split ? 0 : nlist * wave / kWaves;
+        const int q1 = split ? nlist : nlist * (wave + 1) / kWaves;
+        any |= nlist != 0;
+        if (!live && q0 < q1 && rl < 8) S.flag[wave][slot][rl] = 0u;
+        for (int k = 0; k < min(q1 - q0, kSets); k++)
+          if (!(live >> k & 1)) {
+            live |= 1u << k;
+            for (int e = lane; e < kVox; e += 64) {
+              S.sum[wave][k * kVox + e] = Sum{0.f, 0.f, 0.f};
+              if constexpr (kStats) S.st[wave][k * kVox + e] = StatSum{0.f, 0.f, 0.f, 0};
+            }
           }
-          if (rl < 8) S.flag[wave][slot][rl] = 0u;
-          wave_lds();
-        }
-        // this wave's quarter, four tasks at a time
-        const int q0 = nlist * wave / kWaves, q1 = nlist * (wave + 1) / kWaves;
+        wave_lds();
         for (int qb = q0; qb < q1; qb += kSets) {
           const int q = qb + slot;
           const float4* R = rec + (size_t)S.list[min(q, q1 - 1)] * kRec;
@@ -480,7 +489,7 @@ __global__ void __launch_bounds__(kThreads)
             }
             const int imod = nc == 2 ? i & 1 : (i + nc * 1024) % nc;
             const int jmod = nc == 2 ? j0 & 1 : (j0 + nc * 1024) % nc;
-            for (int cls = 0; cls < nc * nc; cls++) {
+            for (int cls = split ? wave : 0; cls < nc * nc; cls += split ? kWaves : 1) {
               const int ca = nc == 2 ? cls & 1 : cls % nc, cb = nc == 2 ? cls >> 1 : cls / nc;
               const int f0 = j0 + (cb >= jmod ? cb - jmod : cb - jmod + nc);
               int c = 0;
@@ -604,7 +613,7 @@ __global__ void __launch_bounds__(kThreads)
         }
       }
     }
-    if (!live) {
+    if (!any) {
       if (tid == 0) {
         pcount[2 * (size_t)b + half] = 0;
         pttd[2 * (size_t)b + half] = 0.0;
@@ -612,6 +621,7 @@ __global__ void __launch_bounds__(kThreads)
       continue;
     }
     // the waves' sums in wave order, into the half-map
+    if (lane == 0) S.live[wave] = live;
     __syncthreads();
     float2* num = half ? num1 : num0;
     float* ctf2 = half ? ctf2_1 : ctf2_0;
@@ -620,6 +630,7 @@ __global__ void __launch_bounds__(kThreads)
       float re = 0.f, im = 0.f, c2 = 0.f;
       for (int q = 0; q < kWaves; q++)
         for (int e = v; e < kSets * kVox; e += kVox) {
+          if (!(S.live[q] >> (e / kVox) & 1)) continue;
           re += S.sum[q][e].re;
           im += S.sum[q][e].im;
           c2 += S.sum[q][e].c2;
@@ -654,13 +665,14 @@ __global__ void __launch_bounds__(kThreads)
     }
   }
   if constexpr (kStats) {
-    if (!live) return;
+    if (!any) return;
     for (int v = tid; v < kVox; v += kThreads) {
       const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
       float s2 = 0.f, sa = 0.f, sp = 0.f;
       int k = 0;
       for (int q = 0; q < kWaves; q++)
         for (int e = v; e < kSets * kVox; e += kVox) {
+          if (!(S.live[q] >> (e / kVox) & 1)) continue;
           s2 += S.st[q][e].v;
           sa += S.st[q][e].a;
           sp += S.st[q][e].p;
