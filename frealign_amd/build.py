@@ -22,6 +22,7 @@ SOURCES = [
     "fr_prep.hip",
     "fr_extract.hip",
     "fr_cc3m.hip",
+    "fr_cc3m_fft.hip",
     "fr_insert.hip",
     "fr_final.hip",
     "fr_stats.hip",

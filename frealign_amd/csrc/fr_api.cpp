@@ -243,6 +243,21 @@ int fr_ctx::cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t) {
   return 0;
 }
 
+int fr_ctx::cc3m_ring(int nsam, int maxr2, float ri2, float ri3, fr::Cc3mRing* t) {
+  const auto k = std::make_tuple(nsam, maxr2, ri2, ri3);
+  auto i = ring_hats.find(k);
+  if (i == ring_hats.end()) {
+    std::vector<float> h;
+    RingTab rt;
+    rt.cnt = fr::cc3m_ring_hat(nsam, ri2, ri3, maxr2, h);
+    if (int r = upload_table(h, &rt.d)) return r;
+    i = ring_hats.emplace(k, rt).first;
+  }
+  t->rhat = i->second.d;
+  t->cnt = i->second.cnt;
+  return 0;
+}
+
 fr_ctx::Tune fr_ctx::tune_for(int nsam) const {
   auto it = tune.find(nsam);
   return it == tune.end() ? Tune{} : it->second;
@@ -315,6 +330,7 @@ int fr_destroy(fr_ctx* c) {
   if (c->hpin) (void)hipHostFree(c->hpin);
   if (c->d_kidx) (void)hipFree(c->d_kidx);
   for (auto& e : c->dft_tabs) (void)hipFree(e.second);
+  for (auto& e : c->ring_hats) (void)hipFree(e.second.d);
   for (auto& e : c->band_dft_tabs) (void)hipFree(e.second);
   for (auto& e : c->band_pair_tabs) (void)hipFree(e.second);
   for (auto& e : c->band_wmap_tabs) (void)hipFree(e.second);
@@ -445,6 +461,17 @@ int fr_cc3_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d
 
 }  // extern "C"
 
+namespace {
+// items per launch of the particle-grid form: its band stays within 192 MB, so
+// that it is read back from the 256 MB cache
+int fft_chunk(int nsam, int maxr2, int n) {
+  const size_t one = fr::cc3m_fft_bytes(nsam, maxr2, 1);
+  const size_t most = ((size_t)192 << 20) / one;
+  const int step = most < 1 ? 1 : most > 65535 ? 65535 : (int)most;
+  return n < step ? n : step;
+}
+}  // namespace
+
 namespace fr {
 int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                const float* d_ctff, const int* d_pidx, const float* d_dm, const float* d_shift,
@@ -460,9 +487,12 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
   Cc3mArgs a{nsam, 0, maxr1, maxr2, rbfact, ring[0], ring[1], ring[2], ring[3]};
   a.cc3 = cc3;
   const fr_ctx::Tune tn = c->tune_for(nsam);
-  if (fr::cc3m_fused_ok(nsam, maxr2) && tn.cc3m_fused) {
-    // the items with AMAG = 1 on the band's own grid, the others (unless there
-    // are none) on the NSAM grid
+  // The items with AMAG = 1 go to the band's own grid, the others (unless there
+  // are none) to the NSAM-grid products, which hold their boxes only.  Any other
+  // box with a band that the grid holds goes there where every AMAG is known to
+  // be 1.
+  const bool any_box = unit_amag && maxr2 <= 32 && maxr2 < nsam / 2;
+  if ((fr::cc3m_fused_ok(nsam, maxr2) || any_box) && tn.cc3m_fused) {
     Cc3mTables tabs;
     Cc3mBandTables band;
     if (int r = c->cc3m_band_tables(a, &band)) return r;
@@ -484,18 +514,18 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
     c->prof_end(pslot);
     return 0;
   }
-  const size_t img = (size_t)nsam * (nsam + 2);
-  // process in chunks so the FFT work buffer stays bounded
-  const int chunk = (int)((size_t)512 * 1024 * 1024 / (img * sizeof(float)));
-  const int step = chunk < 1 ? 1 : (chunk > 65535 ? 65535 : chunk);
+  FR_CHECK(maxr2 < nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", maxr2);
+  Cc3mRing rt;
+  if (int r = c->cc3m_ring(nsam, maxr2, a.ri2, a.ri3, &rt)) return r;
+  const int step = fft_chunk(nsam, maxr2, n);
   int err = 0;
-  float* work = (float*)c->slot(0, img * sizeof(float) * (size_t)(n < step ? n : step), &err);
+  void* work = c->slot(0, fr::cc3m_fft_bytes(nsam, maxr2, step), &err);
   if (!work) return err;
   int pslot = c->prof_begin(kProfCc3m);
   for (int o = 0; o < n; o += step) {
     a.n = n - o < step ? n - o : step;
     if (int r = launch_cc3m(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o, d_dm + 9 * (size_t)o,
-                            d_shift + 2 * (size_t)o, d_amag + o, d_fsct, work, d_score + o))
+                            d_shift + 2 * (size_t)o, d_amag + o, d_fsct, rt, work, d_score + o))
       return r;
   }
   c->prof_end(pslot);
@@ -515,17 +545,17 @@ int fr_presb_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float*
            "null argument");
   FR_CHECK(ring[3] != 0.0f, "HALFW must be non-zero");
   if (n == 0) return 0;
-  const size_t img = (size_t)nsam * (nsam + 2);
-  const int chunk = (int)((size_t)512 * 1024 * 1024 / (img * sizeof(float)));
-  const int step = chunk < 1 ? 1 : (chunk > 65535 ? 65535 : chunk);
+  Cc3mRing rt;
+  if (int r = c->cc3m_ring(nsam, nsam / 2, ring[0], ring[1], &rt)) return r;
+  const int step = fft_chunk(nsam, nsam / 2, n);
   int err = 0;
-  float* work = (float*)c->slot(0, img * sizeof(float) * (size_t)(n < step ? n : step), &err);
+  void* work = c->slot(0, fr::cc3m_fft_bytes(nsam, nsam / 2, step), &err);
   if (!work) return err;
   for (int o = 0; o < n; o += step) {
     int m = n - o < step ? n - o : step;
     if (int r = launch_presb(*c, nsam, m, d_a3df, d_spec, d_ctff, d_pidx + o, d_dm + 9 * (size_t)o,
                              d_shift + 2 * (size_t)o, d_amag + o, ring[0], ring[1], ring[2],
-                             ring[3], work, d_rbin + (size_t)o * nsam))
+                             ring[3], rt, work, d_rbin + (size_t)o * nsam))
       return r;
   }
   return 0;

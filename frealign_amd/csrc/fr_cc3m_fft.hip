@@ -1,0 +1,533 @@
+// fr_cc3m_fft.hip -- CC3M (cc3m.f:8-169) and PRESB (presb.f:8-160) on the
+// particle's grid, for any box, band and AMAG.
+//
+// The section lives on the columns I < MAXR2 of the half-plane only, before and
+// after the mask, so only those are held (a band of CB columns, a multiple of 8)
+// and each step goes over them once:
+//   k_band_cols   gathers 8 columns of an item's section times the CTF straight
+//                 into LDS and runs their backward column FFT
+//   k_band_mean   MASKCOS2's ring mean per item.  The ring sum is linear in the
+//                 section: sum of w_I Re X(I, J) Rhat(I, J), Rhat the transform of
+//                 the ring's pixels, formed in k_band_cols (AMAG = 1); an item of
+//                 another AMAG takes its rows to real space here
+//   k_band_rows   row c2r, (x - mean) w, row r2c, in LDS.  The mean's own term is
+//                 the DC point, which no shell counts
+//   k_band_sums   forward column FFT of 8 columns and their part of the shell sums:
+//                 shell s is s^2-s+1 <= r^2 <= s^2+s, a run of J per column, so a
+//                 thread takes a shell's points of one sign of J in order
+//   k_band_score  the shells of an item, the columns' parts in order
+// Sums run in a fixed order: a rerun gives the same bits.
+//
+// What bounds it: the band goes through memory as write, read, write, read (512
+// items of a 320 box at MAXR2 = 80: 105 MB each time) and its FFTs through LDS;
+// before, whole half-planes went through it twelve times.  That call: 1,122 us as
+// whole planes, now 444.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <type_traits>
+#include <vector>
+
+#include "fr_common.h"
+#include "fr_extract.h"
+#include "fr_fft_dev.h"
+#include "fr_kernels.h"
+
+namespace fr {
+
+namespace {
+
+using namespace fftdev;
+constexpr int kThr = kFftThreads;
+constexpr int kCw = 8;  // columns per workgroup
+constexpr float kPi = 3.1415926535897f;
+
+struct Band {
+  int nsam, nitem, cb, jmax, maxr12, maxr22, nsh;
+  float ri2, ri3, rih, halfw;
+  int flip;
+};
+
+constexpr int rows_nseq(int n) { return n >= 1024 ? 2 : 2048 / n; }
+
+// N > 0: the length is known at compile time (NS sequences of pitch N + 1)
+template <int N, int NS, int SIGN>
+__device__ inline float2* fft_any(float2* buf, float2* tmp, const Plan& pl, int nseq,
+                                  const float2* __restrict__ tw) {
+  if constexpr (N > 0) return lds_fft_t<N, NS, N + 1, SIGN>(buf, tmp, tw);
+  else return lds_fft(buf, tmp, pl, pl.n + 1, nseq, SIGN, tw);
+}
+
+template <int N>
+__global__ void __launch_bounds__(kThr)
+    k_band_cols(Band b, Plan pl, const float2* __restrict__ a3df, const float* __restrict__ dm,
+                const int* __restrict__ pidx, const float2* __restrict__ ctff,
+                const float* __restrict__ rhat, float2* __restrict__ work,
+                float* __restrict__ part, const float2* __restrict__ tw) {
+  extern __shared__ float2 smem[];
+  __shared__ float red[kThr / 64];
+  const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
+  const size_t ic = (size_t)n * jc;
+  float2 *buf = smem, *tmp = smem + kCw * ld;
+  // an item's column blocks in XCD-contiguous order: they share lines
+  const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
+  const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
+  if (it >= b.nitem) return;
+  for (int e = threadIdx.x; e < kCw * ld; e += kThr) buf[e] = make_float2(0.f, 0.f);
+  __syncthreads();
+  const float* d = dm + 9 * (size_t)it;
+  const float2* cp = ctff + (size_t)pidx[it] * 2 * ic;
+  const float scal = 1.0f / (float)n / (float)n;
+  const bool inner = ainterpo_inner(jc, d, b.jmax + 1);
+  float rsum = 0.f;
+#pragma unroll 2
+  for (int e = threadIdx.x; e < kCw * (2 * b.jmax + 1); e += kThr) {
+    const int i = x0 + (e & (kCw - 1)), j = e / kCw - b.jmax, r2 = i * i + j * j;
+    if (r2 < b.maxr12 || r2 >= b.maxr22) continue;
+    const size_t id = (size_t)i + (size_t)jc * wrapn(j, n);
+    const float2 cr = cp[id], cl = cp[id + ic];
+    cf a = inner ? ainterpo_inner_dev(n, jc, a3df, d, i, j) : ainterpo_dev(n, a3df, d, i, j);
+    if (b.flip) {  // cc3.f:86-89
+      if (cr.x + cl.x < 0.0f) a = cf{-a.re, -a.im};
+    } else {
+      a = cmul(a, cf{cr.x + cl.x, cr.y - cl.y});
+    }
+    a = cscale(a, scal);
+    buf[(e & (kCw - 1)) * ld + wrapn(j, n)] = make_float2(a.re, a.im);
+    rsum += (i ? 2.0f : 1.0f) * a.re * rhat[(size_t)abs(j) * b.cb + i];
+  }
+  for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rsum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float s = 0.f;
+    for (int q = 0; q < kThr / 64; q++) s += red[q];
+    part[lb] = s;
+  }
+  const float2* res = fft_any<N, kCw, +1>(buf, tmp, pl, kCw, tw);
+  float2* out = work + (size_t)it * n * b.cb + x0;
+  for (int e = threadIdx.x; e < n * kCw; e += kThr)
+    out[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))] = res[(e & (kCw - 1)) * ld + e / kCw];
+}
+
+// the half spectra of rows 2q and 2q+1 as one sequence: Z_k = A_k + i B_k,
+// Z_{n-k} = conj(A_k) + i conj(B_k), the imaginary parts at k = 0 ignored as the
+// c2r does
+__device__ inline void load_pair(float2* z, const float2* ra, int n, int cb, int k) {
+  float2 a = make_float2(0.f, 0.f), c = a;
+  if (k < cb) {
+    a = ra[k];
+    c = ra[cb + k];
+  }
+  if (k == 0 || 2 * k == n) a.y = c.y = 0.f;
+  z[k] = make_float2(a.x - c.y, a.y + c.x);
+  if (k > 0 && 2 * k < n) z[n - k] = make_float2(a.x + c.y, -a.y + c.x);
+}
+
+// squared wrapped distances of MASKCOS2 (origin 1)
+__device__ inline float wrap2(int v, int n) {
+  const int d = v < n / 2 ? v : v - n;
+  return (float)(d * d);
+}
+
+template <int N>
+__global__ void __launch_bounds__(kThr)
+    k_band_mean(Band b, Plan pl, const float2* __restrict__ work, const float* __restrict__ part,
+                int ring_cnt, const float* __restrict__ amag, float* __restrict__ mean,
+                const float2* __restrict__ tw) {
+  extern __shared__ float2 smem[];
+  __shared__ float red[kThr / 64];
+  __shared__ int redc[kThr / 64];
+  const int n = N ? N : pl.n, ld = n + 1, it = blockIdx.x, nblk = b.cb / kCw;
+  const float am = amag[it];
+  if (am == 1.0f) {
+    if (threadIdx.x == 0) {
+      float s = 0.f;
+      for (int q = 0; q < nblk; q++) s += part[(size_t)it * nblk + q];
+      mean[it] = ring_cnt ? s / (float)ring_cnt : s;
+    }
+    return;
+  }
+  const float ri2p = b.ri2 / am / am, ri3p = b.ri3 / am / am;
+  const int nseq = rows_nseq(n);
+  float2 *buf = smem, *tmp = smem + nseq * ld;
+  float s = 0.f;
+  int cnt = 0;
+  for (int q0 = 0; q0 < n / 2; q0 += nseq) {
+    for (int e = threadIdx.x; e < nseq * (n / 2 + 1); e += kThr) {
+      const int q = e / (n / 2 + 1), k = e - q * (n / 2 + 1);
+      if (q0 + q < n / 2)
+        load_pair(buf + q * ld, work + ((size_t)it * n + 2 * (q0 + q)) * b.cb, n, b.cb, k);
+    }
+    __syncthreads();
+    const float2* res = fft_any<N, N ? rows_nseq(N ? N : 1) : 1, +1>(buf, tmp, pl, nseq, tw);
+    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+      const int q = e / n, x = e - q * n, row = 2 * (q0 + q);
+      if (row >= n) continue;
+      const float2 z = res[q * ld + x];
+      const float ra = wrap2(x, n) + wrap2(row, n), rc = wrap2(x, n) + wrap2(row + 1, n);
+      if (ra > ri2p && ra <= ri3p) s += z.x, cnt++;
+      if (rc > ri2p && rc <= ri3p) s += z.y, cnt++;
+    }
+    __syncthreads();
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    cnt += __shfl_xor(cnt, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = s;
+    redc[threadIdx.x >> 6] = cnt;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s = 0.f;
+    cnt = 0;
+    for (int q = 0; q < kThr / 64; q++) s += red[q], cnt += redc[q];
+    mean[it] = cnt ? s / (float)cnt : s;
+  }
+}
+
+template <int N>
+__global__ void __launch_bounds__(kThr)
+    k_band_rows(Band b, Plan pl, float2* __restrict__ work, const float* __restrict__ amag,
+                const float* __restrict__ mean, const float2* __restrict__ tw) {
+  extern __shared__ float2 smem[];
+  const int n = N ? N : pl.n, ld = n + 1, nh = n / 2, nseq = rows_nseq(n);
+  float2 *buf = smem, *tmp = smem + nseq * ld;
+  const int pair0 = blockIdx.x * nseq, npairs = b.nitem * nh;
+  for (int e = threadIdx.x; e < nseq * (nh + 1); e += kThr) {
+    const int q = e / (nh + 1), k = e - q * (nh + 1);
+    if (pair0 + q < npairs)  // rows of consecutive pairs are consecutive, over items too
+      load_pair(buf + q * ld, work + (size_t)(pair0 + q) * 2 * b.cb, n, b.cb, k);
+  }
+  __syncthreads();
+  float2* res = fft_any<N, N ? rows_nseq(N ? N : 1) : 1, +1>(buf, tmp, pl, nseq, tw);
+  for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+    const int q = e / n, x = e - q * n, pr = pair0 + q;
+    if (pr >= npairs) continue;
+    const int it = pr / nh, row = 2 * (pr - it * nh);
+    const float am = amag[it], mu = mean[it];
+    const float ri2p = b.ri2 / am / am, ri3p = b.ri3 / am / am, rihp = b.rih / am;
+    auto weight = [&](float r2) {
+      if (r2 > ri3p) return 0.0f;
+      if (r2 > ri2p) return (1.0f + cosf(kPi * (sqrtf(r2) - rihp) / b.halfw)) / 2.0f;
+      return 1.0f;
+    };
+    const float dx = wrap2(x, n);
+    const float2 z = res[q * ld + x];
+    res[q * ld + x] = make_float2((z.x - mu) * weight(dx + wrap2(row, n)),
+                                  (z.y - mu) * weight(dx + wrap2(row + 1, n)));
+  }
+  __syncthreads();
+  const float2* out =
+      fft_any<N, N ? rows_nseq(N ? N : 1) : 1, -1>(res, res == buf ? tmp : buf, pl, nseq, tw);
+  for (int e = threadIdx.x; e < nseq * b.cb; e += kThr) {
+    const int q = e / b.cb, k = e - q * b.cb;
+    if (pair0 + q >= npairs) continue;
+    const float2 zk = out[q * ld + k], zm = out[q * ld + (k ? n - k : 0)];
+    float2* ra = work + (size_t)(pair0 + q) * 2 * b.cb + k;
+    ra[0] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
+    ra[b.cb] = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
+  }
+}
+
+// largest j >= 0 with j*j <= v (v >= 0, below 2^20)
+__device__ inline int isqrt(int v) {
+  int j = (int)sqrtf((float)v);
+  if (j * j > v) j--;
+  if ((j + 1) * (j + 1) <= v) j++;
+  return j;
+}
+
+template <int N>
+__global__ void __launch_bounds__(kThr)
+    k_band_sums(Band b, Plan pl, const float2* __restrict__ work, const float2* __restrict__ spec,
+                const int* __restrict__ pidx, const float* __restrict__ shift,
+                float4* __restrict__ psum, const float2* __restrict__ tw) {
+  extern __shared__ float2 smem[];
+  const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
+  float2 *buf = smem, *tmp = smem + kCw * ld;
+  float2* ey = smem + 2 * kCw * ld;  // e^{i SHY J}, J = 0 .. jmax
+  __shared__ float2 ex[kCw];
+  const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
+  const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
+  if (it >= b.nitem) return;
+  const float2* in = work + (size_t)it * n * b.cb + x0;
+  for (int e = threadIdx.x; e < n * kCw; e += kThr)
+    buf[(e & (kCw - 1)) * ld + e / kCw] = in[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))];
+  const float shx = shift[2 * it], shy = shift[2 * it + 1];
+  for (int j = threadIdx.x; j <= b.jmax; j += kThr) {
+    float sn, cs;
+    sincosf(shy * (float)j, &sn, &cs);
+    ey[j] = make_float2(cs, sn);
+  }
+  if (threadIdx.x < kCw) {
+    float sn, cs;
+    sincosf(shx * (float)(x0 + (int)threadIdx.x), &sn, &cs);
+    ex[threadIdx.x] = make_float2(cs, sn);
+  }
+  __syncthreads();
+  float2* res = fft_any<N, kCw, -1>(buf, tmp, pl, kCw, tw);
+  float2* pt = res == buf ? tmp : buf;  // per point (REAL(SAMP CONJG(AINPO)), |SAMP|^2)
+  const float2* sp = spec + (size_t)pidx[it] * n * jc;
+  for (int e = threadIdx.x; e < kCw * (2 * b.jmax + 1); e += kThr) {
+    const int c = e & (kCw - 1), i = x0 + c, j = e / kCw - b.jmax, r2 = i * i + j * j;
+    if (r2 < b.maxr12 || r2 >= b.maxr22) continue;
+    const int row = wrapn(j, n);
+    const float2 s = sp[(size_t)i + (size_t)jc * row], a = res[c * ld + row];
+    const float2 u = ex[c], v = ey[abs(j)];
+    const float vs = j < 0 ? -v.y : v.y;
+    const float cs = u.x * v.x - u.y * vs, sn = u.x * vs + u.y * v.x;
+    const float re = s.x * a.x + s.y * a.y, im = s.y * a.x - s.x * a.y;
+    pt[c * ld + row] = make_float2(re * cs - im * sn, s.x * s.x + s.y * s.y);
+  }
+  __syncthreads();
+  for (int base = 0; base < 2 * b.nsh; base += kThr) {
+    const int e = base + threadIdx.x, s = e >> 1, neg = e & 1;
+    float q = 0.f, s2 = 0.f, a2 = 0.f, cnt = 0.f;
+    if (s < b.nsh) {
+      for (int c = 0; c < kCw; c++) {
+        const int i = x0 + c;
+        const int hi = min(s * s + s, b.maxr22 - 1) - i * i;
+        if (hi < 0) break;
+        const int lo = max(s ? s * s - s + 1 : 0, b.maxr12) - i * i;
+        const int j1 = isqrt(hi);
+        int j0 = lo > 0 ? isqrt(lo - 1) + 1 : 0;
+        if (neg) j0 = max(j0, 1);
+        for (int j = j0; j <= j1; j++) {
+          const int at = c * ld + (neg ? n - j : j);
+          const float2 p = pt[at], a = res[at];
+          q += p.x;
+          s2 += p.y;
+          a2 += a.x * a.x + a.y * a.y;
+          cnt += 1.0f;
+        }
+      }
+    }
+    q += __shfl_xor(q, 1, 64);
+    s2 += __shfl_xor(s2, 1, 64);
+    a2 += __shfl_xor(a2, 1, 64);
+    cnt += __shfl_xor(cnt, 1, 64);
+    if (s < b.nsh && !neg) psum[(size_t)lb * b.nsh + s] = make_float4(q, s2, a2, cnt);
+  }
+}
+
+__device__ inline float4 shell(const float4* psum, const Band& b, int it, int s) {
+  const int nblk = b.cb / kCw;
+  float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = 0; k < nblk; k++) {
+    const float4 p = psum[((size_t)it * nblk + k) * b.nsh + s];
+    t.x += p.x;
+    t.y += p.y;
+    t.z += p.z;
+    t.w += p.w;
+  }
+  return t;
+}
+
+// cc3m.f:139-167 over shells 1 .. NSAM/2-1: one wave per item, FP64 sums reduced
+// by a fixed butterfly
+__global__ void __launch_bounds__(64)
+    k_band_score(Band b, float rbfact, const float4* __restrict__ psum,
+                 const float* __restrict__ fsct, float* __restrict__ score) {
+  const int it = blockIdx.x, lane = threadIdx.x;
+  double s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  for (int s = 1 + lane; s < min(b.nsam / 2, b.nsh); s += 64) {
+    const float4 t = shell(psum, b, it, s);
+    if (t.w == 0.0f) continue;
+    float r = t.x / sqrtf(t.z);
+    if (!b.flip && fsct[s] < 0.95f) r = fabsf(r);
+    const float wgt = expf(-rbfact * (float)(s * s));
+    s3 += (double)(r * wgt);
+    s2 += (double)(wgt * wgt * t.y);
+    s1 += 1.0;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    s1 += __shfl_xor(s1, off, 64);
+    s2 += __shfl_xor(s2, off, 64);
+    s3 += __shfl_xor(s3, off, 64);
+  }
+  if (lane == 0) {
+    if (s1 * s2 != 0.0) s3 = s3 / sqrt(s1 * s2);
+    score[it] = (float)s3;
+  }
+}
+
+// presb.f:95-123: per-shell correlation; shells with no point leave RBIN untouched
+__global__ void __launch_bounds__(64)
+    k_band_presb(Band b, const float4* __restrict__ psum, float* __restrict__ rbin) {
+  const int it = blockIdx.x;
+  float* rb = rbin + (size_t)it * b.nsam;
+  for (int s = threadIdx.x; s < min(b.nsam / 2, b.nsh); s += 64) {
+    const float4 t = shell(psum, b, it, s);
+    if (t.w == 0.0f) continue;
+    rb[2 * s] = t.x / sqrtf(t.y * t.z);
+    rb[2 * s + 1] = 1.0f;
+  }
+}
+
+int band_cb(int maxr2) { return (maxr2 + kCw - 1) / kCw * kCw; }
+int band_nsh(int maxr2) { return maxr2 + 1; }
+
+struct BandWork {
+  float2* band;
+  float4* psum;
+  float *part, *mean;
+};
+
+size_t align16(size_t b) { return (b + 15) & ~(size_t)15; }
+
+BandWork band_work(void* base, int nsam, int maxr2, size_t n, size_t* bytes) {
+  const size_t cb = band_cb(maxr2), nblk = cb / kCw;
+  char* p = static_cast<char*>(base);
+  size_t o = 0;
+  BandWork w;
+  auto take = [&](auto*& q, size_t k) {
+    q = reinterpret_cast<std::remove_reference_t<decltype(q)>>(p + o);
+    o += align16(sizeof(*q) * k);
+  };
+  take(w.band, n * nsam * cb);
+  take(w.psum, n * nblk * band_nsh(maxr2));
+  take(w.part, n * nblk);
+  take(w.mean, n);
+  *bytes = o;
+  return w;
+}
+
+struct BandCall {
+  const float *a3df, *spec, *ctff;
+  const int* pidx;
+  const float *dm, *shift, *amag;
+};
+
+template <int N>
+int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, const BandWork& w) {
+  Plan pl;
+  FR_CHECK(make_plan(b.nsam, &pl), "FFT length %d not supported", b.nsam);
+  const float2* tw = c.twiddles(b.nsam);
+  FR_CHECK(tw != nullptr, "twiddle table allocation failed");
+  const int n = b.nsam, nseq = rows_nseq(n);
+  const int cols = round8(b.nitem * (b.cb / kCw)), npairs = b.nitem * (n / 2);
+  const size_t lc = sizeof(float2) * 2 * kCw * (n + 1), lr = sizeof(float2) * 2 * nseq * (n + 1);
+  const size_t ls = lc + sizeof(float2) * (b.jmax + 1);
+  auto big = [](const void* fn, size_t lds) {
+    return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  };
+  FR_HIP(big((const void*)k_band_cols<N>, lc));
+  FR_HIP(big((const void*)k_band_mean<N>, lr));
+  FR_HIP(big((const void*)k_band_rows<N>, lr));
+  FR_HIP(big((const void*)k_band_sums<N>, ls));
+  hipLaunchKernelGGL(k_band_cols<N>, dim3(cols), dim3(kThr), lc, c.stream, b, pl,
+                     reinterpret_cast<const float2*>(p.a3df), p.dm, p.pidx,
+                     reinterpret_cast<const float2*>(p.ctff), ring.rhat, w.band, w.part, tw);
+  FR_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_band_mean<N>, dim3(b.nitem), dim3(kThr), lr, c.stream, b, pl, w.band,
+                     w.part, ring.cnt, p.amag, w.mean, tw);
+  FR_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_band_rows<N>, dim3((npairs + nseq - 1) / nseq), dim3(kThr), lr, c.stream, b,
+                     pl, w.band, p.amag, w.mean, tw);
+  FR_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_band_sums<N>, dim3(cols), dim3(kThr), ls, c.stream, b, pl, w.band,
+                     reinterpret_cast<const float2*>(p.spec), p.pidx, p.shift, w.psum, tw);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
+// the box sizes of the tests and the benchmark with their length compiled in (an
+// index division or modulus by a run-time length costs more than its butterfly)
+int launch_band(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, const BandWork& w) {
+  switch (b.nsam) {
+    case 64: return launch_n<64>(c, b, p, ring, w);
+    case 96: return launch_n<96>(c, b, p, ring, w);
+    case 128: return launch_n<128>(c, b, p, ring, w);
+    case 160: return launch_n<160>(c, b, p, ring, w);
+    case 192: return launch_n<192>(c, b, p, ring, w);
+    case 256: return launch_n<256>(c, b, p, ring, w);
+    case 320: return launch_n<320>(c, b, p, ring, w);
+    case 384: return launch_n<384>(c, b, p, ring, w);
+    case 512: return launch_n<512>(c, b, p, ring, w);
+    default: return launch_n<0>(c, b, p, ring, w);
+  }
+}
+
+Band make_band(int nsam, int n, int maxr12, int maxr2, float ri2, float ri3, float rih,
+               float halfw, int flip) {
+  int jmax = maxr2 - 1;
+  return Band{nsam, n,   band_cb(maxr2), jmax, maxr12, maxr2 * maxr2, band_nsh(maxr2),
+              ri2,  ri3, rih,            halfw, flip};
+}
+
+}  // namespace
+
+size_t cc3m_fft_bytes(int nsam, int maxr2, size_t n) {
+  size_t bytes = 0;
+  (void)band_work(nullptr, nsam, maxr2, n, &bytes);
+  return bytes;
+}
+
+// Rhat[J][I] = sum over the pixels (x, y) of the MASKCOS2 ring at AMAG = 1 (as the
+// kernels test them) of cos(2 pi I x/N) cos(2 pi J y/N), J < MAXR2, I < CB; in
+// double.  Returns the ring's pixel count.
+int cc3m_ring_hat(int nsam, float ri2, float ri3, int maxr2, std::vector<float>& out) {
+  const int h = nsam / 2, cb = band_cb(maxr2);
+  std::vector<double> co(nsam), row((size_t)(h + 1) * cb, 0.0);
+  for (int k = 0; k < nsam; k++) co[k] = std::cos(2.0 * M_PI * k / nsam);
+  auto mult = [&](int v) { return v == 0 || v == h ? 1 : 2; };
+  long long cnt = 0;
+  for (int y = 0; y <= h; y++)
+    for (int x = 0; x <= h; x++) {
+      const float r2 = (float)(x * x + y * y);
+      if (!(r2 > ri2 && r2 <= ri3)) continue;
+      cnt += (long long)mult(x) * mult(y);
+      for (int i = 0; i < cb; i++)
+        row[(size_t)y * cb + i] += mult(x) * co[(long long)i * x % nsam];
+    }
+  out.assign((size_t)maxr2 * cb, 0.f);
+  for (int j = 0; j < maxr2; j++)
+    for (int i = 0; i < cb; i++) {
+      double s = 0.0;
+      for (int y = 0; y <= h; y++) s += mult(y) * co[(long long)j * y % nsam] * row[(size_t)y * cb + i];
+      out[(size_t)j * cb + i] = (float)s;
+    }
+  return (int)cnt;
+}
+
+int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
+                const int* pidx, const float* dm, const float* shift, const float* amag,
+                const float* fsct, const Cc3mRing& ring, void* work, float* score) {
+  if (a.n <= 0) return 0;
+  FR_CHECK(a.nsam / 2 + 2 <= 260, "box too large for CC3M bins");
+  FR_CHECK(a.maxr2 < a.nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", a.maxr2);
+  FR_CHECK(ring.rhat && work, "CC3M tables missing");
+  const Band b = make_band(a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2, a.ri2, a.ri3, a.rih, a.halfw,
+                           a.cc3);
+  size_t bytes;
+  const BandWork w = band_work(work, a.nsam, a.maxr2, a.n, &bytes);
+  if (int r = launch_band(c, b, BandCall{a3df, spec, ctff, pidx, dm, shift, amag}, ring, w))
+    return r;
+  hipLaunchKernelGGL(k_band_score, dim3(a.n), dim3(64), 0, c.stream, b, a.rbfact, w.psum, fsct,
+                     score);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
+// PRESB for a batch: the CC3M steps over 1 <= r^2 < (NSAM/2)^2
+int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, const float* ctff,
+                 const int* pidx, const float* dm, const float* shift, const float* amag,
+                 float ri2, float ri3, float rih, float halfw, const Cc3mRing& ring, void* work,
+                 float* rbin) {
+  if (n <= 0) return 0;
+  FR_CHECK(nsam / 2 + 2 <= 260, "box too large for PRESB bins");
+  FR_CHECK(ring.rhat && work, "PRESB tables missing");
+  const Band b = make_band(nsam, n, 1, nsam / 2, ri2, ri3, rih, halfw, 0);
+  size_t bytes;
+  const BandWork w = band_work(work, nsam, nsam / 2, n, &bytes);
+  if (int r = launch_band(c, b, BandCall{a3df, spec, ctff, pidx, dm, shift, amag}, ring, w))
+    return r;
+  hipLaunchKernelGGL(k_band_presb, dim3(n), dim3(64), 0, c.stream, b, w.psum, rbin);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
+}  // namespace fr

@@ -22,74 +22,6 @@ namespace {
 
 using namespace fftdev;
 constexpr int kThreads = kFftThreads;
-constexpr int kMaxPass = 12;
-
-struct Plan {
-  int n;
-  int npass;
-  int radix[kMaxPass];
-};
-
-bool make_plan(int n, Plan* p) {
-  if (n < 2 || n > 1024) return false;
-  p->n = n;
-  p->npass = 0;
-  int m = n;
-  while (m % 4 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 4; m /= 4; }
-  while (m % 2 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 2; m /= 2; }
-  while (m % 3 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 3; m /= 3; }
-  while (m % 5 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 5; m /= 5; }
-  return m == 1;
-}
-
-template <int R>
-__device__ inline void stockham_pass(const float2* in, float2* out, int n, int ld, int nseq, int p,
-                                     int sign, const float2* __restrict__ tw) {
-  const int T = n / R;
-  const int stride = n / (p * R);
-  for (int b = threadIdx.x; b < nseq * T; b += blockDim.x) {
-    int s = b / T, i = b - s * T;
-    int k = i % p;
-    const float2* x = in + s * ld;
-    float2 u[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) u[r] = x[i + r * T];
-#pragma unroll
-    for (int r = 1; r < R; r++) {
-      int e = (r * k * stride) % n;
-      float2 w = tw[e];
-      if (sign > 0) w.y = -w.y;
-      u[r] = mul2(u[r], w);
-    }
-    butterfly<R>(u, sign);
-    float2* y = out + s * ld;
-    int base = (i - k) * R + k;
-#pragma unroll
-    for (int q = 0; q < R; q++) y[base + q * p] = u[q];
-  }
-}
-
-// In-LDS FFT of nseq sequences (stride ld); returns the buffer holding the result.
-__device__ float2* lds_fft(float2* buf, float2* tmp, const Plan& pl, int ld, int nseq, int sign,
-                           const float2* __restrict__ tw) {
-  int p = 1;
-  for (int ps = 0; ps < pl.npass; ps++) {
-    int R = pl.radix[ps];
-    switch (R) {
-      case 4: stockham_pass<4>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
-      case 2: stockham_pass<2>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
-      case 3: stockham_pass<3>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
-      default: stockham_pass<5>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
-    }
-    __syncthreads();
-    float2* t = buf;
-    buf = tmp;
-    tmp = t;
-    p *= R;
-  }
-  return buf;
-}
-
 // ---- row pass, forward: rows (2q, 2q+1) -> z = a + i b -> FFT -> unpack to half spectra
 __global__ void __launch_bounds__(kThreads) k_rows_r2c(float* data, Plan pl, int nrows_per_img,
                                                        size_t img_stride, int npairs, int nseq,

@@ -117,6 +117,75 @@ __device__ inline float2* lds_fft_t(float2* buf, float2* tmp, const float2* __re
 }
 
 
+// ---- the same passes with the length known at run time
+constexpr int kMaxPass = 12;
+
+struct Plan {
+  int n;
+  int npass;
+  int radix[kMaxPass];
+};
+
+inline bool make_plan(int n, Plan* p) {
+  if (n < 2 || n > 1024) return false;
+  p->n = n;
+  p->npass = 0;
+  int m = n;
+  while (m % 4 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 4; m /= 4; }
+  while (m % 2 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 2; m /= 2; }
+  while (m % 3 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 3; m /= 3; }
+  while (m % 5 == 0 && p->npass < kMaxPass) { p->radix[p->npass++] = 5; m /= 5; }
+  return m == 1;
+}
+
+template <int R>
+__device__ inline void stockham_pass(const float2* in, float2* out, int n, int ld, int nseq, int p,
+                                     int sign, const float2* __restrict__ tw) {
+  const int T = n / R;
+  const int stride = n / (p * R);
+  for (int b = threadIdx.x; b < nseq * T; b += blockDim.x) {
+    int s = b / T, i = b - s * T;
+    int k = i % p;
+    const float2* x = in + s * ld;
+    float2 u[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) u[r] = x[i + r * T];
+#pragma unroll
+    for (int r = 1; r < R; r++) {
+      int e = (r * k * stride) % n;
+      float2 w = tw[e];
+      if (sign > 0) w.y = -w.y;
+      u[r] = mul2(u[r], w);
+    }
+    butterfly<R>(u, sign);
+    float2* y = out + s * ld;
+    int base = (i - k) * R + k;
+#pragma unroll
+    for (int q = 0; q < R; q++) y[base + q * p] = u[q];
+  }
+}
+
+// In-LDS FFT of nseq sequences (stride ld); returns the buffer holding the result.
+__device__ inline float2* lds_fft(float2* buf, float2* tmp, const Plan& pl, int ld, int nseq, int sign,
+                           const float2* __restrict__ tw) {
+  int p = 1;
+  for (int ps = 0; ps < pl.npass; ps++) {
+    int R = pl.radix[ps];
+    switch (R) {
+      case 4: stockham_pass<4>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
+      case 2: stockham_pass<2>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
+      case 3: stockham_pass<3>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
+      default: stockham_pass<5>(buf, tmp, pl.n, ld, nseq, p, sign, tw); break;
+    }
+    __syncthreads();
+    float2* t = buf;
+    buf = tmp;
+    tmp = t;
+    p *= R;
+  }
+  return buf;
+}
+
 // columns per workgroup of the column pass (16 at 256 measured no faster)
 template <int N>
 constexpr int cols_cw() {

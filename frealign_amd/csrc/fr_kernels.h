@@ -104,12 +104,21 @@ constexpr int kMaskThreads = 1024;
 __global__ void k_scale_mask(int nsam, float* data, size_t img_stride, float scal,
                              const float* amag_arr, int amag_stride, float ri2, float ri3,
                              float rih, float halfw, int origin);
+// On the particle's grid, any box, band and AMAG (fr_cc3m_fft.hip); work:
+// cc3m_fft_bytes for the items of the call (PRESB: MAXR2 = NSAM/2).
+struct Cc3mRing {
+  const float* rhat = nullptr;  // cc3m_ring_hat on the device
+  int cnt = 0;                  // the ring's pixels
+};
+size_t cc3m_fft_bytes(int nsam, int maxr2, size_t n);
+int cc3m_ring_hat(int nsam, float ri2, float ri3, int maxr2, std::vector<float>& out);
 int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
                 const int* pidx, const float* dm, const float* shift, const float* amag,
-                const float* fsct, float* work, float* score);
+                const float* fsct, const Cc3mRing& ring, void* work, float* score);
 int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, const float* ctff,
                  const int* pidx, const float* dm, const float* shift, const float* amag,
-                 float ri2, float ri3, float rih, float halfw, float* work, float* rbin);
+                 float ri2, float ri3, float rih, float halfw, const Cc3mRing& ring, void* work,
+                 float* rbin);
 // SIGMA (sigma.f:8-221) item: PEXTRACT DM, shift, mask centre/radius^2,
 // SIGNSET, particle and band.
 struct SigmaItem {

@@ -40,6 +40,7 @@ struct fr_plan {
   Cc3mArgs ca{};
   Cc3mTables tabs;  // fused CC3M tables (owned by the context)
   Cc3mBandTables band;
+  Cc3mRing ring;
   int nsym = 0;
   int jsym[8] = {};
   float symop[72] = {};
@@ -96,7 +97,7 @@ int enqueue(fr_plan* p) {
       return r;
   } else {
     if (int r = launch_cc3m(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm, p->d_shift,
-                            p->d_amag, p->fsct, p->d_work, p->d_score))
+                            p->d_amag, p->fsct, p->ring, p->d_work, p->d_score))
       return r;
   }
   FR_HIP(hipMemcpyAsync(p->h_score, p->d_score, sizeof(float) * nb, hipMemcpyDeviceToHost,
@@ -230,7 +231,9 @@ int fr_plan_create(fr_ctx* c, int nsam, int nb, const float* d_a3df, const float
       (r = halloc(&p->h_amag, (size_t)nb)) || (r = halloc(&p->h_score, (size_t)nb)) ||
       (r = halloc(&p->h_tasks, (size_t)nb * ncopy)))
     return fail(r);
-  if (!p->fused && (r = dalloc(&p->d_work, img * nb))) return fail(r);
+  if (!p->fused && ((r = dalloc(&p->d_work, cc3m_fft_bytes(nsam, maxr2, nb) / sizeof(float))) ||
+                    (r = c->cc3m_ring(nsam, maxr2, p->ca.ri2, p->ca.ri3, &p->ring))))
+    return fail(r);
   if ((r = dalloc(&p->d_ins, insert_scratch_bytes(nsam, nb, nb * ncopy)))) return fail(r);
   if ((r = dalloc(&p->d_part, 2 * prep_partials_count(nsam, nb)))) return fail(r);
   if (p->fused && ((r = c->cc3m_tables(p->ca, &p->tabs)) ||

@@ -117,3 +117,28 @@ def test_window_equals_scores_at_its_shifts(ctx, nsam, maxr1, maxr2, nsh, amag):
     assert np.abs(sc - want.max(1)).max() <= bar
     assert (want.max(1) - want[np.arange(n), code] <= 2 * bar).all()
     assert np.abs(best[:, 5] - want.reshape(npart, -1).max(1)).max() <= bar
+
+
+@pytest.mark.parametrize("nsam,maxr1,maxr2", [(36, 1, 16), (72, 0, 32), (100, 2, 25), (250, 2, 32),
+                                              (300, 3, 24), (384, 1, 31)])
+def test_band_grid_serves_any_box(ctx, nsam, maxr1, maxr2):
+    """Candidates of a search (AMAG = 1 throughout) at boxes that the products on the
+    particle's grid do not hold, smaller and larger than the band's grid."""
+    npart, k, nbank = 3, 5, 40
+    rng = np.random.default_rng(nsam)
+    ri = 0.42 * nsam
+    ring = np.array([(ri - 3) ** 2, (ri + 3) ** 2, ri - 3, 6.0], np.float32)
+    vol, spec, ctff, _, dm, _, _ = items(nsam, npart, nbank, nsam, False)
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a, d)).to(DEV)  # noqa: E731
+    o, row = rng.integers(0, nbank, (npart, k)), rng.integers(0, 225, (npart, k))
+    nsamr = 2 * ((nsam // 2 + 1) // 2)
+    fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    got, _ = ctx[0].rescore(nsam, vol, spec, ctff, t(o, np.int32), t(row, np.int32),
+                            dm.reshape(nbank, 9), nsamr, maxr1, maxr2, 0.002, fsct, ring)
+    sh = np.stack([row // 15 - 7, row % 15 - 7], -1).astype(np.float32)
+    sh = sh / np.float32(nsamr) * np.float32(2 * 3.1415926535897)
+    want = ctx[1].cc3m(nsam, vol, spec, ctff, t(np.repeat(np.arange(npart), k), np.int32),
+                       dm.reshape(nbank, 9)[t(o.reshape(-1), np.int64)].contiguous(),
+                       t(sh.reshape(-1, 2), np.float32), torch.ones(npart * k, device=DEV), maxr1,
+                       maxr2, 0.002, fsct, ring).reshape(npart, k)
+    assert (got - want).abs().max() <= BAR * want.abs().max()
