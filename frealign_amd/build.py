@@ -31,6 +31,7 @@ SOURCES = [
     "fr_search_sep.hip",
     "fr_search_f32.hip",
     "fr_cnn.hip",
+    "fr_cnn_train.hip",
     "fr_refine.cpp",
     "fr_sigma.hip",
     "fr_plan.cpp",

@@ -1133,8 +1133,11 @@ int fr_cnn_gradients_bf16(fr_ctx* c, int S, int C, int nconv, int K, const float
   FR_CHECK(d_wq && d_img && d_label && d_loss && d_grad && nb >= 1, "null argument");
   CNN_SHAPE(lo);
   int err = 0;
-  float* ws = (float*)c->slot(9, sizeof(float) * cnn_workspace(lo, nb, true), &err);
+  const bool wide = cnn_train_ok(lo);
+  float* ws = (float*)c->slot(
+      9, sizeof(float) * (wide ? cnn_train_workspace(lo, nb) : cnn_workspace(lo, nb, true)), &err);
   if (!ws) return err;
+  if (wide) return cnn_train_backward(*c, lo, d_wq, nb, d_img, d_label, ws, d_loss, d_grad);
   return cnn_backward(*c, lo, d_wq, nb, d_img, d_label, ws, d_loss, d_grad, true);
 }
 

@@ -39,6 +39,17 @@ int cnn_forward_bf16(Ctx& c, const CnnLayout& lo, const float* wq, int B, const 
 // FP32 accumulation (the mixed-precision training step); else FP32 throughout
 int cnn_backward(Ctx& c, const CnnLayout& lo, const float* wq, int B, const float* img,
                  const int* label, float* ws, float* loss, float* grad, bool bf16 = false);
+// output positions of the first convolution (batch x pixels) a training step takes
+constexpr long long kCnnMaxPositions = 64ll * 9 * 16384;
+// the mixed-precision step of a 64-channel network (fr_cnn_train.hip):
+// workspace in floats; results as cnn_backward(..., true)
+bool cnn_train_ok(const CnnLayout& lo);
+size_t cnn_train_workspace(const CnnLayout& lo, int B);
+int cnn_train_backward(Ctx& c, const CnnLayout& lo, const float* wq, int B, const float* img,
+                       const int* label, float* ws, float* loss, float* grad);
+// per-image loss and its gradient (of the batch mean) in rows of ldg >= K
+int cnn_softmax_xent(Ctx& c, int K, int ldg, int B, const float* logits, const int* label,
+                     float* loss, float* grad);
 int cnn_adam(Ctx& c, const CnnLayout& lo, float* master, float* wq, const float* grad, float* m,
              float* v, int step, float lr);
 int cnn_propose(Ctx& c, int K, int B, const float* logits, int topk, int* top, float* prob);

@@ -572,10 +572,11 @@ __device__ inline float block_sum(float v, float* red) {
 }
 
 // softmax cross-entropy of logits[b][*] against label[b]: loss[b] and
-// grad[b][k] = (p_k - [k == label]) / B; one block per sample
+// grad[b][k] = (p_k - [k == label]) / B in rows of ldg (zero beyond K); one
+// block per sample
 __global__ void __launch_bounds__(kT)
-    k_softmax_xent(int K, int B, const float* __restrict__ logits, const int* __restrict__ label,
-                   float* loss, float* grad) {
+    k_softmax_xent(int K, int ldg, int B, const float* __restrict__ logits,
+                   const int* __restrict__ label, float* loss, float* grad) {
   __shared__ float red[kT / 64];
   const int b = blockIdx.x;
   const float* z = logits + (long long)b * K;
@@ -589,8 +590,9 @@ __global__ void __launch_bounds__(kT)
   y = y < 0 ? 0 : (y >= K ? K - 1 : y);  // labels are validated by the caller; stay in bounds
   for (int k = threadIdx.x; k < K; k += kT) {
     float p = expf(z[k] - mx) / s;
-    grad[(long long)b * K + k] = (p - (k == y ? 1.f : 0.f)) / (float)B;
+    grad[(long long)b * ldg + k] = (p - (k == y ? 1.f : 0.f)) / (float)B;
   }
+  for (int k = K + threadIdx.x; k < ldg; k += kT) grad[(long long)b * ldg + k] = 0.f;
   if (threadIdx.x == 0) loss[b] = logf(s) + mx - z[y];
 }
 
@@ -1077,7 +1079,8 @@ struct Ws {
   size_t X, logits, wt, gA, gB, gX, gL, part, total;
 };
 
-constexpr int kMaxSplit = 64;  // splits of the bias-gradient row sums (x9)
+// splits of 16,384 positions of the bias-gradient row sums
+constexpr int kMaxSplit = (int)(kCnnMaxPositions / 16384);
 
 Ws ws_layout(const CnnLayout& lo, int B, bool backward) {
   Ws w{};
@@ -1110,7 +1113,7 @@ Ws ws_layout(const CnnLayout& lo, int B, bool backward) {
     o += (size_t)lo.K * B;
     w.part = o;
     // split-K partials of the weight gradients, or the bias row sums' partials
-    size_t pc = (size_t)lo.C * 9 * kMaxSplit;
+    size_t pc = (size_t)lo.C * kMaxSplit;
     o += (size_t)kPartFloats > pc ? (size_t)kPartFloats : pc;
   }
   w.total = o;
@@ -1211,14 +1214,20 @@ int cnn_forward(Ctx& c, const CnnLayout& lo, const float* wq, int B, const float
   return 0;
 }
 
+int cnn_softmax_xent(Ctx& c, int K, int ldg, int B, const float* logits, const int* label,
+                     float* loss, float* grad) {
+  hipLaunchKernelGGL(k_softmax_xent, dim3(B), dim3(kT), 0, c.stream, K, ldg, B, logits, label, loss,
+                     grad);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
 int cnn_backward(Ctx& c, const CnnLayout& lo, const float* wq, int B, const float* img,
                  const int* label, float* ws, float* loss, float* grad, bool bf16) {
   Ws w = ws_layout(lo, B, true);
   if (int r = forward_impl(c, lo, wq, B, img, ws, w, bf16)) return r;
   const int K = lo.K, F = lo.F();
-  hipLaunchKernelGGL(k_softmax_xent, dim3(B), dim3(kT), 0, c.stream, K, B, ws + w.logits, label,
-                     loss, ws + w.gL);
-  FR_HIP(hipGetLastError());
+  if (int r = cnn_softmax_xent(c, K, K, B, ws + w.logits, label, loss, ws + w.gL)) return r;
   // gWfc[k][f] = sum_b gL[b][k] X[f][b]
   if (int r = gemm(c, K, F, B, ws + w.gL, 1, K, ws + w.X, 1, B, grad + lo.fw_off, F, 1, nullptr,
                    false, false, bf16))
@@ -1249,7 +1258,7 @@ int cnn_backward(Ctx& c, const CnnLayout& lo, const float* wq, int B, const floa
     // the split-K sum above has run), then the splits in order
     const int bchunk = 16384;
     const int bsplit = (int)((NB + bchunk - 1) / bchunk);
-    FR_CHECK(bsplit <= kMaxSplit * 9, "batch too large for the bias reduction");
+    FR_CHECK(NB <= kCnnMaxPositions, "batch too large for the bias reduction");
     hipLaunchKernelGGL(k_rowsum_part, dim3(lo.C, bsplit), dim3(kT), 0, c.stream, (int)NB, NB,
                        bchunk, gcur, ws + w.part);
     FR_HIP(hipGetLastError());
