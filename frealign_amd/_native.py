@@ -32,6 +32,7 @@ SIGNATURES = {
     "fr_fft2d_r2c": ([vp, ci, ci, vp], ci),
     "fr_fft2d_c2r": ([vp, ci, ci, vp], ci),
     "fr_prep_batch": ([vp, ci, ci, vp, vp, vp, vp, ci, vp, vp, vp], ci),
+    "fr_index_range": ([vp, C.c_longlong, vp, pi_, pi_], ci),
     "fr_pextract_batch": ([vp, ci, ci, vp, vp, vp, vp, vp], ci),
     "fr_cc3m_batch": ([vp, ci, ci, vp, vp, vp, vp, vp, vp, vp, ci, ci, cf, vp, vp, vp], ci),
     "fr_cc3_batch": ([vp, ci, ci, vp, vp, vp, vp, vp, vp, vp, ci, ci, cf, vp, vp, vp], ci),

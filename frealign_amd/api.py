@@ -56,6 +56,16 @@ class Context:
         s = torch.cuda.current_stream(self.device).cuda_stream
         N.check(N.lib().fr_set_stream(self.h, C.c_void_p(s)), "fr_set_stream")
 
+    def _inside(self, idx: torch.Tensor, n: int) -> bool:
+        """Whether all of a device tensor of int32 indexes are in 0..n-1."""
+        if idx.device.index != self.device:
+            return 0 <= int(idx.min()) and int(idx.max()) < n
+        lo, hi = C.c_int(), C.c_int()
+        self._sync_stream()
+        N.check(N.lib().fr_index_range(self.h, idx.numel(), _p(idx), C.byref(lo), C.byref(hi)),
+                "fr_index_range")
+        return 0 <= lo.value and hi.value < n
+
     def close(self):
         if self.h:
             N.lib().fr_destroy(self.h)
@@ -132,7 +142,7 @@ class Context:
         npart = ctff.numel() // (2 * nsam * jc)
         if pidx is not None:
             _dev(pidx, torch.int32, "pidx")
-            if pidx.numel() != n or (n and int(pidx.max()) >= npart) or (n and int(pidx.min()) < 0):
+            if pidx.numel() != n or (n and not self._inside(pidx, npart)):
                 raise ValueError("pidx out of range")
         elif n > npart:
             raise ValueError("more sections than CTF tables")
@@ -157,7 +167,7 @@ class Context:
         npart = spec.numel() // (nsam * jc)
         if dm.numel() != 9 * n or shift.numel() != 2 * n or amag.numel() != n:
             raise ValueError("dm/shift/amag sizes do not match pidx")
-        if n and (int(pidx.max()) >= npart or int(pidx.min()) < 0):
+        if n and not self._inside(pidx, npart):
             raise ValueError("pidx out of range")
         if ctff.numel() != 2 * spec.numel() or fsct.numel() < nsam // 2 + 1:
             raise ValueError("ctff/fsct sizes")
@@ -185,7 +195,7 @@ class Context:
         npart = spec.numel() // (nsam * jc)
         if dm.numel() != 9 * n or shift.numel() != 2 * n or amag.numel() != n:
             raise ValueError("dm/shift/amag sizes do not match pidx")
-        if n and (int(pidx.max()) >= npart or int(pidx.min()) < 0):
+        if n and not self._inside(pidx, npart):
             raise ValueError("pidx out of range")
         if ctff.numel() != 2 * spec.numel() or a3df.numel() != nsam * nsam * jc:
             raise ValueError("ctff/a3df sizes")
@@ -675,7 +685,7 @@ class Context:
         _dev(grad, torch.float32, "grad")
         S, K = shape[0], shape[3]
         nb = img.numel() // (S * S)
-        if label.numel() != nb or (nb and (int(label.min()) < 0 or int(label.max()) >= K)):
+        if label.numel() != nb or (nb and not self._inside(label, K)):
             raise ValueError("one label in 0..K-1 per image")
         loss = torch.empty(nb, dtype=torch.float32, device=img.device)
         self._sync_stream()

@@ -328,6 +328,7 @@ int fr_destroy(fr_ctx* c) {
   for (int k = 0; k < fr_ctx::kSlots; k++)
     if (c->slots[k]) (void)hipFree(c->slots[k]);
   if (c->hpin) (void)hipHostFree(c->hpin);
+  if (c->hrange) (void)hipHostFree(c->hrange);
   if (c->d_kidx) (void)hipFree(c->d_kidx);
   for (auto& e : c->dft_tabs) (void)hipFree(e.second);
   for (auto& e : c->ring_hats) (void)hipFree(e.second.d);
@@ -435,6 +436,24 @@ int fr_prep_batch(fr_ctx* c, int nsam, int nb, float* d_data, const float* d_ppa
 }
 
 // ------------------------------------------------------ extraction / scoring
+int fr_index_range(fr_ctx* c, long long n, const int* d_idx, int* lo, int* hi) {
+  CTX_CHECK(c);
+  FR_CHECK(d_idx && lo && hi && n >= 1, "null or empty argument");
+  if (!c->hrange)
+    FR_HIP(hipHostMalloc((void**)&c->hrange, sizeof(int2) * fr_ctx::kRangeBlocks,
+                         hipHostMallocDefault));
+  const int blocks = (int)std::min<long long>(fr_ctx::kRangeBlocks, (n + 4095) / 4096);
+  if (int r = launch_index_range(*c, n, d_idx, blocks, c->hrange)) return r;
+  FR_HIP(hipStreamSynchronize(c->stream));
+  *lo = c->hrange[0].x;
+  *hi = c->hrange[0].y;
+  for (int b = 1; b < blocks; b++) {
+    *lo = std::min(*lo, c->hrange[b].x);
+    *hi = std::max(*hi, c->hrange[b].y);
+  }
+  return 0;
+}
+
 int fr_pextract_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_dm,
                       const int* d_pidx, const float* d_ctff, float* d_outc) {
   CTX_CHECK(c);

@@ -20,6 +20,9 @@ struct fr_ctx : public fr::Ctx {
   void* hpin = nullptr;
   size_t hpin_bytes = 0;
   void* host_pinned(size_t bytes, int* err);
+  // the index checks' results, one pair per workgroup, in host memory
+  static constexpr int kRangeBlocks = 64;
+  int2* hrange = nullptr;
   // search annulus and shift-phase tables, cached per (NSAM, MAXR1, MAXR2)
   int skey[3] = {0, 0, 0};
   int kc = 0, kpad = 0, nsamr = 0;

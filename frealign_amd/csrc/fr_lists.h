@@ -17,4 +17,7 @@ int launch_cand_items(Ctx& c, int np, int k, const int* top_o, const int* top_ro
                       const float* dm_bank, int nsamr, int* pidx, float* dm, float* shift,
                       float* amag);
 int launch_best_cand(Ctx& c, int np, int k, const int* top_o, float* score, int* best);
+// the smallest and largest of idx[0..n) per workgroup into out[0..blocks)
+int launch_index_range(Ctx& c, long long n, const int* idx, int blocks, int2* out);
+
 }  // namespace fr

@@ -99,6 +99,10 @@ int fr_prep_batch(fr_ctx *ctx, int nsam, int nb, float *d_data, const float *d_p
                   const float *d_pssnr, const float *gpar, int ictf, float *d_ctff,
                   float *d_outc, float *d_datc);
 
+/* Smallest and largest of d_idx[0..n) (n >= 1), for checks of device-resident
+ * indexes before a batch: one launch, then the stream is waited for. */
+int fr_index_range(fr_ctx *ctx, long long n, const int *d_idx, int *lo, int *hi);
+
 /* ---------------------------------------------------- extraction / scoring */
 
 /* Replaces PEXTRACT (pextract.f:8-101; IEWALD=0, IPAD=1, IRAD>0): n central
