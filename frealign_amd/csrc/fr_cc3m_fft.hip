@@ -19,11 +19,12 @@
 // Sums run in a fixed order: a rerun gives the same bits.
 //
 // What bounds it: the band goes through memory as write, read, write, read (512
-// items of a 320 box at MAXR2 = 80: 105 MB each time) and its FFTs through LDS;
-// before, whole half-planes went through it twelve times.  That call: 1,122 us as
-// whole planes, now 444.
+// items of a 320 box at MAXR2 = 80: 105 MB each time), the gather and the FFTs'
+// exchanges through LDS; before, whole half-planes went through it twelve times.
+// That call: 1,122 us as whole planes, now 304 (columns 94, rows 133, sums 57).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -50,13 +51,14 @@ struct Band {
 
 constexpr int rows_nseq(int n) { return n >= 1024 ? 2 : 2048 / n; }
 
-// N > 0: the length is known at compile time (NS sequences of pitch N + 1)
-template <int N, int NS, int SIGN>
-__device__ inline float2* fft_any(float2* buf, float2* tmp, const Plan& pl, int nseq,
-                                  const float2* __restrict__ tw) {
-  if constexpr (N > 0) return lds_fft_t<N, NS, N + 1, SIGN>(buf, tmp, tw);
-  else return lds_fft(buf, tmp, pl, pl.n + 1, nseq, SIGN, tw);
-}
+// N > 0: the length is known at compile time; N = 0: passes of a length known at
+// run time between two buffers of sequences of pitch n + 1
+template <int N>
+using Cols = Fft<N ? N : 64, kCw, true>;
+template <int N>
+using Rows = Fft<N ? N : 64, rows_nseq(N ? N : 64), false>;
+template <int N>
+using RowsBack = Fft<N ? N : 64, rows_nseq(N ? N : 64), false, true>;
 
 template <int N>
 __global__ void __launch_bounds__(kThr)
@@ -68,12 +70,14 @@ __global__ void __launch_bounds__(kThr)
   __shared__ float red[kThr / 64];
   const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
   const size_t ic = (size_t)n * jc;
-  float2 *buf = smem, *tmp = smem + kCw * ld;
+  using F = Cols<N>;
+  auto at = [&](int q, int y) { return N ? F::at(q, y) : q * ld + y; };
+  float2* buf = smem;
   // an item's column blocks in XCD-contiguous order: they share lines
   const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
   const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
   if (it >= b.nitem) return;
-  for (int e = threadIdx.x; e < kCw * ld; e += kThr) buf[e] = make_float2(0.f, 0.f);
+  for (int e = threadIdx.x; e < kCw * (N ? F::LD : ld); e += kThr) buf[e] = make_float2(0.f, 0.f);
   __syncthreads();
   const float* d = dm + 9 * (size_t)it;
   const float2* cp = ctff + (size_t)pidx[it] * 2 * ic;
@@ -93,7 +97,7 @@ __global__ void __launch_bounds__(kThr)
       a = cmul(a, cf{cr.x + cl.x, cr.y - cl.y});
     }
     a = cscale(a, scal);
-    buf[(e & (kCw - 1)) * ld + wrapn(j, n)] = make_float2(a.re, a.im);
+    buf[at(e & (kCw - 1), wrapn(j, n))] = make_float2(a.re, a.im);
     rsum += (i ? 2.0f : 1.0f) * a.re * rhat[(size_t)abs(j) * b.cb + i];
   }
   for (int off = 32; off > 0; off >>= 1) rsum += __shfl_xor(rsum, off, 64);
@@ -104,24 +108,68 @@ __global__ void __launch_bounds__(kThr)
     for (int q = 0; q < kThr / 64; q++) s += red[q];
     part[lb] = s;
   }
-  const float2* res = fft_any<N, kCw, +1>(buf, tmp, pl, kCw, tw);
   float2* out = work + (size_t)it * n * b.cb + x0;
-  for (int e = threadIdx.x; e < n * kCw; e += kThr)
-    out[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))] = res[(e & (kCw - 1)) * ld + e / kCw];
+  if constexpr (N > 0) {
+    float2 u[F::IF][F::RF], z[F::IL][F::RL];
+    F::template each<F::RF>([&](int k, int q, int y) {
+#pragma unroll
+      for (int r = 0; r < F::RF; r++) u[k][r] = buf[F::at(q, y + r * F::TF)];
+    });
+    F::template run<+1, true>(u, z, buf, tw);
+    F::template each<F::RL>([&](int k, int q, int y) {
+#pragma unroll
+      for (int r = 0; r < F::RL; r++) out[(size_t)(y + r * F::TL) * b.cb + q] = z[k][r];
+    });
+  } else {
+    const float2* res = lds_fft(buf, smem + kCw * ld, pl, ld, kCw, +1, tw);
+    for (int e = threadIdx.x; e < n * kCw; e += kThr)
+      out[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))] = res[(e & (kCw - 1)) * ld + e / kCw];
+  }
 }
 
-// the half spectra of rows 2q and 2q+1 as one sequence: Z_k = A_k + i B_k,
-// Z_{n-k} = conj(A_k) + i conj(B_k), the imaginary parts at k = 0 ignored as the
-// c2r does
-__device__ inline void load_pair(float2* z, const float2* ra, int n, int cb, int k) {
+// point k of the sequence of rows 2q and 2q+1 (ra: their CB columns each)
+__device__ inline float2 band_pair(const float2* ra, int n, int cb, int k) {
+  const int m = 2 * k <= n ? k : n - k;
   float2 a = make_float2(0.f, 0.f), c = a;
-  if (k < cb) {
-    a = ra[k];
-    c = ra[cb + k];
+  if (m < cb) {
+    a = ra[m];
+    c = ra[cb + m];
   }
-  if (k == 0 || 2 * k == n) a.y = c.y = 0.f;
-  z[k] = make_float2(a.x - c.y, a.y + c.x);
-  if (k > 0 && 2 * k < n) z[n - k] = make_float2(a.x + c.y, -a.y + c.x);
+  return pair_point(a, c, k, n);
+}
+
+// the row pairs pair0 .. of `work` (npairs in all; beyond: the last again)
+// through the c2r: f(q, x, (pixel x of row 2q, of row 2q + 1))
+template <int N, typename F>
+__device__ inline void band_c2r(float2* smem, const Plan& pl, const float2* work, int pair0,
+                                int npairs, int cb, const float2* __restrict__ tw, F f) {
+  const int n = N ? N : pl.n, ld = n + 1, nseq = rows_nseq(n);
+  if constexpr (N > 0) {
+    using T = Rows<N>;
+    float2 u[T::IF][T::RF], z[T::IL][T::RL];
+    T::template each<T::RF>([&](int k, int q, int x) {
+      const float2* ra = work + (size_t)min(pair0 + q, npairs - 1) * 2 * cb;
+#pragma unroll
+      for (int r = 0; r < T::RF; r++) u[k][r] = band_pair(ra, N, cb, x + r * T::TF);
+    });
+    T::template run<+1, true>(u, z, smem, tw);
+    T::template each<T::RL>([&](int k, int q, int x) {
+#pragma unroll
+      for (int r = 0; r < T::RL; r++) f(q, x + r * T::TL, z[k][r]);
+    });
+  } else {
+    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+      const int q = e / n, k = e - q * n;
+      smem[q * ld + k] = band_pair(work + (size_t)min(pair0 + q, npairs - 1) * 2 * cb, n, cb, k);
+    }
+    __syncthreads();
+    const float2* res = lds_fft(smem, smem + nseq * ld, pl, ld, nseq, +1, tw);
+    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+      const int q = e / n, x = e - q * n;
+      f(q, x, res[q * ld + x]);
+    }
+    __syncthreads();
+  }
 }
 
 // squared wrapped distances of MASKCOS2 (origin 1)
@@ -138,7 +186,7 @@ __global__ void __launch_bounds__(kThr)
   extern __shared__ float2 smem[];
   __shared__ float red[kThr / 64];
   __shared__ int redc[kThr / 64];
-  const int n = N ? N : pl.n, ld = n + 1, it = blockIdx.x, nblk = b.cb / kCw;
+  const int n = N ? N : pl.n, it = blockIdx.x, nblk = b.cb / kCw;
   const float am = amag[it];
   if (am == 1.0f) {
     if (threadIdx.x == 0) {
@@ -149,28 +197,17 @@ __global__ void __launch_bounds__(kThr)
     return;
   }
   const float ri2p = b.ri2 / am / am, ri3p = b.ri3 / am / am;
-  const int nseq = rows_nseq(n);
-  float2 *buf = smem, *tmp = smem + nseq * ld;
+  const int nseq = rows_nseq(n), end = (it + 1) * (n / 2);
   float s = 0.f;
   int cnt = 0;
-  for (int q0 = 0; q0 < n / 2; q0 += nseq) {
-    for (int e = threadIdx.x; e < nseq * (n / 2 + 1); e += kThr) {
-      const int q = e / (n / 2 + 1), k = e - q * (n / 2 + 1);
-      if (q0 + q < n / 2)
-        load_pair(buf + q * ld, work + ((size_t)it * n + 2 * (q0 + q)) * b.cb, n, b.cb, k);
-    }
-    __syncthreads();
-    const float2* res = fft_any<N, N ? rows_nseq(N ? N : 1) : 1, +1>(buf, tmp, pl, nseq, tw);
-    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
-      const int q = e / n, x = e - q * n, row = 2 * (q0 + q);
-      if (row >= n) continue;
-      const float2 z = res[q * ld + x];
+  for (int p0 = it * (n / 2); p0 < end; p0 += nseq)
+    band_c2r<N>(smem, pl, work, p0, end, b.cb, tw, [&](int q, int x, float2 z) {
+      if (p0 + q >= end) return;
+      const int row = 2 * (p0 + q - it * (n / 2));
       const float ra = wrap2(x, n) + wrap2(row, n), rc = wrap2(x, n) + wrap2(row + 1, n);
       if (ra > ri2p && ra <= ri3p) s += z.x, cnt++;
       if (rc > ri2p && rc <= ri3p) s += z.y, cnt++;
-    }
-    __syncthreads();
-  }
+    });
   for (int off = 32; off > 0; off >>= 1) {
     s += __shfl_xor(s, off, 64);
     cnt += __shfl_xor(cnt, off, 64);
@@ -194,18 +231,9 @@ __global__ void __launch_bounds__(kThr)
                 const float* __restrict__ mean, const float2* __restrict__ tw) {
   extern __shared__ float2 smem[];
   const int n = N ? N : pl.n, ld = n + 1, nh = n / 2, nseq = rows_nseq(n);
-  float2 *buf = smem, *tmp = smem + nseq * ld;
   const int pair0 = blockIdx.x * nseq, npairs = b.nitem * nh;
-  for (int e = threadIdx.x; e < nseq * (nh + 1); e += kThr) {
-    const int q = e / (nh + 1), k = e - q * (nh + 1);
-    if (pair0 + q < npairs)  // rows of consecutive pairs are consecutive, over items too
-      load_pair(buf + q * ld, work + (size_t)(pair0 + q) * 2 * b.cb, n, b.cb, k);
-  }
-  __syncthreads();
-  float2* res = fft_any<N, N ? rows_nseq(N ? N : 1) : 1, +1>(buf, tmp, pl, nseq, tw);
-  for (int e = threadIdx.x; e < nseq * n; e += kThr) {
-    const int q = e / n, x = e - q * n, pr = pair0 + q;
-    if (pr >= npairs) continue;
+  // (z - mean) weight of pixel x of both rows of pair pr
+  auto masked = [&](int pr, int x, float2 z) {
     const int it = pr / nh, row = 2 * (pr - it * nh);
     const float am = amag[it], mu = mean[it];
     const float ri2p = b.ri2 / am / am, ri3p = b.ri3 / am / am, rihp = b.rih / am;
@@ -215,20 +243,60 @@ __global__ void __launch_bounds__(kThr)
       return 1.0f;
     };
     const float dx = wrap2(x, n);
-    const float2 z = res[q * ld + x];
-    res[q * ld + x] = make_float2((z.x - mu) * weight(dx + wrap2(row, n)),
-                                  (z.y - mu) * weight(dx + wrap2(row + 1, n)));
+    return make_float2((z.x - mu) * weight(dx + wrap2(row, n)),
+                       (z.y - mu) * weight(dx + wrap2(row + 1, n)));
+  };
+  const float2* out;
+  if constexpr (N > 0) {
+    // a thread masks the pixels its last pass leaves it and starts the transform
+    // back with them
+    using F = Rows<N>;
+    using G = RowsBack<N>;
+    static_assert(G::RF == F::RL && G::IF == F::IL, "the passes do not meet");
+    float2 u[F::IF][F::RF], z[F::IL][F::RL], o[G::IL][G::RL];
+    F::template each<F::RF>([&](int k, int q, int x) {
+      const float2* ra = work + (size_t)min(pair0 + q, npairs - 1) * 2 * b.cb;
+#pragma unroll
+      for (int r = 0; r < F::RF; r++) u[k][r] = band_pair(ra, N, b.cb, x + r * F::TF);
+    });
+    F::template run<+1, false>(u, z, smem, tw);
+    F::template each<F::RL>([&](int k, int q, int x) {
+      const int pr = min(pair0 + q, npairs - 1);
+#pragma unroll
+      for (int r = 0; r < F::RL; r++) z[k][r] = masked(pr, x + r * F::TL, z[k][r]);
+    });
+    G::template run<-1, true>(z, o, smem, tw);
+    __syncthreads();
+    G::template each<G::RL>([&](int k, int q, int x) {
+#pragma unroll
+      for (int r = 0; r < G::RL; r++) {
+        const int y = x + r * G::TL;
+        if (y < b.cb || N - y < b.cb) smem[G::at(q, y)] = o[k][r];
+      }
+    });
+    __syncthreads();
+    out = smem;
+  } else {
+    float2* tmp = smem + nseq * ld;
+    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+      const int q = e / n, k = e - q * n;
+      smem[q * ld + k] = band_pair(work + (size_t)min(pair0 + q, npairs - 1) * 2 * b.cb, n, b.cb, k);
+    }
+    __syncthreads();
+    float2* res = lds_fft(smem, tmp, pl, ld, nseq, +1, tw);
+    for (int e = threadIdx.x; e < nseq * n; e += kThr) {
+      const int q = e / n, x = e - q * n;
+      res[q * ld + x] = masked(min(pair0 + q, npairs - 1), x, res[q * ld + x]);
+    }
+    __syncthreads();
+    out = lds_fft(res, res == smem ? tmp : smem, pl, ld, nseq, -1, tw);
   }
-  __syncthreads();
-  const float2* out =
-      fft_any<N, N ? rows_nseq(N ? N : 1) : 1, -1>(res, res == buf ? tmp : buf, pl, nseq, tw);
   for (int e = threadIdx.x; e < nseq * b.cb; e += kThr) {
     const int q = e / b.cb, k = e - q * b.cb;
     if (pair0 + q >= npairs) continue;
-    const float2 zk = out[q * ld + k], zm = out[q * ld + (k ? n - k : 0)];
+    auto at = [&](int x) { return N ? RowsBack<N>::at(q, x) : q * ld + x; };
     float2* ra = work + (size_t)(pair0 + q) * 2 * b.cb + k;
-    ra[0] = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-    ra[b.cb] = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
+    split_pair(out[at(k)], out[at(k ? n - k : 0)], ra[0], ra[b.cb]);
   }
 }
 
@@ -246,16 +314,17 @@ __global__ void __launch_bounds__(kThr)
                 const int* __restrict__ pidx, const float* __restrict__ shift,
                 float4* __restrict__ psum, const float2* __restrict__ tw) {
   extern __shared__ float2 smem[];
+  using F = Cols<N>;
   const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
-  float2 *buf = smem, *tmp = smem + kCw * ld;
-  float2* ey = smem + 2 * kCw * ld;  // e^{i SHY J}, J = 0 .. jmax
+  // the transform's buffers, then per point of the band the masked section and
+  // (REAL(SAMP CONJG(AINPO)), |SAMP|^2): after it (N > 0) or in it
+  const int ldj = 2 * b.jmax + 1;
+  float2* ey = smem + (N ? max(kCw * F::LD, 2 * kCw * ldj) : 2 * kCw * ld);  // e^{i SHY J}
   __shared__ float2 ex[kCw];
   const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
   const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
   if (it >= b.nitem) return;
   const float2* in = work + (size_t)it * n * b.cb + x0;
-  for (int e = threadIdx.x; e < n * kCw; e += kThr)
-    buf[(e & (kCw - 1)) * ld + e / kCw] = in[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))];
   const float shx = shift[2 * it], shy = shift[2 * it + 1];
   for (int j = threadIdx.x; j <= b.jmax; j += kThr) {
     float sn, cs;
@@ -267,20 +336,48 @@ __global__ void __launch_bounds__(kThr)
     sincosf(shx * (float)(x0 + (int)threadIdx.x), &sn, &cs);
     ex[threadIdx.x] = make_float2(cs, sn);
   }
-  __syncthreads();
-  float2* res = fft_any<N, kCw, -1>(buf, tmp, pl, kCw, tw);
-  float2* pt = res == buf ? tmp : buf;  // per point (REAL(SAMP CONJG(AINPO)), |SAMP|^2)
   const float2* sp = spec + (size_t)pidx[it] * n * jc;
-  for (int e = threadIdx.x; e < kCw * (2 * b.jmax + 1); e += kThr) {
-    const int c = e & (kCw - 1), i = x0 + c, j = e / kCw - b.jmax, r2 = i * i + j * j;
-    if (r2 < b.maxr12 || r2 >= b.maxr22) continue;
-    const int row = wrapn(j, n);
-    const float2 s = sp[(size_t)i + (size_t)jc * row], a = res[c * ld + row];
+  auto point = [&](int c, int j, float2 a) {
+    const int i = x0 + c, r2 = i * i + j * j;
+    if (r2 < b.maxr12 || r2 >= b.maxr22) return make_float2(0.f, 0.f);
+    const float2 s = sp[(size_t)i + (size_t)jc * wrapn(j, n)];
     const float2 u = ex[c], v = ey[abs(j)];
     const float vs = j < 0 ? -v.y : v.y;
     const float cs = u.x * v.x - u.y * vs, sn = u.x * vs + u.y * v.x;
     const float re = s.x * a.x + s.y * a.y, im = s.y * a.x - s.x * a.y;
-    pt[c * ld + row] = make_float2(re * cs - im * sn, s.x * s.x + s.y * s.y);
+    return make_float2(re * cs - im * sn, s.x * s.x + s.y * s.y);
+  };
+  float2 *res, *pt;
+  auto pos = [&](int c, int j) { return N ? c * ldj + j + b.jmax : c * ld + (j < 0 ? n + j : j); };
+  if constexpr (N > 0) {
+    float2 u[F::IF][F::RF], z[F::IL][F::RL];
+    F::template each<F::RF>([&](int k, int c, int y) {
+#pragma unroll
+      for (int r = 0; r < F::RF; r++) u[k][r] = in[(size_t)(y + r * F::TF) * b.cb + c];
+    });
+    F::template run<-1, false>(u, z, smem, tw);
+    __syncthreads();
+    res = smem;
+    pt = smem + kCw * ldj;
+    F::template each<F::RL>([&](int k, int c, int y) {
+#pragma unroll
+      for (int r = 0; r < F::RL; r++) {
+        const int row = y + r * F::TL, j = 2 * row <= N ? row : row - N;
+        if (abs(j) > b.jmax) continue;
+        res[pos(c, j)] = z[k][r];
+        pt[pos(c, j)] = point(c, j, z[k][r]);
+      }
+    });
+  } else {
+    for (int e = threadIdx.x; e < n * kCw; e += kThr)
+      smem[(e & (kCw - 1)) * ld + e / kCw] = in[(size_t)(e / kCw) * b.cb + (e & (kCw - 1))];
+    __syncthreads();
+    res = lds_fft(smem, smem + kCw * ld, pl, ld, kCw, -1, tw);
+    pt = res == smem ? smem + kCw * ld : smem;
+    for (int e = threadIdx.x; e < kCw * ldj; e += kThr) {
+      const int c = e & (kCw - 1), j = e / kCw - b.jmax;
+      pt[pos(c, j)] = point(c, j, res[pos(c, j)]);
+    }
   }
   __syncthreads();
   for (int base = 0; base < 2 * b.nsh; base += kThr) {
@@ -296,7 +393,7 @@ __global__ void __launch_bounds__(kThr)
         int j0 = lo > 0 ? isqrt(lo - 1) + 1 : 0;
         if (neg) j0 = max(j0, 1);
         for (int j = j0; j <= j1; j++) {
-          const int at = c * ld + (neg ? n - j : j);
+          const int at = pos(c, neg ? -j : j);
           const float2 p = pt[at], a = res[at];
           q += p.x;
           s2 += p.y;
@@ -409,8 +506,10 @@ int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, con
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
   const int n = b.nsam, nseq = rows_nseq(n);
   const int cols = round8(b.nitem * (b.cb / kCw)), npairs = b.nitem * (n / 2);
-  const size_t lc = sizeof(float2) * 2 * kCw * (n + 1), lr = sizeof(float2) * 2 * nseq * (n + 1);
-  const size_t ls = lc + sizeof(float2) * (b.jmax + 1);
+  const size_t lc = N ? Cols<N>::kLds : sizeof(float2) * 2 * kCw * (n + 1);
+  const size_t lr = N ? Rows<N>::kLds : sizeof(float2) * 2 * nseq * (n + 1);
+  const size_t ls = sizeof(float2) * (b.jmax + 1) +
+                    (N ? std::max(lc, sizeof(float2) * 2 * kCw * (2 * b.jmax + 1)) : lc);
   auto big = [](const void* fn, size_t lds) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   };

@@ -7,8 +7,9 @@
 //
 // Structure: row pass (two real rows packed into one complex sequence),
 // column pass over the JC half-plane columns, both as Stockham autosort FFTs
-// in LDS with radix-4/2/3/5 butterflies and an accurate twiddle table
-// (W_N^k computed on the host in FP64).
+// with an accurate twiddle table (W_N^k computed on the host in FP64): in
+// registers with exchanges through LDS where the length is compiled in, with
+// radix-4/2/3/5 butterflies in LDS where it is not.
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -169,115 +170,112 @@ int row_seqs(int n) {
 // box sizes of the bench and the proposal: 64, 128, 256): every index
 // division and modulus becomes a shift or a constant multiply.
 template <int N>
+using RowFft = Fft<N, 2048 / N, false>;
+template <int N>
+using ColFft = Fft<N, cols_cw<N>(), true>;
+
+template <int N>
 __global__ void __launch_bounds__(kThreads) k_rows_r2c_t(float* data, size_t img_stride,
                                                          int npairs, const float2* __restrict__ tw) {
-  constexpr int NSEQ = 2048 / N, LD = N + 1, JC = N / 2 + 1, PITCH = N + 2;
+  using F = RowFft<N>;
+  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
   extern __shared__ float2 smem[];
-  float2* buf = smem;
-  float2* tmp = smem + NSEQ * LD;
   const int pair0 = blockIdx.x * NSEQ;
-  for (int e = threadIdx.x; e < NSEQ * N; e += kThreads) {
-    const int s = e / N, x = e - s * N;
-    const int pr = pair0 + s;
-    float2 v = f2(0.f, 0.f);
-    if (pr < npairs) {
-      const int img = (2 * pr) / N, row = (2 * pr) % N;
-      const float* ra = data + img * img_stride + (size_t)row * PITCH;
-      v = f2(ra[x], ra[x + PITCH]);
-    }
-    buf[s * LD + x] = v;
-  }
+  // rows of pair pr, as an image's start and the pair's in it
+  auto row = [&](int pr) {
+    return data + (2 * pr / N) * img_stride + (size_t)(2 * pr % N) * PITCH;
+  };
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int s, int i) {
+    const float* ra = row(min(pair0 + s, npairs - 1)) + i;
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) a[it][r] = f2(ra[r * F::TF], ra[r * F::TF + PITCH]);
+  });
+  F::template run<-1, false>(a, z, smem, tw);
   __syncthreads();
-  float2* res = lds_fft_t<N, NSEQ, LD, -1>(buf, tmp, tw);
+  F::template each<F::RL>([&](int it, int s, int i) {
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) smem[F::at(s, i + q * F::TL)] = z[it][q];
+  });
+  __syncthreads();
   for (int e = threadIdx.x; e < NSEQ * JC; e += kThreads) {
     const int s = e / JC, k = e - s * JC;
-    const int pr = pair0 + s;
-    if (pr >= npairs) continue;
-    const float2 zk = res[s * LD + k];
-    const float2 zm = res[s * LD + ((N - k) % N)];
-    const float2 xa = f2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-    const float2 xb = f2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
-    const int img = (2 * pr) / N, row = (2 * pr) % N;
-    float* ra = data + img * img_stride + (size_t)row * PITCH;
-    ra[2 * k] = xa.x;
-    ra[2 * k + 1] = xa.y;
-    ra[PITCH + 2 * k] = xb.x;
-    ra[PITCH + 2 * k + 1] = xb.y;
+    if (pair0 + s >= npairs) continue;
+    float2* ra = reinterpret_cast<float2*>(row(pair0 + s)) + k;
+    split_pair(smem[F::at(s, k)], smem[F::at(s, k ? N - k : 0)], ra[0], ra[JC]);
   }
 }
 
 template <int N>
 __global__ void __launch_bounds__(kThreads) k_rows_c2r_t(float* data, size_t img_stride,
                                                          int npairs, const float2* __restrict__ tw) {
-  constexpr int NSEQ = 2048 / N, LD = N + 1, JC = N / 2 + 1, PITCH = N + 2;
+  using F = RowFft<N>;
+  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
   extern __shared__ float2 smem[];
-  float2* buf = smem;
-  float2* tmp = smem + NSEQ * LD;
   const int pair0 = blockIdx.x * NSEQ;
-  for (int e = threadIdx.x; e < NSEQ * JC; e += kThreads) {
-    const int s = e / JC, k = e - s * JC;
-    const int pr = pair0 + s;
-    float2 a = f2(0.f, 0.f), b = f2(0.f, 0.f);
-    if (pr < npairs) {
-      const int img = (2 * pr) / N, row = (2 * pr) % N;
-      const float* ra = data + img * img_stride + (size_t)row * PITCH;
-      a = f2(ra[2 * k], ra[2 * k + 1]);
-      b = f2(ra[PITCH + 2 * k], ra[PITCH + 2 * k + 1]);
+  auto row = [&](int pr) {
+    return data + (2 * pr / N) * img_stride + (size_t)(2 * pr % N) * PITCH;
+  };
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int s, int i) {
+    const float2* ra = reinterpret_cast<const float2*>(row(min(pair0 + s, npairs - 1)));
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) {
+      const int k = i + r * F::TF, m = 2 * k <= N ? k : N - k;
+      a[it][r] = pair_point(ra[m], ra[m + JC], k, N);
     }
-    if (k == 0 || 2 * k == N) { a.y = 0.f; b.y = 0.f; }
-    buf[s * LD + k] = f2(a.x - b.y, a.y + b.x);
-    if (k > 0 && 2 * k < N) buf[s * LD + (N - k)] = f2(a.x + b.y, -a.y + b.x);
-  }
-  __syncthreads();
-  float2* res = lds_fft_t<N, NSEQ, LD, +1>(buf, tmp, tw);
-  for (int e = threadIdx.x; e < NSEQ * PITCH; e += kThreads) {
-    const int s = e / PITCH, x = e - s * PITCH;
-    const int pr = pair0 + s;
-    if (pr >= npairs) continue;
-    const int img = (2 * pr) / N, row = (2 * pr) % N;
-    float* ra = data + img * img_stride + (size_t)row * PITCH;
-    const float2 z = x < N ? res[s * LD + x] : f2(0.f, 0.f);
-    ra[x] = z.x;
-    ra[PITCH + x] = z.y;
-  }
+  });
+  // every load is in registers once the first exchange's barriers are passed:
+  // the rows may be written in place
+  F::template run<+1, false>(a, z, smem, tw);
+  F::template each<F::RL>([&](int it, int s, int i) {
+    if (pair0 + s >= npairs) return;
+    float* ra = row(pair0 + s);
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) {
+      ra[i + q * F::TL] = z[it][q].x;
+      ra[i + q * F::TL + PITCH] = z[it][q].y;
+    }
+    if (i < 2) ra[N + i] = ra[N + i + PITCH] = 0.f;
+  });
 }
 
 
 template <int N, int SIGN>
 __global__ void __launch_bounds__(kThreads) k_cols_t(float* data, size_t img_stride, int nimg,
                                                      const float2* __restrict__ tw) {
-  constexpr int JC = N / 2 + 1, LD = N + 1;
+  using F = ColFft<N>;
+  constexpr int JC = N / 2 + 1;
   constexpr int CW = cols_cw<N>();
   constexpr int JB = (JC + CW - 1) / CW;
   extern __shared__ float2 smem[];
-  float2* buf = smem;
-  float2* tmp = smem + CW * LD;
   // column blocks of one image in XCD-contiguous order
   const int lb = xcd_block(blockIdx.x, gridDim.x);
   const int img = lb / JB;
   if (img >= nimg) return;
   const int x0 = (lb - img * JB) * CW;
   const int ncol = min(CW, JC - x0);
-  float2* base = reinterpret_cast<float2*>(data + img * img_stride);
-  for (int e = threadIdx.x; e < N * CW; e += kThreads) {
-    const int y = e / CW, c = e - y * CW;
-    float2 v = f2(0.f, 0.f);
-    if (c < ncol) v = base[(size_t)y * JC + x0 + c];
-    buf[c * LD + y] = v;
-  }
-  __syncthreads();
-  float2* res = lds_fft_t<N, CW, LD, SIGN>(buf, tmp, tw);
-  for (int e = threadIdx.x; e < N * CW; e += kThreads) {
-    const int y = e / CW, c = e - y * CW;
-    if (c < ncol) base[(size_t)y * JC + x0 + c] = res[c * LD + y];
-  }
+  float2* base = reinterpret_cast<float2*>(data + img * img_stride) + x0;
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int c, int i) {
+    const float2* col = base + min(c, ncol - 1) + (size_t)i * JC;
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) a[it][r] = col[(size_t)r * F::TF * JC];
+  });
+  F::template run<SIGN, false>(a, z, smem, tw);
+  F::template each<F::RL>([&](int it, int c, int i) {
+    if (c >= ncol) return;
+    float2* col = base + c + (size_t)i * JC;
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) col[(size_t)q * F::TL * JC] = z[it][q];
+  });
 }
 
 template <int N>
 int rows_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, bool fwd, const float2* tw) {
   constexpr int NSEQ = 2048 / N;
   const int npairs = nimg * (N / 2);
-  const size_t lds = sizeof(float2) * 2 * NSEQ * (N + 1);
+  const size_t lds = RowFft<N>::kLds;
   dim3 grid((npairs + NSEQ - 1) / NSEQ);
   if (fwd)
     hipLaunchKernelGGL(k_rows_r2c_t<N>, grid, dim3(kThreads), lds, c.stream, data, img_stride,
@@ -293,7 +291,7 @@ template <int N>
 int cols_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, int sign, const float2* tw) {
   constexpr int JC = N / 2 + 1;
   constexpr int CW = cols_cw<N>();
-  const size_t lds = sizeof(float2) * 2 * CW * (N + 1);
+  const size_t lds = ColFft<N>::kLds;
   const long long nblk = (long long)((JC + CW - 1) / CW) * nimg;
   FR_CHECK(nblk <= (1ll << 30), "too many images in one FFT batch (%d)", nimg);
   dim3 grid(round8((int)nblk));

@@ -1,6 +1,6 @@
 // fr_fft_dev.h -- device building blocks of the batched FFTs: complex
-// helpers, the radix-2/3/4/5 butterflies and the Stockham autosort passes in
-// LDS with the length known at compile time.  Used by the FFT kernels and by
+// helpers, the butterflies and the Stockham autosort passes, with the length
+// known at compile time or at run time.  Used by the FFT kernels and by
 // kernels that run a transform between other work on the same tile.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -18,13 +18,26 @@ constexpr int kFftThreads = 256;  // threads of every workgroup that runs these 
 __device__ inline int xcd_block(int p, int g8) { return (p & 7) * (g8 >> 3) + (p >> 3); }
 inline int round8(int g) { return (g + 7) & ~7; }
 
+// No contraction is left to the compiler in these: it would choose by what
+// surrounds a transform, and the same transform in two kernels would differ in
+// its last bits.
 __device__ inline float2 f2(float a, float b) { return make_float2(a, b); }
-__device__ inline float2 add2(float2 a, float2 b) { return f2(a.x + b.x, a.y + b.y); }
-__device__ inline float2 sub2(float2 a, float2 b) { return f2(a.x - b.x, a.y - b.y); }
-__device__ inline float2 mul2(float2 a, float2 b) {
-  return f2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+__device__ inline float2 add2(float2 a, float2 b) {
+#pragma clang fp contract(off)
+  return f2(a.x + b.x, a.y + b.y);
 }
-__device__ inline float2 scl2(float2 a, float s) { return f2(a.x * s, a.y * s); }
+__device__ inline float2 sub2(float2 a, float2 b) {
+#pragma clang fp contract(off)
+  return f2(a.x - b.x, a.y - b.y);
+}
+__device__ inline float2 mul2(float2 a, float2 b) {
+#pragma clang fp contract(off)
+  return f2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+__device__ inline float2 scl2(float2 a, float s) {
+#pragma clang fp contract(off)
+  return f2(a.x * s, a.y * s);
+}
 // multiply by i*sign
 __device__ inline float2 muli(float2 a, int sign) { return sign > 0 ? f2(-a.y, a.x) : f2(a.y, -a.x); }
 
@@ -41,6 +54,21 @@ __device__ inline void butterfly(float2* u, int sign) {
     u[2] = sub2(a0, b0);
     u[1] = add2(a1, jt);
     u[3] = sub2(a1, jt);
+  } else if constexpr (R == 8) {
+    const float h = 0.70710678118654752440f;
+    float2 e[4] = {u[0], u[2], u[4], u[6]}, o[4] = {u[1], u[3], u[5], u[7]};
+    butterfly<4>(e, sign);
+    butterfly<4>(o, sign);
+    // o[k] times e^{sign i pi k / 4}
+    const float2 j1 = muli(o[1], sign), j3 = muli(o[3], sign);
+    o[1] = scl2(add2(o[1], j1), h);
+    o[2] = muli(o[2], sign);
+    o[3] = scl2(sub2(j3, o[3]), h);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      u[k] = add2(e[k], o[k]);
+      u[k + 4] = sub2(e[k], o[k]);
+    }
   } else if constexpr (R == 3) {
     const float h = 0.86602540378443864676f;
     float2 s = add2(u[1], u[2]), d = sub2(u[1], u[2]);
@@ -68,56 +96,140 @@ __device__ inline void butterfly(float2* u, int sign) {
   }
 }
 
-// Radix of pass i in make_plan's order (0 past the last pass).
-constexpr int radix_at(int n, int i) {
-  int m = n, k = 0;
-  while (m % 4 == 0) { if (k == i) return 4; m /= 4; k++; }
-  while (m % 2 == 0) { if (k == i) return 2; m /= 2; k++; }
-  while (m % 3 == 0) { if (k == i) return 3; m /= 3; k++; }
-  while (m % 5 == 0) { if (k == i) return 5; m /= 5; k++; }
+// ---- transforms whose length is known at compile time
+//
+// A Stockham pass of radix R takes butterfly i (of N / R) of a sequence from the
+// points i + r N / R and leaves it at points N / R apart once it is the last
+// one.  So the first pass takes its points from wherever they are (global
+// memory, a computation) and the last leaves them in registers: LDS only
+// carries the exchanges between passes, two for 8 x 8 x 4 at 256 points, in one
+// buffer (18.5 kB for 2,048 points, so that the waves, not LDS, fill a CU).
+// Radix-4 passes from LDS to LDS, with the tile put there before and read back
+// after, took eight passages through two buffers; a row pass of 512 images of
+// 256^2 ROWS_BEFORE -> ROWS_AFTER us.
+
+// radix of pass i of a length n: eights first, then fours, threes, fives
+constexpr int fft_radix(int n, int i) {
+  int t = 0, m = n;
+  while (m % 2 == 0) { m /= 2; t++; }
+  int n8 = t / 3, n4 = 0, n2 = 0;
+  if (t % 3 == 2) n4 = 1;
+  else if (t % 3 == 1 && n8) { n8--; n4 = 2; }
+  else if (t % 3 == 1) n2 = 1;
+  if (i < n8) return 8;
+  if (i < n8 + n4) return 4;
+  if (i < n8 + n4 + n2) return 2;
+  i -= n8 + n4 + n2;
+  while (m % 3 == 0) { if (i-- == 0) return 3; m /= 3; }
+  while (m % 5 == 0) { if (i-- == 0) return 5; m /= 5; }
   return 0;
 }
 
-template <int R, int N, int P, int NSEQ, int LD, int SIGN>
-__device__ inline void stockham_pass_t(const float2* in, float2* out,
-                                       const float2* __restrict__ tw) {
-  constexpr int T = N / R;
-  constexpr int stride = N / (P * R);
-  for (int b = threadIdx.x; b < NSEQ * T; b += kFftThreads) {
-    const int s = b / T, i = b - s * T;
-    const int k = i % P;
-    const float2* x = in + s * LD;
-    float2 u[R];
+constexpr int fft_npass(int n) {
+  int k = 0;
+  while (fft_radix(n, k)) k++;
+  return k;
+}
+
+// NSEQ sequences of N points by kFftThreads threads.  kCols: neighbouring
+// threads take the same butterfly of neighbouring sequences (columns of an
+// image), else neighbouring butterflies of one sequence.  kRev: the passes in
+// the opposite order; its first pass takes the points where the other order's
+// last pass left them, so that a transform, a step on its points and the
+// transform back need no exchange between them.
+template <int N, int NSEQ, bool kCols, bool kRev = false>
+struct Fft {
+  static constexpr int NP = fft_npass(N);
+  static constexpr int radix(int i) { return fft_radix(N, kRev ? NP - 1 - i : i); }
+  static constexpr int iters(int r) { return (NSEQ * (N / r) + kFftThreads - 1) / kFftThreads; }
+  static constexpr int RF = radix(0), TF = N / RF, IF = iters(RF);            // first pass
+  static constexpr int RL = radix(NP - 1), TL = N / RL, IL = iters(RL);       // last pass
+  // a word after every 8 points and sequences 8 points apart modulo 32: the
+  // strided writes of a pass then fall on different banks, along a sequence
+  // and across columns
+  static constexpr int LP = N + N / 8, LD = LP + (40 - LP % 32) % 32;
+  static constexpr size_t kLds = sizeof(float2) * NSEQ * LD;
+  static __device__ inline int at(int s, int x) { return s * LD + x + (x >> 3); }
+
+  // f(it, s, i) for this thread's butterflies of a pass of radix R
+  template <int R, typename F>
+  static __device__ inline void each(F f) {
+    constexpr int T = N / R;
 #pragma unroll
-    for (int r = 0; r < R; r++) u[r] = x[i + r * T];
-#pragma unroll
-    for (int r = 1; r < R; r++) {
-      float2 w = tw[(r * k * stride) % N];
-      if (SIGN > 0) w.y = -w.y;
-      u[r] = mul2(u[r], w);
+    for (int it = 0; it < iters(R); it++) {
+      const int b = (int)threadIdx.x + it * kFftThreads;
+      if (NSEQ * T % kFftThreads && b >= NSEQ * T) continue;
+      if constexpr (kCols) f(it, b % NSEQ, b / NSEQ);
+      else f(it, b / T, b % T);
     }
-    butterfly<R>(u, SIGN);
-    float2* y = out + s * LD;
-    const int base = (i - k) * R + k;
+  }
+
+  // the passes after pass I's points are in u
+  template <int SIGN, bool kBusy, int I, int P, int IT, int R>
+  static __device__ inline void pass(float2 (&u)[IT][R], float2 (&z)[IL][RL], float2* buf,
+                                     const float2* __restrict__ tw) {
+    each<R>([&](int it, int, int i) {
+      if constexpr (P > 1) {
+        const int k = i % P;
 #pragma unroll
-    for (int q = 0; q < R; q++) y[base + q * P] = u[q];
+        for (int r = 1; r < R; r++) {
+          float2 w = tw[r * k * (N / (P * R))];
+          if (SIGN > 0) w.y = -w.y;
+          u[it][r] = mul2(u[it][r], w);
+        }
+      }
+      butterfly<R>(u[it], SIGN);
+    });
+    if constexpr (I == NP - 1) {
+#pragma unroll
+      for (int it = 0; it < IT; it++)
+#pragma unroll
+        for (int r = 0; r < R; r++) z[it][r] = u[it][r];
+    } else {
+      if (kBusy || I > 0) __syncthreads();
+      each<R>([&](int it, int s, int i) {
+        const int k = i % P, base = (i - k) * R + k;
+#pragma unroll
+        for (int q = 0; q < R; q++) buf[at(s, base + q * P)] = u[it][q];
+      });
+      __syncthreads();
+      constexpr int R2 = radix(I + 1), T2 = N / R2;
+      float2 v[iters(R2)][R2];
+      each<R2>([&](int it, int s, int i) {
+#pragma unroll
+        for (int r = 0; r < R2; r++) v[it][r] = buf[at(s, i + r * T2)];
+      });
+      pass<SIGN, kBusy, I + 1, P * R>(v, z, buf, tw);
+    }
   }
+
+  // a[it][r]: point i + r TF of butterfly (it, s, i) of each<RF>; z[it][q]: point
+  // i + q TL of each<RL>.  kBusy: other threads may still read buf.  They read it
+  // after the return too: a barrier before it is written again.
+  template <int SIGN, bool kBusy>
+  static __device__ inline void run(float2 (&a)[IF][RF], float2 (&z)[IL][RL], float2* buf,
+                                    const float2* __restrict__ tw) {
+    pass<SIGN, kBusy, 0, 1>(a, z, buf, tw);
+  }
+};
+
+// The point k of the sequence that carries two half spectra a and b (of N real
+// values each) as Z = A + i B, from the half planes' points (k or N - k): the
+// imaginary parts at k = 0 and N/2 are ignored, as the c2r does.
+__device__ inline float2 pair_point(float2 a, float2 b, int k, int n) {
+#pragma clang fp contract(off)
+  if (k == 0 || 2 * k == n) a.y = b.y = 0.f;
+  return 2 * k <= n ? make_float2(a.x - b.y, a.y + b.x) : make_float2(a.x + b.y, -a.y + b.x);
 }
 
-template <int N, int NSEQ, int LD, int SIGN, int I = 0, int P = 1>
-__device__ inline float2* lds_fft_t(float2* buf, float2* tmp, const float2* __restrict__ tw) {
-  constexpr int R = radix_at(N, I);
-  if constexpr (R == 0) {
-    return buf;
-  } else {
-    stockham_pass_t<R, N, P, NSEQ, LD, SIGN>(buf, tmp, tw);
-    __syncthreads();
-    return lds_fft_t<N, NSEQ, LD, SIGN, I + 1, P * R>(tmp, buf, tw);
-  }
+// The two half spectra's points k from Z_k and Z_{N-k}.
+__device__ inline void split_pair(float2 zk, float2 zm, float2& a, float2& b) {
+#pragma clang fp contract(off)
+  a = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
+  b = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
 }
 
-
-// ---- the same passes with the length known at run time
+// ---- radix-2/3/4/5 passes from LDS to LDS with the length known at run time
 constexpr int kMaxPass = 12;
 
 struct Plan {

@@ -110,60 +110,66 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
     k_cols_shift(float2* spec, const float* __restrict__ ppar, float2* outc, float2* datc, int nb,
                  const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int JC = N / 2 + 1, LD = N + 1, CW = cols_cw<N>();
+  constexpr int JC = N / 2 + 1, CW = cols_cw<N>();
   constexpr int JB = (JC + CW - 1) / CW;
   constexpr size_t IC = (size_t)N * JC;
+  using F = Fft<N, CW, true>;         // forward
+  using G = Fft<N, CW, true, true>;   // backward, from where the forward leaves its points
+  static_assert(G::RF == F::RL && G::IF == F::IL, "the passes do not meet");
   extern __shared__ float2 cs_smem[];
-  float2* buf = cs_smem;
-  float2* tmp = cs_smem + CW * LD;
   // column blocks of one particle in XCD-contiguous order
   const int lb = xcd_block(blockIdx.x, gridDim.x);
   const int b = lb / JB;
   if (b >= nb) return;
   const int x0 = (lb - b * JB) * CW;
   const int ncol = min(CW, JC - x0);
-  float2* sp = spec + (size_t)b * IC;
-  for (int e = threadIdx.x; e < N * CW; e += kFftThreads) {
-    const int y = e / CW, c = e - y * CW;
-    float2 v = make_float2(0.f, 0.f);
-    if (c < ncol) v = sp[(size_t)y * JC + x0 + c];
-    buf[c * LD + y] = v;
-  }
-  __syncthreads();
-  float2* res = buf;
-  if constexpr (kFwd) {
-    res = lds_fft_t<N, CW, LD, -1>(buf, tmp, tw);
-    for (int e = threadIdx.x; e < N * CW; e += kFftThreads) {
-      const int y = e / CW, c = e - y * CW;
-      if (c < ncol) sp[(size_t)y * JC + x0 + c] = res[c * LD + y];
-    }
-  }
-  float2* oth = res == buf ? tmp : buf;
+  float2* sp = spec + (size_t)b * IC + x0;
   const float* pp = ppar + 8 * b;
-  float2* dc = datc + (size_t)b * IC;
-  // each thread rewrites only the entries it read: no barrier before this loop
-  for (int e = threadIdx.x; e < N * CW; e += kFftThreads) {
-    const int y = e / CW, c = e - y * CW;
-    if (c >= ncol) continue;
-    float2 v, d;
-    shift_point(pp, x0 + c, y >= JC ? y - N : y, res[c * LD + y], v, d);
-    res[c * LD + y] = v;
-    dc[(size_t)y * JC + x0 + c] = d;
+  float2* dc = datc + (size_t)b * IC + x0;
+  float2* oc = outc + (size_t)b * IC + x0;
+  float2 z[F::IL][F::RL];
+  if constexpr (kFwd) {
+    float2 a[F::IF][F::RF];
+    F::template each<F::RF>([&](int it, int c, int i) {
+      const float2* col = sp + min(c, ncol - 1) + (size_t)i * JC;
+#pragma unroll
+      for (int r = 0; r < F::RF; r++) a[it][r] = col[(size_t)r * F::TF * JC];
+    });
+    F::template run<-1, false>(a, z, cs_smem, tw);
+  } else {
+    F::template each<F::RL>([&](int it, int c, int i) {
+      const float2* col = sp + min(c, ncol - 1) + (size_t)i * JC;
+#pragma unroll
+      for (int q = 0; q < F::RL; q++) z[it][q] = col[(size_t)q * F::TL * JC];
+    });
   }
-  __syncthreads();
-  float2* out = lds_fft_t<N, CW, LD, +1>(res, oth, tw);
-  float2* oc = outc + (size_t)b * IC;
-  for (int e = threadIdx.x; e < N * CW; e += kFftThreads) {
-    const int y = e / CW, c = e - y * CW;
-    if (c < ncol) oc[(size_t)y * JC + x0 + c] = out[c * LD + y];
-  }
+  F::template each<F::RL>([&](int it, int c, int i) {
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) {
+      const int y = i + q * F::TL;
+      const float2 p = z[it][q];
+      float2 d;
+      shift_point(pp, x0 + c, y >= JC ? y - N : y, p, z[it][q], d);
+      if (c < ncol) {
+        if constexpr (kFwd) sp[(size_t)y * JC + c] = p;
+        dc[(size_t)y * JC + c] = d;
+      }
+    }
+  });
+  float2 o[G::IL][G::RL];
+  G::template run<+1, true>(z, o, cs_smem, tw);
+  G::template each<G::RL>([&](int it, int c, int i) {
+    if (c >= ncol) return;
+#pragma unroll
+    for (int q = 0; q < G::RL; q++) oc[(size_t)(i + q * G::TL) * JC + c] = o[it][q];
+  });
 }
 
 template <int N>
 int cols_shift_t(Ctx& c, int nb, float* spec, bool fwd, const float* ppar, float* outc,
                  float* datc) {
   constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw<N>();
-  const size_t lds = sizeof(float2) * 2 * CW * (N + 1);
+  const size_t lds = fftdev::Fft<N, CW, true>::kLds;
   const float2* tw = c.twiddles(N);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
   FR_CHECK(nb <= 65535, "too many images in one FFT batch (%d)", nb);
@@ -203,59 +209,55 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
                     float ri2, float ri3, float scal, float2* part,
                     const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int NSEQ = 2048 / N, LD = N + 1, JC = N / 2 + 1, PITCH = N + 2;
+  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
+  using F = Fft<N, NSEQ, false>;
   extern __shared__ float2 rr_smem[];
   __shared__ float red_s[kFftThreads / 64];
   __shared__ int red_c[kFftThreads / 64];
-  float2* buf = rr_smem;
-  float2* tmp = rr_smem + NSEQ * LD;
   const int pair0 = blockIdx.x * NSEQ;
-  for (int e = threadIdx.x; e < NSEQ * JC; e += kFftThreads) {
-    const int s = e / JC, k = e - s * JC;
-    const int pr = pair0 + s;
-    float2 a = make_float2(0.f, 0.f), b = make_float2(0.f, 0.f);
-    if (pr < npairs) {
-      const int img = (2 * pr) / N, row = (2 * pr) % N;
-      const float* ra = data + img * img_stride + (size_t)row * PITCH;
-      a = make_float2(ra[2 * k], ra[2 * k + 1]);
-      b = make_float2(ra[PITCH + 2 * k], ra[PITCH + 2 * k + 1]);
+  auto rows = [&](int pr) {
+    return data + (2 * pr / N) * img_stride + (size_t)(2 * pr % N) * PITCH;
+  };
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int s, int i) {
+    const float2* ra = reinterpret_cast<const float2*>(rows(min(pair0 + s, npairs - 1)));
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) {
+      const int k = i + r * F::TF, m = 2 * k <= N ? k : N - k;
+      a[it][r] = pair_point(ra[m], ra[m + JC], k, N);
     }
-    if (k == 0 || 2 * k == N) { a.y = 0.f; b.y = 0.f; }
-    buf[s * LD + k] = make_float2(a.x - b.y, a.y + b.x);
-    if (k > 0 && 2 * k < N) buf[s * LD + (N - k)] = make_float2(a.x + b.y, -a.y + b.x);
-  }
-  __syncthreads();
-  float2* res = lds_fft_t<N, NSEQ, LD, +1>(buf, tmp, tw);
+  });
+  F::template run<+1, false>(a, z, rr_smem, tw);
   const int img0 = (2 * pair0) / N;
   const float amagp = ppar[8 * (size_t)img0 + 5];
   const float ri2p = ri2 / amagp / amagp, ri3p = ri3 / amagp / amagp;
   const int nmid = N / 2 + 1;
   float sum = 0.f;
   int cnt = 0;
-  for (int e = threadIdx.x; e < NSEQ * PITCH; e += kFftThreads) {
-    const int s = e / PITCH, x = e - s * PITCH;
-    const int pr = pair0 + s;
-    if (pr >= npairs) continue;
-    const int img = (2 * pr) / N, row = (2 * pr) % N;
-    float* ra = data + img * img_stride + (size_t)row * PITCH;
-    if (x >= N) continue;  // the row padding is not read again
-    const float2 z = res[s * LD + x];
-    // pixels beyond RI3' become the ring mean in the masked r2c, which does
-    // not read them: only those within RI3' are stored
-    const float ca = maskcos_r2(row, x, nmid), cb = maskcos_r2(row + 1, x, nmid);
-    if (ca <= ri3p) ra[x] = z.x;
-    if (cb <= ri3p) ra[PITCH + x] = z.y;
-    {
+  // the row padding is not read again
+  F::template each<F::RL>([&](int it, int s, int i) {
+    if (pair0 + s >= npairs) return;
+    const int row = (2 * (pair0 + s)) % N;
+    float* ra = rows(pair0 + s);
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) {
+      const int x = i + q * F::TL;
+      const float2 v = z[it][q];
+      // pixels beyond RI3' become the ring mean in the masked r2c, which does
+      // not read them: only those within RI3' are stored
+      const float ca = maskcos_r2(row, x, nmid), cb = maskcos_r2(row + 1, x, nmid);
+      if (ca <= ri3p) ra[x] = v.x;
+      if (cb <= ri3p) ra[PITCH + x] = v.y;
       if (ca > ri2p && ca <= ri3p) {
-        sum += z.x * scal;
+        sum += v.x * scal;
         cnt++;
       }
       if (cb > ri2p && cb <= ri3p) {
-        sum += z.y * scal;
+        sum += v.y * scal;
         cnt++;
       }
     }
-  }
+  });
   for (int off = 32; off > 0; off >>= 1) {
     sum += __shfl_down(sum, off, 64);
     cnt += __shfl_down(cnt, off, 64);
@@ -287,11 +289,13 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
                     float ri2, float ri3, float rih, float halfw, float scal,
                     const float2* __restrict__ part, const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int NSEQ = 2048 / N, LD = N + 1, JC = N / 2 + 1, PITCH = N + 2;
+  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
   constexpr int WPI = (N / 2) / NSEQ;  // row blocks per image
+  using F = Fft<N, NSEQ, false>;
   extern __shared__ float2 rm_smem[];
-  float2* buf = rm_smem;
-  float2* tmp = rm_smem + NSEQ * LD;
+  auto rows = [&](int pr) {
+    return data + (2 * pr / N) * img_stride + (size_t)(2 * pr % N) * PITCH;
+  };
   const int pair0 = blockIdx.x * NSEQ;
   const int img0 = (2 * pair0) / N;
   float tot = 0.f;
@@ -314,36 +318,31 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
     }
     return v;
   };
-  for (int e = threadIdx.x; e < NSEQ * N; e += kFftThreads) {
-    const int s = e / N, x = e - s * N;
-    const int pr = pair0 + s;
-    float2 v = make_float2(0.f, 0.f);
-    if (pr < npairs) {
-      const int img = (2 * pr) / N, row = (2 * pr) % N;
-      const float* ra = data + img * img_stride + (size_t)row * PITCH;
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int s, int i) {
+    const int pr = min(pair0 + s, npairs - 1), row = (2 * pr) % N;
+    const float* ra = rows(pr);
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) {
+      const int x = i + r * F::TF;
       // beyond RI3' the pixel is the mean: k_rows_c2r_ring did not store it
       const float ca = maskcos_r2(row, x, nmid), cb = maskcos_r2(row + 1, x, nmid);
-      v = make_float2(ca > ri3p ? mean : mask(ra[x] * scal, ca),
-                      cb > ri3p ? mean : mask(ra[x + PITCH] * scal, cb));
+      a[it][r] = make_float2(ca > ri3p ? mean : mask(ra[x] * scal, ca),
+                             cb > ri3p ? mean : mask(ra[x + PITCH] * scal, cb));
     }
-    buf[s * LD + x] = v;
-  }
+  });
+  F::template run<-1, false>(a, z, rm_smem, tw);
   __syncthreads();
-  float2* res = lds_fft_t<N, NSEQ, LD, -1>(buf, tmp, tw);
+  F::template each<F::RL>([&](int it, int s, int i) {
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) rm_smem[F::at(s, i + q * F::TL)] = z[it][q];
+  });
+  __syncthreads();
   for (int e = threadIdx.x; e < NSEQ * JC; e += kFftThreads) {
     const int s = e / JC, k = e - s * JC;
-    const int pr = pair0 + s;
-    if (pr >= npairs) continue;
-    const float2 zk = res[s * LD + k];
-    const float2 zm = res[s * LD + ((N - k) % N)];
-    const float2 xa = make_float2(0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y));
-    const float2 xb = make_float2(0.5f * (zk.y + zm.y), -0.5f * (zk.x - zm.x));
-    const int img = (2 * pr) / N, row = (2 * pr) % N;
-    float* ra = data + img * img_stride + (size_t)row * PITCH;
-    ra[2 * k] = xa.x;
-    ra[2 * k + 1] = xa.y;
-    ra[PITCH + 2 * k] = xb.x;
-    ra[PITCH + 2 * k + 1] = xb.y;
+    if (pair0 + s >= npairs) continue;
+    float2* ra = reinterpret_cast<float2*>(rows(pair0 + s)) + k;
+    split_pair(rm_smem[F::at(s, k)], rm_smem[F::at(s, k ? N - k : 0)], ra[0], ra[JC]);
   }
 }
 
@@ -354,7 +353,7 @@ int rows_mask_t(Ctx& c, int nb, float* outc, const float* ppar, const PrepGlobal
                 float2* part) {
   constexpr int NSEQ = 2048 / N;
   const int npairs = nb * (N / 2);
-  const size_t lds = sizeof(float2) * 2 * NSEQ * (N + 1);
+  const size_t lds = fftdev::Fft<N, NSEQ, false>::kLds;
   const size_t img = (size_t)N * (N + 2);
   const float2* tw = c.twiddles(N);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
