@@ -70,7 +70,7 @@ const float2* Ctx::twiddles(int n) {
 }
 
 float2* Ctx::prep_partials() {
-  if (!prep_part && hipMalloc(&prep_part, sizeof(float2) * 65535 * 16) != hipSuccess)
+  if (!prep_part && hipMalloc(&prep_part, sizeof(float2) * (kRingPartials + kShellPartials)) != hipSuccess)
     prep_part = nullptr;
   return prep_part;
 }

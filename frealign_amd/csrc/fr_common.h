@@ -43,10 +43,12 @@ struct Ctx {
   void prof_end(int slot);
   int ensure_scratch(size_t bytes);
   const float2* twiddles(int n);
-  // the particle preparation's per-row-block ring sums (fr_prep.hip) for
-  // calls on the context's stream: one fixed allocation for the largest
-  // batch (65535 images x 16 row blocks), made on first use and kept (plans,
-  // whose graphs replay on their own streams, bring their own buffer)
+  // the particle preparation's per-row-block ring sums and its shell sums
+  // (fr_prep.hip) for calls on the context's stream: one fixed allocation for
+  // the largest batch (65535 images x 16 row blocks; 32 MB of shells), made on
+  // first use and kept (plans, whose graphs replay on their own streams, bring
+  // their own buffer)
+  static constexpr size_t kRingPartials = 65535 * 16, kShellPartials = (32u << 20) / sizeof(float2);
   float2* prep_part = nullptr;
   float2* prep_partials();
   ~Ctx();
@@ -95,7 +97,5 @@ bool fft_supported(int nsam);
 // the row pass alone (forward r2c of the rows, or backward c2r), for callers
 // that run the column pass themselves
 int fft_rows_2d(Ctx& c, int nsam, int nimg, float* data, size_t img_stride, bool fwd);
-// the column pass alone (sign -1 forward, +1 backward)
-int fft_cols_2d(Ctx& c, int nsam, int nimg, float* data, size_t img_stride, int sign);
 
 }  // namespace fr

@@ -368,11 +368,6 @@ int fft_rows_2d(Ctx& c, int nsam, int nimg, float* data, size_t img_stride, bool
   return rows_pass(c, nsam, nimg, data, img_stride, fwd);
 }
 
-int fft_cols_2d(Ctx& c, int nsam, int nimg, float* data, size_t img_stride, int sign) {
-  if (nimg <= 0) return 0;
-  return cols_pass(c, nsam, nimg, data, img_stride, sign);
-}
-
 int fft_r2c_2d(Ctx& c, int nsam, int nimg, float* data, size_t img_stride) {
   if (nimg <= 0) return 0;
   if (int r = rows_pass(c, nsam, nimg, data, img_stride, true)) return r;

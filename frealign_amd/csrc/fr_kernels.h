@@ -78,7 +78,7 @@ struct PrepGlobals {
   float cs, wl, wgh1, wgh2, thetatr, rih, halfw, ri2, ri3, tx, ty;
   int ictf;
 };
-// part: the ring partial sums of MASKCOS's mean (prep_partials_count(nsam,
+// part: MASKCOS's ring sums and PWEIGHT's shell sums (prep_partials_count(nsam,
 // nb) float2; null: the context's buffer, for calls on the context's stream)
 int launch_prep(Ctx& c, int nsam, int nb, float* data, const float* ppar, const float* pssnr,
                 const PrepGlobals& g, float* ctff, float* outc, float* datc,

@@ -7,14 +7,17 @@
 // in-place double weighting of the Nyquist row and its JC+1 shell aliasing
 // into bin 1's count (the reference calls PWEIGHT(NSAM,OUTC,OUTC,...)).
 //
-// For NSAM 64, 128 and 256 the steps run as seven launches: the CTF table;
-// the r2c's row pass; one column pass that completes the r2c (written back
-// into the image), applies the shift and writes DATC, and runs OUTC's
-// backward column pass; the row c2r, which also sums each row block's part
-// of MASKCOS's ring; the row r2c, which scales and masks as it loads; the
-// forward column pass; the origin shift and PWEIGHT.  Other sizes take the
-// FFT entry points and one kernel per step.
+// For NSAM 64, 128 and 256 the steps run as seven launches: the r2c's row pass;
+// one column pass that completes the r2c (written back into the image), applies
+// the shift and writes DATC, and runs OUTC's backward column pass; the row c2r,
+// which also sums each row block's part of MASKCOS's ring; the row r2c, which
+// scales and masks as it loads; the forward column pass, which also sums each
+// column block's part of PWEIGHT's shells; the shells; the CTF table with the
+// origin shift and PWEIGHT's weights.  Other sizes take the FFT entry points and
+// one kernel per step.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "fr_common.h"
 #include "fr_kernels.h"
@@ -77,24 +80,6 @@ __global__ void __launch_bounds__(kThreads)
   ctff[(size_t)b * 2 * ic + ic + id] = cl;
 }
 
-// ctfapply.f:64-76 alone: the CTF table, one thread per half-plane point
-// (coalesced stores; the fused column pass below applies the shift)
-__global__ void __launch_bounds__(kThreads)
-    k_ctf_table(int nsam, int nb, const float* __restrict__ ppar, PrepGlobals g, float2* ctff) {
-  const int jc = nsam / 2 + 1;
-  const size_t ic = (size_t)nsam * jc;
-  const size_t gid = blockIdx.x * (size_t)kThreads + threadIdx.x;
-  if (gid >= ic * nb) return;
-  const int b = (int)(gid / ic);
-  const int id = (int)(gid - (size_t)b * ic);
-  const int l = id % jc, m = id / jc;
-  const int mm = m >= jc ? m - nsam : m;
-  float2 cr, cl;
-  ctf_point(g, ppar + 8 * b, l, mm, cr, cl);
-  ctff[(size_t)b * 2 * ic + id] = cr;
-  ctff[(size_t)b * 2 * ic + ic + id] = cl;
-}
-
 // The shift step between two column passes, for the box sizes whose FFT
 // length is a compile-time constant: a workgroup takes CW half-plane columns
 // of one particle.  kFwd: `spec` holds the row transforms only; the forward
@@ -104,7 +89,7 @@ __global__ void __launch_bounds__(kThreads)
 // the backward column transform of OUTC, which the row pass completes.  Each
 // value takes the operations of the separate column passes and k_ctf_shift,
 // in their order; two HBM round trips of the batch's spectra are saved.  The
-// CTF table, which needs no spectrum, comes from k_ctf_table.
+// CTF table, which needs no spectrum, is formed where it is used (k_ctf_weight).
 template <int N, bool kFwd>
 __global__ void __launch_bounds__(fftdev::kFftThreads)
     k_cols_shift(float2* spec, const float* __restrict__ ppar, float2* outc, float2* datc, int nb,
@@ -368,18 +353,208 @@ int rows_mask_t(Ctx& c, int nb, float* outc, const float* ppar, const PrepGlobal
   return 0;
 }
 
+// ---- PWEIGHT (pweight.f) on the fused path, in three steps over the whole GPU
+// where one workgroup per particle went over its plane twice: k_cols_shells
+// completes OUTC's transform and, with a block of columns at hand, sums its part
+// of the shells; k_pw_shells adds the blocks and takes the roots; k_ctf_weight
+// weights each point and forms the CTF table there, which PWEIGHT needs and which
+// was written before the FFTs and read back here.  512 images of 256^2: 365 us as
+// table (119), column pass (50) and weighting (197), 239 us like this.
+
+// largest j >= 0 with j*j <= v (v >= 0, below 2^20)
+__device__ inline int isqrt(int v) {
+  int j = (int)sqrtf((float)v);
+  if (j * j > v) j--;
+  if ((j + 1) * (j + 1) <= v) j++;
+  return j;
+}
+
+// The forward column pass of OUTC with the shells' parts: shell s (bin s + 1) is
+// the points s^2-s+1 <= r^2 <= s^2+s below JC^2, a run of J per column; a thread
+// takes a shell's points of one sign of J in order.  The Nyquist row is J = N/2
+// and -N/2 (pweight.f:31-42), so both threads count it.  part[block][s] = (sum of
+// |X|^2, count).
+template <int N>
+__global__ void __launch_bounds__(fftdev::kFftThreads)
+    k_cols_shells(float2* data, int nb, float2* part, const float2* __restrict__ tw) {
+  using namespace fftdev;
+  constexpr int JC = N / 2 + 1, CW = cols_cw<N>(), JB = (JC + CW - 1) / CW, LH = N + 1;
+  using F = Fft<N, CW, true>;
+  extern __shared__ float2 cp_smem[];
+  const int lb = xcd_block(blockIdx.x, gridDim.x);
+  const int img = lb / JB;
+  if (img >= nb) return;
+  const int x0 = (lb - img * JB) * CW;
+  const int ncol = min(CW, JC - x0);
+  float2* base = data + (size_t)img * N * JC + x0;
+  float2 a[F::IF][F::RF], z[F::IL][F::RL];
+  F::template each<F::RF>([&](int it, int c, int i) {
+    const float2* col = base + min(c, ncol - 1) + (size_t)i * JC;
+#pragma unroll
+    for (int r = 0; r < F::RF; r++) a[it][r] = col[(size_t)r * F::TF * JC];
+  });
+  F::template run<-1, false>(a, z, cp_smem, tw);
+  __syncthreads();
+  float* h2 = reinterpret_cast<float*>(cp_smem);
+  static_assert(sizeof(float) * CW * LH <= F::kLds, "the squares do not fit");
+  F::template each<F::RL>([&](int it, int c, int i) {
+#pragma unroll
+    for (int q = 0; q < F::RL; q++) {
+      const int y = i + q * F::TL;
+      if (c < ncol) base[c + (size_t)y * JC] = z[it][q];
+      const float h = hypotf(z[it][q].x, z[it][q].y);
+      h2[c * LH + y] = h * h;
+    }
+  });
+  __syncthreads();
+  for (int e = threadIdx.x; e < 2 * (JC + 1); e += kFftThreads) {
+    const int s = e >> 1, neg = e & 1;
+    float sum = 0.f, cnt = 0.f;
+    for (int c = 0; c < ncol; c++) {
+      const int l = x0 + c, hi = min(s * s + s, JC * JC - 1) - l * l;
+      if (hi < 0) break;
+      const int lo = (s ? s * s - s + 1 : 0) - l * l;
+      const int j1 = isqrt(hi);
+      int j = lo > 0 ? isqrt(lo - 1) + 1 : 0;
+      if (neg) j = max(j, 1);
+      for (; j <= j1; j++) {
+        sum += h2[c * LH + (neg ? N - j : j)];
+        cnt += 1.0f;
+      }
+    }
+    sum += __shfl_xor(sum, 1, 64);
+    cnt += __shfl_xor(cnt, 1, 64);
+    if (!neg) part[(size_t)lb * (JC + 1) + s] = make_float2(sum, cnt);
+  }
+}
+
+// RBUF(1..JC+1) of pweight.f per particle, from its column blocks' parts in
+// order: bins 1..JC are roots of the mean power (1 where it is zero), bin JC+1
+// its sum plus the count of bin 1, whose slot it shares.
+__global__ void __launch_bounds__(kThreads)
+    k_pw_shells(int jc, int jb, const float2* __restrict__ part, float* rbuf) {
+  const float2* p = part + (size_t)blockIdx.x * jb * (jc + 1);
+  float* rb = rbuf + (size_t)blockIdx.x * (jc + 2);
+  auto shell = [&](int s) {
+    float2 t = make_float2(0.f, 0.f);
+    for (int k = 0; k < jb; k++) {
+      const float2 q = p[(size_t)k * (jc + 1) + s];
+      t.x += q.x;
+      t.y += q.y;
+    }
+    return t;
+  };
+  const float2 last = threadIdx.x == 0 ? shell(jc) : make_float2(0.f, 0.f);
+  for (int s = threadIdx.x; s < jc; s += kThreads) {
+    float2 t = shell(s);
+    if (s == 0) {
+      t.y += last.x;
+      rb[jc + 1] = t.y;
+    }
+    float v = t.x;
+    if (t.y != 0.0f) v = sqrtf(v / t.y);
+    rb[s + 1] = v == 0.0f ? 1.0f : v;
+  }
+}
+
+// ctfapply.f:64-76's CTF table and, with it, ctfapply.f:144-158: PWEIGHT's
+// weights and the origin shift of OUTC, one thread per half-plane point.  The
+// Nyquist row takes the weight twice (pweight.f visits it at both signs of J, in
+// place).
+template <int N>
+__global__ void __launch_bounds__(kThreads)
+    k_ctf_weight(const float* __restrict__ ppar, const float* __restrict__ pssnr, PrepGlobals g,
+                 const float* __restrict__ rbuf, float2* ctff, float2* outc) {
+  constexpr int JC = N / 2 + 1, IC = N * JC;
+  const int e = blockIdx.x * kThreads + threadIdx.x, b = blockIdx.y;
+  if (e >= IC) return;
+  const int m = e / JC, l = e - m * JC, mm = m >= JC ? m - N : m;
+  float2 cr, cl;
+  ctf_point(g, ppar + 8 * b, l, mm, cr, cl);
+  float2* cp = ctff + (size_t)b * 2 * IC + e;
+  cp[0] = cr;
+  cp[IC] = cl;
+  const int itemp = l * l + mm * mm;
+  float2* oc = outc + (size_t)b * IC + e;
+  float2 o = make_float2(0.f, 0.f);
+  if (itemp < JC * JC) {
+    const int ibin = (int)(sqrtf((float)itemp) + 0.5f) + 1;
+    o = *oc;
+    const float sg = ((l + mm) & 1) ? -1.0f : 1.0f;
+    float snr = pssnr[ibin - 1];
+    if (g.ictf == 1) {
+      const float h = hypotf(cr.x + cl.x, cr.y - cl.y);
+      snr = snr * (h * h);
+    }
+    const float wgt = snr / (snr + 1.0f) / rbuf[(size_t)b * (JC + 2) + ibin];
+    o.x = o.x * sg * wgt;
+    o.y = o.y * sg * wgt;
+    if (2 * m == N) {
+      o.x *= wgt;
+      o.y *= wgt;
+    }
+  }
+  *oc = o;
+}
+
+// Scratch of the three steps: the parts and RBUF of as many images as 32 MB hold
+// (1,800 of 256^2); more images go in several rounds.
+constexpr size_t kPwBytes = Ctx::kShellPartials * sizeof(float2);
+
+size_t pw_image_bytes(int nsam) {
+  const int jc = nsam / 2 + 1, cw = std::min(2048 / nsam, jc), jb = (jc + cw - 1) / cw;
+  return sizeof(float2) * jb * (jc + 1) + sizeof(float) * (jc + 2);
+}
+
+int pw_chunk(int nsam, int nb) {
+  return (int)std::min<size_t>(nb, kPwBytes / pw_image_bytes(nsam));
+}
+
+template <int N>
+int pweight_t(Ctx& c, int nb, const float* ppar, const float* pssnr, const PrepGlobals& g,
+              float* ctff, float* outc, float2* pw) {
+  constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw<N>(), JB = (JC + CW - 1) / CW;
+  constexpr size_t IC = (size_t)N * JC;
+  const float2* tw = c.twiddles(N);
+  FR_CHECK(tw != nullptr, "twiddle table allocation failed");
+  const int chunk = pw_chunk(N, nb);
+  float* rbuf = reinterpret_cast<float*>(pw + (size_t)chunk * JB * (JC + 1));
+  for (int b0 = 0; b0 < nb; b0 += chunk) {
+    const int n = std::min(chunk, nb - b0);
+    float2* oc = reinterpret_cast<float2*>(outc) + IC * b0;
+    hipLaunchKernelGGL(k_cols_shells<N>, dim3(fftdev::round8(JB * n)), dim3(fftdev::kFftThreads),
+                       (fftdev::Fft<N, CW, true>::kLds), c.stream, oc, n, pw, tw);
+    FR_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_pw_shells, dim3(n), dim3(kThreads), 0, c.stream, JC, JB, pw, rbuf);
+    FR_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_ctf_weight<N>, dim3((unsigned)((IC + kThreads - 1) / kThreads), n),
+                       dim3(kThreads), 0, c.stream, ppar + 8 * (size_t)b0, pssnr, g, rbuf,
+                       reinterpret_cast<float2*>(ctff) + 2 * IC * b0, oc);
+    FR_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
 bool fused_cols(int nsam) { return nsam == 64 || nsam == 128 || nsam == 256; }
+
+// the ring sums' buffer, and the PWEIGHT scratch after it: the caller's, or the
+// context's for its largest batch
+int fused_scratch(Ctx& c, int nsam, int nb, float2*& part, float2*& pw) {
+  FR_CHECK(nb <= 65535, "too many images in one batch (%d)", nb);
+  if (part) {
+    pw = part + (size_t)nsam * nsam / 4096 * nb;
+    return 0;
+  }
+  part = c.prep_partials();
+  FR_CHECK(part != nullptr, "preparation buffer allocation failed");
+  pw = part + Ctx::kRingPartials;
+  return 0;
+}
 
 // the fused path's column pass with the shift (fwd: completing the forward
 // transform first), then OUTC's c2r, MASKCOS and r2c rows
 int fused_shift_mask(Ctx& c, int nsam, int nb, float* spec, bool fwd, const float* ppar,
                      const PrepGlobals& g, float* outc, float* datc, float2* part) {
-  if (!part) {
-    // the context's buffer holds 65535 images' sums
-    FR_CHECK(nb <= 65535, "too many images in one batch (%d)", nb);
-    part = c.prep_partials();
-    FR_CHECK(part != nullptr, "preparation buffer allocation failed");
-  }
   switch (nsam) {
     case 64:
       if (int r = cols_shift_t<64>(c, nb, spec, fwd, ppar, outc, datc)) return r;
@@ -613,31 +788,25 @@ int origin_pweight(Ctx& c, int nsam, int nb, const float* pssnr, const PrepGloba
   return 0;
 }
 
-// the CTF table (first on the fused path: the passes after it then read what
-// the pass before them wrote, while it is still in the caches)
-int ctf_table(Ctx& c, int nsam, int nb, const float* ppar, const PrepGlobals& g, float* ctff) {
-  const size_t tot = (size_t)nsam * (nsam / 2 + 1) * nb;
-  hipLaunchKernelGGL(k_ctf_table, dim3((unsigned)((tot + kThreads - 1) / kThreads)),
-                     dim3(kThreads), 0, c.stream, nsam, nb, ppar, g,
-                     reinterpret_cast<float2*>(ctff));
-  FR_HIP(hipGetLastError());
-  return 0;
-}
-
-// the fused path after its row passes: OUTC's forward column pass, the
-// origin shift and PWEIGHT
-int fused_tail(Ctx& c, int nsam, int nb, const float* pssnr, const PrepGlobals& g,
-               const float* ctff, float* outc) {
-  if (int r = fft_cols_2d(c, nsam, nb, outc, (size_t)nsam * (nsam + 2), -1)) return r;
-  return origin_pweight(c, nsam, nb, pssnr, g, ctff, outc);
+// the fused path after its row passes: OUTC's forward column pass, the origin
+// shift, the CTF table and PWEIGHT
+int fused_tail(Ctx& c, int nsam, int nb, const float* ppar, const float* pssnr,
+               const PrepGlobals& g, float* ctff, float* outc, float2* pw) {
+  switch (nsam) {
+    case 64: return pweight_t<64>(c, nb, ppar, pssnr, g, ctff, outc, pw);
+    case 128: return pweight_t<128>(c, nb, ppar, pssnr, g, ctff, outc, pw);
+    case 256: return pweight_t<256>(c, nb, ppar, pssnr, g, ctff, outc, pw);
+    default: return fail("no fused preparation for NSAM %d", nsam);
+  }
 }
 
 }  // namespace
 
 size_t prep_partials_count(int nsam, int nb) {
   // row blocks of NSEQ = 2048 / NSAM row pairs: NSAM^2 / 4096 per image
-  const size_t per = fused_cols(nsam) ? (size_t)nsam * nsam / 4096 : 1;
-  return per * (size_t)(nb > 0 ? nb : 1);
+  if (!fused_cols(nsam) || nb <= 0) return 1;
+  return (size_t)nsam * nsam / 4096 * nb +
+         (pw_chunk(nsam, nb) * pw_image_bytes(nsam) + sizeof(float2) - 1) / sizeof(float2);
 }
 
 int launch_prep(Ctx& c, int nsam, int nb, float* data, const float* ppar, const float* pssnr,
@@ -653,10 +822,11 @@ int launch_prep(Ctx& c, int nsam, int nb, float* data, const float* ppar, const 
   // lmain.f:459's r2c: its row pass here, its column pass in the fused
   // column kernel, which continues with CTFAPPLY's shift step and OUTC's
   // backward column pass
-  if (int r = ctf_table(c, nsam, nb, ppar, g, ctff)) return r;
+  float2* pw;
+  if (int r = fused_scratch(c, nsam, nb, part, pw)) return r;
   if (int r = fft_rows_2d(c, nsam, nb, data, img, true)) return r;
   if (int r = fused_shift_mask(c, nsam, nb, data, true, ppar, g, outc, datc, part)) return r;
-  return fused_tail(c, nsam, nb, pssnr, g, ctff, outc);
+  return fused_tail(c, nsam, nb, ppar, pssnr, g, ctff, outc, pw);
 }
 
 int launch_ctfapply(Ctx& c, int nsam, int nb, const float* spec, const float* ppar,
@@ -666,11 +836,12 @@ int launch_ctfapply(Ctx& c, int nsam, int nb, const float* spec, const float* pp
   FR_CHECK(nsam / 2 + 1 <= 520, "box too large for PWEIGHT bins");
   if (fused_cols(nsam)) {
     // kFwd false: the spectrum is only read
-    if (int r = ctf_table(c, nsam, nb, ppar, g, ctff)) return r;
+    float2* pw;
+    if (int r = fused_scratch(c, nsam, nb, part, pw)) return r;
     if (int r = fused_shift_mask(c, nsam, nb, const_cast<float*>(spec), false, ppar, g, outc,
                                  datc, part))
       return r;
-    return fused_tail(c, nsam, nb, pssnr, g, ctff, outc);
+    return fused_tail(c, nsam, nb, ppar, pssnr, g, ctff, outc, pw);
   }
   const size_t img = (size_t)nsam * (nsam + 2);
   const size_t tot = (size_t)nsam * (nsam / 2 + 1) * nb;
