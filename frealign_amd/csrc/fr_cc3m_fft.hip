@@ -533,21 +533,8 @@ int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, con
   return 0;
 }
 
-// the box sizes of the tests and the benchmark with their length compiled in (an
-// index division or modulus by a run-time length costs more than its butterfly)
 int launch_band(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, const BandWork& w) {
-  switch (b.nsam) {
-    case 64: return launch_n<64>(c, b, p, ring, w);
-    case 96: return launch_n<96>(c, b, p, ring, w);
-    case 128: return launch_n<128>(c, b, p, ring, w);
-    case 160: return launch_n<160>(c, b, p, ring, w);
-    case 192: return launch_n<192>(c, b, p, ring, w);
-    case 256: return launch_n<256>(c, b, p, ring, w);
-    case 320: return launch_n<320>(c, b, p, ring, w);
-    case 384: return launch_n<384>(c, b, p, ring, w);
-    case 512: return launch_n<512>(c, b, p, ring, w);
-    default: return launch_n<0>(c, b, p, ring, w);
-  }
+  return with_length(b.nsam, [&](auto len) { return launch_n<len()>(c, b, p, ring, w); });
 }
 
 Band make_band(int nsam, int n, int maxr12, int maxr2, float ri2, float ri3, float rih,

@@ -45,10 +45,10 @@ struct Ctx {
   const float2* twiddles(int n);
   // the particle preparation's per-row-block ring sums and its shell sums
   // (fr_prep.hip) for calls on the context's stream: one fixed allocation for
-  // the largest batch (65535 images x 16 row blocks; 32 MB of shells), made on
+  // the largest batch (65535 images x 128 row blocks; 32 MB of shells), made on
   // first use and kept (plans, whose graphs replay on their own streams, bring
   // their own buffer)
-  static constexpr size_t kRingPartials = 65535 * 16, kShellPartials = (32u << 20) / sizeof(float2);
+  static constexpr size_t kRingPartials = 65535 * 128, kShellPartials = (32u << 20) / sizeof(float2);
   float2* prep_part = nullptr;
   float2* prep_partials();
   ~Ctx();

@@ -166,13 +166,11 @@ int row_seqs(int n) {
   return s < 1 ? 1 : s;
 }
 
-// ---- the same three kernels with the length known at compile time (the
-// box sizes of the bench and the proposal: 64, 128, 256): every index
-// division and modulus becomes a shift or a constant multiply.
+// ---- the same three kernels with the length known at compile time
 template <int N>
 using RowFft = Fft<N, 2048 / N, false>;
 template <int N>
-using ColFft = Fft<N, cols_cw<N>(), true>;
+using ColFft = Fft<N, cols_cw(N), true>;
 
 template <int N>
 __global__ void __launch_bounds__(kThreads) k_rows_r2c_t(float* data, size_t img_stride,
@@ -246,7 +244,7 @@ __global__ void __launch_bounds__(kThreads) k_cols_t(float* data, size_t img_str
                                                      const float2* __restrict__ tw) {
   using F = ColFft<N>;
   constexpr int JC = N / 2 + 1;
-  constexpr int CW = cols_cw<N>();
+  constexpr int CW = cols_cw(N);
   constexpr int JB = (JC + CW - 1) / CW;
   extern __shared__ float2 smem[];
   // column blocks of one image in XCD-contiguous order
@@ -290,7 +288,7 @@ int rows_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, bool fwd, cons
 template <int N>
 int cols_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, int sign, const float2* tw) {
   constexpr int JC = N / 2 + 1;
-  constexpr int CW = cols_cw<N>();
+  constexpr int CW = cols_cw(N);
   const size_t lds = ColFft<N>::kLds;
   const long long nblk = (long long)((JC + CW - 1) / CW) * nimg;
   FR_CHECK(nblk <= (1ll << 30), "too many images in one FFT batch (%d)", nimg);
@@ -312,17 +310,25 @@ bool fft_supported(int nsam) {
   return (nsam % 2 == 0) && make_plan(nsam, &p);
 }
 
+static int rows_pass_any(Ctx&, const Plan&, int, float*, size_t, bool, const float2*);
+static int cols_pass_any(Ctx&, const Plan&, int, float*, size_t, int, const float2*);
+
 static int rows_pass(Ctx& c, int nsam, int nimg, float* data, size_t img_stride, bool fwd) {
   Plan pl;
   FR_CHECK(make_plan(nsam, &pl) && nsam % 2 == 0, "FFT length %d not supported", nsam);
   const float2* tw = c.twiddles(nsam);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
-  switch (nsam) {
-    case 64: return rows_pass_t<64>(c, nimg, data, img_stride, fwd, tw);
-    case 128: return rows_pass_t<128>(c, nimg, data, img_stride, fwd, tw);
-    case 256: return rows_pass_t<256>(c, nimg, data, img_stride, fwd, tw);
-    default: break;
-  }
+  return with_length(nsam, [&](auto len) {
+    if constexpr (len() > 0)
+      return rows_pass_t<len()>(c, nimg, data, img_stride, fwd, tw);
+    else
+      return rows_pass_any(c, pl, nimg, data, img_stride, fwd, tw);
+  });
+}
+
+static int rows_pass_any(Ctx& c, const Plan& pl, int nimg, float* data, size_t img_stride, bool fwd,
+                         const float2* tw) {
+  const int nsam = pl.n;
   int npairs = nimg * (nsam / 2);
   int nseq = row_seqs(nsam);
   size_t lds = sizeof(float2) * 2 * nseq * (nsam + 1);
@@ -343,12 +349,17 @@ static int cols_pass(Ctx& c, int nsam, int nimg, float* data, size_t img_stride,
   const float2* tw = c.twiddles(nsam);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
   FR_CHECK(nimg <= 65535, "too many images in one FFT batch (%d)", nimg);
-  switch (nsam) {
-    case 64: return cols_pass_t<64>(c, nimg, data, img_stride, sign, tw);
-    case 128: return cols_pass_t<128>(c, nimg, data, img_stride, sign, tw);
-    case 256: return cols_pass_t<256>(c, nimg, data, img_stride, sign, tw);
-    default: break;
-  }
+  return with_length(nsam, [&](auto len) {
+    if constexpr (len() > 0)
+      return cols_pass_t<len()>(c, nimg, data, img_stride, sign, tw);
+    else
+      return cols_pass_any(c, pl, nimg, data, img_stride, sign, tw);
+  });
+}
+
+static int cols_pass_any(Ctx& c, const Plan& pl, int nimg, float* data, size_t img_stride, int sign,
+                         const float2* tw) {
+  const int nsam = pl.n;
   int jc = nsam / 2 + 1;
   int cw = 2048 / nsam;
   if (cw < 1) cw = 1;

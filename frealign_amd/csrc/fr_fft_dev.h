@@ -5,6 +5,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace fr {
 namespace fftdev {
 
@@ -298,11 +300,64 @@ __device__ inline float2* lds_fft(float2* buf, float2* tmp, const Plan& pl, int 
   return buf;
 }
 
-// columns per workgroup of the column pass (16 at 256 measured no faster)
-template <int N>
-constexpr int cols_cw() {
-  constexpr int JC = N / 2 + 1;
-  return (2048 / N) < JC ? (2048 / N) : JC;
+// The lengths that are compiled in, f(integral_constant<N>): the even ones from
+// 64 to 512 (an index division or modulus by a run-time length costs more than
+// its butterfly: preparing 300 images of 160^2 takes 173 us, 357 with passes of a
+// run-time length).  N = 0, those passes, for any other.
+template <typename F>
+inline int with_length(int n, F f) {
+#define FR_LENGTH(N) \
+  case N: return f(std::integral_constant<int, N>{});
+  switch (n) {
+    FR_LENGTH(64)
+    FR_LENGTH(72)
+    FR_LENGTH(80)
+    FR_LENGTH(90)
+    FR_LENGTH(96)
+    FR_LENGTH(100)
+    FR_LENGTH(108)
+    FR_LENGTH(120)
+    FR_LENGTH(128)
+    FR_LENGTH(144)
+    FR_LENGTH(150)
+    FR_LENGTH(160)
+    FR_LENGTH(162)
+    FR_LENGTH(180)
+    FR_LENGTH(192)
+    FR_LENGTH(200)
+    FR_LENGTH(216)
+    FR_LENGTH(240)
+    FR_LENGTH(250)
+    FR_LENGTH(256)
+    FR_LENGTH(270)
+    FR_LENGTH(288)
+    FR_LENGTH(300)
+    FR_LENGTH(320)
+    FR_LENGTH(324)
+    FR_LENGTH(360)
+    FR_LENGTH(384)
+    FR_LENGTH(400)
+    FR_LENGTH(432)
+    FR_LENGTH(450)
+    FR_LENGTH(480)
+    FR_LENGTH(486)
+    FR_LENGTH(500)
+    FR_LENGTH(512)
+    default: return f(std::integral_constant<int, 0>{});
+  }
+#undef FR_LENGTH
+}
+
+// columns per workgroup of a column pass: 64 bytes or more of a row, and 2,048
+// points where the columns are short (16 at 256 measured no faster)
+constexpr int cols_cw(int n) { return n <= 64 ? 32 : n <= 128 ? 16 : 8; }
+
+// row pairs per workgroup of a row pass that stays in one image: the largest
+// divisor of the image's pairs within 2,048 points
+constexpr int rows_in_image(int n) {
+  int k = 2048 / n;
+  while (n / 2 % k) k--;
+  return k;
 }
 
 }  // namespace fftdev

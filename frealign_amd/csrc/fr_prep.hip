@@ -7,7 +7,7 @@
 // in-place double weighting of the Nyquist row and its JC+1 shell aliasing
 // into bin 1's count (the reference calls PWEIGHT(NSAM,OUTC,OUTC,...)).
 //
-// For NSAM 64, 128 and 256 the steps run as seven launches: the r2c's row pass;
+// Where the FFT's length is compiled in the steps run as seven launches: the r2c's row pass;
 // one column pass that completes the r2c (written back into the image), applies
 // the shift and writes DATC, and runs OUTC's backward column pass; the row c2r,
 // which also sums each row block's part of MASKCOS's ring; the row r2c, which
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
     k_cols_shift(float2* spec, const float* __restrict__ ppar, float2* outc, float2* datc, int nb,
                  const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int JC = N / 2 + 1, CW = cols_cw<N>();
+  constexpr int JC = N / 2 + 1, CW = cols_cw(N);
   constexpr int JB = (JC + CW - 1) / CW;
   constexpr size_t IC = (size_t)N * JC;
   using F = Fft<N, CW, true>;         // forward
@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
 template <int N>
 int cols_shift_t(Ctx& c, int nb, float* spec, bool fwd, const float* ppar, float* outc,
                  float* datc) {
-  constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw<N>();
+  constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw(N);
   const size_t lds = fftdev::Fft<N, CW, true>::kLds;
   const float2* tw = c.twiddles(N);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
                     float ri2, float ri3, float scal, float2* part,
                     const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
+  constexpr int NSEQ = rows_in_image(N), JC = N / 2 + 1, PITCH = N + 2;
   using F = Fft<N, NSEQ, false>;
   extern __shared__ float2 rr_smem[];
   __shared__ float red_s[kFftThreads / 64];
@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
                     float ri2, float ri3, float rih, float halfw, float scal,
                     const float2* __restrict__ part, const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int NSEQ = 2048 / N, JC = N / 2 + 1, PITCH = N + 2;
+  constexpr int NSEQ = rows_in_image(N), JC = N / 2 + 1, PITCH = N + 2;
   constexpr int WPI = (N / 2) / NSEQ;  // row blocks per image
   using F = Fft<N, NSEQ, false>;
   extern __shared__ float2 rm_smem[];
@@ -331,12 +331,12 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
   }
 }
 
-// OUTC's c2r, MASKCOS and r2c rows on the fused path; `part` (NSAM^2/4096
-// float2 per image) carries the ring partial sums between the two launches
+// OUTC's c2r, MASKCOS and r2c rows on the fused path; `part` (a float2 per row
+// block) carries the ring partial sums between the two launches
 template <int N>
 int rows_mask_t(Ctx& c, int nb, float* outc, const float* ppar, const PrepGlobals& g,
                 float2* part) {
-  constexpr int NSEQ = 2048 / N;
+  constexpr int NSEQ = fftdev::rows_in_image(N);
   const int npairs = nb * (N / 2);
   const size_t lds = fftdev::Fft<N, NSEQ, false>::kLds;
   const size_t img = (size_t)N * (N + 2);
@@ -378,7 +378,7 @@ template <int N>
 __global__ void __launch_bounds__(fftdev::kFftThreads)
     k_cols_shells(float2* data, int nb, float2* part, const float2* __restrict__ tw) {
   using namespace fftdev;
-  constexpr int JC = N / 2 + 1, CW = cols_cw<N>(), JB = (JC + CW - 1) / CW, LH = N + 1;
+  constexpr int JC = N / 2 + 1, CW = cols_cw(N), JB = (JC + CW - 1) / CW, LH = N + 1;
   using F = Fft<N, CW, true>;
   extern __shared__ float2 cp_smem[];
   const int lb = xcd_block(blockIdx.x, gridDim.x);
@@ -502,7 +502,7 @@ __global__ void __launch_bounds__(kThreads)
 constexpr size_t kPwBytes = Ctx::kShellPartials * sizeof(float2);
 
 size_t pw_image_bytes(int nsam) {
-  const int jc = nsam / 2 + 1, cw = std::min(2048 / nsam, jc), jb = (jc + cw - 1) / cw;
+  const int jc = nsam / 2 + 1, cw = fftdev::cols_cw(nsam), jb = (jc + cw - 1) / cw;
   return sizeof(float2) * jb * (jc + 1) + sizeof(float) * (jc + 2);
 }
 
@@ -513,7 +513,7 @@ int pw_chunk(int nsam, int nb) {
 template <int N>
 int pweight_t(Ctx& c, int nb, const float* ppar, const float* pssnr, const PrepGlobals& g,
               float* ctff, float* outc, float2* pw) {
-  constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw<N>(), JB = (JC + CW - 1) / CW;
+  constexpr int JC = N / 2 + 1, CW = fftdev::cols_cw(N), JB = (JC + CW - 1) / CW;
   constexpr size_t IC = (size_t)N * JC;
   const float2* tw = c.twiddles(N);
   FR_CHECK(tw != nullptr, "twiddle table allocation failed");
@@ -535,14 +535,19 @@ int pweight_t(Ctx& c, int nb, const float* ppar, const float* pssnr, const PrepG
   return 0;
 }
 
-bool fused_cols(int nsam) { return nsam == 64 || nsam == 128 || nsam == 256; }
+bool fused_cols(int nsam) {
+  return fftdev::with_length(nsam, [](auto len) { return len() > 0; });
+}
+
+// row blocks of an image, whose ring sums k_rows_c2r_ring leaves
+size_t ring_parts(int nsam) { return nsam / 2 / fftdev::rows_in_image(nsam); }
 
 // the ring sums' buffer, and the PWEIGHT scratch after it: the caller's, or the
 // context's for its largest batch
 int fused_scratch(Ctx& c, int nsam, int nb, float2*& part, float2*& pw) {
   FR_CHECK(nb <= 65535, "too many images in one batch (%d)", nb);
   if (part) {
-    pw = part + (size_t)nsam * nsam / 4096 * nb;
+    pw = part + ring_parts(nsam) * nb;
     return 0;
   }
   part = c.prep_partials();
@@ -555,18 +560,14 @@ int fused_scratch(Ctx& c, int nsam, int nb, float2*& part, float2*& pw) {
 // transform first), then OUTC's c2r, MASKCOS and r2c rows
 int fused_shift_mask(Ctx& c, int nsam, int nb, float* spec, bool fwd, const float* ppar,
                      const PrepGlobals& g, float* outc, float* datc, float2* part) {
-  switch (nsam) {
-    case 64:
-      if (int r = cols_shift_t<64>(c, nb, spec, fwd, ppar, outc, datc)) return r;
-      return rows_mask_t<64>(c, nb, outc, ppar, g, part);
-    case 128:
-      if (int r = cols_shift_t<128>(c, nb, spec, fwd, ppar, outc, datc)) return r;
-      return rows_mask_t<128>(c, nb, outc, ppar, g, part);
-    case 256:
-      if (int r = cols_shift_t<256>(c, nb, spec, fwd, ppar, outc, datc)) return r;
-      return rows_mask_t<256>(c, nb, outc, ppar, g, part);
-    default: return fail("no fused column pass for NSAM %d", nsam);
-  }
+  return fftdev::with_length(nsam, [&](auto len) {
+    if constexpr (len() > 0) {
+      if (int r = cols_shift_t<len()>(c, nb, spec, fwd, ppar, outc, datc)) return r;
+      return rows_mask_t<len()>(c, nb, outc, ppar, g, part);
+    } else {
+      return fail("no fused column pass for NSAM %d", nsam);
+    }
+  });
 }
 
 __device__ inline float block_sum(float v, float* red) {
@@ -792,20 +793,19 @@ int origin_pweight(Ctx& c, int nsam, int nb, const float* pssnr, const PrepGloba
 // shift, the CTF table and PWEIGHT
 int fused_tail(Ctx& c, int nsam, int nb, const float* ppar, const float* pssnr,
                const PrepGlobals& g, float* ctff, float* outc, float2* pw) {
-  switch (nsam) {
-    case 64: return pweight_t<64>(c, nb, ppar, pssnr, g, ctff, outc, pw);
-    case 128: return pweight_t<128>(c, nb, ppar, pssnr, g, ctff, outc, pw);
-    case 256: return pweight_t<256>(c, nb, ppar, pssnr, g, ctff, outc, pw);
-    default: return fail("no fused preparation for NSAM %d", nsam);
-  }
+  return fftdev::with_length(nsam, [&](auto len) {
+    if constexpr (len() > 0)
+      return pweight_t<len()>(c, nb, ppar, pssnr, g, ctff, outc, pw);
+    else
+      return fail("no fused preparation for NSAM %d", nsam);
+  });
 }
 
 }  // namespace
 
 size_t prep_partials_count(int nsam, int nb) {
-  // row blocks of NSEQ = 2048 / NSAM row pairs: NSAM^2 / 4096 per image
   if (!fused_cols(nsam) || nb <= 0) return 1;
-  return (size_t)nsam * nsam / 4096 * nb +
+  return ring_parts(nsam) * nb +
          (pw_chunk(nsam, nb) * pw_image_bytes(nsam) + sizeof(float2) - 1) / sizeof(float2);
 }
 

@@ -37,7 +37,7 @@ def _inputs(nsam, nb, rng):
     return g, ps, buf, ppar
 
 
-@pytest.mark.parametrize("nsam", [64, 128, 256])
+@pytest.mark.parametrize("nsam", [64, 72, 80, 90, 128, 162, 200, 250, 256, 432, 500, 512])
 @pytest.mark.parametrize("ictf", [0, 1])
 def test_outc_vs_oracle(nsam, ictf):
     rng = np.random.default_rng(nsam + ictf)
