@@ -1459,15 +1459,14 @@ int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d
   a.maxit = maxit;
   a.sm = sm;
   // one round's items go over in one pinned copy (PIDX | DM | SHIFT | AMAG,
-  // 13 words per item) and its scores come back in one
+  // 13 words per item); its scores, written once each, go to host memory from
+  // the kernels (a copy back is a launch of its own: 6 us of a round's 39)
   auto cc3m = [&](int m, const int* hp, const float* hdm, const float* hsh, const float* ham,
                   float* hscore) -> int {
     int err = 0;
     const size_t words = 13 * (size_t)m;
     char* dbuf = (char*)c->slot(11, sizeof(float) * words, &err);
     if (!dbuf) return err;
-    float* dsc = (float*)c->slot(15, sizeof(float) * (size_t)m, &err);
-    if (!dsc) return err;
     char* h = (char*)c->host_pinned(sizeof(float) * (words + m), &err);
     if (!h) return err;
     const size_t o_dm = sizeof(int) * m, o_sh = o_dm + sizeof(float) * 9 * m,
@@ -1481,10 +1480,9 @@ int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d
     for (int i = 0; i < m; i++) unit &= ham[i] == 1.0f;
     if (int r = cc3m_batch(c, nsam, m, d_a3df, d_spec, d_ctff, (const int*)dbuf,
                            (const float*)(dbuf + o_dm), (const float*)(dbuf + o_sh),
-                           (const float*)(dbuf + o_am), maxr1, maxr2, rbfact, d_fsct, ring, dsc,
-                           0, unit))
+                           (const float*)(dbuf + o_am), maxr1, maxr2, rbfact, d_fsct, ring,
+                           (float*)(h + o_sc), 0, unit))
       return r;
-    FR_HIP(hipMemcpyAsync(h + o_sc, dsc, sizeof(float) * m, hipMemcpyDeviceToHost, c->stream));
     FR_HIP(hipStreamSynchronize(c->stream));
     memcpy(hscore, h + o_sc, sizeof(float) * m);
     return 0;
