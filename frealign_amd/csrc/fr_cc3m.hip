@@ -16,22 +16,27 @@
 // One workgroup per item, persistent over a contiguous run of items (the
 // candidates of one particle reuse its CTF and spectrum, held in registers).
 // Every pass is a product with T[m][2i] = cos(2 pi i m/M), T[m][2i+1] =
-// -sin(2 pi i m/M) on the FP32 matrix cores, folded over the table's
-// symmetry: rows m and M - m of T differ by the sign of the sines, so only
-// m <= M/2 is held and each product gives both.
+// -sin(2 pi i m/M) on the FP32 matrix cores:
 //   column c2c  Y[m][c]   = sum_J T[m][.] B[c][.]   B: the +-J pairs
 //   row c2r     x[r][m]   = sum_I T[r][.] w_I Y[m][.]
 //   mask        y = (x - mean) w, the same w at r and M - r
 //   row r2c     Z[m][k]   = sum_r T[r][k] y[r][m]  (+ M mean at k = 0)
 //   column r2c  out[j][k] = sum_m T[m][j] Z[m][k]
-// then the shell sums of cc3m.f:117-150, each thread its own (I, +-J) pairs,
+// folded over the table's symmetries: rows m and M - m differ by the sign of the
+// sines, rows m and M/2 - m by that of the odd cosines and the even sines.  So
+// the cosine and sine parts of even and odd frequencies, each a product over
+// m < M/4, give all four rows, and the transforms back take the four rows' sums
+// and differences (row M/4 is its own partner, in plain sums).  At MAXR2 <= 16,
+// where 8 frequencies of one parity would not fill a tile, only over M - m.
+// Then the shell sums of cc3m.f:117-150, each thread its own (I, +-J) pairs,
 // reduced by shell in a fixed order.
 //
-// What bounds it: at MAXR2 = 32 an item takes 1,536 16x16x4 FP32 MFMA (5 us
-// of one CU's matrix cores) against 4,896 on a 256 grid.  LDS is 71 KB (149 KB
-// on the 256 grid), so two workgroups share a CU and one's gathers and sums
-// run under the other's products.  8,192 items of a 256 box: 380 us against
-// 1,370 us on the 256 grid.
+// What bounds it: at MAXR2 = 32 an item takes 768 16x16x4 FP32 MFMA (2.5 us of
+// one CU's matrix cores; 1,536 folded once, 4,896 on a 256 grid), 3,200 gathered
+// points and the barriers between the passes.  LDS is 71 KB (149 KB on the 256
+// grid), so two workgroups share a CU and one's gathers and sums run under the
+// other's products.  8,192 items of a 256 box: 300 us (1,370 on the 256 grid,
+// 393 folded once).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -68,6 +73,9 @@ template <int RB, int M>
 struct BandShape {
   static constexpr int kThreads = RB == 32 ? 512 : 256;
   static constexpr int kWaves = kThreads / 64;
+  // the products folded over quarters of the grid, a wave's tile 16 frequencies
+  // of one parity: 16 of RB = 32 fill it, 8 of RB = 16 would not
+  static constexpr bool kQuarter = RB == 32;
   static constexpr int kK = 2 * RB;      // reals per row: RB frequencies
   static constexpr int kP = kK + 4;      // LDS row pitch (floats): conflict-free operand reads
   static constexpr int kPairs = RB * RB / kThreads;  // (I, |J|) pairs per thread
@@ -105,6 +113,7 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
   const int jc = nsam / 2 + 1;
   const size_t ic = (size_t)nsam * jc;
   auto ld2 = [](const float* p) { return *reinterpret_cast<const float2*>(p); };
+  auto ld4 = [](const float* p) { return *reinterpret_cast<const fx4*>(p); };
 
   const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
   const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
@@ -213,9 +222,53 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     if (lane == 0) red_s[wave] = rsum;
     __syncthreads();
 
-    // ---- column c2c, times the c2r weight: for m < M/2, E against the cosine
-    // rows of B and O against its sine rows give Y[m] = E + O, Y[M-m] = E - O
-    {
+    // ---- column c2c, times the c2r weight
+    if constexpr (S::kQuarter) {
+      // m < M/4 and the frequencies' parity: Ee, Eo, Oe, Oo give Y at m, M - m,
+      // M/2 - m and M/2 + m
+      const int y0 = (wave / (kK / 16)) * 16, c0 = (wave % (kK / 16)) * 16;
+      fx4 ee = {0.f, 0.f, 0.f, 0.f}, eo = ee, oe = ee, oo = ee;
+#pragma unroll
+      for (int s = 0; s < RB / 8; s++) {
+        const fx4 tv = ld4(Ts + (y0 + la) * kP + 16 * s + 4 * lg);
+        const fx4 bv = ld4(Bs + (c0 + la) * kP + 16 * s + 4 * lg);
+        ee = mfma4(tv[0], bv[0], ee);
+        oe = mfma4(tv[1], bv[1], oe);
+        eo = mfma4(tv[2], bv[2], eo);
+        oo = mfma4(tv[3], bv[3], oo);
+      }
+      const float wc = (c0 + la) < 2 ? 1.0f : 2.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int y = y0 + 4 * lg + i;
+        if (M % 128 && y >= M / 4) continue;
+        float* yp = Ys + c0 + la;
+        const float ep = ee[i] + eo[i], em = ee[i] - eo[i];
+        const float op = oe[i] + oo[i], om = oe[i] - oo[i];
+        yp[y * kP] = (ep + op) * wc;
+        yp[(H - y) * kP] = (em - om) * wc;
+        if (y) {
+          yp[(M - y) * kP] = (ep - op) * wc;
+          yp[(H + y) * kP] = (em + om) * wc;
+        }
+      }
+      // rows M/4 and 3M/4, eight threads per column: even J by the cosines, odd J
+      // by the sines
+      const int c = tid >> 3, q = tid & 7;
+      float v = 0.f;
+#pragma unroll
+      for (int j = 0; j < RB; j += 8) v += Bs[c * kP + 2 * (j + q) + (q & 1)];
+      if ((q ^ (q >> 1)) & 1) v = -v;
+      v += __shfl_xor(v, 2, 64);
+      v += __shfl_xor(v, 4, 64);
+      const float o = __shfl_xor(v, 1, 64);
+      if (q == 0) {
+        Ys[(M / 4) * kP + c] = (v + o) * (c < 2 ? 1.0f : 2.0f);
+        Ys[(3 * M / 4) * kP + c] = (v - o) * (c < 2 ? 1.0f : 2.0f);
+      }
+    } else {
+      // m < M/2: E against the cosine rows of B and O against its sine rows give
+      // Y[m] = E + O, Y[M-m] = E - O
       constexpr int kTiles = (H / 16) * (kK / 16);
 #pragma unroll
       for (int t0 = 0; t0 < kTiles; t0 += S::kWaves) {
@@ -251,9 +304,94 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
     }
     __syncthreads();
 
-    // ---- rows of this wave's block: E and O of a tile of T rows r < M/2 give
-    // x[r] = E + O and x[M-r] = E - O; y = (x - mean) w (the same w at r and
-    // M - r); Z's cosine part takes y[r] + y[M-r], its sine part y[r] - y[M-r]
+    // ---- rows of this wave's block: x = c2r of Y, y = (x - mean) w, Z = r2c of y
+    float tot = 0.f;
+#pragma unroll
+    for (int k = 0; k < S::kWaves; k++) tot += red_s[k];
+    const float mean = ring_cnt ? tot / (float)ring_cnt : tot;
+    if constexpr (S::kQuarter) {
+      // r < M/4 by parity as above: w is the same at r and M - r, and at M/2 - r
+      // and M/2 + r.  Z at even and odd k takes the sums and differences of the
+      // four y over the halves
+      if (rows) {
+        constexpr int kQt = (M / 4 + 15) / 16;
+        fx4 w[kQt], wm[kQt];
+#pragma unroll
+        for (int t = 0; t < kQt; t++) {
+          w[t] = ld4(wtab + (size_t)m * M + 16 * t + 4 * lg);
+#pragma unroll
+          for (int i = 0; i < 4; i++) wm[t][i] = wtab[(size_t)m * M + H - (16 * t + 4 * lg + i)];
+        }
+        const float wq = wtab[(size_t)m * M + M / 4];
+        fx4 yv[RB / 8];
+#pragma unroll
+        for (int s = 0; s < RB / 8; s++) yv[s] = ld4(Ys + m * kP + 16 * s + 4 * lg);
+        fx4 zce = {0.f, 0.f, 0.f, 0.f}, zse = zce, zco = zce, zso = zce;
+#pragma unroll
+        for (int t = 0; t < kQt; t++) {
+          __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
+          fx4 ee = {0.f, 0.f, 0.f, 0.f}, eo = ee, oe = ee, oo = ee, ce, se, co, so;
+#pragma unroll
+          for (int s = 0; s < RB / 8; s++) {
+            const fx4 tv = ld4(Ts + (16 * t + la) * kP + 16 * s + 4 * lg);
+            ee = mfma4(tv[0], yv[s][0], ee);
+            oe = mfma4(tv[1], yv[s][1], oe);
+            eo = mfma4(tv[2], yv[s][2], eo);
+            oo = mfma4(tv[3], yv[s][3], oo);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const float ep = ee[i] + eo[i] - mean, em = ee[i] - eo[i] - mean;
+            const float op = oe[i] + oo[i], om = oe[i] - oo[i];
+            float ya = (ep + op) * w[t][i], yb = (ep - op) * w[t][i];
+            float yc = (em - om) * wm[t][i], yd = (em + om) * wm[t][i];
+            if (t == 0 && i == 0 && lg == 0) yb = yd = 0.f;  // r = 0 and M/2: their own partners
+            if (M % 64 && 16 * t + 4 * lg + i >= M / 4) ya = yb = yc = yd = 0.f;
+            const float p = ya + yb, q = yc + yd, u = ya - yb, v = yc - yd;
+            ce[i] = p + q;
+            co[i] = p - q;
+            se[i] = u - v;
+            so[i] = u + v;
+          }
+          // k-step i takes r = 16t + 4 lg + i: the C layout of the sums is the B layout
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const fx4 tv = ld4(Ts + (16 * t + 4 * lg + i) * kP + 4 * la);
+            zce = mfma4(tv[0], ce[i], zce);
+            zse = mfma4(tv[1], se[i], zse);
+            zco = mfma4(tv[2], co[i], zco);
+            zso = mfma4(tv[3], so[i], zso);
+          }
+        }
+        // rows M/4 and 3M/4: x = P + Q and P - Q, P of the even I (8 s + 2 lg), Q of the odd
+        float xp = 0.f, xq = 0.f;
+#pragma unroll
+        for (int s = 0; s < RB / 8; s++) {
+          xp += yv[s][0];
+          xq -= yv[s][3];
+        }
+        if (lg & 1) xp = -xp, xq = -xq;
+        xp += __shfl_xor(xp, 16, 64);
+        xq += __shfl_xor(xq, 16, 64);
+        xp += __shfl_xor(xp, 32, 64);
+        xq += __shfl_xor(xq, 32, 64);
+        const float ya = (xp + xq - mean) * wq, yb = (xp - xq - mean) * wq;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          zce[i] += (i & 1) ? -(ya + yb) : ya + yb;
+          zso[i] += (i & 1) ? ya - yb : yb - ya;
+        }
+        if (lg == 0) zce[0] += mean * (float)M;  // k = 0, the mean's own term
+        // this wave alone read rows m0 .. m0 + 15 of Ys
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          *reinterpret_cast<fx4*>(Ys + m * kP + 4 * (4 * lg + i)) =
+              fx4{zce[i], zse[i], zco[i], zso[i]};
+      }
+    } else {
+      // E and O of a tile of T rows r < M/2 give x[r] = E + O and x[M-r] = E - O
+      // (the same w at both); Z's cosine part takes y[r] + y[M-r], its sine part
+      // y[r] - y[M-r]
     fx4 w[M / 32];
     float wh = 0.f;
     if (rows) {
@@ -262,10 +400,6 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
         w[t] = *reinterpret_cast<const fx4*>(wtab + (size_t)m * M + 16 * t + 4 * lg);
       wh = wtab[(size_t)m * M + H];
     }
-    float tot = 0.f;
-#pragma unroll
-    for (int k = 0; k < S::kWaves; k++) tot += red_s[k];
-    const float mean = ring_cnt ? tot / (float)ring_cnt : tot;
     if (rows) {
       float2 yv[RB / 4];
 #pragma unroll
@@ -322,6 +456,7 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
           *reinterpret_cast<float2*>(Ys + m * kP + 2 * (16 * kt + 4 * lg + i)) =
               make_float2(zc[kt][i], zs[kt][i]);
     }
+    }
     __syncthreads();
 
     // the pairs' spectrum, in flight under the column r2c
@@ -336,9 +471,38 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
         sneg[u] = sp[(size_t)jc * wrapn(-jj, nsam)];
       }
     }
-    // ---- column r2c, folded over m: cosine rows take Z[m] + Z[M-m], sine
-    // rows Z[m] - Z[M-m] (m = 0 and M/2 are their own partners)
-    {
+    // ---- column r2c, folded over m
+    if constexpr (S::kQuarter) {
+      // a wave's 16 j of one parity: cosine rows take (Z[m] + Z[M-m]) +- (Z[M/2-m] +
+      // Z[M/2+m]), sine rows (Z[m] - Z[M-m]) -+ (Z[M/2-m] - Z[M/2+m])
+      const int par = wave / (kK / 16), c0 = (wave % (kK / 16)) * 16;
+      const float sg = par ? -1.0f : 1.0f;
+      fx4 ac = {0.f, 0.f, 0.f, 0.f}, as = ac;
+      const float* zp = Ys + c0 + la;
+      const float* tp = Ts + lg * kP + 4 * la + 2 * par;
+#pragma unroll
+      for (int s = 0; s < M / 16; s++) {
+        const int mm = 4 * s + lg;
+        // m = 0 and M/2 have no partner (row M does not exist)
+        const bool alone = s == 0 && lg == 0;
+        const float za = zp[mm * kP], zc = zp[(H - mm) * kP], zd = zp[(H + mm) * kP];
+        const float zb = zp[(alone ? 0 : M - mm) * kP];
+        const float2 tv = ld2(tp + 4 * s * kP);
+        ac = mfma4(tv.x, alone ? za + sg * zc : (za + zb) + sg * (zc + zd), ac);
+        as = mfma4(tv.y, alone ? 0.f : (za - zb) - sg * (zc - zd), as);
+      }
+      // m = M/4 and 3M/4: the cosines of even j and the sines of odd j are +-1
+      const float z1 = zp[(M / 4) * kP], z3 = zp[(3 * M / 4) * kP];
+      const float ec = par ? 0.f : z1 + z3, es = par ? z3 - z1 : 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int j = 2 * (4 * lg + i) + par;
+        Bs[j * kP + c0 + la] = ac[i] + ((i & 1) ? -ec : ec);
+        Bs[(RB + j) * kP + c0 + la] = as[i] + ((i & 1) ? -es : es);
+      }
+    } else {
+      // cosine rows take Z[m] + Z[M-m], sine rows Z[m] - Z[M-m] (m = 0 and M/2 are
+      // their own partners)
       constexpr int kTiles = (RB / 16) * (kK / 16);
       if (wave < kTiles) {
         const int j0 = (wave / (kK / 16)) * 16, c0 = (wave % (kK / 16)) * 16;
