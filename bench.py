@@ -17,8 +17,8 @@ the timed steps cycle over a pool of 5,120 distinct particles.  Searches:
     particles whose top class probability is below 0.3 take the exhaustive
     search instead;
   * exhaustive BF16: every orientation, the same separable BF16 search;
-  * plain FP32: every orientation, the 225-shift FP32 MFMA GEMM (the
-    baseline of the metric);
+  * plain FP32: every orientation, the FP32 search (the baseline of the
+    metric; its shifts applied in two separable FP32 matrix-core stages too);
   * reference-exact PSEARCH on a few particles: CCP with PAD and ROTATE2D as
     the reference computes them.
 The network is trained first, on the GPU, on projections of the same
@@ -101,26 +101,15 @@ PEAK_FP32_MFMA = 157.3e12
 PEAK_HBM = 8.0e12
 
 
-def cc3m_issued_mfma(nsam, ri3):
-    """16x16x4 FP32 MFMA issued per fused CC3M item with MAXR2 = 32 (the
-    band-pruned transforms, folded over the cos/sin symmetry of the DFT
-    table): the column c2c takes (N/2 / 16) x 4 folded tiles of 16 products,
-    the row pass 32 per folded tile (16 forward, 16 back) for each 16-row
-    block and each tile that reaches inside the mask radius^2 ri3 (the
-    kernel's own test), the column r2c 8 waves x (N/4 / 2 + 1) x 4; 2048
-    flops each.  The ring-mean pass (AMAG != 1 only) is not counted."""
-    h = nsam // 2
-
-    def lo(v0):
-        a = v0 if v0 < h else v0 - nsam
-        b = a + 15
-        return 0 if a <= 0 <= b else min(a * a, b * b)
-    rows = sum(1 for rb in range(nsam // 16) for nt in range(h // 16)
-               if not lo(16 * nt) + lo(16 * rb) > ri3)
-    return (h // 16) * 4 * 16 + rows * 32 + 8 * (nsam // 8 + 1) * 4
+def cc3m_issued_mfma():
+    """16x16x4 FP32 MFMA issued per CC3M item on the band's 128-point grid
+    (MAXR2 = 32, AMAG = 1), folded over quarters of it: the column c2c takes 2 x 4
+    tiles of 16 products, each of the 8 16-row blocks 2 tiles of 16 forward and 16
+    back, the column r2c 8 tiles of 16; 2048 flops each."""
+    return 2 * 4 * 16 + 8 * 2 * 32 + 8 * 16
 
 
-CC3M_FLOPS = cc3m_issued_mfma(NSAM, (RI + 3.0) ** 2) * 2048.0
+CC3M_FLOPS = cc3m_issued_mfma() * 2048.0
 # the algorithmic unit of one CC3M evaluation: its two NSAM^2 FFTs (the c2r
 # and r2c of cc3m.f:113-115), 5 N^2 log2(N^2) flops each
 CC3M_FFT_FLOPS = 2 * 5.0 * NSAM * NSAM * math.log2(NSAM * NSAM)
@@ -427,7 +416,7 @@ def main():
             f"particles/s")
 
     # ------------------------------------------------------------ roofline
-    # dominant kernel of the learned step: the FP32 CC3M rescoring or the search GEMM
+    # dominant kernel of the learned step: the FP32 CC3M rescoring or the list search
     ncand = float(np.mean(valid))
     gemm_avg_s = gemm_ms / 1e3 / max(gemm_n, 1)
     cc3m_avg_s = cc3m_ms / 1e3 / max(cc3m_n, 1)
@@ -435,9 +424,9 @@ def main():
         items = B * TOPK
         flops = items * CC3M_FFT_FLOPS
         achieved = flops / cc3m_avg_s
-        roof = {"kernel": "k_cc3m_fused (FP32 MFMA)", "bound": "mfma", "achieved": achieved / 1e12,
+        roof = {"kernel": "k_cc3m_band (FP32 MFMA)", "bound": "mfma", "achieved": achieved / 1e12,
                 "peak": PEAK_FP32_MFMA / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_MFMA,
-                "traffic": measured_traffic(f"k_cc3m_fused_{items}"),
+                "traffic": measured_traffic(f"k_cc3m_band_{items}"),
                 "traffic_source": os.path.relpath(TRAFFIC_FILE, os.path.dirname(TRAFFIC_FILE) + "/.."),
                 "launch_ms": cc3m_avg_s * 1e3,
                 "algorithmic_unit": "two NSAM^2 FFTs per item, 2 x 5 N^2 log2(N^2) = "

@@ -527,7 +527,7 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
       if (unit_amag) continue;
       if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o,
                                     d_dm + 9 * (size_t)o, d_shift + 2 * (size_t)o, d_amag + o,
-                                    d_fsct, tabs, d_score + o, -1, nullptr, nullptr, true))
+                                    d_fsct, tabs, d_score + o, -1))
         return r;
     }
     c->prof_end(pslot);

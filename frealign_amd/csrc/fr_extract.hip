@@ -5,9 +5,9 @@
 //   negative-coordinate correction, the JC-1 clamps that double-weight the
 //   x = NSAM/2 plane) reproduced exactly.
 // k_pextract: PEXTRACT (pextract.f:8-101) for a batch of (particle, DM).
-// launch_cc3m: CC3M (cc3m.f:8-169) for a batch of (particle, DM, shift)
-//   items: annulus extraction x CTF x 1/NSAM^2 -> c2r -> MASKCOS2 -> r2c ->
-//   per-shell sums -> FP64 shell combination.
+// k_cc3m_fused: CC3M (cc3m.f:8-169) of a (particle, DM, shift) item on the NSAM
+//   grid in one workgroup, for AMAG other than 1: annulus extraction x CTF x
+//   1/NSAM^2 -> c2r -> MASKCOS2 -> r2c -> per-shell sums -> FP64 shell combination.
 #include <hip/hip_runtime.h>
 
 #include "fr_common.h"
@@ -108,7 +108,10 @@ __device__ inline void tile_r2(int v0, int nsamh, int nsam, int& lo, int& hi) {
 constexpr int cc3m_pts_words() { return (kCc3mPtsHdr + 32 * (2 * kFJ + 1) + 1) & ~1; }
 
 // kWin: the score at every shift of a window around the item's shift (the
-// best of them and its index), instead of at the item's shift alone
+// best of them and its index), instead of at the item's shift alone.  Without a
+// window the items with AMAG = 1 are the band grid's (fr_cc3m.hip) and left
+// alone; a window takes every item, those with AMAG = 1 by the tables of one
+// ring and mask.
 template <bool kWin>
 __global__ void __launch_bounds__(kFT)
     k_cc3m_fused(int nsam, int nitem, int maxr12, int maxr22, float rbfact,
@@ -120,7 +123,7 @@ __global__ void __launch_bounds__(kFT)
                  const int* __restrict__ pts, const float* __restrict__ ring_tab, int ring_cnt,
                  const float* __restrict__ wmap, float ri2,
                  float ri3, float rih, float halfw, float* score, Cc3mWindow win,
-                 int* __restrict__ wcode, int flip, int skip_unit) {
+                 int* __restrict__ wcode, int flip) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int hrow = nsam / 2 + 1;
   float* Ts = lds;                      // [nsam/2 + 1][kFP]: the folded table TF
@@ -154,7 +157,7 @@ __global__ void __launch_bounds__(kFT)
   // particle (a particle's candidates) reuse its band spectrum in LDS
   const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
   const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
-  if (skip_unit) {
+  if constexpr (!kWin) {
     bool any = false;
     for (int it = it0 + tid; it < it1; it += kFT) any |= amag_arr[it] != 1.0f;
     if (!__syncthreads_or(any)) return;
@@ -172,10 +175,10 @@ __global__ void __launch_bounds__(kFT)
   static_assert(64 * 64 % kFT == 0, "Q entries per thread");
   float qv[64 * 64 / kFT];
 #pragma unroll
-  for (int r = 0; r < 64 * 64 / kFT; r++) qv[r] = ring_tab ? ring_tab[tid + r * kFT] : 0.f;
+  for (int r = 0; r < 64 * 64 / kFT; r++) qv[r] = kWin ? ring_tab[tid + r * kFT] : 0.f;
   int pprev = -1;
   for (int it = it0; it < it1; it++) {
-  if (skip_unit && amag_arr[it] == 1.0f) continue;
+  if (!kWin && amag_arr[it] == 1.0f) continue;  // the band grid's item
   const int p = pidx[it];
   const bool newp = p != pprev;
   pprev = p;
@@ -224,7 +227,7 @@ __global__ void __launch_bounds__(kFT)
   // B(X)^T[c][k]: column c = (I, re|im), k = (|J|, cos|sin).  At AMAG = 1
   // the MASKCOS2 ring sum is linear in B: sum_{c,k} Q[c][k] B^T[c][k] with the
   // precomputed Q (the ring's rows of T through both transforms)
-  const bool ringq = ring_tab != nullptr && amagp == 1.0f;
+  const bool ringq = kWin && amagp == 1.0f;
   float rsum = 0.f;
   int rcnt = 0;
 #pragma unroll
@@ -306,7 +309,7 @@ __global__ void __launch_bounds__(kFT)
   }
   __syncthreads();
 
-  const bool use_wmap = wmap != nullptr && amagp == 1.0f;
+  const bool use_wmap = kWin && amagp == 1.0f;
   // ---- MASKCOS2 ring mean: x over ri2' < r^2 <= ri3'.  At AMAG = 1 the
   // ring sum was taken from B above; otherwise a pass over the ring tiles on
   // the matrix cores.
@@ -932,10 +935,10 @@ int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks
 int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
                       const float* ctff, const int* pidx, const float* dm, const float* shift,
                       const float* amag, const float* fsct, const Cc3mTables& t, float* score,
-                      int blocks, const Cc3mWindow* win, int* wcode, bool skip_unit) {
+                      int blocks, const Cc3mWindow* win, int* wcode) {
   if (a.n <= 0) return 0;
   FR_CHECK(cc3m_fused_ok(a.nsam, a.maxr2), "fused CC3M needs NSAM %% 32 == 0, NSAM <= 256, MAXR2 <= 32");
-  FR_CHECK(t.dft && t.pts, "fused CC3M tables missing");
+  FR_CHECK(t.dft && t.pts && t.ring && t.wmap, "fused CC3M tables missing");
   const size_t lds = cc3m_fused_lds(a.nsam);
   Cc3mWindow w{1, 1, 0.f, 0.f};
   if (win) {
@@ -958,7 +961,7 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
                        t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w, wcode,
-                       a.cc3, (int)skip_unit);
+                       a.cc3);
   else
     hipLaunchKernelGGL(k_cc3m_fused<false>, dim3((unsigned)grid), dim3(kFT), lds, c.stream,
                        a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2 * a.maxr2, a.rbfact,
@@ -966,7 +969,7 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
                        t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w,
-                       (int*)nullptr, a.cc3, (int)skip_unit);
+                       (int*)nullptr, a.cc3);
   FR_HIP(hipGetLastError());
   return 0;
 }

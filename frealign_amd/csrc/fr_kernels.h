@@ -99,11 +99,8 @@ struct Cc3mArgs {
   float rbfact, ri2, ri3, rih, halfw;
   int cc3 = 0;  // 1: CC3 (cc3.f): the section phase-flipped by the CTF sign, no |R| branch
 };
-// Scale by `scal`, then MASKCOS (origin=0) / MASKCOS2 (origin=1); one workgroup per image.
+
 constexpr int kMaskThreads = 1024;
-__global__ void k_scale_mask(int nsam, float* data, size_t img_stride, float scal,
-                             const float* amag_arr, int amag_stride, float ri2, float ri3,
-                             float rih, float halfw, int origin);
 // On the particle's grid, any box, band and AMAG (fr_cc3m_fft.hip); work:
 // cc3m_fft_bytes for the items of the call (PRESB: MAXR2 = NSAM/2).
 struct Cc3mRing {
@@ -168,12 +165,11 @@ struct Cc3mWindow {
   int nsx, nsy;
   float dsx, dsy;
 };
-// skip_unit: leave the items with AMAG = 1 alone
+// Without a window the items with AMAG = 1 are left alone.
 int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
                       const float* ctff, const int* pidx, const float* dm, const float* shift,
                       const float* amag, const float* fsct, const Cc3mTables& t, float* score,
-                      int blocks = 0, const Cc3mWindow* win = nullptr, int* wcode = nullptr,
-                      bool skip_unit = false);
+                      int blocks = 0, const Cc3mWindow* win = nullptr, int* wcode = nullptr);
 // The launch's workgroups: `blocks` (0: one per item; below 0: what the device
 // holds at once), at most one per item.
 int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks, int* grid);

@@ -92,8 +92,7 @@ int enqueue(fr_plan* p) {
                                  p->d_shift, p->d_amag, p->fsct, p->band, p->d_score, p->blocks))
       return r;
     if (int r = launch_cc3m_fused(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm,
-                                  p->d_shift, p->d_amag, p->fsct, p->tabs, p->d_score, -1,
-                                  nullptr, nullptr, true))
+                                  p->d_shift, p->d_amag, p->fsct, p->tabs, p->d_score, -1))
       return r;
   } else {
     if (int r = launch_cc3m(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm, p->d_shift,

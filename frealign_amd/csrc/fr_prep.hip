@@ -583,31 +583,25 @@ __device__ inline float block_sum(float v, float* red) {
 
 }  // namespace
 
-// ctfapply.f:107-122 and maskcos.f / maskcos2.f: scale, then cosine-edged
-// real-space mask.  origin=0 centres the disc at NSAM/2+1 (MASKCOS), origin=1
-// at the FFT origin (MASKCOS2).  One workgroup per image: a read-only pass for
+// ctfapply.f:107-122 and maskcos.f: scale, then the cosine-edged real-space mask
+// centred at NSAM/2+1.  One workgroup per image: a read-only pass for
 // the mean of the scaled ring, then one pass that scales, masks and writes.
 // Threads take fixed columns and step over rows (no per-pixel division).
 __global__ void __launch_bounds__(kMaskThreads)
     k_scale_mask(int nsam, float* data, size_t img_stride, float scal, const float* amag_arr,
-                 int amag_stride, float ri2, float ri3, float rih, float halfw, int origin) {
+                 int amag_stride, float ri2, float ri3, float rih, float halfw) {
   __shared__ float red[kMaskThreads / 64];
   __shared__ int redi[kMaskThreads / 64];
   float* img = data + blockIdx.x * img_stride;
   const float amagp = amag_arr[(size_t)blockIdx.x * amag_stride];
   const float rihp = rih / amagp, ri2p = ri2 / amagp / amagp, ri3p = ri3 / amagp / amagp;
-  const int nmid = origin ? 1 : nsam / 2 + 1, nsamh = nsam / 2, pitch = nsam + 2;
+  const int nmid = nsam / 2 + 1, pitch = nsam + 2;
   const int nt = blockDim.x;
   const int cols = nsam < nt ? nsam : nt, rstep = nt / cols;
   const int c0 = threadIdx.x % cols, r0 = threadIdx.x / cols;
   const bool act = r0 < rstep;
   auto rad2 = [&](int i, int jx) {  // 1-based pixel (i, jx)
-    int ii = i, jj = jx;
-    if (origin) {
-      if (ii > nsamh) ii -= nsam;
-      if (jj > nsamh) jj -= nsam;
-    }
-    float d1 = (float)(ii - nmid), d2 = (float)(jj - nmid);
+    float d1 = (float)(i - nmid), d2 = (float)(jx - nmid);
     float crad2;
     {
 #pragma clang fp contract(off)
@@ -853,8 +847,7 @@ int launch_ctfapply(Ctx& c, int nsam, int nb, const float* spec, const float* pp
   if (int r = fft_c2r_2d(c, nsam, nb, outc, img)) return r;
   // ctfapply.f:107-122; per-particle AMAGP is column 5 of ppar
   hipLaunchKernelGGL(k_scale_mask, dim3(nb), dim3(kMaskThreads), 0, c.stream, nsam, outc, img,
-                     1.0f / (float)nsam / (float)nsam, ppar + 5, 8, g.ri2, g.ri3, g.rih, g.halfw,
-                     0);
+                     1.0f / (float)nsam / (float)nsam, ppar + 5, 8, g.ri2, g.ri3, g.rih, g.halfw);
   FR_HIP(hipGetLastError());
   if (int r = fft_r2c_2d(c, nsam, nb, outc, img)) return r;
   return origin_pweight(c, nsam, nb, pssnr, g, ctff, outc);

@@ -282,7 +282,8 @@ int fr_storeshift(fr_ctx *ctx, int nsam, double std_, double vtd, int iredun, co
  * orientation) is scored as CCP scores a view: argmax over -6..6 (x outer,
  * first max wins), 3x3 box sum /9, normalised by sqrt(sum|cT|^2 sum|X|^2).
  * dtype 1 runs the correlation as a BF16 MFMA GEMM with FP32 accumulation,
- * dtype 0 as an FP32 MFMA GEMM.  dtype 2 (MAXR2 <= 32) evaluates the same
+ * dtype 0 in FP32 (MAXR2 <= 32: the shifts in two separable stages; wider
+ * bands: an FP32 MFMA GEMM).  dtype 2 (MAXR2 <= 32) evaluates the same
  * 15x15 map on the BF16 matrix cores in two separable stages (the J phase,
  * then the I phase) from a bank in the separable layout. */
 
