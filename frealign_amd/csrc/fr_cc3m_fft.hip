@@ -566,16 +566,23 @@ int cc3m_ring_hat(int nsam, float ri2, float ri3, int maxr2, std::vector<float>&
       const float r2 = (float)(x * x + y * y);
       if (!(r2 > ri2 && r2 <= ri3)) continue;
       cnt += (long long)mult(x) * mult(y);
-      for (int i = 0; i < cb; i++)
-        row[(size_t)y * cb + i] += mult(x) * co[(long long)i * x % nsam];
+      for (int i = 0, at = 0; i < cb; i++) {
+        row[(size_t)y * cb + i] += mult(x) * co[at];
+        at += x;
+        if (at >= nsam) at -= nsam;
+      }
     }
   out.assign((size_t)maxr2 * cb, 0.f);
-  for (int j = 0; j < maxr2; j++)
-    for (int i = 0; i < cb; i++) {
-      double s = 0.0;
-      for (int y = 0; y <= h; y++) s += mult(y) * co[(long long)j * y % nsam] * row[(size_t)y * cb + i];
-      out[(size_t)j * cb + i] = (float)s;
+  std::vector<double> sum(cb);
+  for (int j = 0; j < maxr2; j++) {
+    std::fill(sum.begin(), sum.end(), 0.0);
+    for (int y = 0; y <= h; y++) {
+      const double c = mult(y) * co[(long long)j * y % nsam];
+      const double* r = &row[(size_t)y * cb];
+      for (int i = 0; i < cb; i++) sum[i] += c * r[i];
     }
+    for (int i = 0; i < cb; i++) out[(size_t)j * cb + i] = (float)sum[i];
+  }
   return (int)cnt;
 }
 
