@@ -1060,13 +1060,20 @@ int fr_search_batch(fr_ctx* c, int nsam, int maxr1, int maxr2, float rbfact, int
   if (int r = launch_search_feats(*c, nsam, np, c->kc, c->kpad, maxr2 * maxr2, rbfact, d_outc,
                                   d_ctff, c->d_kidx, ap, c2, sum2))
     return r;
-  // FP32 with separable shifts where its registers hold the band; a wider band
-  // takes the 225-row product (64 particles x 46,800 templates at MAXR2 = 32:
-  // 40.4 ms as the product)
-  if (dtype == 0 && maxr2 <= kSepMaxR2) {
+  // FP32 with separable shifts where its registers hold the band and the band is
+  // worth its fixed work: 32 particles x 46,800 templates at MAXR2 = 4 take 845 us
+  // as the 225-row product and 1,174 separable, at 6 1,226 and 1,180, at 8 1,812 and
+  // 1,192; 64 at MAXR2 = 32 40.5 and 7.4 ms
+  if (dtype == 0 && maxr2 >= 6 && maxr2 <= kSepMaxR2) {
+    int* ties = (int*)c->slot(2, sizeof(int) * ((size_t)np * norient + np), &err);
+    if (!ties) return err;
+    int* ntie = ties + (size_t)np * norient;
     int pslot = c->prof_begin(kProfSearchGemm);
     if (int r = launch_search_sep32(*c, np, norient, maxr2, c->kc, c->kpad, c->nsamr, c->d_kidx,
-                                    d_bank, ap, c2, sum2, score, brow))
+                                    d_bank, ap, c2, sum2, score, brow, ntie, ties))
+      return r;
+    if (int r = launch_search_ties(*c, np, norient, c->kpad, d_bank, ntie, ties, ap, c2, sum2,
+                                   c->d_shx, c->d_shy, score, brow))
       return r;
     c->prof_end(pslot);
     return launch_topk(*c, norient, np, norient, group, nullptr, nullptr, nullptr, 0, topk, score,

@@ -42,10 +42,15 @@ int launch_search_sep(Ctx& c, int np, int nbank, int nsamr, int nrow, const int*
                       const int* ord = nullptr);
 // the exhaustive FP32 search with separable shifts (fr_search_f32.hip), MAXR2 <=
 // kSepMaxR2: the annulus bank (kc points of kidx, rows of kpad floats) against the
-// particle terms of launch_search_feats
+// particle terms of launch_search_feats.  ntie[p] and ties[p * norient ..]: the
+// orientations whose peak it leaves to launch_search_ties
 int launch_search_sep32(Ctx& c, int np, int norient, int maxr2, int kc, int kpad, int nsamr,
                         const int* kidx, const void* bank, const float* ap, const float* c2,
-                        const float* sum2, float* score, int* best_row);
+                        const float* sum2, float* score, int* best_row, int* ntie, int* ties);
+// those pairs by the 225-row product, as a list search has them
+int launch_search_ties(Ctx& c, int np, int nbank, int kpad, const void* bank, const int* ntie,
+                       const int* ties, const float* ap, const float* c2, const float* sum2,
+                       const float* shx_tab, const float* shy_tab, float* score, int* best_row);
 int launch_topk(Ctx& c, int nbank, int np, int n, int group, const int* loff, const int* grp,
                 const int* cand, int cap, int topk, const float* score, const int* best_row,
                 int* top_o, int* top_row, float* top_s);

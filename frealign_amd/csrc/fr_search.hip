@@ -24,6 +24,8 @@
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "fr_common.h"
 #include "fr_extract.h"
 #include "fr_search.h"
@@ -195,47 +197,43 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 // ---------------------------------------------------------------- GEMM
-constexpr int kGemmThreads = 512;  // 8 waves: 4 row groups x 2 column groups
+constexpr int kGemmThreads = 512;  // 8 waves: 4 row groups x 2 column groups of CT x 16
 
-template <typename T>
-__device__ inline void mma_step(const T* As, const T* Bs, floatx4 (&acc)[4][8], int wr, int wc,
-                                int lane);
-
-template <>
-__device__ inline void mma_step<__bf16>(const __bf16* As, const __bf16* Bs,
-                                        floatx4 (&acc)[4][8], int wr, int wc, int lane) {
+template <int CT>
+__device__ inline void mma_step(const __bf16* As, const __bf16* Bs, floatx4 (&acc)[4][CT], int wr,
+                                int wc, int lane) {
   constexpr int P = Elem<__bf16>::kPad;
   const int lr = lane & 15, kq = (lane >> 4) * 8;
-  bf16x8 a[4], b[8];
+  bf16x8 a[4], b[CT];
 #pragma unroll
   for (int rt = 0; rt < 4; rt++)
     a[rt] = *reinterpret_cast<const bf16x8*>(As + (wr * 64 + rt * 16 + lr) * P + kq);
 #pragma unroll
-  for (int ct = 0; ct < 8; ct++)
-    b[ct] = *reinterpret_cast<const bf16x8*>(Bs + (wc * 128 + ct * 16 + lr) * P + kq);
+  for (int ct = 0; ct < CT; ct++)
+    b[ct] = *reinterpret_cast<const bf16x8*>(Bs + (wc * CT * 16 + ct * 16 + lr) * P + kq);
 #pragma unroll
   for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-    for (int ct = 0; ct < 8; ct++)
+    for (int ct = 0; ct < CT; ct++)
       acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], b[ct], acc[rt][ct], 0, 0, 0);
 }
 
-template <>
-__device__ inline void mma_step<float>(const float* As, const float* Bs, floatx4 (&acc)[4][8],
-                                       int wr, int wc, int lane) {
+template <int CT>
+__device__ inline void mma_step(const float* As, const float* Bs, floatx4 (&acc)[4][CT], int wr,
+                                int wc, int lane) {
   constexpr int P = Elem<float>::kPad;
   const int lr = lane & 15, kq = lane >> 4;
 #pragma unroll
   for (int kk = 0; kk < kKStep; kk += 4) {
-    float a[4], b[8];
+    float a[4], b[CT];
 #pragma unroll
     for (int rt = 0; rt < 4; rt++) a[rt] = As[(wr * 64 + rt * 16 + lr) * P + kk + kq];
 #pragma unroll
-    for (int ct = 0; ct < 8; ct++) b[ct] = Bs[(wc * 128 + ct * 16 + lr) * P + kk + kq];
+    for (int ct = 0; ct < CT; ct++) b[ct] = Bs[(wc * CT * 16 + ct * 16 + lr) * P + kk + kq];
 #pragma unroll
     for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-      for (int ct = 0; ct < 8; ct++)
+      for (int ct = 0; ct < CT; ct++)
         acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt], b[ct], acc[rt][ct], 0, 0, 0);
   }
 }
@@ -244,11 +242,11 @@ __device__ inline void mma_step<float>(const float* As, const float* Bs, floatx4
 // and three table buffers, each holding the chunk's 16x15 X'(k) e^{i I sx}
 // and 16x15 e^{i J sy} phase entries and its 16 weights |c_p(k)|^2.  The
 // epilogue map [kRows][65] floats aliases the operand buffers; the column
-// norms' partial sums alias the table buffers.
-template <typename T>
+// norms' partial sums alias the table buffers.  NC: columns of the tile.
+template <typename T, int NC = kCols>
 struct Lds {
   static constexpr size_t a_bytes = (size_t)kRows * Elem<T>::kPad * sizeof(T);
-  static constexpr size_t b_bytes = (size_t)kCols * Elem<T>::kPad * sizeof(T);
+  static constexpr size_t b_bytes = (size_t)NC * Elem<T>::kPad * sizeof(T);
   static constexpr size_t op_bytes = a_bytes + b_bytes;  // one buffer
   static constexpr int tab_entries = 2 * 16 * kShift + 16;
   static constexpr size_t tab_one = tab_entries * sizeof(float2);
@@ -265,16 +263,17 @@ constexpr size_t lds_total() {
   return Lds<T>::total;
 }
 
-// B chunk transfer: kCols templates x 32 reals, in 16-byte pieces.
-template <typename T>
+// B chunk transfer: NC templates x 32 reals, in 16-byte pieces.
+template <typename T, int NC>
 struct BPieces {
   static constexpr int per_row = 32 * sizeof(T) / 16;      // 4 (bf16) or 8 (fp32)
-  static constexpr int total = kCols * per_row;             // 1024 or 2048
-  static constexpr int per_thread = total / kGemmThreads;   // 2 or 4
+  static constexpr int total = NC * per_row;
+  static constexpr int per_thread = total / kGemmThreads;   // 2 or 4 for kCols
+  static_assert(total % kGemmThreads == 0, "whole pieces per thread");
   static constexpr int elems = 16 / sizeof(T);              // elements per piece
 };
 
-// One tile: the 225 shift rows of particle p against columns o0..o0+255 of
+// One tile: the 225 shift rows of particle p against columns o0..o0+NC-1 of
 // its template list (list entry cand_p[o], or o itself when cand_p is null;
 // entries outside 0..nbank-1 are empty columns).  The normalisation
 // sum_k |c_p(k)|^2 |T_o(k)|^2 (SUM of ccp.f:211-214 with the CTF folded on
@@ -283,8 +282,9 @@ struct BPieces {
 // pays where the template rows are gathered (candidate lists) and the K
 // loop waits on memory, not where it streams the bank (the exhaustive
 // search, whose norms k_search_norm computes).  Outputs are indexed by list
-// position.
-template <typename T, bool kFused, bool kLoop>
+// position, or with kAtCand by list entry.  A column's sums do not depend on the
+// tile it is in: every form gives it the same map, bit for bit.
+template <typename T, bool kFused, bool kLoop, int NC = kCols, bool kAtCand = false>
 __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int ncol, int nbank,
                                           int kpad, const T* __restrict__ bank,
                                           const int* __restrict__ cand_p,
@@ -295,8 +295,9 @@ __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int n
                                           const float2* __restrict__ shy_tab, float* score_p,
                                           int* brow_p) {
   constexpr int P = Elem<T>::kPad;
-  using L = Lds<T>;
-  using BP = BPieces<T>;
+  constexpr int CT = NC / 32;  // a wave's column blocks of 16
+  using L = Lds<T, NC>;
+  using BP = BPieces<T, NC>;
   auto As = [&](int buf) { return reinterpret_cast<T*>(smem_raw + buf * L::op_bytes); };
   auto Bs = [&](int buf) { return reinterpret_cast<T*>(smem_raw + buf * L::op_bytes + L::a_bytes); };
   auto tabx = [&](int buf) {
@@ -309,11 +310,11 @@ __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int n
   const int half = kpad / 2;
   const int nchunk = half / 16;
 
-  floatx4 acc[4][8];
+  floatx4 acc[4][CT];
 #pragma unroll
   for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-    for (int ct = 0; ct < 8; ct++) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < CT; ct++) acc[rt][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
   float nacc = 0.f;  // norm partial: column tid/2, complex 8*(tid%2)..+7 of each chunk
 
   // this thread's B pieces: piece bq of templates bc0 + u * bstep, for the
@@ -436,8 +437,8 @@ __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int n
       const int cur = kc & 1, nxt = cur ^ 1;
       const bool more = kc + 1 < nchunk;
       if (kc + 2 < nchunk) load_tab(kc + 2);
-      mma_step<T>(As(cur), Bs(cur), acc, wr, wc, lane);
-      if (kFused) norm_step(cur, kc % 3);
+      mma_step<CT>(As(cur), Bs(cur), acc, wr, wc, lane);
+      if (kFused && (NC == kCols || row < NC)) norm_step(cur, kc % 3);
       if (more) {
         gen_a(nxt, (kc + 1) % 3);
         store_b(nxt, breg[(d + 1) % kBDepth]);
@@ -453,18 +454,19 @@ __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int n
   float* nl = reinterpret_cast<float*>(smem_raw + L::tab_off);
   if (kFused) nl[tid] = nacc;
 #pragma unroll
-  for (int q4 = 0; q4 < 4; q4++) {  // 64-column quarters of the 256 templates
+  for (int q4 = 0; q4 < NC / 64; q4++) {  // the templates 64 columns at a time
     if (q4) __syncthreads();
-    if (wc == (q4 >> 1)) {
+    constexpr int W = CT < 4 ? CT : 4;    // of the wave's blocks, those in the 64
+    if (NC == 64 || wc == (q4 >> 1)) {
 #pragma unroll
       for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++)
+        for (int ct = 0; ct < W; ct++)
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             int r = wr * 64 + rt * 16 + (lane >> 4) * 4 + i;
-            int c = ct * 16 + (lane & 15);
-            ep[r * 65 + c] = acc[rt][ct + 4 * (q4 & 1)][i];
+            int c = (NC == 64 ? wc * W * 16 : 0) + ct * 16 + (lane & 15);
+            ep[r * 65 + c] = acc[rt][NC == 64 ? ct : ct + 4 * (q4 & 1)][i];
           }
     }
     __syncthreads();
@@ -485,8 +487,9 @@ __device__ __forceinline__ void gemm_tile(unsigned char* smem_raw, int o0, int n
       if (o < ncol) {
         float n = kFused ? nl[2 * cc] + nl[2 * cc + 1] : nrm_p[o];
         float v = (n > 0.f && s2 > 0.f) ? box / sqrtf(n) / sqrtf(s2) / 9.0f : -3.0e38f;
-        score_p[o] = v;
-        brow_p[o] = (bx + 7) * kShift + (by + 7);
+        const int at = kAtCand ? cand_p[o] : o;
+        score_p[at] = v;
+        brow_p[at] = (bx + 7) * kShift + (by + 7);
       }
     }
   }
@@ -553,6 +556,28 @@ __global__ void __launch_bounds__(kGemmThreads)
                        cand + base, ap + (size_t)p * half, c2 + (size_t)p * half, nullptr,
                        sum2[p], shx_tab, shy_tab, score + base, best_row + base);
   }
+}
+
+// The pairs whose peak the separable FP32 search left undecided
+// (fr_search_f32.hip): particle p's ntie[p] orientations in ties[p * nbank ..],
+// their scores and rows put where the orientation's are.  Tiles of 64 columns:
+// a particle has some tens of them, and a tile's time is its columns'.
+constexpr int kTieCols = 64;
+
+__global__ void __launch_bounds__(kGemmThreads)
+    k_search_gemm_ties(int np, int nbank, int kpad, const float* __restrict__ bank,
+                       const int* __restrict__ ntie, const int* __restrict__ ties,
+                       const float2* __restrict__ ap, const float* __restrict__ c2,
+                       const float* __restrict__ sum2, const float2* __restrict__ shx_tab,
+                       const float2* __restrict__ shy_tab, float* score, int* best_row) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int p = blockIdx.x % np, n = ntie[p], half = kpad / 2;
+  const size_t base = (size_t)p * nbank;
+  const int step = (int)(gridDim.x / np) * kTieCols;
+  for (int o0 = (int)(blockIdx.x / np) * kTieCols; o0 < n; o0 += step)
+    gemm_tile<float, true, true, kTieCols, true>(
+        smem_raw, o0, n, nbank, kpad, bank, ties + base, ap + (size_t)p * half,
+        c2 + (size_t)p * half, nullptr, sum2[p], shx_tab, shy_tab, score + base, best_row + base);
 }
 
 // ---------------------------------------------------------------- top-K
@@ -797,6 +822,28 @@ int launch_search_gemm_ragged(Ctx& c, int np, int nbank, int kpad, const void* b
     hipLaunchKernelGGL(k_search_gemm_ragged<float>, dim3(grid), dim3(kGemmThreads), lds,
                        c.stream, np, nbank, kpad, reinterpret_cast<const float*>(bank), loff, toff,
                        cand, cap, apv, c2, sum2, sx, sy, score, best_row);
+  FR_HIP(hipGetLastError());
+  return 0;
+}
+
+int launch_search_ties(Ctx& c, int np, int nbank, int kpad, const void* bank, const int* ntie,
+                       const int* ties, const float* ap, const float* c2, const float* sum2,
+                       const float* shx_tab, const float* shy_tab, float* score, int* best_row) {
+  const size_t lds = Lds<float, kTieCols>::total;
+  if (int r = set_gemm_lds<float>((const void*)k_search_gemm_ties, lds)) return r;
+  if (c.cus <= 0) {
+    hipDeviceProp_t prop;
+    FR_HIP(hipGetDeviceProperties(&prop, c.device));
+    c.cus = prop.multiProcessorCount;
+  }
+  // a place for every workgroup of a CU each; a particle's workgroups share its tiles
+  const int most = (nbank + kTieCols - 1) / kTieCols;
+  const int per = std::max(1, std::min(most, c.cus / np));
+  hipLaunchKernelGGL(k_search_gemm_ties, dim3((unsigned)(per * np)), dim3(kGemmThreads), lds,
+                     c.stream, np, nbank, kpad, reinterpret_cast<const float*>(bank), ntie, ties,
+                     reinterpret_cast<const float2*>(ap), c2, sum2,
+                     reinterpret_cast<const float2*>(shx_tab),
+                     reinterpret_cast<const float2*>(shy_tab), score, best_row);
   FR_HIP(hipGetLastError());
   return 0;
 }

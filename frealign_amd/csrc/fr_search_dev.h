@@ -47,10 +47,11 @@ __device__ inline void phase(int a, int n, float& c, float& s) {
 // first maximum: the maximum value across the wave, then the first (sx, sy)
 // holding it from the lanes' ballots (of the lanes of one i, the lowest has the
 // smallest sx and then the smallest sy); the 3 x 3 box sum around it by lane
-// reads.  Uniform results.
-__device__ __forceinline__ void ccp_peak(const floatx4& map, int g, int n, float& box, int& row) {
+// reads.  Uniform results; m is the maximum.
+__device__ __forceinline__ void ccp_peak(const floatx4& map, int g, int n, float& box, int& row,
+                                         float& m) {
   bool ok[4];
-  float m = -3.4e38f;
+  m = -3.4e38f;
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int sx = 4 * g + i;

@@ -20,9 +20,19 @@
 // template is written while this one is used); the particle's terms stay in
 // registers.  Sum |c T|^2 for the normalisation accumulates beside the products.
 //
+// CCP takes the first maximum of the map's inner 13 x 13 and then a 3 x 3 box
+// about it, so where two cells tie to a rounding the order of the sums decides, and
+// the two boxes may differ by a percent.  A pair whose second cell lies within kTie
+// of its first is therefore noted and its peak taken from the 225-row product
+// (k_search_gemm_ties), by which list searches decide: the same pair has the same
+// peak in both.  kTie: a cell is at most 2 x 1,640 products summed in FP32, each
+// step rounded to 2^-24 of at most sqrt(sum |c T|^2 sum |X|^2); as a random walk
+// sqrt(3280) 2^-24, times 4: 2^-16 of that root.  Two orders of the sums differ by
+// up to 4.0e-6 of it over 50,400 pairs at MAXR2 = 32, a quarter; 0.3% of them tie.
+//
 // What bounds it: the matrix cores (76 x 32 cycles a pair) with about 430 vector
 // instructions a pair beside them.  64 particles x 46,800 templates at MAXR2 = 32:
-// 7.1 ms, 40.3 ms as the 225-row product with its separate norms.
+// 7.4 ms (0.3 of it the ties), 40.5 ms as the 225-row product with its separate norms.
 #include <hip/hip_runtime.h>
 
 #include "fr_common.h"
@@ -34,6 +44,7 @@ namespace fr {
 namespace {
 
 constexpr int kThr = 256;
+constexpr float kTie = 0x1p-16f;
 
 template <int R>
 struct Shape32 {
@@ -50,7 +61,7 @@ __global__ void __launch_bounds__(kThr, 2)
                    const int2* __restrict__ kidx, const float2* __restrict__ bank,
                    const float2* __restrict__ ap, const float* __restrict__ c2,
                    const float* __restrict__ sum2, float* __restrict__ score,
-                   int* __restrict__ best_row) {
+                   int* __restrict__ best_row, int* __restrict__ ntie, int* __restrict__ ties) {
   using S = Shape32<R>;
   constexpr int kNT = S::kNT, kKS = S::kKS, kPer = S::kPer, kF = kNT * kKS;
   // [buffer][block][lane]: (+J, -J) of the lane's point
@@ -173,9 +184,20 @@ __global__ void __launch_bounds__(kThr, 2)
       floatx4 map;
 #pragma unroll
       for (int i = 0; i < 4; i++) map[i] = m[0][i] - m[1][i];
-      float box;
+      float box, top;
       int row;
-      ccp_peak(map, g, n, box, row);
+      ccp_peak(map, g, n, box, row, top);
+      // cells at the top; none where the map has no ordered value
+      const float tied = top - kTie * sqrtf(nacc * s2);
+      int near = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int sx = 4 * g + i;
+        const bool in = sx >= 1 && sx <= 13 && n >= 1 && n <= 13;
+        near += __popcll(__ballot(in && map[i] >= tied));
+      }
+      if (near != 1 && nacc > 0.f && s2 > 0.f && lane == 0)
+        ties[(size_t)p * norient + atomicAdd(&ntie[p], 1)] = o;
       const int slot = (o - lo) & 63;
       if (lane == slot) {
         box_l = box;
@@ -194,10 +216,15 @@ __global__ void __launch_bounds__(kThr, 2)
   }
 }
 
+__global__ void k_no_ties(int np, int* ntie) {
+  const int p = blockIdx.x * kThr + threadIdx.x;
+  if (p < np) ntie[p] = 0;
+}
+
 template <int R>
 int launch_r(Ctx& c, int np, int norient, int kc, int pitch, int nsamr, const int* kidx,
              const void* bank, const float* ap, const float* c2, const float* sum2, float* score,
-             int* best_row) {
+             int* best_row, int* ntie, int* ties) {
   if (c.cus <= 0) {
     hipDeviceProp_t prop;
     FR_HIP(hipGetDeviceProperties(&prop, c.device));
@@ -211,10 +238,12 @@ int launch_r(Ctx& c, int np, int norient, int kc, int pitch, int nsamr, const in
   const int ntile = (norient + tile - 1) / tile;
   const size_t nblk = (size_t)((ntile + 7) / 8 * 8) * npq;
   FR_CHECK(nblk < (1u << 31), "search grid too large");
+  hipLaunchKernelGGL(k_no_ties, dim3((np + kThr - 1) / kThr), dim3(kThr), 0, c.stream, np, ntie);
+  FR_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_search_sep32<R>, dim3((unsigned)nblk), dim3(kThr), 0, c.stream, np, norient,
                      kc, pitch, nsamr, ntile, tile, reinterpret_cast<const int2*>(kidx),
                      reinterpret_cast<const float2*>(bank), reinterpret_cast<const float2*>(ap),
-                     c2, sum2, score, best_row);
+                     c2, sum2, score, best_row, ntie, ties);
   FR_HIP(hipGetLastError());
   return 0;
 }
@@ -223,11 +252,12 @@ int launch_r(Ctx& c, int np, int norient, int kc, int pitch, int nsamr, const in
 
 int launch_search_sep32(Ctx& c, int np, int norient, int maxr2, int kc, int kpad, int nsamr,
                         const int* kidx, const void* bank, const float* ap, const float* c2,
-                        const float* sum2, float* score, int* best_row) {
+                        const float* sum2, float* score, int* best_row, int* ntie, int* ties) {
   if (np <= 0 || norient <= 0) return 0;
   FR_CHECK(maxr2 <= kSepMaxR2, "the separable search holds MAXR2 <= %d (got %d)", kSepMaxR2, maxr2);
   auto go = [&](auto fn) {
-    return fn(c, np, norient, kc, kpad / 2, nsamr, kidx, bank, ap, c2, sum2, score, best_row);
+    return fn(c, np, norient, kc, kpad / 2, nsamr, kidx, bank, ap, c2, sum2, score, best_row, ntie,
+              ties);
   };
   if (maxr2 <= 16) return go(launch_r<16>);
   if (maxr2 <= 24) return go(launch_r<24>);

@@ -288,9 +288,9 @@ __global__ void __launch_bounds__(kSepThreads, 2)
     floatx4 acc2;
 #pragma unroll
     for (int i = 0; i < 4; i++) acc2[i] = acc2h[0][i] + acc2h[1][i];
-    float box;
+    float box, top;
     int row;
-    ccp_peak(acc2, g, n, box, row);
+    ccp_peak(acc2, g, n, box, row, top);
     if (lane == at) {
       box_l = box;
       norm_l = nacc;
