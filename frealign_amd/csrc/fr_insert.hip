@@ -43,7 +43,12 @@
 // The _SE variant (PINSERT_TRILIN_SE with NNSTAT = 1,
 // pinsert_trilin_se.f:186-194) also sums, per voxel, the count, |term|^2,
 // |term| and the phase difference to the reference transform of the terms it
-// receives, over both halves: its workgroups take the two halves in turn.
+// receives, over both halves: a second launch of the same form, whose sums are
+// these and whose lists hold both halves' tasks.  A point's eight terms are its
+// sample times real weights, so their size and phase are formed once, and the
+// reference's phases once per tile.  In one launch with the sums, both took
+// 112 KB, one workgroup a CU: 4 particles at 256^3 450 us, 64 particles 1,458,
+// 300 at 150^3 1,296; now 224, 711 and 650 (as the gather 237, 711 and 1,534).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -287,11 +292,34 @@ __device__ inline bool plane_reaches(const float4& g, float xl, float xh, float 
   return cx * cx + cy * cy + cz * cz <= g.w;
 }
 
-// pdiff.f:8-24: |phase of b conj(r)|, 0 where the product is 0
-__device__ inline float pdiff_dev(float br, float bi, float2 r) {
-  const float cr = br * r.x + bi * r.y, ci = bi * r.x - br * r.y;
-  if (cr == 0.0f && ci == 0.0f) return 0.0f;
-  return fabsf(atan2f(ci, cr));
+// Phases as whole turns times 2^32, whose differences wrap by themselves: exact
+// octants and the arctangent of a ratio up to 1, scaled in 64 bits.  Against 64
+// bits a difference is 4.0e-8 radians off (rms of 2e7, most 2.1e-7), as the
+// arctangent of the product formed in FP32 is (4.0e-8, 2.9e-7).
+__device__ inline unsigned turns(float x, float y) {
+  const float ax = fabsf(x), ay = fabsf(y), mx = fmaxf(ax, ay);
+  const double a = atanf(mx > 0.f ? fminf(ax, ay) / mx : 0.f);
+  unsigned u = (unsigned)(a * 683565275.57643158 + 0.5);  // 2^32 / 2 pi
+  if (ay > ax) u = (1u << 30) - u;
+  if (x < 0.f) u = (1u << 31) - u;
+  return y < 0.f ? 0u - u : u;
+}
+
+// A voxel's reference phase, odd; kNoPhase where the value is zero (pdiff.f:8-24:
+// no difference), kBadPhase where it is no number
+constexpr unsigned kNoPhase = 0u, kBadPhase = 2u;
+__device__ inline unsigned ref_phase(float2 r) {
+  if (!(fabsf(r.x) <= 3.4e38f && fabsf(r.y) <= 3.4e38f)) return kBadPhase;
+  return r.x == 0.f && r.y == 0.f ? kNoPhase : turns(r.x, r.y) | 1u;
+}
+
+// pdiff.f:8-24: |phase of b conj(r)| of a term of size ab and phase p
+__device__ inline float pdiff_dev(float ab, unsigned p, unsigned ref) {
+  if (ref == kBadPhase) return __int_as_float(0x7fc00000);
+  const int d = (int)(p - ref);
+  const unsigned m = d < 0 ? 0u - (unsigned)d : (unsigned)d;
+  const float v = (float)((double)m * 1.4629180792671596e-9);  // 2 pi / 2^32
+  return ab == 0.f || ref == kNoPhase ? 0.f : v + (ab - ab);
 }
 
 // inclusive prefix sum over each 32 lanes, on the vector ALU
@@ -316,6 +344,11 @@ __device__ inline void wave_lds() {
 
 struct Sum {
   float re, im, c2;  // numerator, CTF^2
+  __device__ void add(const Sum& o) {
+    re += o.re;
+    im += o.im;
+    c2 += o.c2;
+  }
 };
 constexpr int kOut = 1 << 20;             // byte offset of a corner outside the tile
 
@@ -345,12 +378,19 @@ struct Axis {
 struct StatSum {
   float v, a, p;  // |term|^2, |term|, phase difference
   int n;
+  __device__ void add(const StatSum& o) {
+    v += o.v;
+    a += o.a;
+    p += o.p;
+    n += o.n;
+  }
 };
 
 template <bool kStats>
 struct TileSums {
-  Sum sum[kWaves][kSets * kVox];
-  StatSum st[kStats ? kWaves : 1][kStats ? kSets * kVox : 1];
+  using Acc = std::conditional_t<kStats, StatSum, Sum>;
+  Acc sum[kWaves][kSets * kVox];
+  unsigned ref[kStats ? kVox : 1];     // the reference transform's phases in the tile
   int list[kList];
   int tot[kWaves];
   int2 row[kWaves][kSets][kLanes];     // I | first J << 16, start
@@ -360,6 +400,7 @@ struct TileSums {
   double rt[kWaves];
 };
 
+// kStats: the statistics of the terms, both halves' together, instead of their sums
 template <bool kStats>
 __global__ void __launch_bounds__(kThreads)
     k_insert_scatter(int nsam, int ntask, int tx, int ty, int tz, const int* __restrict__ n0p,
@@ -367,12 +408,16 @@ __global__ void __launch_bounds__(kThreads)
                      const float4* __restrict__ pts, float2* num0, float* ctf2_0, float2* num1,
                      float* ctf2_1, unsigned long long* pcount, double* pttd, InsertStats st) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  using Acc = typename TileSums<kStats>::Acc;
   TileSums<kStats>& S = *reinterpret_cast<TileSums<kStats>*>(lds_raw);
   const int jc = nsam / 2 + 1, h = nsam / 2, w = 2 * jc - 1;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // a tile's two halves are neighbouring workgroups (one workgroup with statistics)
+  // a tile's two halves are neighbouring workgroups (one workgroup for statistics)
   const int b = kStats ? blockIdx.x : blockIdx.x >> 1;
+  const int half = kStats ? 0 : blockIdx.x & 1;
+  // no term in the tile: the sums' launch has counted them
+  if (kStats && (pcount[2 * (size_t)b] | pcount[2 * (size_t)b + 1]) == 0) return;
   // tiles go out slab by slab in order of |logical n|, rows in order of
   // |logical m| (storage rows 0, last, 1, last - 1, ...): the tiles near the
   // origin, which every plane crosses, start first instead of last
@@ -391,8 +436,8 @@ __global__ void __launch_bounds__(kThreads)
   const unsigned long long lt = (1ull << lane) - 1ull;
   char* const set = reinterpret_cast<char*>(&S.sum[wave][slot * kVox]);
 
-  for (int half = kStats ? 0 : blockIdx.x & 1; half < (kStats ? 2 : (blockIdx.x & 1) + 1); half++) {
-    const int k0 = half ? *n0p : 0, k1 = half ? ntask : *n0p;
+  {
+    const int k0 = half ? *n0p : 0, k1 = half || kStats ? ntask : *n0p;
     unsigned cnt = 0u;
     unsigned long long cnt64 = 0ull;
     double ttd = 0.0;
@@ -400,7 +445,7 @@ __global__ void __launch_bounds__(kThreads)
       const int ml = mlo[box % nmr], mh = mhi[box % nmr];
       const int nl = nlo[box / nmr], nh = nhi[box / nmr];
       // where the box starts in the tile's sums, in bytes
-      constexpr int kB = sizeof(Sum), kM = kTile * kB, kN = kTile * kM;
+      constexpr int kB = sizeof(Acc), kM = kTile * kB, kN = kTile * kM;
       const int ms = ((ml < 0 ? nsam : 0) - m0 + ml) * kM, ns = ((nl < 0 ? nsam : 0) - n0 + nl) * kN;
       const float cx = 0.5f * (float)(l0 + l1), hx = 0.5f * (float)(l1 - l0) + 1.02f;
       const float cy = 0.5f * (float)(ml + mh), hy = 0.5f * (float)(mh - ml) + 1.02f;
@@ -431,15 +476,22 @@ __global__ void __launch_bounds__(kThreads)
         const bool split = nlist < kSplit;
         const int q0 = split ? 0 : nlist * wave / kWaves;
         const int q1 = split ? nlist : nlist * (wave + 1) / kWaves;
+        if constexpr (kStats)
+          if (nlist && !any) {  // read per term they were most of a pass: 600 cycles each of eight
+            for (int v = tid; v < kVox; v += kThreads) {
+              const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
+              if (l < jc && m < nsam && n < nsam)
+                S.ref[v] = ref_phase(reinterpret_cast<const float2*>(
+                    st.ref)[(size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n)]);
+            }
+            __syncthreads();
+          }
         any |= nlist != 0;
         if (!live && q0 < q1 && rl < 8) S.flag[wave][slot][rl] = 0u;
         for (int k = 0; k < min(q1 - q0, kSets); k++)
           if (!(live >> k & 1)) {
             live |= 1u << k;
-            for (int e = lane; e < kVox; e += 64) {
-              S.sum[wave][k * kVox + e] = Sum{0.f, 0.f, 0.f};
-              if constexpr (kStats) S.st[wave][k * kVox + e] = StatSum{0.f, 0.f, 0.f, 0};
-            }
+            for (int e = lane; e < kVox; e += 64) S.sum[wave][k * kVox + e] = Acc{};
           }
         wave_lds();
         for (int qb = q0; qb < q1; qb += kSets) {
@@ -528,30 +580,34 @@ __global__ void __launch_bounds__(kThreads)
                   }
                   const Axis X(x3), Y(y3), Z(z3);
                   const bool inside = on && pi * pi + pj * pj <= ir2;
+                  // a point's terms are its sample times real weights: one size and
+                  // one phase for the eight
+                  float pab = 0.f;
+                  unsigned pph = 0u;
+                  if constexpr (kStats) {
+                    pab = hypotf(pv.x, pv.y);
+                    pph = turns(pv.x, pv.y);
+                  }
                   // corner (kx, ky, kz) of every lane's point: pinsert_trilin.f:113-131,
                   // the weights' product in its order
                   auto corner = [&](int off, float bxy, float bz) {
                     const float box = bxy * bz;
                     if (off < kOut) {
-                      Sum& t = *reinterpret_cast<Sum*>(set + off);
-                      Sum u = t;
-                      u.re += pv.x * box;
-                      u.im += pv.y * box;
-                      u.c2 += pv.z * box;
-                      t = u;
+                      Acc& t = *reinterpret_cast<Acc*>(set + off);
+                      Acc u = t;
                       if constexpr (kStats) {
-                        const int v = off / (int)sizeof(Sum);
-                        const int vm = m0 + (v >> 3 & 7), vn = n0 + (v >> 6);
-                        const float2 ref = reinterpret_cast<const float2*>(
-                            st.ref)[(size_t)(l0 + (v & 7)) +
-                                    (size_t)jc * ((size_t)vm + (size_t)nsam * vn)];
-                        const float br = pv.x * box, bi = pv.y * box, ab = hypotf(br, bi);
-                        StatSum& q2 = S.st[wave][slot * kVox + v];
-                        q2.v += ab * ab;
-                        q2.a += ab;
-                        q2.p += pdiff_dev(br, bi, ref);
-                        q2.n++;
+                        const float ab = pab * fabsf(box);  // a weight may round to -1e-7
+                        u.v += ab * ab;
+                        u.a += ab;
+                        u.p += pdiff_dev(ab, pph + (__float_as_uint(box) & 1u << 31),
+                                         S.ref[off / kB]);
+                        u.n++;
+                      } else {
+                        u.re += pv.x * box;
+                        u.im += pv.y * box;
+                        u.c2 += pv.z * box;
                       }
+                      t = u;
                     }
                     wave_lds();  // another lane's next corner may be this voxel
                   };
@@ -614,35 +670,47 @@ __global__ void __launch_bounds__(kThreads)
       }
     }
     if (!any) {
-      if (tid == 0) {
+      if (!kStats && tid == 0) {
         pcount[2 * (size_t)b + half] = 0;
         pttd[2 * (size_t)b + half] = 0.0;
       }
-      continue;
+      return;
     }
-    // the waves' sums in wave order, into the half-map
+    // the waves' sums in wave order, into the half-map or the statistics: every
+    // set's value is read, those in use added, so that eight loads are in flight
+    // instead of one after the other
     if (lane == 0) S.live[wave] = live;
     __syncthreads();
-    float2* num = half ? num1 : num0;
-    float* ctf2 = half ? ctf2_1 : ctf2_0;
+    unsigned use[kWaves];
+#pragma unroll
+    for (int q = 0; q < kWaves; q++) use[q] = S.live[q];
     for (int v = tid; v < kVox; v += kThreads) {
       const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
-      float re = 0.f, im = 0.f, c2 = 0.f;
+      const size_t at = (size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n);
+      Acc t{};
+#pragma unroll
       for (int q = 0; q < kWaves; q++)
-        for (int e = v; e < kSets * kVox; e += kVox) {
-          if (!(S.live[q] >> (e / kVox) & 1)) continue;
-          re += S.sum[q][e].re;
-          im += S.sum[q][e].im;
-          c2 += S.sum[q][e].c2;
-          if (kStats) S.sum[q][e] = Sum{0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < kSets; k++) {
+          const Acc u = S.sum[q][k * kVox + v];
+          if (use[q] >> k & 1) t.add(u);
         }
-      if (l < jc && m < nsam && n < nsam && (re != 0.f || im != 0.f || c2 != 0.f)) {
-        const size_t at = (size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n);
+      if (l >= jc || m >= nsam || n >= nsam) continue;
+      if constexpr (kStats) {
+        if (!t.n) continue;
+        st.ksum[at] += t.n;
+        st.vsum[at] += t.v;
+        st.psum[at] += t.p;
+        st.asum[at] += t.a;
+      } else if (t.re != 0.f || t.im != 0.f || t.c2 != 0.f) {
+        float2* num = half ? num1 : num0;
+        float* ctf2 = half ? ctf2_1 : ctf2_0;
         const float2 o = num[at];
-        num[at] = make_float2(o.x + re, o.y + im);
-        ctf2[at] += c2;
+        num[at] = make_float2(o.x + t.re, o.y + t.im);
+        ctf2[at] += t.c2;
       }
     }
+    if (kStats) return;
     // the tile's NKSUM and TTD: a fixed reduction order
     for (int off = 32; off > 0; off >>= 1) {
       cnt64 += __shfl_xor(cnt64, off, 64);
@@ -662,29 +730,6 @@ __global__ void __launch_bounds__(kThreads)
       }
       pcount[2 * (size_t)b + half] = uc;
       pttd[2 * (size_t)b + half] = ut;
-    }
-  }
-  if constexpr (kStats) {
-    if (!any) return;
-    for (int v = tid; v < kVox; v += kThreads) {
-      const int l = l0 + (v & 7), m = m0 + (v >> 3 & 7), n = n0 + (v >> 6);
-      float s2 = 0.f, sa = 0.f, sp = 0.f;
-      int k = 0;
-      for (int q = 0; q < kWaves; q++)
-        for (int e = v; e < kSets * kVox; e += kVox) {
-          if (!(S.live[q] >> (e / kVox) & 1)) continue;
-          s2 += S.st[q][e].v;
-          sa += S.st[q][e].a;
-          sp += S.st[q][e].p;
-          k += S.st[q][e].n;
-        }
-      if (l < jc && m < nsam && n < nsam && k) {
-        const size_t at = (size_t)l + (size_t)jc * ((size_t)m + (size_t)nsam * n);
-        st.ksum[at] += k;
-        st.vsum[at] += s2;
-        st.psum[at] += sp;
-        st.asum[at] += sa;
-      }
     }
   }
 }
@@ -746,6 +791,8 @@ int launch_insert(Ctx& c, int nsam, int nb, int ntask, const InsertTask* d_tasks
   if (ntask <= 0 || nb <= 0) return 0;
   FR_CHECK(scratch != nullptr, "insertion scratch missing");
   FR_CHECK(nb <= 65535, "too many particles in one insertion (%d)", nb);
+  FR_CHECK(!stats || (stats->ref && stats->ksum && stats->vsum && stats->psum && stats->asum),
+           "insertion statistics arrays missing");
   const int jc = nsam / 2 + 1, w = 2 * jc - 1;
   int tx, ty, tz;
   tile_counts(nsam, &tx, &ty, &tz);
@@ -762,21 +809,19 @@ int launch_insert(Ctx& c, int nsam, int nb, int ntask, const InsertTask* d_tasks
   hipLaunchKernelGGL(k_insert_geo, dim3((ntask + kThreads - 1) / kThreads), dim3(kThreads), 0,
                      c.stream, ntask, nb, nsam, d_tasks, s.ord, s.hit, s.rec);
   FR_HIP(hipGetLastError());
+  const size_t lds = sizeof(TileSums<false>);
+  hipLaunchKernelGGL(k_insert_scatter<false>, dim3(2 * ntiles), dim3(kThreads), lds, c.stream,
+                     nsam, ntask, tx, ty, tz, s.n0, s.hit, s.rec, s.pts,
+                     reinterpret_cast<float2*>(num0), ctf2_0, reinterpret_cast<float2*>(num1),
+                     ctf2_1, s.pcount, s.pttd, InsertStats{});
   if (stats) {
-    FR_CHECK(stats->ref && stats->ksum && stats->vsum && stats->psum && stats->asum,
-             "insertion statistics arrays missing");
-    const size_t lds = sizeof(TileSums<true>);
+    FR_HIP(hipGetLastError());
+    const size_t lds_st = sizeof(TileSums<true>);
     FR_HIP(hipFuncSetAttribute((const void*)k_insert_scatter<true>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_insert_scatter<true>, dim3(ntiles), dim3(kThreads), lds, c.stream, nsam,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_st));
+    hipLaunchKernelGGL(k_insert_scatter<true>, dim3(ntiles), dim3(kThreads), lds_st, c.stream, nsam,
                        ntask, tx, ty, tz, s.n0, s.hit, s.rec, s.pts, reinterpret_cast<float2*>(num0),
                        ctf2_0, reinterpret_cast<float2*>(num1), ctf2_1, s.pcount, s.pttd, *stats);
-  } else {
-    const size_t lds = sizeof(TileSums<false>);
-    hipLaunchKernelGGL(k_insert_scatter<false>, dim3(2 * ntiles), dim3(kThreads), lds, c.stream,
-                       nsam, ntask, tx, ty, tz, s.n0, s.hit, s.rec, s.pts,
-                       reinterpret_cast<float2*>(num0), ctf2_0, reinterpret_cast<float2*>(num1),
-                       ctf2_1, s.pcount, s.pttd, InsertStats{});
   }
   FR_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_insert_reduce, dim3(1), dim3(kReduceThreads), 0, c.stream, ntiles,

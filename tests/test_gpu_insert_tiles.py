@@ -76,3 +76,47 @@ def test_insert_tiles_vs_oracle(nsam, nb, asym, nasym, amag, rrec, aligned):
         for g, w in zip(got, (num, c2)):
             assert np.linalg.norm(g - w) <= 1.6e-5 * np.linalg.norm(w)
         assert abs(outs[0][5][h] - ttd.value) <= 1e-6 * abs(ttd.value)
+
+
+@pytest.mark.parametrize("nsam", [16, 36])
+def test_statistics_phases(nsam):
+    """PSUM of one particle on the volume's own grid, a term a voxel: the phase
+    difference to the reference on the octants' edges, across the half turn and in
+    between, zero where the reference is.  Bar: two arctangents and the result rounded
+    to 2^-24 of pi: 4e-7."""
+    rng = np.random.default_rng(nsam)
+    jc = nsam // 2 + 1
+
+    def phases(*shape):
+        a = rng.integers(-8, 9, shape) * np.pi / 8 + rng.choice([0, 0, 1e-6, -1e-6], shape)
+        a = np.where(rng.uniform(size=shape) < 0.3, rng.uniform(-np.pi, np.pi, shape), a)
+        return (10 ** rng.uniform(-3, 3, shape) * np.exp(1j * a)).astype(np.complex64)
+
+    datc, ref = phases(1, nsam, jc), phases(nsam, nsam, jc)
+    axis = np.array([1, -1, 1j, -1j], np.complex64)  # exact axes, with signed zeros
+    datc[0, ::3, ::2] = axis[rng.integers(0, 4, datc[0, ::3, ::2].shape)]
+    ref[0, ::2, ::3] = -axis[rng.integers(0, 4, ref[0, ::2, ::3].shape)]
+    ref[0, 1, ::2] = 0
+    ctff = np.zeros((1, 2, nsam, jc), np.complex64)
+    ctff[:, 0] = 1
+    recb = np.zeros((1, 10), np.float32)
+    recb[0, 5:10] = 1, 1, 1, 0.5, 0.45
+    ctx = api.Context(0)
+    vols = api.HalfMaps.zeros(nsam)
+    stats = api.VoxelStats.zeros(nsam, torch.from_numpy(ref).to(DEV))
+    ctx.insert(nsam, torch.from_numpy(datc).to(DEV), torch.from_numpy(ctff).to(DEV), recb,
+               np.zeros(1, np.int32), api.point_group("C", 1), 5.0, 40.0, 1.5, vols, stats=stats)
+    ctx.close()
+    j = np.arange(nsam)
+    j = np.where(j >= jc, j - nsam, j)
+    r2 = j[:, None] ** 2 + np.arange(jc)[None] ** 2
+    on = (r2 <= int(nsam * np.float32(0.45)) ** 2) & (r2 > 0)
+    d, r = datc[0].astype(np.complex128), ref[0].astype(np.complex128)
+    want = np.where(r == 0, 0.0, np.abs(np.angle(d * np.conj(r))))
+    got, cnt = stats.psum.cpu().numpy(), stats.ksum.cpu().numpy()
+    assert (cnt[0][on] >= 1).all() and on.sum() > 40
+    assert np.abs(got[0] - want)[on].max() <= 4e-7
+    size = stats.asum.cpu().numpy()[0]
+    term = np.abs(vols.num[0].cpu().numpy()[0].astype(np.complex128))
+    assert (np.abs(size - term)[on] <= 1e-6 * term[on]).all()
+    assert np.abs(got[2:]).max() == 0
