@@ -244,17 +244,23 @@ int fr_ctx::cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t) {
 }
 
 int fr_ctx::cc3m_ring(int nsam, int maxr2, float ri2, float ri3, fr::Cc3mRing* t) {
+  FR_CHECK(nsam <= fr::kCc3mMaxBox, "box too large for the shells of CC3M and PRESB (%d)", nsam);
   const auto k = std::make_tuple(nsam, maxr2, ri2, ri3);
   auto i = ring_hats.find(k);
   if (i == ring_hats.end()) {
-    std::vector<float> h;
-    RingTab rt;
-    rt.cnt = fr::cc3m_ring_hat(nsam, ri2, ri3, maxr2, h);
-    if (int r = upload_table(h, &rt.d)) return r;
+    RingHat rt{nullptr, {}};
+    rt.ring.cnt = fr::cc3m_ring_count(nsam, ri2, ri3);
+    FR_HIP(hipMalloc(&rt.buf, fr::cc3m_ring_bytes(nsam, maxr2)));
+    int r = fr::launch_ring_hat(*this, nsam, ri2, ri3, maxr2, rt.buf, &rt.ring.rhat);
+    // other streams may be next to read it
+    if (!r && hipStreamSynchronize(stream) != hipSuccess) r = fr::fail("ring table failed");
+    if (r) {
+      (void)hipFree(rt.buf);
+      return r;
+    }
     i = ring_hats.emplace(k, rt).first;
   }
-  t->rhat = i->second.d;
-  t->cnt = i->second.cnt;
+  *t = i->second.ring;
   return 0;
 }
 
@@ -331,7 +337,7 @@ int fr_destroy(fr_ctx* c) {
   if (c->hrange) (void)hipHostFree(c->hrange);
   if (c->d_kidx) (void)hipFree(c->d_kidx);
   for (auto& e : c->dft_tabs) (void)hipFree(e.second);
-  for (auto& e : c->ring_hats) (void)hipFree(e.second.d);
+  for (auto& e : c->ring_hats) (void)hipFree(e.second.buf);
   for (auto& e : c->band_dft_tabs) (void)hipFree(e.second);
   for (auto& e : c->band_pair_tabs) (void)hipFree(e.second);
   for (auto& e : c->band_wmap_tabs) (void)hipFree(e.second);

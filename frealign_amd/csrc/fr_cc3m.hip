@@ -39,6 +39,7 @@
 // 393 folded once).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -807,42 +808,54 @@ void cc3m_band_wmap(int nsam, int M, const std::vector<float>& full, std::vector
     w = full;
     return;
   }
+  // Every step runs along rows, so that the compiler vectorises it, and over a
+  // quarter of the result: on a 256 box 1.1 ms, 11.0 as sums
+  // per element.
   const int h = nsam / 2, Q = M / 2;  // frequencies 0 .. Q - 1
-  std::vector<double> cosn(nsam), cosm(M);
-  for (int k = 0; k < nsam; k++) cosn[k] = std::cos(2.0 * M_PI * k / nsam);
-  for (int k = 0; k < M; k++) cosm[k] = std::cos(2.0 * M_PI * k / M);
+  auto table = [&](int rows, int cols, int n) {  // [r][c] = cos(2 pi r c/n)
+    std::vector<double> co(n), t((size_t)rows * cols);
+    for (int k = 0; k < n; k++) co[k] = std::cos(2.0 * M_PI * k / n);
+    for (int r = 0; r < rows; r++)
+      for (int c = 0, at = 0; c < cols; c++) {
+        t[(size_t)r * cols + c] = co[at];
+        at = (at + r) % n;
+      }
+    return t;
+  };
+  // y += v x
+  auto add = [](int n, double v, const double* x, double* y) {
+    for (int k = 0; k < n; k++) y[k] += v * x[k];
+  };
   auto mult = [&](int n) { return n == 0 || n == h ? 1.0 : 2.0; };
-  // a[q][m] = sum_n w[m][n] cos(2 pi q n/N), m = 0 .. N/2
-  std::vector<double> a((size_t)Q * (h + 1), 0.0), f((size_t)Q * Q, 0.0);
-  for (int q = 0; q < Q; q++)
-    for (int m = 0; m <= h; m++) {
-      double s = 0.0;
-      for (int n = 0; n <= h; n++)
-        s += mult(n) * (double)full[(size_t)m * nsam + n] * cosn[(long long)q * n % nsam];
-      a[(size_t)q * (h + 1) + m] = s;
-    }
-  for (int q = 0; q < Q; q++)
-    for (int p = 0; p < Q; p++) {
-      double s = 0.0;
-      for (int m = 0; m <= h; m++)
-        s += mult(m) * a[(size_t)q * (h + 1) + m] * cosn[(long long)p * m % nsam];
-      f[(size_t)p * Q + q] = s / ((double)nsam * nsam) * (p ? 2.0 : 1.0) * (q ? 2.0 : 1.0);
-    }
-  // b[p][n] = sum_q f[p][q] cos(2 pi q n/M), then the rows
-  std::vector<double> b((size_t)Q * M, 0.0);
+  const std::vector<double> cn = table(h + 1, Q, nsam), cm = table(Q, Q + 1, M);
+  // a[m][q] = sum_n w[m][n] cos(2 pi q n/N), then f[p][q] over m
+  std::vector<double> a((size_t)(h + 1) * Q, 0.0), f((size_t)Q * Q, 0.0);
+  for (int m = 0; m <= h; m++) {
+    double* am = &a[(size_t)m * Q];
+    for (int n = 0; n <= h; n++)
+      if (const float v = full[(size_t)m * nsam + n])
+        add(Q, mult(n) * (double)v, &cn[(size_t)n * Q], am);
+    for (int p = 0; p < Q; p++) add(Q, mult(m) * cn[(size_t)m * Q + p], am, &f[(size_t)p * Q]);
+  }
   for (int p = 0; p < Q; p++)
-    for (int n = 0; n < M; n++) {
-      double s = 0.0;
-      for (int q = 0; q < Q; q++) s += f[(size_t)p * Q + q] * cosm[q * n % M];
-      b[(size_t)p * M + n] = s;
-    }
+    for (int q = 0; q < Q; q++)
+      f[(size_t)p * Q + q] *= (p ? 2.0 : 1.0) * (q ? 2.0 : 1.0) / ((double)nsam * nsam);
+  // b[p][n] = sum_q f[p][q] cos(2 pi q n/M), n <= M/2, then the rows
+  std::vector<double> b((size_t)Q * (Q + 1), 0.0), row(Q + 1);
+  for (int p = 0; p < Q; p++)
+    for (int q = 0; q < Q; q++)
+      add(Q + 1, f[(size_t)p * Q + q], &cm[(size_t)q * (Q + 1)], &b[(size_t)p * (Q + 1)]);
   w.assign((size_t)M * M, 0.f);
-  for (int m = 0; m < M; m++)
-    for (int n = 0; n < M; n++) {
-      double s = 0.0;
-      for (int p = 0; p < Q; p++) s += b[(size_t)p * M + n] * cosm[p * m % M];
-      w[(size_t)m * M + n] = (float)s;
+  for (int m = 0; m <= Q; m++) {
+    std::fill(row.begin(), row.end(), 0.0);
+    for (int p = 0; p < Q; p++)
+      add(Q + 1, cm[(size_t)p * (Q + 1) + m], &b[(size_t)p * (Q + 1)], row.data());
+    for (int n = 0; n <= Q; n++) {
+      const float v = (float)row[n];
+      for (int y : {m, (M - m) % M})
+        for (int x : {n, (M - n) % M}) w[(size_t)y * M + x] = v;
     }
+  }
 }
 
 int cc3m_band_npair(int maxr12, int maxr22, int rb) {

@@ -464,6 +464,36 @@ __global__ void __launch_bounds__(64)
   }
 }
 
+// The ring's sums on the device: on the host they were 2 ms of the first PRESB of a
+// 256 box
+__device__ inline double ring_mult(int v, int n) { return v == 0 || 2 * v == n ? 1.0 : 2.0; }
+
+__global__ void __launch_bounds__(kThr)
+    k_ring_rows(int n, int cb, float ri2, float ri3, double* __restrict__ row) {
+  const int y = blockIdx.x;
+  for (int i = threadIdx.x; i < cb; i += kThr) {
+    double s = 0.0;
+    for (int x = 0; 2 * x <= n; x++) {
+      const float r2 = (float)(x * x + y * y);
+      if (r2 > ri2 && r2 <= ri3) s += ring_mult(x, n) * cospi(2.0 * (i * x % n) / n);
+    }
+    row[(size_t)y * cb + i] = ring_mult(y, n) * s;
+  }
+}
+
+__global__ void __launch_bounds__(kThr)
+    k_ring_hat(int n, int cb, const double* __restrict__ row, float* __restrict__ out) {
+  __shared__ double co[kCc3mMaxBox / 2 + 1];
+  const int j = blockIdx.x;
+  for (int y = threadIdx.x; 2 * y <= n; y += kThr) co[y] = cospi(2.0 * (j * y % n) / n);
+  __syncthreads();
+  for (int i = threadIdx.x; i < cb; i += kThr) {
+    double s = 0.0;
+    for (int y = 0; 2 * y <= n; y++) s += co[y] * row[(size_t)y * cb + i];
+    out[(size_t)j * cb + i] = (float)s;
+  }
+}
+
 int band_cb(int maxr2) { return (maxr2 + kCw - 1) / kCw * kCw; }
 int band_nsh(int maxr2) { return maxr2 + 1; }
 
@@ -552,45 +582,44 @@ size_t cc3m_fft_bytes(int nsam, int maxr2, size_t n) {
   return bytes;
 }
 
-// Rhat[J][I] = sum over the pixels (x, y) of the MASKCOS2 ring at AMAG = 1 (as the
-// kernels test them) of cos(2 pi I x/N) cos(2 pi J y/N), J < MAXR2, I < CB; in
-// double.  Returns the ring's pixel count.
-int cc3m_ring_hat(int nsam, float ri2, float ri3, int maxr2, std::vector<float>& out) {
-  const int h = nsam / 2, cb = band_cb(maxr2);
-  std::vector<double> co(nsam), row((size_t)(h + 1) * cb, 0.0);
-  for (int k = 0; k < nsam; k++) co[k] = std::cos(2.0 * M_PI * k / nsam);
+// Pixels of the MASKCOS2 ring at AMAG = 1, as the kernels test them.
+int cc3m_ring_count(int nsam, float ri2, float ri3) {
+  const int h = nsam / 2;
   auto mult = [&](int v) { return v == 0 || v == h ? 1 : 2; };
-  long long cnt = 0;
+  int cnt = 0;
   for (int y = 0; y <= h; y++)
     for (int x = 0; x <= h; x++) {
       const float r2 = (float)(x * x + y * y);
-      if (!(r2 > ri2 && r2 <= ri3)) continue;
-      cnt += (long long)mult(x) * mult(y);
-      for (int i = 0, at = 0; i < cb; i++) {
-        row[(size_t)y * cb + i] += mult(x) * co[at];
-        at += x;
-        if (at >= nsam) at -= nsam;
-      }
+      if (r2 > ri2 && r2 <= ri3) cnt += mult(x) * mult(y);
     }
-  out.assign((size_t)maxr2 * cb, 0.f);
-  std::vector<double> sum(cb);
-  for (int j = 0; j < maxr2; j++) {
-    std::fill(sum.begin(), sum.end(), 0.0);
-    for (int y = 0; y <= h; y++) {
-      const double c = mult(y) * co[(long long)j * y % nsam];
-      const double* r = &row[(size_t)y * cb];
-      for (int i = 0; i < cb; i++) sum[i] += c * r[i];
-    }
-    for (int i = 0; i < cb; i++) out[(size_t)j * cb + i] = (float)sum[i];
-  }
-  return (int)cnt;
+  return cnt;
+}
+
+size_t cc3m_ring_bytes(int nsam, int maxr2) {
+  return band_cb(maxr2) * (sizeof(double) * (nsam / 2 + 1) + sizeof(float) * (size_t)maxr2);
+}
+
+// Rhat[J][I] = sum over the ring's pixels (x, y) of cos(2 pi I x/N) cos(2 pi J y/N),
+// J < MAXR2, I < CB, in 64 bits; in front of it, for the launch alone, the rows' sums
+// over x.
+int launch_ring_hat(Ctx& c, int nsam, float ri2, float ri3, int maxr2, void* buf,
+                    const float** rhat) {
+  const int h = nsam / 2, cb = band_cb(maxr2);
+  double* row = static_cast<double*>(buf);
+  float* out = reinterpret_cast<float*>(row + (size_t)(h + 1) * cb);
+  hipLaunchKernelGGL(k_ring_rows, dim3(h + 1), dim3(kThr), 0, c.stream, nsam, cb, ri2, ri3, row);
+  FR_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_ring_hat, dim3(maxr2), dim3(kThr), 0, c.stream, nsam, cb, row, out);
+  FR_HIP(hipGetLastError());
+  *rhat = out;
+  return 0;
 }
 
 int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
                 const int* pidx, const float* dm, const float* shift, const float* amag,
                 const float* fsct, const Cc3mRing& ring, void* work, float* score) {
   if (a.n <= 0) return 0;
-  FR_CHECK(a.nsam / 2 + 2 <= 260, "box too large for CC3M bins");
+  FR_CHECK(a.nsam <= kCc3mMaxBox, "box too large for CC3M bins");
   FR_CHECK(a.maxr2 < a.nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", a.maxr2);
   FR_CHECK(ring.rhat && work, "CC3M tables missing");
   const Band b = make_band(a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2, a.ri2, a.ri3, a.rih, a.halfw,
@@ -611,7 +640,7 @@ int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, 
                  float ri2, float ri3, float rih, float halfw, const Cc3mRing& ring, void* work,
                  float* rbin) {
   if (n <= 0) return 0;
-  FR_CHECK(nsam / 2 + 2 <= 260, "box too large for PRESB bins");
+  FR_CHECK(nsam <= kCc3mMaxBox, "box too large for PRESB bins");
   FR_CHECK(ring.rhat && work, "PRESB tables missing");
   const Band b = make_band(nsam, n, 1, nsam / 2, ri2, ri3, rih, halfw, 0);
   size_t bytes;

@@ -45,7 +45,11 @@ struct fr_ctx : public fr::Ctx {
   std::map<std::pair<int, int>, int*> band_pair_tabs;          // per (MAXR1^2, MAXR2^2)
   // per (NSAM, M, RI2, RI3, RIH, HALFW)
   std::map<std::tuple<int, int, float, float, float, float>, float*> band_wmap_tabs;
-  std::map<std::tuple<int, int, float, float>, RingTab> ring_hats;  // per (NSAM, MAXR2, RI2, RI3)
+  struct RingHat {
+    void* buf;
+    fr::Cc3mRing ring;
+  };
+  std::map<std::tuple<int, int, float, float>, RingHat> ring_hats;  // per (NSAM, MAXR2, RI2, RI3)
   int cc3m_ring(int nsam, int maxr2, float ri2, float ri3, fr::Cc3mRing* t);
   int cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t);
   // launch choices per box size (set by fr_autotune_cc3m)

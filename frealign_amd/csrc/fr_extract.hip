@@ -886,13 +886,15 @@ int cc3m_fused_ring_q(int nsam, float ri2, float ri3, std::vector<float>& q) {
       t[(size_t)m * kFK + 2 * i] = std::cos(ph);
       t[(size_t)m * kFK + 2 * i + 1] = -std::sin(ph);
     }
-  q.assign((size_t)kFK * kFK, 0.f);
-  for (int c = 0; c < kFK; c++)
-    for (int k = 0; k < kFK; k++) {
-      double acc = 0.0;
-      for (int m = 0; m < nsam; m++) acc += t[(size_t)m * kFK + k] * (double)ring[(size_t)m * kFK + c];
-      q[(size_t)c * kFK + k] = (float)((c < 2 ? 1.0 : 2.0) * acc);
+  std::vector<double> sum((size_t)kFK * kFK, 0.0);
+  for (int m = 0; m < nsam; m++)
+    for (int c = 0; c < kFK; c++) {
+      const double r = ring[(size_t)m * kFK + c];
+      const double* tm = &t[(size_t)m * kFK];
+      for (int k = 0; k < kFK; k++) sum[(size_t)c * kFK + k] += tm[k] * r;
     }
+  q.resize((size_t)kFK * kFK);
+  for (int e = 0; e < kFK * kFK; e++) q[e] = (float)((e < 2 * kFK ? 1.0 : 2.0) * sum[e]);
   return cnt;
 }
 

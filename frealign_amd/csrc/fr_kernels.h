@@ -101,14 +101,18 @@ struct Cc3mArgs {
 };
 
 constexpr int kMaskThreads = 1024;
+constexpr int kCc3mMaxBox = 516;  // the largest box of CC3M and PRESB
 // On the particle's grid, any box, band and AMAG (fr_cc3m_fft.hip); work:
 // cc3m_fft_bytes for the items of the call (PRESB: MAXR2 = NSAM/2).
 struct Cc3mRing {
-  const float* rhat = nullptr;  // cc3m_ring_hat on the device
+  const float* rhat = nullptr;  // launch_ring_hat
   int cnt = 0;                  // the ring's pixels
 };
 size_t cc3m_fft_bytes(int nsam, int maxr2, size_t n);
-int cc3m_ring_hat(int nsam, float ri2, float ri3, int maxr2, std::vector<float>& out);
+int cc3m_ring_count(int nsam, float ri2, float ri3);
+size_t cc3m_ring_bytes(int nsam, int maxr2);
+int launch_ring_hat(Ctx& c, int nsam, float ri2, float ri3, int maxr2, void* buf,
+                    const float** rhat);
 int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
                 const int* pidx, const float* dm, const float* shift, const float* amag,
                 const float* fsct, const Cc3mRing& ring, void* work, float* score);
