@@ -637,13 +637,15 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
 //   T3 = sum Im S sin aI cos bJ,   T4 = sum Re D sin aI sin bJ,
 // and -a or -b only change signs: four products over a quarter of the window.
 // Per shell each is a matrix product of 16 items by the shell's pairs with the
-// pairs by the quarter's shifts, on the FP32 matrix cores.  One wave takes 16
-// items; the phase factors are formed from two small tables, and a shell's
-// terms join FP64 sums per shift, as in the score.
+// pairs by the quarter's shifts, on the FP32 matrix cores; the phase factors are
+// formed from two small tables.  A workgroup takes 16 items at a time, its eight
+// waves the shells in zig-zag; a shell's terms join the wave's FP64 sums per shift,
+// and these add up in LDS in wave order: the same sums whatever the launch holds.
 // On the vector units, one item a workgroup and one shift a lane, the sums were
 // most of the window's time: 52,728 items of a 128 box x 81 shifts took 10.6 ms,
-// and take 2.6 ms.
-constexpr int kWinWaves = 4, kWinItems = 16 * kWinWaves;
+// and take 2.05 ms.  With all of an item's shells in one wave and four such waves of
+// 16 items a workgroup, this kernel took 107 us for 27 items and 111 for 500; 30 and 31 now.
+constexpr int kWinWaves = 8, kWinItems = 16;
 constexpr int kWinHalf = kCc3mWinMax / 2 + 1;  // offsets 0 .. 5 per axis
 
 template <int NT>
@@ -652,9 +654,12 @@ __global__ void __launch_bounds__(64 * kWinWaves)
                   const float* __restrict__ fsct, const float* __restrict__ amag_arr, int flip,
                   Cc3mWindow win, Cc3mWinBuf wb, float* __restrict__ score,
                   int* __restrict__ code) {
+  constexpr int kN = 16 * NT + 4;  // pitch: conflict-free
   __shared__ float2 tx[32][kWinHalf], ty[32][kWinHalf];  // (cos, sin) of a dsx I, b dsy J
   __shared__ unsigned short ij[32 * 32];                 // the pairs in shell order
+  __shared__ double sums[4][kWinItems][kN];              // [signs][item][quarter shift]
   const int tid = threadIdx.x, lane = tid & 63, la = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int e = tid; e < 32 * kWinHalf; e += 64 * kWinWaves) {
     const int i = e / kWinHalf, a = e % kWinHalf;
     float sn, cs;
@@ -668,8 +673,6 @@ __global__ void __launch_bounds__(64 * kWinWaves)
     if (p >= 0) ij[p] = (unsigned short)((e / rb) | ((e % rb) << 8));
   }
   __syncthreads();
-  const int base = (blockIdx.x * kWinWaves + (tid >> 6)) * 16;
-  if (base >= nitem) return;
   const int hx = win.nsx / 2, hy = win.nsy / 2, nq = (hx + 1) * (hy + 1);
   int qa[NT], qb[NT];
 #pragma unroll
@@ -678,85 +681,102 @@ __global__ void __launch_bounds__(64 * kWinWaves)
     qa[t] = n / (hy + 1);
     qb[t] = n % (hy + 1);
   }
-  const float4* row = wb.cross + (size_t)min(base + la, nitem - 1) * wb.npair;
-  double acc[NT][4][4];
-#pragma unroll
-  for (int t = 0; t < NT; t++)
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int k = 0; k < 4; k++) acc[t][i][k] = 0.0;
-  for (int sh = 1; sh < top && sh <= rb; sh++) {
-    const int b0 = pairs[sh], b1 = pairs[sh + 1];
-    if (b0 == b1) continue;
-    fx4 T[NT][4];
+  for (int base = blockIdx.x * kWinItems; base < nitem; base += gridDim.x * kWinItems) {
+    const float4* row = wb.cross + (size_t)min(base + la, nitem - 1) * wb.npair;
+    double acc[NT][4][4];
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) T[t][k] = fx4{0.f, 0.f, 0.f, 0.f};
-    for (int e0 = b0; e0 < b1; e0 += 4) {
-      const int e = e0 + lg;
-      float4 v = row[min(e, b1 - 1)];
-      if (e >= b1) v = make_float4(0.f, 0.f, 0.f, 0.f);
-      const int pk = ij[min(e, b1 - 1)], i = pk & 0xff, j = pk >> 8;
+      for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int t = 0; t < NT; t++) {
-        const float2 x = tx[i][qa[t]], y = ty[j][qb[t]];
-        T[t][0] = mfma4(v.x, x.x * y.x, T[t][0]);
-        T[t][1] = mfma4(v.w, x.x * y.y, T[t][1]);
-        T[t][2] = mfma4(v.y, x.y * y.x, T[t][2]);
-        T[t][3] = mfma4(v.z, x.y * y.y, T[t][3]);
+        for (int k = 0; k < 4; k++) acc[t][i][k] = 0.0;
+    for (int sh = 1; sh < top && sh <= rb; sh++) {
+      const int z = sh & (2 * kWinWaves - 1);
+      if ((z < kWinWaves ? z : 2 * kWinWaves - 1 - z) != wave) continue;
+      const int b0 = pairs[sh], b1 = pairs[sh + 1];
+      if (b0 == b1) continue;
+      fx4 T[NT][4];
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) T[t][k] = fx4{0.f, 0.f, 0.f, 0.f};
+      for (int e0 = b0; e0 < b1; e0 += 4) {
+        const int e = e0 + lg;
+        float4 v = row[min(e, b1 - 1)];
+        if (e >= b1) v = make_float4(0.f, 0.f, 0.f, 0.f);
+        const int pk = ij[min(e, b1 - 1)], i = pk & 0xff, j = pk >> 8;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          const float2 x = tx[i][qa[t]], y = ty[j][qb[t]];
+          T[t][0] = mfma4(v.x, x.x * y.x, T[t][0]);
+          T[t][1] = mfma4(v.w, x.x * y.y, T[t][1]);
+          T[t][2] = mfma4(v.y, x.y * y.x, T[t][2]);
+          T[t][3] = mfma4(v.z, x.y * y.y, T[t][3]);
+        }
       }
-    }
-    const float wgt = expf(-rbfact * (float)(sh * sh));
-    const bool absr = !flip && fsct[sh] < 0.95f;
+      const float wgt = expf(-rbfact * (float)(sh * sh));
+      const bool absr = !flip && fsct[sh] < 0.95f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int it = min(base + 4 * lg + i, nitem - 1);
-      const float ra = sqrtf(wb.a2[(size_t)it * kCc3mWinShells + sh - 1]);
+      for (int i = 0; i < 4; i++) {
+        const int it = min(base + 4 * lg + i, nitem - 1);
+        const float ra = sqrtf(wb.a2[(size_t)it * kCc3mWinShells + sh - 1]);
 #pragma unroll
-      for (int t = 0; t < NT; t++) {
-        const float u = T[t][0][i], w = T[t][1][i], x = T[t][2][i], y = T[t][3][i];
-        float r[4] = {(u - w) - (x + y), (u + w) - (x - y), (u - w) + (x + y), (u + w) + (x - y)};
+        for (int t = 0; t < NT; t++) {
+          const float u = T[t][0][i], w = T[t][1][i], x = T[t][2][i], y = T[t][3][i];
+          float r[4] = {(u - w) - (x + y), (u + w) - (x - y), (u - w) + (x + y),
+                        (u + w) + (x - y)};
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-          r[k] = r[k] / ra;
-          if (absr) r[k] = fabsf(r[k]);
-          acc[t][i][k] += (double)(r[k] * wgt);
+          for (int k = 0; k < 4; k++) {
+            r[k] = r[k] / ra;
+            if (absr) r[k] = fabsf(r[k]);
+            acc[t][i][k] += (double)(r[k] * wgt);
+          }
         }
       }
     }
-  }
-  // the first maximum of each item in window order (IX outer, IY inner)
+    for (int w = 0; w < kWinWaves; w++) {
+      if (wave == w)
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int it = base + 4 * lg + i;
-    const double norm = wb.norm[min(it, nitem - 1)];
-    float bv = -3.0e38f;
-    int bs = 0x7fffffff;
+        for (int t = 0; t < NT; t++)
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+          for (int i = 0; i < 4; i++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const float v = (float)(acc[t][i][k] / norm);
-        const int s = (hx + (k & 2 ? -qa[t] : qa[t])) * win.nsy + hy + (k & 1 ? -qb[t] : qb[t]);
+            for (int k = 0; k < 4; k++) {
+              double& s = sums[k][4 * lg + i][16 * t + la];
+              s = w ? s + acc[t][i][k] : acc[t][i][k];
+            }
+      __syncthreads();
+    }
+    // the first maximum of each item in window order (IX outer, IY inner)
+    for (int m = wave; m < kWinItems; m += kWinWaves) {
+      const int it = base + m;
+      if (it >= nitem) break;
+      const double norm = wb.norm[it];
+      float bv = -3.0e38f;
+      int bs = 0x7fffffff;
+      for (int e = lane; e < 4 * nq; e += 64) {
+        const int n = e >> 2, k = e & 3, a = n / (hy + 1), b = n % (hy + 1);
+        const float v = (float)(sums[k][m][n] / norm);
+        const int s = (hx + (k & 2 ? -a : a)) * win.nsy + hy + (k & 1 ? -b : b);
         if (v > bv || (v == bv && s < bs)) {
           bv = v;
           bs = s;
         }
       }
-    for (int off = 8; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(bv, off, 64);
-      const int os = __shfl_xor(bs, off, 64);
-      if (ov > bv || (ov == bv && os < bs)) {
-        bv = ov;
-        bs = os;
+      for (int off = 32; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(bv, off, 64);
+        const int os = __shfl_xor(bs, off, 64);
+        if (ov > bv || (ov == bv && os < bs)) {
+          bv = ov;
+          bs = os;
+        }
+      }
+      if (lane == 0 && amag_arr[it] == 1.0f) {
+        score[it] = bv;
+        code[it] = bs < win.nsx * win.nsy ? bs : 0;
       }
     }
-    if (la == 0 && it < nitem && amag_arr[it] == 1.0f) {
-      score[it] = bv;
-      code[it] = bs < win.nsx * win.nsy ? bs : 0;
-    }
+    __syncthreads();  // the sums are written again
   }
 }
 
@@ -921,8 +941,11 @@ int launch_window(Ctx& c, const Cc3mArgs& a, const float* fsct, const float* ama
                   const Cc3mBandTables& t, const Cc3mWindow& win, const Cc3mWinBuf& wb,
                   float* score, int* code) {
   const int top = a.nsam / 2 < kCc3mShells ? a.nsam / 2 : kCc3mShells;
-  hipLaunchKernelGGL(k_cc3m_window<NT>, dim3((unsigned)((a.n + kWinItems - 1) / kWinItems)),
-                     dim3(64 * kWinWaves), 0, c.stream, a.n, cc3m_band_rb(a.maxr2), top, a.rbfact,
+  int grid = 0;
+  if (int r = cc3m_grid(c, (const void*)k_cc3m_window<NT>, 64 * kWinWaves, 0,
+                        (a.n + kWinItems - 1) / kWinItems, -1, &grid))
+    return r;
+  hipLaunchKernelGGL(k_cc3m_window<NT>, dim3((unsigned)grid), dim3(64 * kWinWaves), 0, c.stream, a.n, cc3m_band_rb(a.maxr2), top, a.rbfact,
                      t.pairs, fsct, amag, a.cc3, win, wb, score, code);
   FR_HIP(hipGetLastError());
   return 0;
