@@ -173,27 +173,6 @@ int fr_ctx::cc3m_tables(const fr::Cc3mArgs& a, fr::Cc3mTables* t) {
     pi = pts_tabs.emplace(pk, d).first;
   }
   t->pts = pi->second;
-  const auto rk = std::make_tuple(a.nsam, a.ri2, a.ri3);
-  auto ri = ring_tabs.find(rk);
-  if (ri == ring_tabs.end()) {
-    std::vector<float> ring;
-    RingTab rt;
-    rt.cnt = fr::cc3m_fused_ring_q(a.nsam, a.ri2, a.ri3, ring);
-    if (int r = upload_table(ring, &rt.d)) return r;
-    ri = ring_tabs.emplace(rk, rt).first;
-  }
-  t->ring = ri->second.d;
-  t->ring_cnt = ri->second.cnt;
-  const auto wk = std::make_tuple(a.nsam, a.ri2, a.ri3, a.rih, a.halfw);
-  auto wi = wmap_tabs.find(wk);
-  if (wi == wmap_tabs.end()) {
-    std::vector<float> w;
-    fr::cc3m_fused_wmap(a.nsam, a.ri2, a.ri3, a.rih, a.halfw, w);
-    float* d = nullptr;
-    if (int r = upload_table(w, &d)) return r;
-    wi = wmap_tabs.emplace(wk, d).first;
-  }
-  t->wmap = wi->second;
   return 0;
 }
 
@@ -343,7 +322,6 @@ int fr_destroy(fr_ctx* c) {
   for (auto& e : c->band_wmap_tabs) (void)hipFree(e.second);
   for (auto& e : c->pts_tabs) (void)hipFree(e.second);
   for (auto& e : c->ring_tabs) (void)hipFree(e.second.d);
-  for (auto& e : c->wmap_tabs) (void)hipFree(e.second);
   for (auto& e : c->ccp_tabs) {
     (void)hipFree((void*)e.second.d);
     (void)hipFree((void*)e.second.k);

@@ -38,8 +38,6 @@ struct fr_ctx : public fr::Ctx {
     int cnt = 0;
   };
   std::map<std::tuple<int, float, float>, RingTab> ring_tabs;  // per (NSAM, RI2, RI3)
-  // per (NSAM, RI2, RI3, RIH, HALFW)
-  std::map<std::tuple<int, float, float, float, float>, float*> wmap_tabs;
   int cc3m_tables(const fr::Cc3mArgs& a, fr::Cc3mTables* t);
   std::map<std::pair<int, int>, float*> band_dft_tabs;         // per (M, frequencies held)
   std::map<std::pair<int, int>, int*> band_pair_tabs;          // per (MAXR1^2, MAXR2^2)

@@ -108,10 +108,8 @@ __device__ inline void tile_r2(int v0, int nsamh, int nsam, int& lo, int& hi) {
 constexpr int cc3m_pts_words() { return (kCc3mPtsHdr + 32 * (2 * kFJ + 1) + 1) & ~1; }
 
 // kWin: the score at every shift of a window around the item's shift (the
-// best of them and its index), instead of at the item's shift alone.  Without a
-// window the items with AMAG = 1 are the band grid's (fr_cc3m.hip) and left
-// alone; a window takes every item, those with AMAG = 1 by the tables of one
-// ring and mask.
+// best of them and its index), instead of at the item's shift alone.  Items with
+// AMAG = 1 are the band grid's (fr_cc3m.hip) and left alone.
 template <bool kWin>
 __global__ void __launch_bounds__(kFT)
     k_cc3m_fused(int nsam, int nitem, int maxr12, int maxr22, float rbfact,
@@ -120,10 +118,8 @@ __global__ void __launch_bounds__(kFT)
                  const float2* __restrict__ ctff, const float2* __restrict__ spec,
                  const float* __restrict__ shift, const float* __restrict__ amag_arr,
                  const float* __restrict__ fsct, const float* __restrict__ tab,
-                 const int* __restrict__ pts, const float* __restrict__ ring_tab, int ring_cnt,
-                 const float* __restrict__ wmap, float ri2,
-                 float ri3, float rih, float halfw, float* score, Cc3mWindow win,
-                 int* __restrict__ wcode, int flip) {
+                 const int* __restrict__ pts, float ri2, float ri3, float rih, float halfw,
+                 float* score, Cc3mWindow win, int* __restrict__ wcode, int flip) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int hrow = nsam / 2 + 1;
   float* Ts = lds;                      // [nsam/2 + 1][kFP]: the folded table TF
@@ -157,11 +153,9 @@ __global__ void __launch_bounds__(kFT)
   // particle (a particle's candidates) reuse its band spectrum in LDS
   const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
   const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
-  if constexpr (!kWin) {
-    bool any = false;
-    for (int it = it0 + tid; it < it1; it += kFT) any |= amag_arr[it] != 1.0f;
-    if (!__syncthreads_or(any)) return;
-  }
+  bool any = false;
+  for (int it = it0 + tid; it < it1; it += kFT) any |= amag_arr[it] != 1.0f;
+  if (!__syncthreads_or(any)) return;
   // ---- stage TF once; the workgroup then takes its items
   for (int e = tid; e < hrow * (kFK / 4); e += kFT) {
     int n = e / (kFK / 4), q = e % (kFK / 4);
@@ -170,15 +164,9 @@ __global__ void __launch_bounds__(kFT)
   }
   // the band point table, once (item independent)
   for (int e = tid; e < kCc3mPtsHdr + pts[kCc3mShells]; e += kFT) pts_s[e] = pts[e];
-  // this thread's entries e = tid + 512 r of the ring's Q table (the same for
-  // every item), held in registers across the items
-  static_assert(64 * 64 % kFT == 0, "Q entries per thread");
-  float qv[64 * 64 / kFT];
-#pragma unroll
-  for (int r = 0; r < 64 * 64 / kFT; r++) qv[r] = kWin ? ring_tab[tid + r * kFT] : 0.f;
   int pprev = -1;
   for (int it = it0; it < it1; it++) {
-  if (!kWin && amag_arr[it] == 1.0f) continue;  // the band grid's item
+  if (amag_arr[it] == 1.0f) continue;  // the band grid's item
   const int p = pidx[it];
   const bool newp = p != pprev;
   pprev = p;
@@ -224,12 +212,10 @@ __global__ void __launch_bounds__(kFT)
     }
   }
   __syncthreads();
-  // B(X)^T[c][k]: column c = (I, re|im), k = (|J|, cos|sin).  At AMAG = 1
-  // the MASKCOS2 ring sum is linear in B: sum_{c,k} Q[c][k] B^T[c][k] with the
-  // precomputed Q (the ring's rows of T through both transforms)
-  const bool ringq = kWin && amagp == 1.0f;
+  // B(X)^T[c][k]: column c = (I, re|im), k = (|J|, cos|sin)
   float rsum = 0.f;
   int rcnt = 0;
+  static_assert(64 * 64 % kFT == 0, "B entries per thread");
 #pragma unroll
   for (int r = 0; r < 64 * 64 / kFT; r++) {
     const int e = tid + r * kFT;
@@ -243,7 +229,6 @@ __global__ void __launch_bounds__(kFT)
     if (!(c & 1)) v = (k & 1) ? Q.y : P.x;   // Y_re = P_re T_re + Q_im T_im
     else v = (k & 1) ? -Q.x : P.y;           // Y_im = P_im T_re - Q_re T_im
     Bs[c * kFP + k] = v;
-    if (ringq) rsum += qv[r] * v;
   }
   __syncthreads();
 
@@ -309,13 +294,8 @@ __global__ void __launch_bounds__(kFT)
   }
   __syncthreads();
 
-  const bool use_wmap = kWin && amagp == 1.0f;
-  // ---- MASKCOS2 ring mean: x over ri2' < r^2 <= ri3'.  At AMAG = 1 the
-  // ring sum was taken from B above; otherwise a pass over the ring tiles on
-  // the matrix cores.
-  if (ringq) {
-    rcnt = tid == 0 ? ring_cnt : 0;
-  } else
+  // ---- MASKCOS2 ring mean: x over ri2' < r^2 <= ri3', a pass over the ring
+  // tiles on the matrix cores
   for (int rb = wave; rb < mt; rb += kFT / 64) {
     const int m0 = rb * 16;
     int mlo, mhi;
@@ -400,12 +380,11 @@ __global__ void __launch_bounds__(kFT)
       if (!((float)(nlo + mlo) > ri3p)) act |= 1u << nt;
     }
     // MASKCOS2 weights w of this lane's pixels (n0 + 4 lg + i, m) of a tile:
-    // 1 inside RI2', from the precomputed map at AMAG = 1, else per pixel
+    // 1 inside RI2', else per pixel
     auto weights = [&](int n0) -> fx4 {
       int nlo, nhi;
       tile_r2(n0, nsamh, nsam, nlo, nhi);
       if (!((float)(nhi + mhi) > ri2p)) return fx4{1.f, 1.f, 1.f, 1.f};
-      if (use_wmap) return *reinterpret_cast<const fx4*>(wmap + (size_t)m * nsam + n0 + 4 * lg);
       fx4 w;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -510,7 +489,6 @@ __global__ void __launch_bounds__(kFT)
         xs += __shfl_xor(xs, 32, 64);
         float w = 1.0f;
         if (crad2 > ri3p) w = 0.0f;
-        else if (use_wmap) w = wmap[(size_t)m * nsam + nsamh];
         else if (crad2 > ri2p) w = (1.0f + cosf(kPi * (sqrtf(crad2) - rihp) / halfw)) / 2.0f;
         const float y = (xs - mean) * w;
 #pragma unroll
@@ -940,7 +918,7 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                       int blocks, const Cc3mWindow* win, int* wcode) {
   if (a.n <= 0) return 0;
   FR_CHECK(cc3m_fused_ok(a.nsam, a.maxr2), "fused CC3M needs NSAM %% 32 == 0, NSAM <= 256, MAXR2 <= 32");
-  FR_CHECK(t.dft && t.pts && t.ring && t.wmap, "fused CC3M tables missing");
+  FR_CHECK(t.dft && t.pts, "fused CC3M tables missing");
   const size_t lds = cc3m_fused_lds(a.nsam);
   Cc3mWindow w{1, 1, 0.f, 0.f};
   if (win) {
@@ -962,16 +940,14 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
                        reinterpret_cast<const float2*>(a3df), dm, pidx,
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
-                       t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w, wcode,
-                       a.cc3);
+                       a.ri2, a.ri3, a.rih, a.halfw, score, w, wcode, a.cc3);
   else
     hipLaunchKernelGGL(k_cc3m_fused<false>, dim3((unsigned)grid), dim3(kFT), lds, c.stream,
                        a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2 * a.maxr2, a.rbfact,
                        reinterpret_cast<const float2*>(a3df), dm, pidx,
                        reinterpret_cast<const float2*>(ctff),
                        reinterpret_cast<const float2*>(spec), shift, amag, fsct, t.dft, t.pts,
-                       t.ring, t.ring_cnt, t.wmap, a.ri2, a.ri3, a.rih, a.halfw, score, w,
-                       (int*)nullptr, a.cc3);
+                       a.ri2, a.ri3, a.rih, a.halfw, score, w, (int*)nullptr, a.cc3);
   FR_HIP(hipGetLastError());
   return 0;
 }

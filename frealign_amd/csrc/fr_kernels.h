@@ -137,21 +137,12 @@ size_t cc3m_fused_lds(int nsam);
 //        -sin(2 pi i r/N), r = 0..N/2, i < 32 (T[n][2i] = cos(2 pi i n/N),
 //        T[n][2i+1] = -sin(2 pi i n/N) for every n is read from it);
 //   pts  kCc3mShells+1 shell offsets, then the band points (I | (J+64) << 8)
-//        sorted by shell INT(SQRT(I*I+J*J)+0.5), (I, J) order within a shell;
-//   ring Q[c][k] = w_c sum_m T[m][k] R[m][c], R[m][k] the sum over the
-//        MASKCOS2 ring pixels n of row m of T[n][k] (w_c the c2r weight): the
-//        ring sum is sum Q B^T, for AMAG = 1 (null: the ring mean is taken by a
-//        pass on the matrix cores);
-//   wmap the MASKCOS2 weight of every pixel [m][n] at AMAG = 1 (null:
-//        evaluated per pixel).
+//        sorted by shell INT(SQRT(I*I+J*J)+0.5), (I, J) order within a shell.
 constexpr int kCc3mShells = 34;
 constexpr int kCc3mPtsHdr = 36;
 struct Cc3mTables {
   const float* dft = nullptr;
   const int* pts = nullptr;
-  const float* ring = nullptr;
-  int ring_cnt = 0;
-  const float* wmap = nullptr;
 };
 void cc3m_fused_table(int nsam, std::vector<float>& tab);
 void cc3m_fused_table_folded(int nsam, std::vector<float>& tab);
@@ -169,7 +160,7 @@ struct Cc3mWindow {
   int nsx, nsy;
   float dsx, dsy;
 };
-// Without a window the items with AMAG = 1 are left alone.
+// Items with AMAG = 1 are left alone.
 int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec,
                       const float* ctff, const int* pidx, const float* dm, const float* shift,
                       const float* amag, const float* fsct, const Cc3mTables& t, float* score,
@@ -183,8 +174,10 @@ int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks
 int cc3m_band_grid(int nsam, int maxr2);
 int cc3m_band_rb(int maxr2);  // frequencies per axis the kernel holds: 16 or 32
 // Constant tables (device pointers, owned by the context): the DFT table of the
-// M grid, the band's (I, |J|) pairs in shell order, Q and the ring's pixel
-// count as in Cc3mTables, the mask on the M grid.
+// M grid, the band's (I, |J|) pairs in shell order, the ring's Q and its pixel
+// count, the mask on the M grid.  Q[c][k] = w_c sum_m T[m][k] R[m][c] on the NSAM
+// grid, R[m][k] the sum over the MASKCOS2 ring pixels n of row m of T[n][k] (w_c
+// the c2r weight): the ring sum is sum Q B^T.
 constexpr int kCc3mPairHdr = 36;    // shell offsets in front of the pairs' places
 constexpr int kCc3mRingPitch = 64;  // row length of Q
 struct Cc3mBandTables {

@@ -36,11 +36,12 @@ using namespace fr;
 
 namespace {
 
-// Items i = q * norient + o of particles p0 + q: o = (a * n + b) * n + c.
+// Items i = q * norient + o of particles who[q]: o = (a * n + b) * n + c.
 // trig: per particle, [angle 0..2][offset 0..n-1] (COS, SIN).  Writes DM,
 // the particle index, the window centre and the magnification per item.
-__global__ void k_local_dm(int nitem, int n, int p0, const float* __restrict__ trig,
-                           const float* __restrict__ amag, const float* __restrict__ centre,
+__global__ void k_local_dm(int nitem, int n, const int* __restrict__ who,
+                           const float* __restrict__ trig, const float* __restrict__ amag,
+                           const float* __restrict__ centre,
                            const float* __restrict__ sm, float* __restrict__ dm,
                            int* __restrict__ pidx, float* __restrict__ shift,
                            float* __restrict__ amag_it) {
@@ -48,9 +49,9 @@ __global__ void k_local_dm(int nitem, int n, int p0, const float* __restrict__ t
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nitem) return;
   const int norient = n * n * n;
-  const int q = i / norient, o = i % norient;
+  const int p = who[i / norient], o = i % norient;
   const int a = o / (n * n), b = (o / n) % n, c = o % n;
-  const float* t = trig + (size_t)(p0 + q) * 6 * n;
+  const float* t = trig + (size_t)p * 6 * n;
   const float cphi = t[2 * a], sphi = t[2 * a + 1];
   const float cthe = t[2 * (n + b)], sthe = t[2 * (n + b) + 1];
   const float cpsi = t[2 * (2 * n + c)], spsi = t[2 * (2 * n + c) + 1];
@@ -64,7 +65,7 @@ __global__ void k_local_dm(int nitem, int n, int p0, const float* __restrict__ t
   d[6] = sthe * cphi;
   d[7] = sthe * sphi;
   d[8] = cthe;
-  const float am = amag[p0 + q];
+  const float am = amag[p];
   if (am != 0.0f) {
     const float ab = fabsf(am);
     for (int k = 0; k < 9; k++) d[k] = d[k] / ab;
@@ -81,18 +82,20 @@ __global__ void k_local_dm(int nitem, int n, int p0, const float* __restrict__ t
   } else {
     for (int k = 0; k < 9; k++) out[k] = d[k];
   }
-  pidx[i] = p0 + q;
-  shift[2 * (size_t)i] = centre[2 * (size_t)(p0 + q)];
-  shift[2 * (size_t)i + 1] = centre[2 * (size_t)(p0 + q) + 1];
+  pidx[i] = p;
+  shift[2 * (size_t)i] = centre[2 * (size_t)p];
+  shift[2 * (size_t)i + 1] = centre[2 * (size_t)p + 1];
   amag_it[i] = fabsf(am);
 }
 
 // one wave per particle: the first maximum of its norient scores; writes
-// (orientation, shift index, score) to out[3 q ..]
+// (orientation, shift index, score) to out[3 who[q] ..], and all scores and indexes to
+// its place in all_s and all_c where these are given
 __global__ void __launch_bounds__(64)
     k_local_best(int norient, const float* __restrict__ score, const int* __restrict__ code,
-                 int* __restrict__ out) {
-  const int q = blockIdx.x, lane = threadIdx.x;
+                 const int* __restrict__ who, int* __restrict__ out, float* __restrict__ all_s,
+                 int* __restrict__ all_c) {
+  const int q = blockIdx.x, lane = threadIdx.x, p = who[q];
   const float* s = score + (size_t)q * norient;
   float bv = -3.0e38f;
   int bo = 0x7fffffff;
@@ -113,10 +116,15 @@ __global__ void __launch_bounds__(64)
   }
   if (lane == 0) {
     const int o = bo < norient ? bo : 0;
-    out[3 * q] = o;
-    out[3 * q + 1] = code[(size_t)q * norient + o];
-    out[3 * q + 2] = __float_as_int(s[o]);
+    out[3 * p] = o;
+    out[3 * p + 1] = code[(size_t)q * norient + o];
+    out[3 * p + 2] = __float_as_int(s[o]);
   }
+  if (all_s)
+    for (int o = lane; o < norient; o += 64) all_s[(size_t)p * norient + o] = s[o];
+  if (all_c)
+    for (int o = lane; o < norient; o += 64)
+      all_c[(size_t)p * norient + o] = code[(size_t)q * norient + o];
 }
 
 constexpr int kItemBudget = 1 << 16;  // items per launch
@@ -157,28 +165,41 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
     centre[2 * p] = x[3];
     centre[2 * p + 1] = x[4];
   }
-  std::vector<float> am(amag, amag + np);
-  // on the band's own grid where every AMAG is 1, else on the NSAM grid
-  bool unit = true;
-  for (int p = 0; p < np; p++) unit &= fabsf(am[p]) == 1.0f;
+  // A particle with AMAG = 1 goes to the band's own grid, another to the NSAM grid,
+  // whatever the others of the batch are: they are taken in that order
+  std::vector<float> am(np);
+  std::vector<int> who;
+  who.reserve(np);
+  for (int kind = 0; kind < 2; kind++)
+    for (int p = 0; p < np; p++) {
+      am[p] = fabsf(amag[p]);
+      if ((am[p] == 1.0f) == (kind == 0)) who.push_back(p);
+    }
+  const int ones = (int)std::count(am.begin(), am.end(), 1.0f);
+  const bool two = ones > 0 && ones < np;
   const size_t win_bytes = cc3m_window_bytes(
       cc3m_band_npair(maxr1 * maxr1, maxr2 * maxr2, cc3m_band_rb(maxr2)));
-  const size_t budget = unit ? std::min<size_t>(kItemBudget, kWinBudget / win_bytes) : kItemBudget;
+  const size_t budget = ones ? std::min<size_t>(kItemBudget, kWinBudget / win_bytes) : kItemBudget;
   const int chunk_p = std::max(1, std::min(np, (int)budget / norient));
   const size_t chunk_items = (size_t)chunk_p * norient;
   int err = 0;
-  float* d_trig = (float*)c->slot(6, sizeof(float) * (trig.size() + centre.size() + np + 9), &err);
+  // everything that goes over, in one copy: a particle's 27 orientations 88 us, 118 with
+  // five
+  std::vector<float> up(trig);
+  up.insert(up.end(), centre.begin(), centre.end());
+  up.insert(up.end(), am.begin(), am.end());
+  const size_t o_sm = up.size(), o_who = o_sm + 9;
+  up.resize(o_who + np);
+  if (sm) memcpy(&up[o_sm], sm, sizeof(float) * 9);
+  memcpy(&up[o_who], who.data(), sizeof(int) * (size_t)np);
+  float* d_trig = (float*)c->slot(6, sizeof(float) * up.size(), &err);
   if (!d_trig) return err;
   float* d_centre = d_trig + trig.size();
   float* d_am = d_centre + centre.size();
-  float* d_sm = d_am + np;
-  FR_HIP(hipMemcpyAsync(d_trig, trig.data(), sizeof(float) * trig.size(), hipMemcpyHostToDevice,
+  float* d_sm = d_trig + o_sm;
+  int* d_who = (int*)(d_trig + o_who);
+  FR_HIP(hipMemcpyAsync(d_trig, up.data(), sizeof(float) * up.size(), hipMemcpyHostToDevice,
                         c->stream));
-  FR_HIP(hipMemcpyAsync(d_centre, centre.data(), sizeof(float) * centre.size(),
-                        hipMemcpyHostToDevice, c->stream));
-  FR_HIP(hipMemcpyAsync(d_am, am.data(), sizeof(float) * np, hipMemcpyHostToDevice, c->stream));
-  if (sm)
-    FR_HIP(hipMemcpyAsync(d_sm, sm, sizeof(float) * 9, hipMemcpyHostToDevice, c->stream));
   // per-chunk item arrays: DM, particle, window centre, magnification, score, index
   const size_t per_item = 9 * sizeof(float) + sizeof(int) + 2 * sizeof(float) + sizeof(float) +
                           sizeof(float) + sizeof(int);
@@ -196,39 +217,41 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
   Cc3mTables tabs;
   Cc3mBandTables band;
   void* d_win = nullptr;
-  if (unit) {
+  if (ones) {
     if (int r = c->cc3m_band_tables(a, &band)) return r;
     d_win = c->slot(12, win_bytes * chunk_items, &err);
     if (!d_win) return err;
-  } else if (int r = c->cc3m_tables(a, &tabs)) {
-    return r;
   }
+  if (ones < np)
+    if (int r = c->cc3m_tables(a, &tabs)) return r;
   const Cc3mWindow win{2 * nsh + 1, 2 * nsh + 1, dsh, dsh};
   const fr_ctx::Tune tn = c->tune_for(nsam);
-  std::vector<int> best(3 * (size_t)np);
-  for (int p0 = 0; p0 < np; p0 += chunk_p) {
-    const int pc = std::min(chunk_p, np - p0);
-    const int ni = pc * norient;
-    hipLaunchKernelGGL(k_local_dm, dim3((ni + 255) / 256), dim3(256), 0, c->stream, ni, n, p0,
+  for (int q0 = 0; q0 < np; q0 += chunk_p) {
+    const int pc = std::min(chunk_p, np - q0), ni = pc * norient;
+    const int* d_w = d_who + q0;
+    hipLaunchKernelGGL(k_local_dm, dim3((ni + 255) / 256), dim3(256), 0, c->stream, ni, n, d_w,
                        d_trig, d_am, d_centre, sm ? d_sm : nullptr, d_dm, d_pi, d_sh, d_ai);
     FR_HIP(hipGetLastError());
-    a.n = ni;
-    float* sc = d_scores ? d_scores + (size_t)p0 * norient : d_sc;
-    int* cd = d_codes ? d_codes + (size_t)p0 * norient : d_cd;
+    // the caller's arrays directly where the list is the batch in order
+    float* sc = d_scores && !two ? d_scores + (size_t)q0 * norient : d_sc;
+    int* cd = d_codes && !two ? d_codes + (size_t)q0 * norient : d_cd;
+    const int n1 = std::max(0, std::min(pc, ones - q0)) * norient;  // items with AMAG = 1
     int pslot = c->prof_begin(kProfCc3m);
-    if (unit) {
-      if (int r = launch_cc3m_band_window(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
-                                          d_fsct, band, win, d_win, sc, cd, tn.cc3m_blocks))
-        return r;
-    } else if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
-                                         d_fsct, tabs, sc, tn.cc3m_blocks, &win, cd)) {
+    a.n = n1;
+    if (int r = launch_cc3m_band_window(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
+                                        d_fsct, band, win, d_win, sc, cd, tn.cc3m_blocks))
       return r;
-    }
+    a.n = ni - n1;
+    if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pi + n1,
+                                  d_dm + 9 * (size_t)n1, d_sh + 2 * (size_t)n1, d_ai + n1, d_fsct,
+                                  tabs, sc + n1, tn.cc3m_blocks, &win, cd + n1))
+      return r;
     c->prof_end(pslot);
-    hipLaunchKernelGGL(k_local_best, dim3(pc), dim3(64), 0, c->stream, norient, sc, cd,
-                       d_best + 3 * (size_t)p0);
+    hipLaunchKernelGGL(k_local_best, dim3(pc), dim3(64), 0, c->stream, norient, sc, cd, d_w, d_best,
+                       two ? d_scores : nullptr, two ? d_codes : nullptr);
     FR_HIP(hipGetLastError());
   }
+  std::vector<int> best(3 * (size_t)np);
   FR_HIP(hipMemcpyAsync(best.data(), d_best, sizeof(int) * best.size(), hipMemcpyDeviceToHost,
                         c->stream));
   FR_HIP(hipStreamSynchronize(c->stream));

@@ -142,3 +142,32 @@ def test_band_grid_serves_any_box(ctx, nsam, maxr1, maxr2):
                        t(sh.reshape(-1, 2), np.float32), torch.ones(npart * k, device=DEV), maxr1,
                        maxr2, 0.002, fsct, ring).reshape(npart, k)
     assert (got - want).abs().max() <= BAR * want.abs().max()
+
+
+def mask(nsam):
+    ri = 0.42 * nsam
+    return np.array([(ri - 3) ** 2, (ri + 3) ** 2, ri - 3, 6.0], np.float32)
+
+
+def test_local_search_does_not_depend_on_the_other_particles(ctx):
+    """Particles with AMAG 1, 1.04, 1, -1 together and one by one: the same bits."""
+    nsam, maxr2, n = 128, 25, 4
+    a3df, spec, ctff = items(nsam, n, n, 3, False)[:3]
+    fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    rng = np.random.default_rng(11)
+    par = np.concatenate([synth.random_orientations(n, rng), rng.normal(0, 0.1, (n, 2))],
+                         1).astype(np.float32)
+    amag = np.array([1.0, 1.04, 1.0, -1.0], np.float32)
+
+    def search(k):
+        return ctx[0].local_search(nsam, a3df, spec[k].contiguous(), ctff[k].contiguous(), par[k],
+                                   nang=1, dang=0.02, nsh=4, dsh=float(np.float32(2 * np.pi / nsam)),
+                                   maxr1=2, maxr2=maxr2, rbfact=0.002, fsct=fsct, ring=mask(nsam),
+                                   amag=amag[k], all_scores=True)
+
+    best, sc, code = search([0, 1, 2, 3])
+    for k in range(n):
+        b, s, c = search([k])
+        assert np.array_equal(b[0].view(np.int32), best[k].view(np.int32))
+        assert torch.equal(s.reshape(-1), sc.reshape(n, -1)[k])
+        assert torch.equal(c.reshape(-1), code.reshape(n, -1)[k])
