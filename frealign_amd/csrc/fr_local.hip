@@ -128,8 +128,9 @@ __global__ void __launch_bounds__(64)
 }
 
 constexpr int kItemBudget = 1 << 16;  // items per launch
-// bytes of the cross spectra between the two kernels of a launch: they stay in
-// the 256 MB cache next to what else the launch reads
+// bytes of the cross spectra between the two kernels of the band grid: they stay
+// in the 256 MB cache next to what else is read.  A chunk's items go there in as
+// many pairs of launches as that takes, one particle's among them.
 constexpr size_t kWinBudget = (size_t)160 << 20;
 
 }  // namespace
@@ -179,9 +180,9 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
   const bool two = ones > 0 && ones < np;
   const size_t win_bytes = cc3m_window_bytes(
       cc3m_band_npair(maxr1 * maxr1, maxr2 * maxr2, cc3m_band_rb(maxr2)));
-  const size_t budget = ones ? std::min<size_t>(kItemBudget, kWinBudget / win_bytes) : kItemBudget;
-  const int chunk_p = std::max(1, std::min(np, (int)budget / norient));
+  const int chunk_p = std::max(1, std::min(np, kItemBudget / norient));
   const size_t chunk_items = (size_t)chunk_p * norient;
+  const int win_items = (int)std::min<size_t>(chunk_items, kWinBudget / win_bytes);
   int err = 0;
   // everything that goes over, in one copy: a particle's 27 orientations 88 us, 118 with
   // five
@@ -219,7 +220,7 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
   void* d_win = nullptr;
   if (ones) {
     if (int r = c->cc3m_band_tables(a, &band)) return r;
-    d_win = c->slot(12, win_bytes * chunk_items, &err);
+    d_win = c->slot(12, win_bytes * win_items, &err);
     if (!d_win) return err;
   }
   if (ones < np)
@@ -237,10 +238,14 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
     int* cd = d_codes && !two ? d_codes + (size_t)q0 * norient : d_cd;
     const int n1 = std::max(0, std::min(pc, ones - q0)) * norient;  // items with AMAG = 1
     int pslot = c->prof_begin(kProfCc3m);
-    a.n = n1;
-    if (int r = launch_cc3m_band_window(*c, a, d_a3df, d_spec, d_ctff, d_pi, d_dm, d_sh, d_ai,
-                                        d_fsct, band, win, d_win, sc, cd, tn.cc3m_blocks))
-      return r;
+    for (int o = 0; o < n1; o += win_items) {
+      a.n = std::min(win_items, n1 - o);
+      if (int r = launch_cc3m_band_window(*c, a, d_a3df, d_spec, d_ctff, d_pi + o,
+                                          d_dm + 9 * (size_t)o, d_sh + 2 * (size_t)o, d_ai + o,
+                                          d_fsct, band, win, d_win, sc + o, cd + o,
+                                          tn.cc3m_blocks))
+        return r;
+    }
     a.n = ni - n1;
     if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pi + n1,
                                   d_dm + 9 * (size_t)n1, d_sh + 2 * (size_t)n1, d_ai + n1, d_fsct,

@@ -171,3 +171,21 @@ def test_local_search_does_not_depend_on_the_other_particles(ctx):
         assert np.array_equal(b[0].view(np.int32), best[k].view(np.int32))
         assert torch.equal(s.reshape(-1), sc.reshape(n, -1)[k])
         assert torch.equal(c.reshape(-1), code.reshape(n, -1)[k])
+
+
+def test_local_search_of_more_orientations_than_one_launch_holds(ctx):
+    """15,625 orientations: the cross spectra go through their buffer in two parts.
+    The orientations of a smaller grid about the same centre keep their bits."""
+    nsam, maxr2 = 64, 31
+    a3df, spec, ctff = items(nsam, 1, 1, 4, False)[:3]
+    fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    par = np.array([[0.3, 0.8, -0.4, 0.02, -0.01]], np.float32)
+    out = {}
+    for nang in (2, 12):
+        _, s, c = ctx[0].local_search(nsam, a3df, spec, ctff, par, nang=nang, dang=0.02, nsh=2,
+                                      dsh=0.1, maxr1=1, maxr2=maxr2, rbfact=0.002, fsct=fsct,
+                                      ring=mask(nsam), all_scores=True)
+        m, w = 2 * nang + 1, slice(nang - 2, nang + 3)
+        out[nang] = (s.reshape(m, m, m)[w, w, w], c.reshape(m, m, m)[w, w, w])
+        assert torch.isfinite(s).all()
+    assert torch.equal(out[2][0], out[12][0]) and torch.equal(out[2][1], out[12][1])
