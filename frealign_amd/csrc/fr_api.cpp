@@ -494,7 +494,7 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
   // are none) to the NSAM-grid products, which hold their boxes only.  Any other
   // box with a band that the grid holds goes there where every AMAG is known to
   // be 1.
-  const bool any_box = unit_amag && maxr2 <= 32 && maxr2 < nsam / 2;
+  const bool any_box = unit_amag && maxr2 <= 32 && maxr2 < nsam / 2 && nsam <= kCc3mMaxBox;
   if ((fr::cc3m_fused_ok(nsam, maxr2) || any_box) && tn.cc3m_fused) {
     Cc3mTables tabs;
     Cc3mBandTables band;

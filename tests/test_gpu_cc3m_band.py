@@ -189,3 +189,20 @@ def test_local_search_of_more_orientations_than_one_launch_holds(ctx):
         out[nang] = (s.reshape(m, m, m)[w, w, w], c.reshape(m, m, m)[w, w, w])
         assert torch.isfinite(s).all()
     assert torch.equal(out[2][0], out[12][0]) and torch.equal(out[2][1], out[12][1])
+
+
+def test_boxes_beyond_the_largest_are_refused(ctx):
+    """CC3M holds boxes up to 516: a rescoring of a larger one is refused whatever
+    its band, as a score of it is."""
+    nsam, k = 540, 2
+    jc = nsam // 2 + 1
+    z = lambda *s: torch.zeros(s, dtype=torch.complex64, device=DEV)  # noqa: E731
+    vol, spec, ctff = z(nsam, nsam, jc), z(1, nsam, jc), z(1, 2, nsam, jc)
+    o = torch.zeros((1, k), dtype=torch.int32, device=DEV)
+    dm = torch.from_numpy(api.rotation(np.zeros((1, 3), np.float32), amag=1.0)).to(DEV)
+    fsct = torch.ones(jc, device=DEV)
+    with pytest.raises(N.NativeError, match="box too large"):
+        ctx[0].cc3m(nsam, vol, spec, ctff, o[0, :1].contiguous(), dm, torch.zeros((1, 2), device=DEV),
+                    torch.ones(1, device=DEV), 2, 20, 0.0, fsct, mask(nsam))
+    with pytest.raises(N.NativeError, match="box too large"):
+        ctx[0].rescore(nsam, vol, spec, ctff, o, o + 112, dm, 270, 2, 20, 0.0, fsct, mask(nsam))
