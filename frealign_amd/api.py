@@ -167,7 +167,8 @@ class Context:
         npart = spec.numel() // (nsam * jc)
         if dm.numel() != 9 * n or shift.numel() != 2 * n or amag.numel() != n:
             raise ValueError("dm/shift/amag sizes do not match pidx")
-        if n and not self._inside(pidx, npart):
+        here = pidx.device.index == amag.device.index == self.device
+        if n and not here and not self._inside(pidx, npart):
             raise ValueError("pidx out of range")
         if ctff.numel() != 2 * spec.numel() or fsct.numel() < nsam // 2 + 1:
             raise ValueError("ctff/fsct sizes")
@@ -176,9 +177,16 @@ class Context:
         r = np.asarray(ring, dtype=np.float32)
         out = torch.empty(n, dtype=torch.float32, device=a3df.device)
         self._sync_stream()
-        N.check(N.lib().fr_cc3m_batch(self.h, nsam, n, _p(a3df), _p(spec), _p(ctff), _p(pidx),
-                                      _p(dm), _p(shift), _p(amag), maxr1, maxr2, float(rbfact),
-                                      _p(fsct), _p(r), _p(out)), "fr_cc3m_batch")
+        args = (_p(a3df), _p(spec), _p(ctff), _p(pidx), _p(dm), _p(shift), _p(amag), maxr1, maxr2,
+                float(rbfact), _p(fsct), _p(r), _p(out))
+        if not here:
+            N.check(N.lib().fr_cc3m_batch(self.h, nsam, n, *args), "fr_cc3m_batch")
+            return out
+        inside = C.c_int(1)
+        N.check(N.lib().fr_cc3m_checked(self.h, nsam, n, npart, *args, C.byref(inside)),
+                "fr_cc3m_checked")
+        if not inside.value:
+            raise ValueError("pidx out of range")
         return out
 
     def presb(self, nsam: int, a3df, spec, ctff, pidx, dm, shift, amag, ring,

@@ -243,6 +243,26 @@ int fr_ctx::cc3m_ring(int nsam, int maxr2, float ri2, float ri3, fr::Cc3mRing* t
   return 0;
 }
 
+int fr_ctx::index_range(long long n, const int* d_idx, const float* d_amag, int* lo, int* hi,
+                        fr::AmagMix* mix) {
+  if (!hrange)
+    FR_HIP(hipHostMalloc((void**)&hrange, sizeof(int4) * kRangeBlocks, hipHostMallocDefault));
+  const int blocks = (int)std::min<long long>(kRangeBlocks, (n + 4095) / 4096);
+  if (int r = fr::launch_index_range(*this, n, d_idx, d_amag, blocks, hrange)) return r;
+  FR_HIP(hipStreamSynchronize(stream));
+  int4 t = hrange[0];
+  for (int b = 1; b < blocks; b++) {
+    t.x = std::min(t.x, hrange[b].x);
+    t.y = std::max(t.y, hrange[b].y);
+    t.z |= hrange[b].z;
+    t.w |= hrange[b].w;
+  }
+  *lo = t.x;
+  *hi = t.y;
+  if (mix) *mix = fr::AmagMix{t.z != 0, t.w != 0};
+  return 0;
+}
+
 fr_ctx::Tune fr_ctx::tune_for(int nsam) const {
   auto it = tune.find(nsam);
   return it == tune.end() ? Tune{} : it->second;
@@ -423,19 +443,7 @@ int fr_prep_batch(fr_ctx* c, int nsam, int nb, float* d_data, const float* d_ppa
 int fr_index_range(fr_ctx* c, long long n, const int* d_idx, int* lo, int* hi) {
   CTX_CHECK(c);
   FR_CHECK(d_idx && lo && hi && n >= 1, "null or empty argument");
-  if (!c->hrange)
-    FR_HIP(hipHostMalloc((void**)&c->hrange, sizeof(int2) * fr_ctx::kRangeBlocks,
-                         hipHostMallocDefault));
-  const int blocks = (int)std::min<long long>(fr_ctx::kRangeBlocks, (n + 4095) / 4096);
-  if (int r = launch_index_range(*c, n, d_idx, blocks, c->hrange)) return r;
-  FR_HIP(hipStreamSynchronize(c->stream));
-  *lo = c->hrange[0].x;
-  *hi = c->hrange[0].y;
-  for (int b = 1; b < blocks; b++) {
-    *lo = std::min(*lo, c->hrange[b].x);
-    *hi = std::max(*hi, c->hrange[b].y);
-  }
-  return 0;
+  return c->index_range(n, d_idx, nullptr, lo, hi, nullptr);
 }
 
 int fr_pextract_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_dm,
@@ -452,6 +460,24 @@ int fr_cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* 
                   const float* d_fsct, const float* ring, float* d_score) {
   return fr::cc3m_batch(c, nsam, n, d_a3df, d_spec, d_ctff, d_pidx, d_dm, d_shift, d_amag, maxr1,
                         maxr2, rbfact, d_fsct, ring, d_score, 0);
+}
+
+int fr_cc3m_checked(fr_ctx* c, int nsam, int n, int npart, const float* d_a3df,
+                    const float* d_spec, const float* d_ctff, const int* d_pidx,
+                    const float* d_dm, const float* d_shift, const float* d_amag, int maxr1,
+                    int maxr2, float rbfact, const float* d_fsct, const float* ring,
+                    float* d_score, int* inside) {
+  CTX_CHECK(c);
+  FR_CHECK(n >= 0 && d_pidx && d_amag && inside, "null argument");
+  AmagMix mix;
+  if (n > 0) {
+    int lo = 0, hi = 0;
+    if (int r = c->index_range(n, d_pidx, d_amag, &lo, &hi, &mix)) return r;
+    if (!(*inside = lo >= 0 && hi < npart)) return 0;
+  }
+  *inside = 1;
+  return fr::cc3m_batch(c, nsam, n, d_a3df, d_spec, d_ctff, d_pidx, d_dm, d_shift, d_amag, maxr1,
+                        maxr2, rbfact, d_fsct, ring, d_score, 0, mix);
 }
 
 int fr_cc3_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
@@ -479,7 +505,7 @@ namespace fr {
 int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                const float* d_ctff, const int* d_pidx, const float* d_dm, const float* d_shift,
                const float* d_amag, int maxr1, int maxr2, float rbfact, const float* d_fsct,
-               const float* ring, float* d_score, int cc3, bool unit_amag) {
+               const float* ring, float* d_score, int cc3, AmagMix mix) {
   CTX_CHECK(c);
   SIZE_CHECK(nsam);
   FR_CHECK(n >= 0 && d_a3df && d_spec && d_ctff && d_pidx && d_dm && d_shift && d_amag &&
@@ -490,45 +516,45 @@ int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_s
   Cc3mArgs a{nsam, 0, maxr1, maxr2, rbfact, ring[0], ring[1], ring[2], ring[3]};
   a.cc3 = cc3;
   const fr_ctx::Tune tn = c->tune_for(nsam);
-  // The items with AMAG = 1 go to the band's own grid, the others (unless there
-  // are none) to the NSAM-grid products, which hold their boxes only.  Any other
-  // box with a band that the grid holds goes there where every AMAG is known to
-  // be 1.
-  const bool any_box = unit_amag && maxr2 <= 32 && maxr2 < nsam / 2 && nsam <= kCc3mMaxBox;
-  if ((fr::cc3m_fused_ok(nsam, maxr2) || any_box) && tn.cc3m_fused) {
-    Cc3mTables tabs;
-    Cc3mBandTables band;
-    if (int r = c->cc3m_band_tables(a, &band)) return r;
-    if (!unit_amag)
-      if (int r = c->cc3m_tables(a, &tabs)) return r;
-    int pslot = c->prof_begin(kProfCc3m);
-    for (int o = 0; o < n; o += 65535) {
-      a.n = n - o < 65535 ? n - o : 65535;
-      if (int r = launch_cc3m_band(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o,
-                                   d_dm + 9 * (size_t)o, d_shift + 2 * (size_t)o, d_amag + o,
-                                   d_fsct, band, d_score + o, tn.cc3m_blocks))
-        return r;
-      if (unit_amag) continue;
-      if (int r = launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o,
-                                    d_dm + 9 * (size_t)o, d_shift + 2 * (size_t)o, d_amag + o,
-                                    d_fsct, tabs, d_score + o, -1))
-        return r;
-    }
-    c->prof_end(pslot);
-    return 0;
-  }
-  FR_CHECK(maxr2 < nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", maxr2);
+  // An item's path follows from its box, its band and its own AMAG, never from
+  // the other items of the call: AMAG = 1 goes to the band's own grid wherever that
+  // holds the band, the rest to the NSAM-grid products where these hold the box,
+  // else to the particle's grid.
+  const bool band = tn.cc3m_fused && cc3m_band_ok(nsam, maxr2);
+  const bool fused = tn.cc3m_fused && cc3m_fused_ok(nsam, maxr2);
+  const bool rest = !band || mix.other;
+  a.mixed = mix.unit && mix.other;
+  Cc3mTables tabs;
+  Cc3mBandTables bt;
   Cc3mRing rt;
-  if (int r = c->cc3m_ring(nsam, maxr2, a.ri2, a.ri3, &rt)) return r;
-  const int step = fft_chunk(nsam, maxr2, n);
-  int err = 0;
-  void* work = c->slot(0, fr::cc3m_fft_bytes(nsam, maxr2, step), &err);
-  if (!work) return err;
+  void* work = nullptr;
+  int step = 65535;
+  if (band && mix.unit)
+    if (int r = c->cc3m_band_tables(a, &bt)) return r;
+  if (rest && fused) {
+    if (int r = c->cc3m_tables(a, &tabs)) return r;
+  } else if (rest) {
+    FR_CHECK(maxr2 < nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", maxr2);
+    if (int r = c->cc3m_ring(nsam, maxr2, a.ri2, a.ri3, &rt)) return r;
+    step = fft_chunk(nsam, maxr2, n);
+    int err = 0;
+    if (!(work = c->slot(0, fr::cc3m_fft_bytes(nsam, maxr2, step), &err))) return err;
+  }
   int pslot = c->prof_begin(kProfCc3m);
-  for (int o = 0; o < n; o += step) {
+  for (int o = 0; band && mix.unit && o < n; o += 65535) {
+    a.n = n - o < 65535 ? n - o : 65535;
+    if (int r = launch_cc3m_band(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o, d_dm + 9 * (size_t)o,
+                                 d_shift + 2 * (size_t)o, d_amag + o, d_fsct, bt, d_score + o,
+                                 tn.cc3m_blocks))
+      return r;
+  }
+  for (int o = 0; rest && o < n; o += step) {
     a.n = n - o < step ? n - o : step;
-    if (int r = launch_cc3m(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o, d_dm + 9 * (size_t)o,
-                            d_shift + 2 * (size_t)o, d_amag + o, d_fsct, rt, work, d_score + o))
+    const float *dm = d_dm + 9 * (size_t)o, *sh = d_shift + 2 * (size_t)o;
+    if (int r = fused ? launch_cc3m_fused(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o, dm, sh,
+                                          d_amag + o, d_fsct, tabs, d_score + o, -1)
+                      : launch_cc3m(*c, a, d_a3df, d_spec, d_ctff, d_pidx + o, dm, sh, d_amag + o,
+                                    d_fsct, rt, work, d_score + o, band))
       return r;
   }
   c->prof_end(pslot);
@@ -1393,7 +1419,7 @@ int fr_rescore_batch(fr_ctx* c, int nsam, int np, int k, const float* d_a3df, co
                                 sh, am))
     return r;
   if (int r = cc3m_batch(c, nsam, (int)n, d_a3df, d_outc, d_ctff, pidx, dm, sh, am, maxr1, maxr2,
-                         rbfact, d_fsct, ring, d_score, 0, true))
+                         rbfact, d_fsct, ring, d_score, 0, AmagMix{true, false}))
     return r;
   return launch_best_cand(*c, np, k, d_top_o, d_score, d_best);
 }
@@ -1467,12 +1493,10 @@ int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d
     memcpy(h + o_sh, hsh, sizeof(float) * 2 * m);
     memcpy(h + o_am, ham, sizeof(float) * m);
     FR_HIP(hipMemcpyAsync(dbuf, h, o_sc, hipMemcpyHostToDevice, c->stream));
-    bool unit = true;
-    for (int i = 0; i < m; i++) unit &= ham[i] == 1.0f;
     if (int r = cc3m_batch(c, nsam, m, d_a3df, d_spec, d_ctff, (const int*)dbuf,
                            (const float*)(dbuf + o_dm), (const float*)(dbuf + o_sh),
                            (const float*)(dbuf + o_am), maxr1, maxr2, rbfact, d_fsct, ring,
-                           (float*)(h + o_sc), 0, unit))
+                           (float*)(h + o_sc), 0, amag_mix(ham, m)))
       return r;
     FR_HIP(hipStreamSynchronize(c->stream));
     memcpy(hscore, h + o_sc, sizeof(float) * m);

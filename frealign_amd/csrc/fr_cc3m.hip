@@ -98,7 +98,7 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
                 const float* __restrict__ amag_arr, const float* __restrict__ fsct,
                 const float* __restrict__ tab, const int* __restrict__ pairs,
                 const float* __restrict__ ring_tab, int ring_cnt,
-                const float* __restrict__ wmap, float* __restrict__ score, int flip,
+                const float* __restrict__ wmap, float* __restrict__ score, int flip, int mixed,
                 Cc3mWinBuf wb) {
   using S = BandShape<RB, M>;
   constexpr int kThr = S::kThreads, kK = S::kK, kP = S::kP, kPr = S::kPairs, H = M / 2;
@@ -119,6 +119,11 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
   const int per = (nitem + (int)gridDim.x - 1) / (int)gridDim.x;
   const int it0 = blockIdx.x * per, it1 = min(nitem, it0 + per);
 
+  if (mixed) {  // no item of this form: nothing to set up
+    bool any = false;
+    for (int it = it0 + tid0; it < it1; it += kThr) any |= amag_arr[it] == 1.0f;
+    if (!__syncthreads_or(any)) return;
+  }
   // ---- what does not depend on the item
   for (int e = tid0; e < (H + 1) * (kK / 4); e += kThr) {
     const int r = e / (kK / 4), q = e % (kK / 4);
@@ -782,6 +787,15 @@ __global__ void __launch_bounds__(64 * kWinWaves)
 
 }  // namespace
 
+// Every band that the kernel's registers hold, at the boxes of the NSAM-grid form
+// and, below NSAM/2, at the boxes of the particle's grid: an item with AMAG = 1
+// comes here at any of them (8,192 items of a 250 box at MAXR2 32: 274 us, on the
+// particle's grid 1,928)
+bool cc3m_band_ok(int nsam, int maxr2) {
+  return maxr2 >= 1 && maxr2 <= 32 &&
+         (cc3m_fused_ok(nsam, maxr2) || (maxr2 < nsam / 2 && nsam <= kCc3mMaxBox));
+}
+
 int cc3m_band_grid(int nsam, int maxr2) {
   if (maxr2 > 32 || maxr2 < 1) return 0;
   const int need = maxr2 <= 16 ? 64 : maxr2 <= 24 ? 96 : 128;
@@ -919,7 +933,7 @@ int launch_band(Ctx& c, const Cc3mArgs& a, const BandCall& p, const Cc3mBandTabl
                      a.rbfact, reinterpret_cast<const float2*>(p.a3df), p.dm, p.pidx,
                      reinterpret_cast<const float2*>(p.ctff),
                      reinterpret_cast<const float2*>(p.spec), p.shift, p.amag, p.fsct, t.dft,
-                     t.pairs, t.ring, t.ring_cnt, t.wmap, score, a.cc3, wb);
+                     t.pairs, t.ring, t.ring_cnt, t.wmap, score, a.cc3, a.mixed, wb);
   FR_HIP(hipGetLastError());
   return 0;
 }

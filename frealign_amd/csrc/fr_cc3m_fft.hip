@@ -47,6 +47,8 @@ struct Band {
   int nsam, nitem, cb, jmax, maxr12, maxr22, nsh;
   float ri2, ri3, rih, halfw;
   int flip;
+  int skip;  // items with AMAG = 1 are the band grid's (fr_cc3m.hip): left alone
+  __device__ bool left(float amag) const { return skip && amag == 1.0f; }
 };
 
 constexpr int rows_nseq(int n) { return n >= 1024 ? 2 : 2048 / n; }
@@ -64,8 +66,9 @@ template <int N>
 __global__ void __launch_bounds__(kThr)
     k_band_cols(Band b, Plan pl, const float2* __restrict__ a3df, const float* __restrict__ dm,
                 const int* __restrict__ pidx, const float2* __restrict__ ctff,
-                const float* __restrict__ rhat, float2* __restrict__ work,
-                float* __restrict__ part, const float2* __restrict__ tw) {
+                const float* __restrict__ rhat, const float* __restrict__ amag,
+                float2* __restrict__ work, float* __restrict__ part,
+                const float2* __restrict__ tw) {
   extern __shared__ float2 smem[];
   __shared__ float red[kThr / 64];
   const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
@@ -76,7 +79,7 @@ __global__ void __launch_bounds__(kThr)
   // an item's column blocks in XCD-contiguous order: they share lines
   const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
   const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
-  if (it >= b.nitem) return;
+  if (it >= b.nitem || b.left(amag[it])) return;
   for (int e = threadIdx.x; e < kCw * (N ? F::LD : ld); e += kThr) buf[e] = make_float2(0.f, 0.f);
   __syncthreads();
   const float* d = dm + 9 * (size_t)it;
@@ -189,7 +192,7 @@ __global__ void __launch_bounds__(kThr)
   const int n = N ? N : pl.n, it = blockIdx.x, nblk = b.cb / kCw;
   const float am = amag[it];
   if (am == 1.0f) {
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && !b.skip) {
       float s = 0.f;
       for (int q = 0; q < nblk; q++) s += part[(size_t)it * nblk + q];
       mean[it] = ring_cnt ? s / (float)ring_cnt : s;
@@ -232,6 +235,12 @@ __global__ void __launch_bounds__(kThr)
   extern __shared__ float2 smem[];
   const int n = N ? N : pl.n, ld = n + 1, nh = n / 2, nseq = rows_nseq(n);
   const int pair0 = blockIdx.x * nseq, npairs = b.nitem * nh;
+  if (b.skip) {  // rows of items that are left alone only
+    const int last = min(pair0 + nseq, npairs) - 1;
+    bool any = false;
+    for (int it = pair0 / nh; it <= last / nh; it++) any |= !b.left(amag[it]);
+    if (!any) return;
+  }
   // (z - mean) weight of pixel x of both rows of pair pr
   auto masked = [&](int pr, int x, float2 z) {
     const int it = pr / nh, row = 2 * (pr - it * nh);
@@ -312,7 +321,8 @@ template <int N>
 __global__ void __launch_bounds__(kThr)
     k_band_sums(Band b, Plan pl, const float2* __restrict__ work, const float2* __restrict__ spec,
                 const int* __restrict__ pidx, const float* __restrict__ shift,
-                float4* __restrict__ psum, const float2* __restrict__ tw) {
+                const float* __restrict__ amag, float4* __restrict__ psum,
+                const float2* __restrict__ tw) {
   extern __shared__ float2 smem[];
   using F = Cols<N>;
   const int n = N ? N : pl.n, ld = n + 1, jc = n / 2 + 1;
@@ -323,7 +333,7 @@ __global__ void __launch_bounds__(kThr)
   __shared__ float2 ex[kCw];
   const int nblk = b.cb / kCw, lb = xcd_block(blockIdx.x, gridDim.x);
   const int it = lb / nblk, x0 = (lb - it * nblk) * kCw;
-  if (it >= b.nitem) return;
+  if (it >= b.nitem || b.left(amag[it])) return;
   const float2* in = work + (size_t)it * n * b.cb + x0;
   const float shx = shift[2 * it], shy = shift[2 * it + 1];
   for (int j = threadIdx.x; j <= b.jmax; j += kThr) {
@@ -427,8 +437,10 @@ __device__ inline float4 shell(const float4* psum, const Band& b, int it, int s)
 // by a fixed butterfly
 __global__ void __launch_bounds__(64)
     k_band_score(Band b, float rbfact, const float4* __restrict__ psum,
-                 const float* __restrict__ fsct, float* __restrict__ score) {
+                 const float* __restrict__ fsct, const float* __restrict__ amag,
+                 float* __restrict__ score) {
   const int it = blockIdx.x, lane = threadIdx.x;
+  if (b.left(amag[it])) return;
   double s1 = 0.0, s2 = 0.0, s3 = 0.0;
   for (int s = 1 + lane; s < min(b.nsam / 2, b.nsh); s += 64) {
     const float4 t = shell(psum, b, it, s);
@@ -549,7 +561,8 @@ int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, con
   FR_HIP(big((const void*)k_band_sums<N>, ls));
   hipLaunchKernelGGL(k_band_cols<N>, dim3(cols), dim3(kThr), lc, c.stream, b, pl,
                      reinterpret_cast<const float2*>(p.a3df), p.dm, p.pidx,
-                     reinterpret_cast<const float2*>(p.ctff), ring.rhat, w.band, w.part, tw);
+                     reinterpret_cast<const float2*>(p.ctff), ring.rhat, p.amag, w.band, w.part,
+                     tw);
   FR_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_band_mean<N>, dim3(b.nitem), dim3(kThr), lr, c.stream, b, pl, w.band,
                      w.part, ring.cnt, p.amag, w.mean, tw);
@@ -558,7 +571,8 @@ int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, con
                      pl, w.band, p.amag, w.mean, tw);
   FR_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_band_sums<N>, dim3(cols), dim3(kThr), ls, c.stream, b, pl, w.band,
-                     reinterpret_cast<const float2*>(p.spec), p.pidx, p.shift, w.psum, tw);
+                     reinterpret_cast<const float2*>(p.spec), p.pidx, p.shift, p.amag, w.psum,
+                     tw);
   FR_HIP(hipGetLastError());
   return 0;
 }
@@ -568,10 +582,10 @@ int launch_band(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, 
 }
 
 Band make_band(int nsam, int n, int maxr12, int maxr2, float ri2, float ri3, float rih,
-               float halfw, int flip) {
+               float halfw, int flip, int skip) {
   int jmax = maxr2 - 1;
   return Band{nsam, n,   band_cb(maxr2), jmax, maxr12, maxr2 * maxr2, band_nsh(maxr2),
-              ri2,  ri3, rih,            halfw, flip};
+              ri2,  ri3, rih,            halfw, flip,   skip};
 }
 
 }  // namespace
@@ -617,19 +631,20 @@ int launch_ring_hat(Ctx& c, int nsam, float ri2, float ri3, int maxr2, void* buf
 
 int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
                 const int* pidx, const float* dm, const float* shift, const float* amag,
-                const float* fsct, const Cc3mRing& ring, void* work, float* score) {
+                const float* fsct, const Cc3mRing& ring, void* work, float* score,
+                bool skip_unit) {
   if (a.n <= 0) return 0;
   FR_CHECK(a.nsam <= kCc3mMaxBox, "box too large for CC3M bins");
   FR_CHECK(a.maxr2 < a.nsam / 2, "CC3M needs MAXR2 < NSAM/2 (got %d)", a.maxr2);
   FR_CHECK(ring.rhat && work, "CC3M tables missing");
   const Band b = make_band(a.nsam, a.n, a.maxr1 * a.maxr1, a.maxr2, a.ri2, a.ri3, a.rih, a.halfw,
-                           a.cc3);
+                           a.cc3, skip_unit);
   size_t bytes;
   const BandWork w = band_work(work, a.nsam, a.maxr2, a.n, &bytes);
   if (int r = launch_band(c, b, BandCall{a3df, spec, ctff, pidx, dm, shift, amag}, ring, w))
     return r;
   hipLaunchKernelGGL(k_band_score, dim3(a.n), dim3(64), 0, c.stream, b, a.rbfact, w.psum, fsct,
-                     score);
+                     amag, score);
   FR_HIP(hipGetLastError());
   return 0;
 }
@@ -642,7 +657,7 @@ int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, 
   if (n <= 0) return 0;
   FR_CHECK(nsam <= kCc3mMaxBox, "box too large for PRESB bins");
   FR_CHECK(ring.rhat && work, "PRESB tables missing");
-  const Band b = make_band(nsam, n, 1, nsam / 2, ri2, ri3, rih, halfw, 0);
+  const Band b = make_band(nsam, n, 1, nsam / 2, ri2, ri3, rih, halfw, 0, 0);
   size_t bytes;
   const BandWork w = band_work(work, nsam, nsam / 2, n, &bytes);
   if (int r = launch_band(c, b, BandCall{a3df, spec, ctff, pidx, dm, shift, amag}, ring, w))

@@ -185,7 +185,8 @@ int run(fr_ctx* c, const Job& j, float* out, int* nevals) {
       if (int r = cc3m_batch(c, nsam, cnt, j.d_a3df, d_outc, d_ctff, d_pi + k0,
                              d_it + 9 * (size_t)k0, d_it + 9 * (size_t)m + 2 * (size_t)k0,
                              d_it + 11 * (size_t)m + k0, kv.first.first, kv.first.second,
-                             j.rbfact, d_fs, j.ring, d_sc + k0, 1))
+                             j.rbfact, d_fs, j.ring, d_sc + k0, 1,
+                             amag_mix(&items[11 * (size_t)m + k0], cnt)))
         return r;
       k0 += cnt;
     }

@@ -20,9 +20,11 @@ struct fr_ctx : public fr::Ctx {
   void* hpin = nullptr;
   size_t hpin_bytes = 0;
   void* host_pinned(size_t bytes, int* err);
-  // the index checks' results, one pair per workgroup, in host memory
+  // the index checks' results, one record per workgroup, in host memory
   static constexpr int kRangeBlocks = 64;
-  int2* hrange = nullptr;
+  int4* hrange = nullptr;
+  int index_range(long long n, const int* d_idx, const float* d_amag, int* lo, int* hi,
+                  fr::AmagMix* mix);
   // search annulus and shift-phase tables, cached per (NSAM, MAXR1, MAXR2)
   int skey[3] = {0, 0, 0};
   int kc = 0, kpad = 0, nsamr = 0;
@@ -64,12 +66,12 @@ struct fr_ctx : public fr::Ctx {
 };
 
 namespace fr {
-// fr_cc3m_batch (cc3 = 0) and fr_cc3_batch (cc3 = 1).  unit_amag: the caller
-// knows that every AMAG is 1
+// fr_cc3m_batch (cc3 = 0) and fr_cc3_batch (cc3 = 1).  mix: what the caller knows of
+// the items' AMAG (it saves launches; an item's path does not depend on it)
 int cc3m_batch(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                const float* d_ctff, const int* d_pidx, const float* d_dm, const float* d_shift,
                const float* d_amag, int maxr1, int maxr2, float rbfact, const float* d_fsct,
-               const float* ring, float* d_score, int cc3, bool unit_amag = false);
+               const float* ring, float* d_score, int cc3, fr::AmagMix mix = {});
 // fr_refine_batch with the symmetry matrix SM applied to every DM (null: identity)
 int refine_items(fr_ctx* c, int nsam, int n, const float* d_a3df, const float* d_spec,
                  const float* d_ctff, const int* pidx, const float* amag, float* par,

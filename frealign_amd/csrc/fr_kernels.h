@@ -98,12 +98,25 @@ struct Cc3mArgs {
   int nsam, n, maxr1, maxr2;
   float rbfact, ri2, ri3, rih, halfw;
   int cc3 = 0;  // 1: CC3 (cc3.f): the section phase-flipped by the CTF sign, no |R| branch
+  // each form of the launch takes the items of its own AMAG; 0 where the caller
+  // knows that these are all items
+  int mixed = 1;
 };
+// What the caller knows of the items' AMAG: whether any may be 1, any may not.
+struct AmagMix {
+  bool unit = true, other = true;
+};
+inline AmagMix amag_mix(const float* amag, size_t n) {
+  AmagMix m{false, false};
+  for (size_t i = 0; i < n; i++) (amag[i] == 1.0f ? m.unit : m.other) = true;
+  return m;
+}
 
 constexpr int kMaskThreads = 1024;
 constexpr int kCc3mMaxBox = 516;  // the largest box of CC3M and PRESB
 // On the particle's grid, any box, band and AMAG (fr_cc3m_fft.hip); work:
-// cc3m_fft_bytes for the items of the call (PRESB: MAXR2 = NSAM/2).
+// cc3m_fft_bytes for the items of the call (PRESB: MAXR2 = NSAM/2).  skip_unit:
+// items with AMAG = 1 are left alone (the band's grid takes them).
 struct Cc3mRing {
   const float* rhat = nullptr;  // launch_ring_hat
   int cnt = 0;                  // the ring's pixels
@@ -115,7 +128,8 @@ int launch_ring_hat(Ctx& c, int nsam, float ri2, float ri3, int maxr2, void* buf
                     const float** rhat);
 int launch_cc3m(Ctx& c, const Cc3mArgs& a, const float* a3df, const float* spec, const float* ctff,
                 const int* pidx, const float* dm, const float* shift, const float* amag,
-                const float* fsct, const Cc3mRing& ring, void* work, float* score);
+                const float* fsct, const Cc3mRing& ring, void* work, float* score,
+                bool skip_unit = false);
 int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, const float* ctff,
                  const int* pidx, const float* dm, const float* shift, const float* amag,
                  float ri2, float ri3, float rih, float halfw, const Cc3mRing& ring, void* work,
@@ -170,7 +184,9 @@ int launch_cc3m_fused(Ctx& c, const Cc3mArgs& a, const float* a3df, const float*
 int cc3m_grid(Ctx& c, const void* fn, int threads, size_t lds, int n, int blocks, int* grid);
 
 // CC3M on the band's own M x M grid (fr_cc3m.hip), for the items with AMAG = 1;
-// the others are left alone.  cc3m_band_grid: M, or 0 where there is none.
+// the others are left alone.  cc3m_band_ok: whether the grid holds the band and
+// the box.  cc3m_band_grid: M, or 0 where there is none.
+bool cc3m_band_ok(int nsam, int maxr2);
 int cc3m_band_grid(int nsam, int maxr2);
 int cc3m_band_rb(int maxr2);  // frequencies per axis the kernel holds: 16 or 32
 // Constant tables (device pointers, owned by the context): the DFT table of the

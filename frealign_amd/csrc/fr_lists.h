@@ -17,7 +17,9 @@ int launch_cand_items(Ctx& c, int np, int k, const int* top_o, const int* top_ro
                       const float* dm_bank, int nsamr, int* pidx, float* dm, float* shift,
                       float* amag);
 int launch_best_cand(Ctx& c, int np, int k, const int* top_o, float* score, int* best);
-// the smallest and largest of idx[0..n) per workgroup into out[0..blocks)
-int launch_index_range(Ctx& c, long long n, const int* idx, int blocks, int2* out);
+// per workgroup into out[0..blocks): the smallest and largest of idx[0..n), and
+// whether any of amag[0..n) (may be null) is 1, any is not
+int launch_index_range(Ctx& c, long long n, const int* idx, const float* amag, int blocks,
+                       int4* out);
 
 }  // namespace fr

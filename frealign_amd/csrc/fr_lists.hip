@@ -28,20 +28,25 @@ constexpr int kFill = 256;
 constexpr int kTile = 256;   // template columns per GEMM tile
 constexpr float kPi = 3.1415926535897f;
 
-// The smallest and largest of n indexes: one pair per workgroup, in host memory
-// that the device writes, so that the caller's check costs one launch and one
-// wait.  Two library reductions, each with a copy and a wait of its own, were
-// nearly half of a score of 8 items (56 us; 31 us with this).
+// The smallest and largest of n indexes and, with amag, whether any of its n
+// values is 1 and any is not: one record per workgroup, in host memory that the
+// device writes, so that the caller's check costs one launch and one wait.  Two
+// library reductions, each with a copy and a wait of its own, were nearly half of
+// a score of 8 items (56 us; 31 us with this).
 __global__ void __launch_bounds__(kFill)
-    k_index_range(long long n, const int* __restrict__ idx, int2* out) {
+    k_index_range(long long n, const int* __restrict__ idx, const float* __restrict__ amag,
+                  int4* out) {
   __shared__ int2 red[kFill / 64];
-  int lo = 0x7fffffff, hi = -0x7fffffff - 1;
+  int lo = 0x7fffffff, hi = -0x7fffffff - 1, unit = 0, other = 0;
   for (long long i = blockIdx.x * (long long)kFill + threadIdx.x; i < n;
        i += (long long)gridDim.x * kFill) {
     const int v = idx[i];
     lo = min(lo, v);
     hi = max(hi, v);
+    if (amag) (amag[i] == 1.0f ? unit : other) = 1;
   }
+  unit = __syncthreads_or(unit);
+  other = __syncthreads_or(other);
   for (int off = 32; off > 0; off >>= 1) {
     lo = min(lo, __shfl_xor(lo, off, 64));
     hi = max(hi, __shfl_xor(hi, off, 64));
@@ -53,7 +58,7 @@ __global__ void __launch_bounds__(kFill)
       lo = min(lo, red[w].x);
       hi = max(hi, red[w].y);
     }
-    out[blockIdx.x] = make_int2(lo, hi);
+    out[blockIdx.x] = make_int4(lo, hi, unit != 0, other != 0);
   }
 }
 
@@ -315,8 +320,9 @@ int launch_best_cand(Ctx& c, int np, int k, const int* top_o, float* score, int*
   return 0;
 }
 
-int launch_index_range(Ctx& c, long long n, const int* idx, int blocks, int2* out) {
-  hipLaunchKernelGGL(k_index_range, dim3(blocks), dim3(kFill), 0, c.stream, n, idx, out);
+int launch_index_range(Ctx& c, long long n, const int* idx, const float* amag, int blocks,
+                       int4* out) {
+  hipLaunchKernelGGL(k_index_range, dim3(blocks), dim3(kFill), 0, c.stream, n, idx, amag, out);
   FR_HIP(hipGetLastError());
   return 0;
 }

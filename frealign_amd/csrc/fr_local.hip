@@ -215,6 +215,7 @@ int fr_local_search_batch(fr_ctx* c, int nsam, int np, const float* d_a3df, cons
   int* d_best = (int*)c->slot(8, 3 * sizeof(int) * (size_t)np, &err);
   if (!d_best) return err;
   Cc3mArgs a{nsam, 0, maxr1, maxr2, rbfact, ring[0], ring[1], ring[2], ring[3]};
+  a.mixed = 0;
   Cc3mTables tabs;
   Cc3mBandTables band;
   void* d_win = nullptr;

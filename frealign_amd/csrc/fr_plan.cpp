@@ -31,7 +31,7 @@ using namespace fr;
 
 struct fr_plan {
   fr_ctx* c = nullptr;
-  int nsam = 0, nb = 0, ncopy = 0, fused = 0, blocks = 0;
+  int nsam = 0, nb = 0, ncopy = 0, fused = 0, onband = 0, blocks = 0;
   // bound arguments
   const float* a3df = nullptr;
   const float* pssnr = nullptr;
@@ -87,16 +87,18 @@ int enqueue(fr_plan* p) {
                         c->stream));
   Cc3mArgs a = p->ca;
   a.n = nb;
-  if (p->fused) {  // as cc3m_batch: a batch's AMAG is not known at capture
+  // as cc3m_batch: a batch's AMAG is not known at capture
+  if (p->onband)
     if (int r = launch_cc3m_band(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm,
                                  p->d_shift, p->d_amag, p->fsct, p->band, p->d_score, p->blocks))
       return r;
+  if (p->fused) {
     if (int r = launch_cc3m_fused(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm,
                                   p->d_shift, p->d_amag, p->fsct, p->tabs, p->d_score, -1))
       return r;
   } else {
     if (int r = launch_cc3m(*c, a, p->a3df, p->d_outc, p->d_ctff, p->d_pidx, p->d_dm, p->d_shift,
-                            p->d_amag, p->fsct, p->ring, p->d_work, p->d_score))
+                            p->d_amag, p->fsct, p->ring, p->d_work, p->d_score, p->onband))
       return r;
   }
   FR_HIP(hipMemcpyAsync(p->h_score, p->d_score, sizeof(float) * nb, hipMemcpyDeviceToHost,
@@ -213,6 +215,7 @@ int fr_plan_create(fr_ctx* c, int nsam, int nb, const float* d_a3df, const float
   p->ttd = d_ttd;
   const fr_ctx::Tune tn = c->tune_for(nsam);
   p->fused = cc3m_fused_ok(nsam, maxr2) && tn.cc3m_fused;
+  p->onband = cc3m_band_ok(nsam, maxr2) && tn.cc3m_fused;
   p->blocks = tn.cc3m_blocks;
   const size_t ic = (size_t)nsam * (nsam / 2 + 1), img = (size_t)nsam * (nsam + 2);
   int r = 0;
@@ -235,9 +238,8 @@ int fr_plan_create(fr_ctx* c, int nsam, int nb, const float* d_a3df, const float
     return fail(r);
   if ((r = dalloc(&p->d_ins, insert_scratch_bytes(nsam, nb, nb * ncopy)))) return fail(r);
   if ((r = dalloc(&p->d_part, 2 * prep_partials_count(nsam, nb)))) return fail(r);
-  if (p->fused && ((r = c->cc3m_tables(p->ca, &p->tabs)) ||
-                   (r = c->cc3m_band_tables(p->ca, &p->band))))
-    return fail(r);
+  if (p->fused && (r = c->cc3m_tables(p->ca, &p->tabs))) return fail(r);
+  if (p->onband && (r = c->cc3m_band_tables(p->ca, &p->band))) return fail(r);
   std::vector<int> pid(nb);
   for (int b = 0; b < nb; b++) pid[b] = b;
   if (hipMemcpy(p->d_pidx, pid.data(), sizeof(int) * nb, hipMemcpyHostToDevice) != hipSuccess)
@@ -351,7 +353,7 @@ int fr_autotune_cc3m(fr_ctx* c, int nsam, int n, const float* d_a3df, const floa
     float ms;
   };
   std::vector<Cand> cands;
-  if (cc3m_fused_ok(nsam, maxr2)) {
+  if (cc3m_band_ok(nsam, maxr2)) {
     int cus = 256;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, c->device) == hipSuccess) cus = prop.multiProcessorCount;

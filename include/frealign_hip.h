@@ -121,6 +121,15 @@ int fr_cc3m_batch(fr_ctx *ctx, int nsam, int n, const float *d_a3df, const float
                   const float *d_shift, const float *d_amag, int maxr1, int maxr2, float rbfact,
                   const float *d_fsct, const float *ring, float *d_score);
 
+/* fr_cc3m_batch after a check that every d_pidx[k] is in 0..npart-1 (one launch
+ * and one wait, which also tell which items have AMAG 1, so that only the kernels
+ * for these or the others are launched).  *inside = 0 and no scores otherwise. */
+int fr_cc3m_checked(fr_ctx *ctx, int nsam, int n, int npart, const float *d_a3df,
+                    const float *d_spec, const float *d_ctff, const int *d_pidx,
+                    const float *d_dm, const float *d_shift, const float *d_amag, int maxr1,
+                    int maxr2, float rbfact, const float *d_fsct, const float *ring,
+                    float *d_score, int *inside);
+
 /* Replaces CC3 (cc3.f:8-159; IEWALD=0, IBUF=0), the score of the defocus and
  * magnification refinements (calcfx.f:63-140): as fr_cc3m_batch with the
  * section multiplied by the sign of REAL(CTFR+CONJG(CTFL)) instead of the CTF

@@ -1,6 +1,7 @@
 """CC3M on the band's own grid against the FFT path on the particle's grid.
 
-The two agree up to FP32 rounding for every box size, band and mask: bands at
+The two agree up to FP32 rounding for every box size, band and mask, and an item's
+score has the same bits whatever the other items of its call are: bands at
 the edges of the grids (MAXR2 16 | 17, 24 | 25, 32), boxes smaller than, equal
 to and larger than the grid, one item and more items than workgroups, and
 items whose AMAG is not 1 (taken by another kernel) between the others.  The
@@ -133,6 +134,7 @@ def test_band_grid_serves_any_box(ctx, nsam, maxr1, maxr2):
     o, row = rng.integers(0, nbank, (npart, k)), rng.integers(0, 225, (npart, k))
     nsamr = 2 * ((nsam // 2 + 1) // 2)
     fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    ctx[1].set_cc3m_variant(nsam, False)
     got, _ = ctx[0].rescore(nsam, vol, spec, ctff, t(o, np.int32), t(row, np.int32),
                             dm.reshape(nbank, 9), nsamr, maxr1, maxr2, 0.002, fsct, ring)
     sh = np.stack([row // 15 - 7, row % 15 - 7], -1).astype(np.float32)
@@ -142,11 +144,64 @@ def test_band_grid_serves_any_box(ctx, nsam, maxr1, maxr2):
                        t(sh.reshape(-1, 2), np.float32), torch.ones(npart * k, device=DEV), maxr1,
                        maxr2, 0.002, fsct, ring).reshape(npart, k)
     assert (got - want).abs().max() <= BAR * want.abs().max()
+    ctx[1].set_cc3m_variant(nsam, True)  # the score entry takes the same way
+    same = ctx[1].cc3m(nsam, vol, spec, ctff, t(np.repeat(np.arange(npart), k), np.int32),
+                       dm.reshape(nbank, 9)[t(o.reshape(-1), np.int64)].contiguous(),
+                       t(sh.reshape(-1, 2), np.float32), torch.ones(npart * k, device=DEV), maxr1,
+                       maxr2, 0.002, fsct, ring).reshape(npart, k)
+    assert torch.equal(got, same)
 
 
 def mask(nsam):
     ri = 0.42 * nsam
     return np.array([(ri - 3) ** 2, (ri + 3) ** 2, ri - 3, 6.0], np.float32)
+
+
+@pytest.mark.parametrize("nsam,maxr1,maxr2", [(36, 1, 16), (72, 0, 32), (100, 2, 25), (128, 2, 24),
+                                              (250, 2, 16)])
+@pytest.mark.parametrize("cc3", [False, True])
+def test_a_score_does_not_depend_on_the_other_items(ctx, nsam, maxr1, maxr2, cc3):
+    """Items with AMAG 1 and 1.04 in one call, against each kind and each item by
+    itself: the same bits, and all against the particle's grid."""
+    a = items(nsam, 3, 40, nsam, True)
+    amag = a[-1].cpu().numpy()
+    whole = score(ctx[0], nsam, a, maxr1, maxr2, mask(nsam), cc3)
+    few = [[k] for k in (0, 1, 2, 39)] + [np.flatnonzero(amag == 1), np.flatnonzero(amag != 1)]
+    assert all(len(k) for k in few)
+    for k in few:
+        idx = torch.as_tensor(np.asarray(k), device=DEV)
+        part = a[:3] + tuple(x[idx].contiguous() for x in a[3:])
+        assert np.array_equal(score(ctx[0], nsam, part, maxr1, maxr2, mask(nsam), cc3), whole[k])
+    if not cc3:  # the checked entry knows which items there are
+        fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+        got = ctx[0].cc3m(nsam, *a, maxr1, maxr2, 0.002, fsct, mask(nsam)).cpu().numpy()
+        assert np.array_equal(got, whole)
+    ctx[1].set_cc3m_variant(nsam, False)
+    want = score(ctx[1], nsam, a, maxr1, maxr2, mask(nsam), cc3)
+    assert np.abs(whole - want).max() <= BAR * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nsam,maxr2", [(72, 32), (100, 25), (128, 24)])
+def test_refinement_does_not_depend_on_the_other_particles(ctx, nsam, maxr2):
+    """PREFINE of AMAG 1, 1.04, 1 together and one by one: the same bits."""
+    n = 3
+    a3df, spec, ctff = items(nsam, n, n, 7 * nsam, False)[:3]
+    fsct = torch.linspace(1.0, 0.5, nsam // 2 + 1, device=DEV)
+    rng = np.random.default_rng(nsam)
+    par = np.zeros((n, 6), np.float32)
+    par[:, :3], par[:, 3:5] = synth.random_orientations(n, rng), rng.normal(0, 0.05, (n, 2))
+    prior = np.tile(np.array([0, 0, 0.3, 0.3, 0.01], np.float32), (n, 1))
+    amag = np.array([1.0, 1.04, 1.0], np.float32)
+
+    def refine(k):
+        return ctx[0].refine(nsam, a3df, spec, ctff, np.asarray(k, np.int32), amag[k], par[k],
+                             np.ones(5, np.int32), 2, maxr2, 0.0, fsct, mask(nsam), prior[k])
+
+    whole, nev = refine([0, 1, 2])
+    assert len(set(nev.tolist())) > 1  # they do not all converge in the same round
+    for k in range(n):
+        got, ne = refine([k])
+        assert ne[0] == nev[k] and np.array_equal(got[0].view(np.int32), whole[k].view(np.int32))
 
 
 def test_local_search_does_not_depend_on_the_other_particles(ctx):

@@ -38,6 +38,7 @@ def _records(parts, rng, nb):
     recb[:, 0:3] = parts.euler + np.radians(rng.normal(0, 2, (nb, 3))).astype(np.float32)
     recb[:, 3:5] = parts.shift
     recb[:, 5] = 1.0
+    recb[1::3, 5] = 1.03  # scored by another kernel
     recb[:, 6] = 1.0
     recb[:, 6][::5] = 0.0  # some particles carry no occupancy: nothing inserted
     recb[:, 7] = 1.0
@@ -47,7 +48,8 @@ def _records(parts, rng, nb):
     return recb, half
 
 
-@pytest.mark.parametrize("nsam,asym,nasym", [(64, "C", 1), (96, "D", 7), (128, "C", 2)])
+@pytest.mark.parametrize("nsam,asym,nasym", [(64, "C", 1), (96, "D", 7), (128, "C", 2),
+                                             (100, "C", 1)])
 def test_plan_replays_equal_eager(ctx, nsam, asym, nasym):
     psize, ri, nb = 2.0, 0.4 * nsam, 8
     optics = synth.Optics(psize=psize)
