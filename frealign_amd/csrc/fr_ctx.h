@@ -52,6 +52,12 @@ struct fr_ctx : public fr::Ctx {
   std::map<std::tuple<int, int, float, float>, RingHat> ring_hats;  // per (NSAM, MAXR2, RI2, RI3)
   int cc3m_ring(int nsam, int maxr2, float ri2, float ri3, fr::Cc3mRing* t);
   int cc3m_band_tables(const fr::Cc3mArgs& a, fr::Cc3mBandTables* t);
+  // a second stream, for the part of a batch that other kernels take than the rest.
+  // side_open orders it after what the context's stream holds; who uses it waits for
+  // it on the host before returning.
+  hipStream_t side = nullptr;
+  hipEvent_t side_fork = nullptr;
+  int side_open();
   // launch choices per box size (set by fr_autotune_cc3m)
   struct Tune {
     int cc3m_fused = 1;   // band-pruned fused CC3M where it applies

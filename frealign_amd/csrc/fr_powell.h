@@ -57,12 +57,18 @@ struct RefineArgs {
   const float* sm = nullptr;    // SM of the DMs (cc3m.f:66, MATMUL_T); null: identity
 };
 
-// Objective values in one launch: score[q] = CC3M of particle pidx[q] at
-// (dm[9q..], shift[2q..], amag[q]) for q < m (host arrays).
-using Cc3mFn = std::function<int(int m, const int* pidx, const float* dm, const float* shift,
-                                 const float* amag, float* score)>;
+// A round of objective values: submit starts CC3M of particle pidx[q] at
+// (dm[9q..], shift[2q..], amag[q]) for q < m (host arrays, free after the call), wait
+// ends it and gives the scores.  Each lane, 0 for items with AMAG = 1 and 1 for the
+// others, has at most one round under way; both may at once.
+struct Cc3mRounds {
+  std::function<int(int lane, int m, const int* pidx, const float* dm, const float* shift,
+                    const float* amag)>
+      submit;
+  std::function<int(int lane, int m, float* score)> wait;
+};
 
 // par: host n x 6, PHI THETA PSI DSHX DSHY in, refined values and PRESA out.
-int refine_batch(Ctx& c, const RefineArgs& a, float* par, int* nevals, const Cc3mFn& cc3m);
+int refine_batch(const RefineArgs& a, float* par, int* nevals, const Cc3mRounds& cc3m);
 
 }  // namespace fr

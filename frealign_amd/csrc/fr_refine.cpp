@@ -366,14 +366,14 @@ inline float fsh(float sig2, float x, float y, float xm, float ym, float sx, flo
 
 }  // namespace
 
-int refine_batch(Ctx& c, const RefineArgs& a, float* par, int* nevals, const Cc3mFn& cc3m) {
-  (void)c;
+int refine_batch(const RefineArgs& a, float* par, int* nevals, const Cc3mRounds& cc3m) {
   constexpr float kPi = 3.1415926535897f;
   const float epar[6] = {0.1f, 0.1f, 0.1f, 0.01f, 0.01f, 0.001f};  // prefine.f:46
   const int n = a.n;
   std::vector<Powell> pw(n);
   std::vector<int> npar(n, 0);
-  std::vector<int> active;
+  auto lane_of = [&](int i) { return a.amag[i] == 1.0f ? 0 : 1; };
+  std::vector<int> active[2], idle[2];  // per lane
   // prefine.f:56-66: the refined subset of (PHI, THETA, PSI, DSHX, DSHY)
   for (int i = 0; i < n; i++) {
     float xm[6], em[6];
@@ -387,25 +387,22 @@ int refine_batch(Ctx& c, const RefineArgs& a, float* par, int* nevals, const Cc3
     npar[i] = np;
     if (np > 0) {
       pw[i].start(xm, em, np, 100.0f, 1, a.maxit);
-      active.push_back(i);
     }
+    (np > 0 ? active : idle)[lane_of(i)].push_back(i);
   }
-  std::vector<int> want;
   std::vector<int> pidx;
-  std::vector<float> dm, shift, amag, score;
-  // objective at each item's current parameters: -CC3M - FSH + penalties
-  auto evaluate = [&](const std::vector<int>& items, std::vector<float>& fval,
-                      std::vector<float>& cc) -> int {
+  std::vector<float> dm, shift, amag, xp[2], score;
+  // the round of a lane's items at their current parameters
+  auto submit = [&](int lane, const std::vector<int>& items) -> int {
     const int m = (int)items.size();
     pidx.resize(m);
     dm.resize(9 * (size_t)m);
     shift.resize(2 * (size_t)m);
     amag.resize(m);
-    score.resize(m);
-    std::vector<float> xp(6 * (size_t)m);
+    xp[lane].resize(6 * (size_t)m);
     for (int q = 0; q < m; q++) {
       const int i = items[q];
-      float* x = &xp[6 * (size_t)q];
+      float* x = &xp[lane][6 * (size_t)q];
       for (int j = 0; j < 5; j++) x[j] = par[6 * i + j];
       if (npar[i] > 0) {
         const float* v = pw[i].x();
@@ -420,12 +417,17 @@ int refine_batch(Ctx& c, const RefineArgs& a, float* par, int* nevals, const Cc3
       shift[2 * q + 1] = x[4];
       amag[q] = x[5];
     }
-    if (int r = cc3m(m, pidx.data(), dm.data(), shift.data(), amag.data(), score.data())) return r;
+    return cc3m.submit(lane, m, pidx.data(), dm.data(), shift.data(), amag.data());
+  };
+  // its objectives: -CC3M - FSH + penalties
+  auto finish = [&](int lane, const std::vector<int>& items, std::vector<float>& fval) -> int {
+    const int m = (int)items.size();
+    score.resize(m);
+    if (int r = cc3m.wait(lane, m, score.data())) return r;
     fval.resize(m);
-    cc.resize(m);
     for (int q = 0; q < m; q++) {
       const int i = items[q];
-      const float* x = &xp[6 * (size_t)q];
+      const float* x = &xp[lane][6 * (size_t)q];
       const float* pr = a.prior + 5 * (size_t)i;
       float rft = -score[q] - fsh(pr[4], x[3], x[4], pr[0], pr[1], pr[2], pr[3]);
       if (fabsf(x[0]) > kPi) rft = rft + (kPi - fabsf(x[0])) * (kPi - fabsf(x[0]));
@@ -434,38 +436,43 @@ int refine_batch(Ctx& c, const RefineArgs& a, float* par, int* nevals, const Cc3
       if (fabsf(x[3]) > 1.0f) rft = rft + (1.0f - fabsf(x[3])) * (1.0f - fabsf(x[3]));
       if (fabsf(x[4]) > 1.0f) rft = rft + (1.0f - fabsf(x[4])) * (1.0f - fabsf(x[4]));
       fval[q] = rft;
-      cc[q] = score[q];
     }
     return 0;
   };
-  std::vector<float> fval, cc;
+  std::vector<float> fval;
   // items with nothing to refine: PRESA = CC3M + FSH at the start (prefine.f:68-84, 155)
-  {
-    std::vector<int> idle;
-    for (int i = 0; i < n; i++)
-      if (npar[i] == 0) idle.push_back(i);
-    if (!idle.empty()) {
-      if (int r = evaluate(idle, fval, cc)) return r;
-      for (size_t q = 0; q < idle.size(); q++) {
-        const int i = idle[q];
-        const float* pr = a.prior + 5 * (size_t)i;
-        par[6 * i + 5] = cc[q] + fsh(pr[4], par[6 * i + 3], par[6 * i + 4], pr[0], pr[1], pr[2], pr[3]);
-        if (nevals) nevals[i] = 1;
+  for (int lane = 0; lane < 2; lane++) {
+    if (idle[lane].empty()) continue;
+    if (int r = submit(lane, idle[lane])) return r;
+    if (int r = finish(lane, idle[lane], fval)) return r;
+    for (size_t q = 0; q < idle[lane].size(); q++) {
+      const int i = idle[lane][q];
+      const float* pr = a.prior + 5 * (size_t)i;
+      par[6 * i + 5] =
+          score[q] + fsh(pr[4], par[6 * i + 3], par[6 * i + 4], pr[0], pr[1], pr[2], pr[3]);
+      if (nevals) nevals[i] = 1;
+    }
+  }
+  // lock-stepped minimisations, the lanes' rounds in turn
+  for (int lane : {1, 0}) {
+    for (int i : active[lane]) pw[i].run();
+    if (!active[lane].empty())
+      if (int r = submit(lane, active[lane])) return r;
+  }
+  while (!active[0].empty() || !active[1].empty())
+    for (int lane : {0, 1}) {
+      if (active[lane].empty()) continue;
+      if (int r = finish(lane, active[lane], fval)) return r;
+      std::vector<int> next;
+      for (size_t q = 0; q < active[lane].size(); q++) {
+        const int i = active[lane][q];
+        pw[i].supply(fval[q]);
+        if (pw[i].run()) next.push_back(i);
       }
+      active[lane].swap(next);
+      if (!active[lane].empty())
+        if (int r = submit(lane, active[lane])) return r;
     }
-  }
-  // lock-stepped minimisations
-  for (int i : active) pw[i].run();
-  while (!active.empty()) {
-    if (int r = evaluate(active, fval, cc)) return r;
-    std::vector<int> next;
-    for (size_t q = 0; q < active.size(); q++) {
-      const int i = active[q];
-      pw[i].supply(fval[q]);
-      if (pw[i].run()) next.push_back(i);
-    }
-    active.swap(next);
-  }
   for (int i = 0; i < n; i++) {
     if (npar[i] == 0) continue;
     const float* v = pw[i].x();

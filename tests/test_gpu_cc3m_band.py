@@ -193,15 +193,17 @@ def test_refinement_does_not_depend_on_the_other_particles(ctx, nsam, maxr2):
     prior = np.tile(np.array([0, 0, 0.3, 0.3, 0.01], np.float32), (n, 1))
     amag = np.array([1.0, 1.04, 1.0], np.float32)
 
-    def refine(k):
+    def refine(k, free):
         return ctx[0].refine(nsam, a3df, spec, ctff, np.asarray(k, np.int32), amag[k], par[k],
-                             np.ones(5, np.int32), 2, maxr2, 0.0, fsct, mask(nsam), prior[k])
+                             np.full(5, free, np.int32), 2, maxr2, 0.0, fsct, mask(nsam), prior[k])
 
-    whole, nev = refine([0, 1, 2])
-    assert len(set(nev.tolist())) > 1  # they do not all converge in the same round
-    for k in range(n):
-        got, ne = refine([k])
-        assert ne[0] == nev[k] and np.array_equal(got[0].view(np.int32), whole[k].view(np.int32))
+    for free in (1, 0):  # 0: nothing to refine, PRESA alone
+        whole, nev = refine([0, 1, 2], free)
+        assert not free or len(set(nev.tolist())) > 1  # not all converge in the same round
+        for k in range(n):
+            got, ne = refine([k], free)
+            assert ne[0] == nev[k]
+            assert np.array_equal(got[0].view(np.int32), whole[k].view(np.int32))
 
 
 def test_local_search_does_not_depend_on_the_other_particles(ctx):
