@@ -35,7 +35,7 @@
 // one CU's matrix cores; 1,536 folded once, 4,896 on a 256 grid), 3,200 gathered
 // points and the barriers between the passes.  LDS is 71 KB (149 KB on the 256
 // grid), so two workgroups share a CU and one's gathers and sums run under the
-// other's products.  8,192 items of a 256 box: 300 us (1,370 on the 256 grid,
+// other's products.  8,192 items of a 256 box: 291 us (1,370 on the 256 grid,
 // 393 folded once).
 #include <hip/hip_runtime.h>
 
@@ -398,70 +398,70 @@ __global__ void __launch_bounds__((BandShape<RB, M>::kThreads), 4)
       // E and O of a tile of T rows r < M/2 give x[r] = E + O and x[M-r] = E - O
       // (the same w at both); Z's cosine part takes y[r] + y[M-r], its sine part
       // y[r] - y[M-r]
-    fx4 w[M / 32];
-    float wh = 0.f;
-    if (rows) {
+      fx4 w[M / 32];
+      float wh = 0.f;
+      if (rows) {
 #pragma unroll
-      for (int t = 0; t < M / 32; t++)
-        w[t] = *reinterpret_cast<const fx4*>(wtab + (size_t)m * M + 16 * t + 4 * lg);
-      wh = wtab[(size_t)m * M + H];
-    }
-    if (rows) {
-      float2 yv[RB / 4];
-#pragma unroll
-      for (int ks = 0; ks < RB / 4; ks++) yv[ks] = ld2(Ys + m * kP + 8 * ks + 2 * lg);
-      fx4 zc[RB / 16], zs[RB / 16];
-#pragma unroll
-      for (int kt = 0; kt < RB / 16; kt++) zc[kt] = zs[kt] = fx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < M / 32; t++) {
-        __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
-        fx4 e = {0.f, 0.f, 0.f, 0.f}, o = e, sp, sm;
-#pragma unroll
-        for (int ks = 0; ks < RB / 4; ks++) {
-          const float2 tv = ld2(Ts + (16 * t + la) * kP + 8 * ks + 2 * lg);
-          e = mfma4(tv.x, yv[ks].x, e);
-          o = mfma4(tv.y, yv[ks].y, o);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float ya = (e[i] + o[i] - mean) * w[t][i];
-          float yb = (e[i] - o[i] - mean) * w[t][i];
-          if (t == 0 && i == 0 && lg == 0) yb = 0.f;  // r = 0: its own partner
-          sp[i] = ya + yb;
-          sm[i] = ya - yb;
-        }
-        // k-step i takes r = 16t + 4 lg + i: the C layout of E, O is the B layout
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-          for (int kt = 0; kt < RB / 16; kt++) {
-            const float2 tv = ld2(Ts + (16 * t + 4 * lg + i) * kP + 2 * (16 * kt + la));
-            zc[kt] = mfma4(tv.x, sp[i], zc[kt]);
-            zs[kt] = mfma4(tv.y, sm[i], zs[kt]);
-          }
+        for (int t = 0; t < M / 32; t++)
+          w[t] = *reinterpret_cast<const fx4*>(wtab + (size_t)m * M + 16 * t + 4 * lg);
+        wh = wtab[(size_t)m * M + H];
       }
-      // row M/2: x = sum_I (-1)^I wYre[m][I], I = 4 ks + lg
-      float xs = 0.f;
+      if (rows) {
+        float2 yv[RB / 4];
 #pragma unroll
-      for (int ks = 0; ks < RB / 4; ks++) xs += yv[ks].x;
-      xs = (lg & 1) ? -xs : xs;
-      xs += __shfl_xor(xs, 16, 64);
-      xs += __shfl_xor(xs, 32, 64);
-      const float yh = (xs - mean) * wh;
+        for (int ks = 0; ks < RB / 4; ks++) yv[ks] = ld2(Ys + m * kP + 8 * ks + 2 * lg);
+        fx4 zc[RB / 16], zs[RB / 16];
 #pragma unroll
-      for (int kt = 0; kt < RB / 16; kt++)
+        for (int kt = 0; kt < RB / 16; kt++) zc[kt] = zs[kt] = fx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; i++) zc[kt][i] += (i & 1) ? -yh : yh;
-      if (lg == 0) zc[0][0] += mean * (float)M;  // k = 0, the mean's own term
-      // this wave alone read rows m0 .. m0 + 15 of Ys
+        for (int t = 0; t < M / 32; t++) {
+          __builtin_amdgcn_sched_barrier(0);  // one tile's operands at a time
+          fx4 e = {0.f, 0.f, 0.f, 0.f}, o = e, sp, sm;
 #pragma unroll
-      for (int kt = 0; kt < RB / 16; kt++)
+          for (int ks = 0; ks < RB / 4; ks++) {
+            const float2 tv = ld2(Ts + (16 * t + la) * kP + 8 * ks + 2 * lg);
+            e = mfma4(tv.x, yv[ks].x, e);
+            o = mfma4(tv.y, yv[ks].y, o);
+          }
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-          *reinterpret_cast<float2*>(Ys + m * kP + 2 * (16 * kt + 4 * lg + i)) =
-              make_float2(zc[kt][i], zs[kt][i]);
-    }
+          for (int i = 0; i < 4; i++) {
+            const float ya = (e[i] + o[i] - mean) * w[t][i];
+            float yb = (e[i] - o[i] - mean) * w[t][i];
+            if (t == 0 && i == 0 && lg == 0) yb = 0.f;  // r = 0: its own partner
+            sp[i] = ya + yb;
+            sm[i] = ya - yb;
+          }
+          // k-step i takes r = 16t + 4 lg + i: the C layout of E, O is the B layout
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int kt = 0; kt < RB / 16; kt++) {
+              const float2 tv = ld2(Ts + (16 * t + 4 * lg + i) * kP + 2 * (16 * kt + la));
+              zc[kt] = mfma4(tv.x, sp[i], zc[kt]);
+              zs[kt] = mfma4(tv.y, sm[i], zs[kt]);
+            }
+        }
+        // row M/2: x = sum_I (-1)^I wYre[m][I], I = 4 ks + lg
+        float xs = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < RB / 4; ks++) xs += yv[ks].x;
+        xs = (lg & 1) ? -xs : xs;
+        xs += __shfl_xor(xs, 16, 64);
+        xs += __shfl_xor(xs, 32, 64);
+        const float yh = (xs - mean) * wh;
+#pragma unroll
+        for (int kt = 0; kt < RB / 16; kt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) zc[kt][i] += (i & 1) ? -yh : yh;
+        if (lg == 0) zc[0][0] += mean * (float)M;  // k = 0, the mean's own term
+        // this wave alone read rows m0 .. m0 + 15 of Ys
+#pragma unroll
+        for (int kt = 0; kt < RB / 16; kt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            *reinterpret_cast<float2*>(Ys + m * kP + 2 * (16 * kt + 4 * lg + i)) =
+                make_float2(zc[kt][i], zs[kt][i]);
+      }
     }
     __syncthreads();
 
@@ -959,8 +959,9 @@ int launch_window(Ctx& c, const Cc3mArgs& a, const float* fsct, const float* ama
   if (int r = cc3m_grid(c, (const void*)k_cc3m_window<NT>, 64 * kWinWaves, 0,
                         (a.n + kWinItems - 1) / kWinItems, -1, &grid))
     return r;
-  hipLaunchKernelGGL(k_cc3m_window<NT>, dim3((unsigned)grid), dim3(64 * kWinWaves), 0, c.stream, a.n, cc3m_band_rb(a.maxr2), top, a.rbfact,
-                     t.pairs, fsct, amag, a.cc3, win, wb, score, code);
+  hipLaunchKernelGGL(k_cc3m_window<NT>, dim3((unsigned)grid), dim3(64 * kWinWaves), 0, c.stream,
+                     a.n, cc3m_band_rb(a.maxr2), top, a.rbfact, t.pairs, fsct, amag, a.cc3, win,
+                     wb, score, code);
   FR_HIP(hipGetLastError());
   return 0;
 }

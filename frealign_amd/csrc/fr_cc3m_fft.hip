@@ -309,14 +309,6 @@ __global__ void __launch_bounds__(kThr)
   }
 }
 
-// largest j >= 0 with j*j <= v (v >= 0, below 2^20)
-__device__ inline int isqrt(int v) {
-  int j = (int)sqrtf((float)v);
-  if (j * j > v) j--;
-  if ((j + 1) * (j + 1) <= v) j++;
-  return j;
-}
-
 template <int N>
 __global__ void __launch_bounds__(kThr)
     k_band_sums(Band b, Plan pl, const float2* __restrict__ work, const float2* __restrict__ spec,

@@ -26,7 +26,7 @@
 // fragment order once per step.
 //
 // Measured, forward and backward of that batch with 4 convolutions:
-// 857 -> 269 us (convolution 1 forward 73 -> 27, its input gradient 161 -> 31,
+// 857 -> 251 us (convolution 1 forward 73 -> 27, its input gradient 161 -> 31,
 // its weight gradient with its sums 142 -> 50).
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>

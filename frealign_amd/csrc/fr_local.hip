@@ -11,7 +11,7 @@
 //     path; k_local_dm forms DM from them with the products of cc3m.f:48-65 in
 //     the same order without contraction, so each DM is the one the host's
 //     rotation gives for the same angles, bit for bit.
-//   * The scores come from the fused CC3M kernel with a shift window: one
+//   * The scores come from CC3M's kernels with a shift window: one
 //     extraction, masking and transform pair per orientation, the shell sums
 //     at every shift from one set of cross-spectrum products.
 //   * k_local_best takes each particle's first maximum over its orientations

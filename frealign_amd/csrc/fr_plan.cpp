@@ -1,9 +1,10 @@
 // fr_plan.cpp -- persistent, graph-captured batches and the launch autotuner.
 //
 // fr_autotune_cc3m: times the CC3M launch variants that apply to a box size
-// (the fused band-pruned kernel at several persistent grid sizes, and the
-// FFT path) on the caller's data, keeps the fastest for that NSAM in the
-// context and returns the measurements as JSON.
+// ("fused": the band's grid at several persistent grid sizes, with the NSAM-grid
+// form beside it; "fft": the particle's grid for every item) on the caller's data,
+// keeps the fastest for that NSAM in the context and returns the measurements as
+// JSON.  Untuned, the band's grid runs as many workgroups as the device holds.
 //
 // fr_plan: one box size, one batch size.  The score-and-insert pipeline of a
 // batch -- CTFAPPLY (fr_prep_batch), CC3M at the particles' current

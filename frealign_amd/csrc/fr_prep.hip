@@ -361,14 +361,6 @@ int rows_mask_t(Ctx& c, int nb, float* outc, const float* ppar, const PrepGlobal
 // was written before the FFTs and read back here.  512 images of 256^2: 365 us as
 // table (119), column pass (50) and weighting (197), 239 us like this.
 
-// largest j >= 0 with j*j <= v (v >= 0, below 2^20)
-__device__ inline int isqrt(int v) {
-  int j = (int)sqrtf((float)v);
-  if (j * j > v) j--;
-  if ((j + 1) * (j + 1) <= v) j++;
-  return j;
-}
-
 // The forward column pass of OUTC with the shells' parts: shell s (bin s + 1) is
 // the points s^2-s+1 <= r^2 <= s^2+s below JC^2, a run of J per column; a thread
 // takes a shell's points of one sign of J in order.  The Nyquist row is J = N/2

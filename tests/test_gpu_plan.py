@@ -3,14 +3,14 @@
 A plan's replay must equal the eager sequence fr_prep_batch ->
 fr_cc3m_batch -> fr_insert_batch on the same batch bit for bit (NKSUM, CC3M
 scores, TTD and the half-maps): every kernel on the path sums in a fixed
-order.  Box sizes 64 and 128 take the fused preparation (its ring sums in
-the plan's own buffer), 96 the one-kernel-per-step form.  The graph is
+order.  All boxes here take the fused preparation, its ring sums in the
+plan's own buffer.  The graph is
 replayed several times on different batches, with eager work between the
 replays, and every replay is checked.  The
 autotuner's choice must be one of its measured candidates, and each CC3M
-variant it can choose must give the same scores (1e-6 between persistent
-grid sizes of the fused kernel, whose shell sums use LDS float atomics; 1e-4
-against the FFT path).
+variant it can choose must give the same scores (the same bits between grid
+sizes, 1e-4 against the particle's grid).  Some particles have another AMAG, and
+100 is a box off the NSAM grid's sizes: those scores come from other kernels.
 """
 import numpy as np
 import pytest
