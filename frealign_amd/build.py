@@ -5,6 +5,7 @@ python -m frealign_amd.build            # compile every source, link the library
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -45,6 +46,9 @@ SOURCES = [
     "fr_finalize.cpp",
 ]
 
+# compiled once more for each FFT length (fr_fft_dev.h): a code object per length
+LENGTH_SOURCES = ["fr_prep.hip", "fr_cc3m_fft.hip", "fr_fft.hip"]
+
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("FR_ARCH", "gfx950")
 COMMON = [
@@ -55,10 +59,17 @@ COMMON = [
 ]
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+def lengths() -> list[str]:
+    with open(os.path.join(CSRC, "fr_fft_dev.h")) as f:
+        macro = re.search(r"#define FR_LENGTHS\(X\)((?:.*\\\n)+.*\n)", f.read()).group(1)
+    return re.findall(r"X\((\d+)\)", macro)
+
+
+def _compile(job: tuple[str, str]) -> str:
+    src, length = job
+    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ("_" + length if length else "") + ".o")
     path = os.path.join(CSRC, src)
-    cmd = [HIPCC, *COMMON, "-c", path, "-o", obj]
+    cmd = [HIPCC, *COMMON, *([f"-DFR_LEN={length}"] if length else []), "-c", path, "-o", obj]
     if src.endswith(".cpp"):
         cmd[1:1] = ["-x", "hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -72,8 +83,9 @@ def build(verbose: bool = True) -> str:
         raise RuntimeError(f"hipcc not found at {HIPCC}")
     os.makedirs(BUILD, exist_ok=True)
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
-        objs = list(ex.map(_compile, srcs))
+    jobs = [(s, "") for s in srcs] + [(s, n) for s in LENGTH_SOURCES for n in lengths()]
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        objs = list(ex.map(_compile, jobs))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, "-shared", f"--offload-arch={ARCH}", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)

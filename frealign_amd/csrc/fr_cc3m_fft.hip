@@ -36,12 +36,7 @@
 
 namespace fr {
 
-namespace {
-
-using namespace fftdev;
-constexpr int kThr = kFftThreads;
-constexpr int kCw = 8;  // columns per workgroup
-constexpr float kPi = 3.1415926535897f;
+namespace bandfft {
 
 struct Band {
   int nsam, nitem, cb, jmax, maxr12, maxr22, nsh;
@@ -50,6 +45,30 @@ struct Band {
   int skip;  // items with AMAG = 1 are the band grid's (fr_cc3m.hip): left alone
   __device__ bool left(float amag) const { return skip && amag == 1.0f; }
 };
+
+struct BandWork {
+  float2* band;
+  float4* psum;
+  float *part, *mean;
+};
+
+struct BandCall {
+  const float *a3df, *spec, *ctff;
+  const int* pidx;
+  const float *dm, *shift, *amag;
+};
+
+}  // namespace bandfft
+
+namespace {
+
+using namespace fftdev;
+using bandfft::Band;
+using bandfft::BandCall;
+using bandfft::BandWork;
+constexpr int kThr = kFftThreads;
+constexpr int kCw = 8;  // columns per workgroup
+constexpr float kPi = 3.1415926535897f;
 
 constexpr int rows_nseq(int n) { return n >= 1024 ? 2 : 2048 / n; }
 
@@ -412,6 +431,7 @@ __global__ void __launch_bounds__(kThr)
   }
 }
 
+#ifndef FR_LEN
 __device__ inline float4 shell(const float4* psum, const Band& b, int it, int s) {
   const int nblk = b.cb / kCw;
   float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -501,12 +521,6 @@ __global__ void __launch_bounds__(kThr)
 int band_cb(int maxr2) { return (maxr2 + kCw - 1) / kCw * kCw; }
 int band_nsh(int maxr2) { return maxr2 + 1; }
 
-struct BandWork {
-  float2* band;
-  float4* psum;
-  float *part, *mean;
-};
-
 size_t align16(size_t b) { return (b + 15) & ~(size_t)15; }
 
 BandWork band_work(void* base, int nsam, int maxr2, size_t n, size_t* bytes) {
@@ -525,15 +539,13 @@ BandWork band_work(void* base, int nsam, int maxr2, size_t n, size_t* bytes) {
   *bytes = o;
   return w;
 }
+#endif  // FR_LEN
 
-struct BandCall {
-  const float *a3df, *spec, *ctff;
-  const int* pidx;
-  const float *dm, *shift, *amag;
-};
+}  // namespace
 
 template <int N>
-int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, const BandWork& w) {
+int launch_band_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring,
+                  const BandWork& w) {
   Plan pl;
   FR_CHECK(make_plan(b.nsam, &pl), "FFT length %d not supported", b.nsam);
   const float2* tw = c.twiddles(b.nsam);
@@ -569,8 +581,19 @@ int launch_n(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, con
   return 0;
 }
 
+#ifdef FR_LEN
+template int launch_band_n<FR_LEN>(Ctx&, const Band&, const BandCall&, const Cc3mRing&,
+                                   const BandWork&);
+#else
+#define FR_EXTERN(N)                                                                        \
+  extern template int launch_band_n<N>(Ctx&, const Band&, const BandCall&, const Cc3mRing&, \
+                                       const BandWork&);
+FR_LENGTHS(FR_EXTERN)
+
+namespace {
+
 int launch_band(Ctx& c, const Band& b, const BandCall& p, const Cc3mRing& ring, const BandWork& w) {
-  return with_length(b.nsam, [&](auto len) { return launch_n<len()>(c, b, p, ring, w); });
+  return with_length(b.nsam, [&](auto len) { return launch_band_n<len()>(c, b, p, ring, w); });
 }
 
 Band make_band(int nsam, int n, int maxr12, int maxr2, float ri2, float ri3, float rih,
@@ -658,5 +681,7 @@ int launch_presb(Ctx& c, int nsam, int n, const float* a3df, const float* spec, 
   FR_HIP(hipGetLastError());
   return 0;
 }
+
+#endif  // FR_LEN
 
 }  // namespace fr

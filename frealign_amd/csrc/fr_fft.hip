@@ -23,6 +23,7 @@ namespace {
 
 using namespace fftdev;
 constexpr int kThreads = kFftThreads;
+#ifndef FR_LEN
 // ---- row pass, forward: rows (2q, 2q+1) -> z = a + i b -> FFT -> unpack to half spectra
 __global__ void __launch_bounds__(kThreads) k_rows_r2c(float* data, Plan pl, int nrows_per_img,
                                                        size_t img_stride, int npairs, int nseq,
@@ -165,6 +166,7 @@ int row_seqs(int n) {
   int s = 2048 / n;
   return s < 1 ? 1 : s;
 }
+#endif
 
 // ---- the same three kernels with the length known at compile time
 template <int N>
@@ -269,6 +271,8 @@ __global__ void __launch_bounds__(kThreads) k_cols_t(float* data, size_t img_str
   });
 }
 
+}  // namespace
+
 template <int N>
 int rows_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, bool fwd, const float2* tw) {
   constexpr int NSEQ = 2048 / N;
@@ -303,7 +307,14 @@ int cols_pass_t(Ctx& c, int nimg, float* data, size_t img_stride, int sign, cons
   return 0;
 }
 
-}  // namespace
+#ifdef FR_LEN
+template int rows_pass_t<FR_LEN>(Ctx&, int, float*, size_t, bool, const float2*);
+template int cols_pass_t<FR_LEN>(Ctx&, int, float*, size_t, int, const float2*);
+#else
+#define FR_EXTERN(N)                                                                  \
+  extern template int rows_pass_t<N>(Ctx&, int, float*, size_t, bool, const float2*); \
+  extern template int cols_pass_t<N>(Ctx&, int, float*, size_t, int, const float2*);
+FR_LENGTHS(FR_EXTERN)
 
 bool fft_supported(int nsam) {
   Plan p;
@@ -421,5 +432,7 @@ int fft_c2r_3d(Ctx& c, int nsam, float* data) {
   if (int r = z_pass(c, nsam, data, +1)) return r;
   return fft_c2r_2d(c, nsam, nsam, data, img);
 }
+
+#endif  // FR_LEN
 
 }  // namespace fr

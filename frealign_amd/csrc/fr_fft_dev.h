@@ -308,52 +308,29 @@ __device__ inline float2* lds_fft(float2* buf, float2* tmp, const Plan& pl, int 
   return buf;
 }
 
-// The lengths that are compiled in, f(integral_constant<N>): the even ones from
-// 64 to 512 (an index division or modulus by a run-time length costs more than
-// its butterfly: preparing 300 images of 160^2 takes 173 us, 357 with passes of a
-// run-time length).  N = 0, those passes, for any other.
+// The lengths that are compiled in: the even ones from 64 to 512 (an index division
+// or modulus by a run-time length costs more than its butterfly: preparing 300
+// images of 160^2 takes 173 us, 357 with passes of a run-time length).  A source with
+// kernels of a length is compiled once per length as well, with FR_LEN defined, and
+// then holds that length's alone: the device code is loaded where a program first
+// uses it, and all lengths of the preparation's kernels together were 11 ms of its
+// first call.
+#define FR_LENGTHS(X) \
+  X(64) X(72) X(80) X(90) X(96) X(100) X(108) X(120) X(128) \
+  X(144) X(150) X(160) X(162) X(180) X(192) X(200) X(216) X(240) \
+  X(250) X(256) X(270) X(288) X(300) X(320) X(324) X(360) X(384) \
+  X(400) X(432) X(450) X(480) X(486) X(500) X(512)
+
+// f(integral_constant<N>), or N = 0, the passes of a run-time length, for any other
 template <typename F>
 inline int with_length(int n, F f) {
-#define FR_LENGTH(N) \
+#define FR_CASE(N) \
   case N: return f(std::integral_constant<int, N>{});
   switch (n) {
-    FR_LENGTH(64)
-    FR_LENGTH(72)
-    FR_LENGTH(80)
-    FR_LENGTH(90)
-    FR_LENGTH(96)
-    FR_LENGTH(100)
-    FR_LENGTH(108)
-    FR_LENGTH(120)
-    FR_LENGTH(128)
-    FR_LENGTH(144)
-    FR_LENGTH(150)
-    FR_LENGTH(160)
-    FR_LENGTH(162)
-    FR_LENGTH(180)
-    FR_LENGTH(192)
-    FR_LENGTH(200)
-    FR_LENGTH(216)
-    FR_LENGTH(240)
-    FR_LENGTH(250)
-    FR_LENGTH(256)
-    FR_LENGTH(270)
-    FR_LENGTH(288)
-    FR_LENGTH(300)
-    FR_LENGTH(320)
-    FR_LENGTH(324)
-    FR_LENGTH(360)
-    FR_LENGTH(384)
-    FR_LENGTH(400)
-    FR_LENGTH(432)
-    FR_LENGTH(450)
-    FR_LENGTH(480)
-    FR_LENGTH(486)
-    FR_LENGTH(500)
-    FR_LENGTH(512)
+    FR_LENGTHS(FR_CASE)
     default: return f(std::integral_constant<int, 0>{});
   }
-#undef FR_LENGTH
+#undef FR_CASE
 }
 
 // columns per workgroup of a column pass: 64 bytes or more of a row, and 2,048

@@ -58,6 +58,7 @@ __device__ inline void ctf_point(const PrepGlobals& g, const float* pp, int l, i
   cl = make_float2(b.re, b.im);
 }
 
+#ifndef FR_LEN
 // ctfapply.f:64-80: CTF table and shifted spectrum; one thread per half-plane point
 __global__ void __launch_bounds__(kThreads)
     k_ctf_shift(int nsam, int nb, const float2* __restrict__ spec, const float* __restrict__ ppar,
@@ -79,6 +80,7 @@ __global__ void __launch_bounds__(kThreads)
   ctff[(size_t)b * 2 * ic + id] = cr;
   ctff[(size_t)b * 2 * ic + ic + id] = cl;
 }
+#endif
 
 // The shift step between two column passes, for the box sizes whose FFT
 // length is a compile-time constant: a workgroup takes CW half-plane columns
@@ -150,6 +152,8 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
   });
 }
 
+}  // namespace
+
 template <int N>
 int cols_shift_t(Ctx& c, int nb, float* spec, bool fwd, const float* ppar, float* outc,
                  float* datc) {
@@ -171,6 +175,8 @@ int cols_shift_t(Ctx& c, int nb, float* spec, bool fwd, const float* ppar, float
   FR_HIP(hipGetLastError());
   return 0;
 }
+
+namespace {
 
 // MASKCOS's squared distance of 0-based pixel (row, x) from the centre
 // NSAM/2+1 of 1-based coordinates, as k_scale_mask forms it
@@ -331,6 +337,8 @@ __global__ void __launch_bounds__(fftdev::kFftThreads)
   }
 }
 
+}  // namespace
+
 // OUTC's c2r, MASKCOS and r2c rows on the fused path; `part` (a float2 per row
 // block) carries the ring partial sums between the two launches
 template <int N>
@@ -352,6 +360,8 @@ int rows_mask_t(Ctx& c, int nb, float* outc, const float* ppar, const PrepGlobal
   FR_HIP(hipGetLastError());
   return 0;
 }
+
+namespace {
 
 // ---- PWEIGHT (pweight.f) on the fused path, in three steps over the whole GPU
 // where one workgroup per particle went over its plane twice: k_cols_shells
@@ -502,6 +512,8 @@ int pw_chunk(int nsam, int nb) {
   return (int)std::min<size_t>(nb, kPwBytes / pw_image_bytes(nsam));
 }
 
+}  // namespace
+
 template <int N>
 int pweight_t(Ctx& c, int nb, const float* ppar, const float* pssnr, const PrepGlobals& g,
               float* ctff, float* outc, float2* pw) {
@@ -526,6 +538,22 @@ int pweight_t(Ctx& c, int nb, const float* ppar, const float* pssnr, const PrepG
   }
   return 0;
 }
+
+#ifdef FR_LEN
+template int cols_shift_t<FR_LEN>(Ctx&, int, float*, bool, const float*, float*, float*);
+template int rows_mask_t<FR_LEN>(Ctx&, int, float*, const float*, const PrepGlobals&, float2*);
+template int pweight_t<FR_LEN>(Ctx&, int, const float*, const float*, const PrepGlobals&, float*,
+                               float*, float2*);
+#else
+#define FR_EXTERN(N)                                                                             \
+  extern template int cols_shift_t<N>(Ctx&, int, float*, bool, const float*, float*, float*);    \
+  extern template int rows_mask_t<N>(Ctx&, int, float*, const float*, const PrepGlobals&,        \
+                                     float2*);                                                   \
+  extern template int pweight_t<N>(Ctx&, int, const float*, const float*, const PrepGlobals&,    \
+                                   float*, float*, float2*);
+FR_LENGTHS(FR_EXTERN)
+
+namespace {
 
 bool fused_cols(int nsam) {
   return fftdev::with_length(nsam, [](auto len) { return len() > 0; });
@@ -844,5 +872,7 @@ int launch_ctfapply(Ctx& c, int nsam, int nb, const float* spec, const float* pp
   if (int r = fft_r2c_2d(c, nsam, nb, outc, img)) return r;
   return origin_pweight(c, nsam, nb, pssnr, g, ctff, outc);
 }
+
+#endif  // FR_LEN
 
 }  // namespace fr
